@@ -8,9 +8,11 @@ input block already resident in HBM.
 
 The reported value is the split-precision mode (SG4_PREC_F32X2: mode
 contractions on the matrix cores with three bf16 limbs per FP32 operand and
-FP32 accumulation; kinetic part, term sum and result in FP64); the plain FP64
-apply of the same operator is timed beside it with the same number of steps,
-and their ratio is reported.  The eigenvalue error condition of the metric is
+FP32 accumulation; kinetic part, term sum and result in FP64); the FP64 term
+kernel of the same operator is timed beside it with the same number of steps,
+and their ratio is reported.  FP64 applies of this operator (a sum of one- and
+two-mode functions) run as one sparse matrix unless told otherwise; that
+apply is timed as "fp64_sparse", and the Davidson runs use it.  The eigenvalue error condition of the metric is
 measured by block Davidson runs for the 20 lowest levels: FP64, split
 precision followed by an FP64 phase, and split precision alone, each
 compared with the FP64 levels; each run is timed after an untimed run of the
@@ -258,6 +260,8 @@ def main():
         elif not args.no_autotune:
             op.autotune(nvec, PREC[pname])
 
+    op.set_sparse(False)        # FP64 through the term kernels, as the other modes
+
     def timed(p, steps, warmup):
         for _ in range(warmup):
             op.apply(Xc, Y, p)
@@ -297,6 +301,17 @@ def main():
         if oname == "fp64":   # H.psi error of the reported mode against FP64, same input
             e2 = (torch.linalg.norm(Yrep - Y, dim=1) / torch.linalg.norm(Y, dim=1)).max().item()
             other["hpsi_rel_err_2norm_of_reported_vs_fp64"] = e2
+    # FP64 as one sparse matrix over the packed rows (the default FP64 path)
+    op.set_sparse(True)
+    sparse = None
+    taken, nnz = op.sparse_info()
+    if taken:
+        dts, kavgs = timed(PREC["fp64"], args.steps, args.warmup)
+        moved = 12.0 * nnz + 16.0 * b.nb_ba * nvec
+        sparse = {"H·psi/s": nvec * args.steps / dts, "ms_per_step": dts / args.steps * 1e3,
+                  "kernel": "k_nm_spmm", "kernel_ms": kavgs * 1e3, "entries": nnz,
+                  "bytes": moved, "GBps": moved / kavgs / 1e9, "peak_GBps": PEAK_HBM_GBPS}
+    op.set_sparse(False)
     # the apply replayed from one captured HIP graph, in the rows layout the
     # device-side drivers use (kinetic rows and term kernel in one graph)
     graph = None
@@ -314,6 +329,7 @@ def main():
             torch.cuda.synchronize()
             tg = time.perf_counter() - t0
             graph[pname] = {"H·psi/s": nvec * args.steps / tg, "ms_per_step": tg / args.steps * 1e3}
+    op.set_sparse(True)
     F1 = reference_flops(b, nvec)
     kname = KERNEL[args.prec] if split or args.prec == "f32x2" else (
         "k_hpsi_t1_" + ("f64" if args.prec == "fp64" else "f32"))
@@ -374,7 +390,9 @@ def main():
         line["graph_replay"] = graph
     if other is not None:
         line["other_precision"] = other
-        line[f"speedup_vs_{oname}"] = (nvec * args.steps / dt) / other["H·psi/s"]
+        line[f"speedup_vs_{oname}_term_kernel" if oname == "fp64" else f"speedup_vs_{oname}"] = (nvec * args.steps / dt) / other["H·psi/s"]
+    if sparse is not None:
+        line["fp64_sparse"] = sparse
     if args.nlev and args.prec != "fp64":
         from elvibrot_amd.davidson import sub_propagation_Davidson
         runs = {}

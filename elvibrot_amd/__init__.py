@@ -269,6 +269,17 @@ class SG4Operator:
         _capi.check(lib().sg4_plan_split_info(self._h, C.byref(sp), C.byref(nnz)))
         return bool(sp.value), nnz.value
 
+    def set_sparse(self, on=True):
+        """FP64 applies as one sparse matrix where the operator has that form
+        (default), or always by the term kernels."""
+        _capi.check(lib().sg4_plan_set_option(self._h, _capi.OPT_SPARSE, 1 if on else 0))
+
+    def sparse_info(self):
+        """(FP64 applies run as one sparse matrix, its stored entries)"""
+        sp, nnz = C.c_int32(), C.c_int64()
+        _capi.check(lib().sg4_plan_sparse_info(self._h, C.byref(sp), C.byref(nnz)))
+        return bool(sp.value), nnz.value
+
     def timing(self, enable=True):
         _capi.check(lib().sg4_plan_timing(self._h, 1 if enable else 0))
 

@@ -11,6 +11,7 @@ I_P = C.POINTER(C.c_int32)
 PREC_FP64, PREC_F32, PREC_F32X2 = 0, 1, 2
 OPT_GROUPING = 1
 OPT_DETERMINISTIC = 2
+OPT_SPARSE = 3
 # return codes (include/sg4hpsi.h)
 OK, ERR_ARG, ERR_HIP, ERR_OOM, ERR_UNSUPPORTED, ERR_STATE = 0, -1, -2, -3, -4, -5
 BASIS_HO, BASIS_LEGENDRE = 0, 1
@@ -23,7 +24,7 @@ EXPORTS = [
     "sg4_plan_set_stream", "sg4_plan_set_operator", "sg4_plan_set_henon_heiles", "sg4_plan_set_jacobi_triatomic", "sg4_apply",
     "sg4_apply_host", "sg4_apply_rows", "sg4_plan_stats", "sg4_plan_timing",
     "sg4_plan_kernel_times", "sg4_grad_V", "sg4_plan_set_field", "sg4_plan_autotune", "sg4_plan_config", "sg4_plan_set_config",
-    "sg4_apply_graph", "sg4_plan_set_option", "sg4_plan_split_info", "sg4_plan_mfma_stats",
+    "sg4_apply_graph", "sg4_plan_set_option", "sg4_plan_split_info", "sg4_plan_sparse_info", "sg4_plan_mfma_stats",
     "sg4_plan_destroy", "sg4_apply_noalloc", "sg4_cheby_propagate", "sg4_cheby_field_gradient",
     "sg4_plan_grid_dipole", "sg4_plan_set_operator_type1", "sg4_taylor_propagate",
     "sg4_block_gram_work", "sg4_block_gram", "sg4_block_combine",
@@ -104,6 +105,7 @@ def lib():
         L.sg4_plan_set_jacobi_triatomic.argtypes = [vp, C.POINTER(C.c_double)]
         L.sg4_setup_packed.argtypes = [vp, C.POINTER(i32)]
         L.sg4_plan_split_info.argtypes = [vp, C.POINTER(i32), C.POINTER(C.c_int64)]
+        L.sg4_plan_sparse_info.argtypes = [vp, C.POINTER(i32), C.POINTER(C.c_int64)]
         L.sg4_plan_mfma_stats.argtypes = [vp, C.POINTER(C.c_double), C.POINTER(C.c_int64)]
         L.sg4_plan_destroy.argtypes = [vp]
         L.sg4_plan_grid_dipole.argtypes = [vp, vp]

@@ -9,7 +9,7 @@
 // (term, chunk of vectors) work item in LDS, in passes over groups of up to
 // three modes whose slabs a thread holds in registers while it multiplies
 // them by the small 1-D matrices (entries wave-uniform, read through the
-// scalar cache).  Three type-1 paths:
+// scalar cache).  Four type-1 paths:
 //   split path (k_kin_rows + k_hpsi_t1s_*): the kinetic part as one sparse
 //     matrix over the packed rows, the terms keep only basis->grid, the
 //     potential and grid->basis, with the gather and the weighted scatter-add
@@ -17,6 +17,8 @@
 //   grouped grid path (k_hpsi_t1_*, term_t1_grouped): the reference's
 //     structure with the kinetic derivatives on the grid;
 //   per-mode grid path (k_hpsi_t1_*, term_t1): one pass per mode, any sizes.
+//   sparse path (sg4_nmode.hip): FP64, potentials that are sums of one- and
+//     two-mode functions: all of H as one sparse matrix over the packed rows.
 // Type 10 (d1 G d1): k_hpsi_t10_f64.  Eigenvalue gradients: k_grad_v.
 #include <hip/hip_runtime.h>
 
@@ -28,11 +30,13 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
 #include "sg4_mfma.h"
+#include "sg4_nmode.h"
 
 namespace sg4 {
 
@@ -236,25 +240,6 @@ __global__ void k_grid_jacobi(JacArgs a) {
 // ---------------------------------------------------------------------------
 // plan
 // ---------------------------------------------------------------------------
-struct DevBuf {
-  void* p = nullptr;
-  size_t n = 0;
-  ~DevBuf() { if (p) (void)hipFree(p); }
-  int alloc(size_t bytes) {
-    if (p) { (void)hipFree(p); p = nullptr; }
-    n = bytes;
-    if (bytes == 0) return SG4_OK;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      set_error("device allocation of " + std::to_string(bytes) + " bytes failed");
-      p = nullptr;
-      return SG4_ERR_OOM;
-    }
-    return SG4_OK;
-  }
-  template <class T> T* as() const { return (T*)p; }
-};
-
 struct ItemPlan {
   DevBuf items, scratch;
   int64_t nitems = 0, nbig = 0, slot_size = 0;
@@ -337,6 +322,17 @@ struct sg4_plan {
   std::vector<int32_t> h_map;
   std::vector<double> h_mats;
   sg4::DevBuf d_kptr, d_kcol, d_kval;
+  std::vector<double> h_T;       // T_k(m) per (mode, level), rounding entries zeroed
+  std::vector<int64_t> h_toff;
+  std::vector<int> inst_L;       // largest |l| of every instance's terms
+  double flops_split = 0;        // algorithmic flops per vector of the split path's terms
+  // the field-free H as one sparse matrix (sg4_nmode.hip); field_on: V holds a
+  // field term
+  sg4::NModeTables* nmt = nullptr;
+  sg4::NModeMat nm;
+  bool field_on = false, nm_off = false;
+  bool sparse = true;            // SG4_OPT_SPARSE
+  std::set<int> nm_seen;         // block widths applied since the operator was set
   // split-precision MFMA path (SG4_PREC_F32X2): terms cut into mode groups,
   // group matrices in A-operand lane order
   bool mfma_valid = false;
@@ -349,6 +345,7 @@ struct sg4_plan {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pairs;
   size_t ev_used = 0;
   ~sg4_plan() {
+    sg4::nmode_tables_destroy(nmt);
     for (auto& e : ev_pairs) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.exec);
     if (own_stream) (void)hipStreamDestroy(own_stream);
@@ -387,6 +384,8 @@ static void invalidate(sg4_plan* P) {
   P->items.clear();
   P->f32_valid = false;
   P->mfma_valid = false;
+  P->nm.valid = false;
+  P->nm_seen.clear();
 }
 
 // Greedy grouping of consecutive active modes into the shapes of
@@ -492,6 +491,13 @@ static int build_kinetic(sg4_plan* P) {
       }
     tcut[i] = 1e-12 * tmax;
   }
+  P->h_T = tm;
+  P->h_toff = toff;
+  for (size_t i = 0; i < nmd; ++i) {
+    const int n = P->h_md[i].nq;
+    for (int e = 0; e < n * n; ++e)
+      if (e / n != e % n && std::fabs(tm[toff[i] + e]) <= tcut[i]) P->h_T[toff[i] + e] = 0.0;
+  }
   // Smolyak structure of every instance
   std::vector<int> Linst(P->inst.size());
   for (size_t ii = 0; ii < P->inst.size(); ++ii) {
@@ -515,6 +521,7 @@ static int build_kinetic(sg4_plan* P) {
     }
     Linst[ii] = L;
   }
+  P->inst_L = Linst;
   // two sweeps over (row, mode) pairs: count, then fill
   const int64_t nrows = P->nb_ba;
   std::vector<int64_t> ptr(nrows + 1, 0);
@@ -612,8 +619,33 @@ static int build_kinetic(sg4_plan* P) {
   return SG4_OK;
 }
 
+// What the sparse-matrix construction reads of the plan.
+static NModeIn nmode_in(const sg4_plan* P) {
+  NModeIn in;
+  for (size_t i = 0; i < P->inst.size(); ++i) {
+    const sg4_plan::Inst& I = P->inst[i];
+    in.inst.push_back(NModeInst{I.D, P->inst_L[i], I.Lmax, I.nterms, I.nb_ba, I.term0, I.row0, I.md0, I.ck0, I.lev0});
+  }
+  in.levels = &P->h_levels; in.nq = &P->h_nq; in.qoff = &P->h_qoff; in.ck = &P->h_ck;
+  in.T = &P->h_T; in.toff = &P->h_toff;
+  in.d_terms = P->d_terms.as<TermDev>(); in.d_md = P->d_md.as<MatDev>(); in.d_mats = P->d_mats.as<double>();
+  in.d_levels = P->d_levels.as<int32_t>(); in.d_map = P->d_map.as<int32_t>();
+  in.sum_nq = P->sum_nq; in.rows = P->nb_ba; in.stream = P->stream;
+  return in;
+}
+
+// The field-free operator as one sparse matrix, where it has that form.
+static int build_nmode(sg4_plan* P) {
+  P->nm.valid = false;
+  if (!P->split_ok) return SG4_OK;
+  const NModeIn in = nmode_in(P);
+  if (!P->nmt && !(P->nmt = nmode_tables_create(in))) return SG4_ERR_HIP;
+  return nmode_build(P->nmt, in, P->d_V0.p ? P->d_V0.as<double>() : P->d_V.as<double>(), nullptr, P->nm);
+}
+
 static int build_terms(sg4_plan* P) {
   P->mfma_valid = false;
+  P->flops_split = 0.0;
   P->h_terms.resize(P->nterms);
   std::vector<double> ck = P->h_ck;
   if ((int)ck.size() < P->nck) ck.assign(P->nck, 0.0);
@@ -651,13 +683,17 @@ static int build_terms(sg4_plan* P) {
       T.vshift = vs;
       T.ngrp = (P->grouping && P->type_op == 1 && nact > 0) ? make_groups(P, T) : 0;
       P->h_terms[t] = T;
+      double f = 0.0;
+      for (int q = 0; q < nact; ++q) f += 4.0 * (double)T.nq * P->h_md[T.mat[q]].nq;
+      P->flops_split += f + (double)T.nq;
     }
   }
   int rc = P->d_terms.alloc(sizeof(TermDev) * P->h_terms.size());
   if (rc) return rc;
   HIP_TRY(hipMemcpy(P->d_terms.p, P->h_terms.data(), sizeof(TermDev) * P->h_terms.size(),
                     hipMemcpyHostToDevice));
-  return build_kinetic(P);
+  if ((rc = build_kinetic(P))) return rc;
+  return build_nmode(P);
 }
 
 struct HItem { Item it; double cost; bool large; };
@@ -1138,6 +1174,12 @@ static bool use_split_for(const sg4_plan* P, int prec) {
   return prec == SG4_PREC_F32X2 ? use_split_alg(P) : use_split(P);
 }
 
+// FP64 applies of a field-free operator that is a sparse matrix.
+static bool use_nmode(const sg4_plan* P, int prec) {
+  return prec == SG4_PREC_FP64 && P->nm.valid && P->sparse && !P->field_on && !P->nm_off && !P->deterministic &&
+         use_split_alg(P);
+}
+
 // Launch configuration for (nvec, prec): the one tuned or set for it, else
 // the one set for the nearest block width of the same precision (the
 // narrowest wider one first): the best launch shape depends on the term set
@@ -1202,10 +1244,55 @@ static int pad_width(const sg4_plan* p, int nvec) {
   return W <= p->max_nvec ? W : nvec;
 }
 
+// the next pair of timing events of the plan
+static int next_events(sg4_plan* P) {
+  if (P->ev_used == P->ev_pairs.size()) {
+    hipEvent_t e0, e1;
+    HIP_TRY(hipEventCreate(&e0));
+    HIP_TRY(hipEventCreate(&e1));
+    P->ev_pairs.emplace_back(e0, e1);
+  }
+  P->ev0 = P->ev_pairs[P->ev_used].first;
+  P->ev1 = P->ev_pairs[P->ev_used].second;
+  ++P->ev_used;
+  return SG4_OK;
+}
+
+// FP64 apply of the sparse path.  ri: a rows-layout staging block for
+// column-major blocks of nvec vectors (W columns, or null: rows layout).
+static int apply_nmode(sg4_plan* P, int nvec, int W, const double* psi, double* hpsi, double* ri, double* ro) {
+  int rc;
+  if (P->no_alloc && !P->nm_seen.count(W)) return not_prepared();
+  if (!P->no_alloc) P->nm_seen.insert(W);
+  P->last_items = P->nterms;
+  P->last_flops = P->flops_split * W;
+  const bool direct = ri && nmode_cols_direct(P->nm, W);
+  if (ri && !direct)
+    hipLaunchKernelGGL(k_cols_to_rows, tile_grid(P->nb_ba, W), dim3(256), 0, P->stream, psi, ri, P->nb_ba, nvec, W);
+  if (P->timing) {
+    if ((rc = next_events(P))) return rc;
+    HIP_TRY(hipEventRecord(P->ev0, P->stream));
+  }
+  bool back = false;
+  if (!ri) rc = nmode_apply(P->nm, nvec, psi, hpsi, P->stream);
+  else if (direct) rc = nmode_apply_cols(P->nm, W, nvec, psi, hpsi, P->stream);
+  else if ((rc = nmode_apply_to_cols(P->nm, W, nvec, ri, hpsi, P->stream)) > 0) {
+    rc = nmode_apply(P->nm, W, ri, ro, P->stream);
+    back = true;
+  }
+  if (rc) return rc;
+  if (P->timing) HIP_TRY(hipEventRecord(P->ev1, P->stream));
+  if (back)
+    hipLaunchKernelGGL(k_rows_to_cols, tile_grid(P->nb_ba, W), dim3(256), 0, P->stream, ro, hpsi, P->nb_ba, nvec, W);
+  HIP_TRY(hipGetLastError());
+  return SG4_OK;
+}
+
 static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, int prec,
                       const LaunchCfg* cfgp = nullptr) {
   int rc;
   if ((rc = check_apply(P, nvec, prec))) return rc;
+  if (use_nmode(P, prec)) return apply_nmode(P, nvec, nvec, psi, hpsi, nullptr, nullptr);
   const LaunchCfg cfg = cfgp ? *cfgp : cfg_for(P, nvec, prec);
   ItemPlan* ip = nullptr;
   if ((rc = prepare(P, nvec, prec, cfg, &ip))) return rc;
@@ -1238,15 +1325,7 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
   P->last_flops = ip->flops_main;
   P->last_flops_mfma = ip->flops_mfma;
   if (P->timing) {
-    if (P->ev_used == P->ev_pairs.size()) {
-      hipEvent_t e0, e1;
-      HIP_TRY(hipEventCreate(&e0));
-      HIP_TRY(hipEventCreate(&e1));
-      P->ev_pairs.emplace_back(e0, e1);
-    }
-    P->ev0 = P->ev_pairs[P->ev_used].first;
-    P->ev1 = P->ev_pairs[P->ev_used].second;
-    ++P->ev_used;
+    if ((rc = next_events(P))) return rc;
     if (!split) HIP_TRY(hipEventRecord(P->ev0, P->stream));
   }
   const unsigned grid = (unsigned)((cfg.grid > 0 && cfg.grid < ip->nitems) ? cfg.grid : ip->nitems);
@@ -1691,6 +1770,7 @@ int sg4_plan_set_operator(sg4_plan* p, const sg4_operator* op) {
   p->type_op = op->type_op;
   HIP_TRY(hipMemcpy(p->d_V.p, op->V, sizeof(double) * p->sum_nq, hipMemcpyHostToDevice));
   (void)p->d_V0.alloc(0);
+  p->field_on = false;
   return build_terms(p);
 }
 
@@ -1713,6 +1793,7 @@ int sg4_plan_set_operator_type1(sg4_plan* p, int32_t nder, const int32_t* der, c
   p->type_op = 11;
   p->h_ck.assign(p->nck, 0.0);
   (void)p->d_V0.alloc(0);
+  p->field_on = false;
   return build_terms(p);
 }
 
@@ -1735,6 +1816,7 @@ int sg4_plan_set_henon_heiles(sg4_plan* p, double lambda) {
   HIP_TRY(hipGetLastError());
   p->type_op = 1;
   (void)p->d_V0.alloc(0);
+  p->field_on = false;
   p->h_ck.assign(p->nck, -0.5);
   int rc;
   if ((rc = p->d_ck.alloc(sizeof(double) * p->nck))) return rc;
@@ -1796,6 +1878,7 @@ int sg4_plan_set_jacobi_triatomic(sg4_plan* p, const double* prm) {
   HIP_TRY(hipGetLastError());
   p->type_op = 10;
   (void)p->d_V0.alloc(0);
+  p->field_on = false;
   p->h_ck.assign(p->nck, 0.0);
   rc = build_terms(p);
   if (rc) return rc;
@@ -1821,6 +1904,7 @@ int sg4_apply(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi, int32_
     return apply_rows(p, 1, psi, hpsi, prec);
   }
   const int W = pad_width(p, nvec);
+  if (p->type_op && use_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
   hipLaunchKernelGGL(k_cols_to_rows, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, psi, ri, p->nb_ba, nvec, W);
   int rc = apply_rows(p, W, ri, ro, prec);
   if (rc) return rc;
@@ -1884,6 +1968,7 @@ int sg4_apply_noalloc(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi
   if (nvec == 1) return apply_rows(p, 1, psi, hpsi, prec);
   double* ri = base;
   double* ro = base + n;
+  if (use_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
   hipLaunchKernelGGL(k_cols_to_rows, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, psi, ri, p->nb_ba, nvec, W);
   if ((rc = apply_rows(p, W, ri, ro, prec))) return rc;
   hipLaunchKernelGGL(k_rows_to_cols, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, ro, hpsi, p->nb_ba, nvec, W);
@@ -1934,6 +2019,13 @@ int sg4_plan_split_info(const sg4_plan* p, int32_t* split, int64_t* kin_nnz) {
   return SG4_OK;
 }
 
+int sg4_plan_sparse_info(const sg4_plan* p, int32_t* sparse, int64_t* nnz) {
+  if (!p) { set_error("null plan"); return SG4_ERR_ARG; }
+  if (sparse) *sparse = use_nmode(p, SG4_PREC_FP64) ? 1 : 0;
+  if (nnz) *nnz = p->nm.valid ? p->nm.nnz : 0;
+  return SG4_OK;
+}
+
 int sg4_plan_set_field(sg4_plan* p, const double* mu, double eps) {
   if (!p) { set_error("null plan"); return SG4_ERR_ARG; }
   if (p->type_op == 0) { set_error("no operator set on the plan"); return SG4_ERR_STATE; }
@@ -1952,6 +2044,9 @@ int sg4_plan_set_field(sg4_plan* p, const double* mu, double eps) {
                      p->d_V0.as<double>(), mu, eps, p->d_V.as<double>(), p->sum_nq);
   HIP_TRY(hipGetLastError());
   p->f32_valid = false;
+  // FP64 graphs of the sparse path do not read V: a field changes the path
+  if (p->field_on != (mu != nullptr) && p->nm.valid) drop_graphs(p);
+  p->field_on = mu != nullptr;
   return SG4_OK;
 }
 
@@ -2001,6 +2096,7 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
   HIP_TRY(hipEventCreate(&e1));
   const bool timing = p->timing;
   p->timing = false;
+  p->nm_off = true;    // tune the term kernels also where FP64 takes the sparse path
   LaunchCfg best;
   float bms = 1e30f;
   int cus = 256;
@@ -2037,6 +2133,17 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
                     nvec, prec, c.nthreads, c.lds_budget, c.grid, c.xcd, ms);
           if (ms < bms) { bms = ms; best = c; }
         }
+  p->nm_off = false;
+  if (!rc && use_nmode(p, prec)) {   // the time of the path that later applies take
+    for (int r = 0; r < 4 && !rc; ++r) {
+      if (r == 1) HIP_TRY(hipEventRecord(e0, p->stream));
+      rc = apply_rows(p, nvec, x.as<double>(), y.as<double>(), prec);
+    }
+    HIP_TRY(hipEventRecord(e1, p->stream));
+    HIP_TRY(hipEventSynchronize(e1));
+    HIP_TRY(hipEventElapsedTime(&bms, e0, e1));
+    bms /= 3;
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   p->timing = timing;
@@ -2124,6 +2231,11 @@ int sg4_plan_set_option(sg4_plan* p, int32_t option, int32_t value) {
   if (option == SG4_OPT_DETERMINISTIC) {
     drop_graphs(p);
     p->deterministic = value != 0;
+    return SG4_OK;
+  }
+  if (option == SG4_OPT_SPARSE) {
+    drop_graphs(p);
+    p->sparse = value != 0;
     return SG4_OK;
   }
   if (option != SG4_OPT_GROUPING) { set_error("unknown option"); return SG4_ERR_ARG; }

@@ -1,0 +1,1039 @@
+// Potentials that are sums of one- and two-mode functions,
+//   V(q) = V0 + sum_a f_a(q_a) + sum_{a<b} f_ab(q_a, q_b)
+// (Henon-Heiles, vibronic-coupling models, quadratic and cubic pair force
+// fields): the whole type-1 H as one sparse matrix over the packed rows.
+//
+// With B^T W B = I in every mode (checked for the split path) a term's matrix
+// of f_ab is M_ab(l_a, l_b) = (BtW_a x BtW_b) f_ab (B_a x B_b) in modes a, b and
+// the identity in the others, so the Smolyak sum over the levels of the other
+// modes telescopes as it does for the kinetic part: with Lambda the sum of the
+// smallest levels holding the indices of the other modes, the weights of fixed
+// (l_a, l_b) sum to the coefficient of z^u, u = L - Lambda - l_a - l_b, in
+// (1 - z)^-(D-2) (1 - z)^(D-1) = 1 - z.  Hence with m = L - Lambda
+//   <r|V|r'> = sum_{l_a + l_b = m} M_ab - sum_{l_a + l_b = m - 1} M_ab
+// (levels that hold both rows' indices), the two-mode combination technique,
+// and for f_a (and c_a d_a^2) the one-mode matrix at level m = L - Lambda_a.
+// This is the operator the term-by-term sum gives, without its cancellation.
+//
+// f_a and f_ab are read off the grid V on cuts through the middle point of the
+// other modes (odd rules), then the sum is compared with V on EVERY grid
+// point; V that differs beyond rounding keeps the term kernels.  Matrix
+// elements below the rounding error of their own quadrature sum are zero
+// (parity, band structure of polynomials) and are not stored.
+//
+// What bounds it: the gathers of psi rows, one 128-byte line per stored entry
+// and 16 vectors, from beyond L2.  10D L=8 Henon-Heiles (32.2 M entries, 0.39
+// GB): 0.75 ms at 16 vectors (4.1 GB of gathers, 5.5 TB/s), 0.14 ms at one
+// (matrix 2.8 TB/s); the term kernels and the kinetic rows take 5.1 and 1.2 ms.
+// sg4_apply of 16 column-major vectors: 0.85 ms against 5.2.  One group of W
+// lanes per row (W vectors, the entries loaded once per group) in row order;
+// measured slower at 16 / 1 vectors: 8 loads in flight 0.77 / 0.16 ms, a
+// contiguous chunk of rows per XCD 0.80 / 0.15, non-temporal matrix loads 0.94 /
+// 0.18, two slices of entries per row (16 vectors) 0.87.
+#include "sg4_nmode.h"
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <map>
+#include <memory>
+#include <string>
+
+namespace sg4 {
+
+#define NM_TRY(expr)                                                              \
+  do {                                                                            \
+    hipError_t _e = (expr);                                                       \
+    if (_e != hipSuccess) {                                                       \
+      set_error(std::string("HIP error: ") + hipGetErrorString(_e) + " at " #expr); \
+      return SG4_ERR_HIP;                                                         \
+    }                                                                             \
+  } while (0)
+
+namespace {
+
+constexpr int NI = SG4_MAX_N;         // 1-D indices per mode
+constexpr int RT = 128;               // rows per workgroup of the row kernels
+constexpr double EPS = 2.220446049250313e-16;
+// A grid value may differ from the sum of its parts by the rounding of the
+// parts (each the difference of up to four grid values): 64 eps of the sum of
+// their magnitudes.  A matrix element below 16 eps of the absolute sum of its
+// quadrature terms is rounding.
+constexpr double TOL_V = 64 * EPS, TOL_M = 16 * EPS;
+// Stored entries per grid point up to which the matrix is taken: an entry
+// costs ~1.5 ps per vector at 10D L=8 (gather of one psi value), a grid point
+// ~9.5 ps in the FP64 term kernel.
+constexpr double NNZ_PER_POINT = 4.0;
+constexpr int64_t NNZ_SMALL = 1 << 18;        // always taken: the apply is one short launch
+// A column-major block is read in place while nnz W^2 <= 2^26 (W columns, a
+// gather touches W lines instead of one), else staged in the rows layout (one
+// more launch).  In place / staged, us: 6D L=6 x16 9.4 / 11.3, 8D L=6 x8
+// 17.8 / 17.8, x16 36.6 / 30.4, 10D L=6 x4 46.9 / 47.8, x8 60.5 / 48.0, 12D L=6
+// x2 50.5 / 52.8, x4 127 / 114.
+constexpr int64_t COLS_DIRECT = (int64_t)1 << 26;
+constexpr int64_t MAX_E = (int64_t)1 << 27;   // entries of the two-mode tables
+
+// Device view of an instance.
+struct NmDev {
+  int D, L, LB, L1;            // L1 = Lmax + 1 (stride of the md tables)
+  int64_t term0, nterms, row0, nrows;
+  const int32_t* levels;       // D per term
+  const MatDev* md;            // [k * L1 + l]
+  const int32_t* n;            // [k * (L+1) + l] points
+  const uint8_t* lam;          // [k * NI + i] smallest level holding index i
+  const int32_t* pre;          // [(k * (LB+1) + b) * (NI+1) + i] rank prefix
+  const int32_t* f1off;        // [k * (L+1) + l] offset of the mode's cut, -1: none
+  const int32_t* f2off;        // [(p * (L+1) + la) * (L+1) + lb], -1: none
+  const int32_t* s2n;          // [p * (L+1) + m] pair indices of level <= m
+  const int32_t* s2off;        // [p] offset in s2 / pos
+  const uint16_t* s2;          // (ja | jb << 8), by level
+  const int32_t* posoff;       // [p]
+  const int16_t* pos;          // [ia * nbL + ib] position in s2
+  const uint8_t* pa;           // [p] modes of the pair
+  const uint8_t* pb;
+  const double* T;             // kinetic matrices of the instance
+  const int32_t* toff;         // [k * (L+1) + l]
+  const double* ck;            // D
+  const int32_t* g1off;        // [k * (L+1) + l] offset in g1
+  int64_t c1base;              // the instance's cuts: c1[c1base] = V0
+  int npair, pair0;            // pair0: first global pair (flags, eoff)
+};
+
+// A cut of V: along one mode (nb = 1) or two.
+struct Cut {
+  int64_t off;                 // grid value at the middle point of the other modes, indices 0
+  int32_t sa, sb, na, nb;
+  int64_t out;                 // where the cut goes in c1 / f2
+  int64_t fa, fb, v0;          // two modes: the one-mode cuts and V0 in c1
+  int32_t pair;                // global pair, or -1
+};
+
+// work item of the two-mode matrices
+struct EWork { int32_t inst, pair, m; int32_t pad; int64_t off; };
+
+__device__ __forceinline__ int find_inst(const int64_t* first, int ninst, int64_t x) {
+  int lo = 0, hi = ninst;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    if (first[mid] <= x) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
+// the map's entries are the lexicographic ranks of their mode indices
+// (-1 beyond the basis level), the last mode's index fastest
+__global__ __launch_bounds__(256) void k_nm_check_map(const NmDev* insts, const int64_t* term0,
+                                                      int ninst, int64_t nterms, const TermDev* terms,
+                                                      const int32_t* map, int* bad) {
+  for (int64_t t = blockIdx.x; t < nterms; t += gridDim.x) {
+    const NmDev& I = insts[find_inst(term0, ninst, t)];
+    const int32_t* lev = I.levels + (t - I.term0) * I.D;
+    const TermDev& T = terms[t];
+    for (int e = threadIdx.x; e < T.nb; e += blockDim.x) {
+      int rest = e, b = I.LB;
+      int64_t r = 0;
+      for (int k = 0; k < I.D && r >= 0; ++k) {
+        const int n = I.n[k * (I.L + 1) + lev[k]];
+        const int i = rest % n;
+        rest /= n;
+        const int li = I.lam[k * NI + i];
+        if (li > b) { r = -1; break; }
+        r += I.pre[(k * (I.LB + 1) + b) * (NI + 1) + i];
+        b -= li;
+      }
+      if (map[T.boff + e] != (r < 0 ? -1 : (int32_t)(r + I.row0))) *bad = 1;
+    }
+  }
+}
+
+__global__ __launch_bounds__(64) void k_nm_cut1(const Cut* cuts, const double* V, double* c1) {
+  const Cut c = cuts[blockIdx.x];
+  for (int i = threadIdx.x; i < c.na; i += 64) c1[c.out + i] = V[c.off + (int64_t)i * c.sa];
+}
+
+// f_ab on its cut; a pair whose cuts are all rounding stays flagged zero
+__global__ __launch_bounds__(64) void k_nm_cut2(const Cut* cuts, const double* V, const double* c1,
+                                                double* f2, int* flag) {
+  const Cut c = cuts[blockIdx.x];
+  const double v0 = c1[c.v0];
+  bool nz = false;
+  for (int e = threadIdx.x; e < c.na * c.nb; e += 64) {
+    const int ia = e % c.na, ib = e / c.na;
+    const double v = V[c.off + (int64_t)ia * c.sa + (int64_t)ib * c.sb];
+    const double va = c1[c.fa + ia], vb = c1[c.fb + ib];
+    const double f = (v - va) - (vb - v0);
+    f2[c.out + e] = f;
+    nz = nz || !(fabs(f) <= TOL_V * (fabs(v) + fabs(va) + fabs(vb) + fabs(v0)));
+  }
+  if (nz) flag[c.pair] = 1;
+}
+
+// V against the sum of its parts on every grid point of every term
+__global__ __launch_bounds__(256) void k_nm_verify(const NmDev* insts, const int64_t* term0, int ninst,
+                                                   int64_t nterms, const TermDev* terms, const double* V,
+                                                   const double* c1, const double* f2, const int* flag,
+                                                   int* bad) {
+  __shared__ int an[MAXACT], af[MAXACT], act[MAXACT], np, stop, px[120], py[120], pf[120];
+  __shared__ uint8_t dig[MAXACT][256];
+  const int tid = threadIdx.x;
+  for (int64_t t = blockIdx.x; t < nterms; t += gridDim.x) {
+    __syncthreads();                   // the previous term's tables are no longer read
+    if (tid == 0) { stop = *(volatile int*)bad; np = 0; }
+    __syncthreads();
+    if (stop) return;                  // the same for the whole workgroup
+    const NmDev& I = insts[find_inst(term0, ninst, t)];
+    const int32_t* lev = I.levels + (t - I.term0) * I.D;
+    const int L1 = I.L + 1;
+    int na = 0;
+    for (int k = 0; k < I.D; ++k)
+      if (lev[k] > 0 && I.n[k * L1 + lev[k]] > 1) {
+        if (tid == 0 && na < MAXACT) {
+          act[na] = k;
+          an[na] = I.n[k * L1 + lev[k]];
+          af[na] = I.f1off[k * L1 + lev[k]];
+        }
+        ++na;
+      }
+    __syncthreads();
+    if (na > MAXACT) { if (tid == 0) *bad = 1; return; }
+    for (int e = tid; e < na * na; e += 256) {
+      const int x = e / na, y = e % na;
+      if (x >= y) continue;
+      const int a = act[x], b = act[y];
+      const int p = a * (2 * I.D - a - 1) / 2 + (b - a - 1);
+      if (!flag[I.pair0 + p]) continue;
+      const int s = atomicAdd(&np, 1);
+      px[s] = x; py[s] = y;
+      pf[s] = I.f2off[(p * L1 + lev[a]) * L1 + lev[b]];
+    }
+    __syncthreads();
+    const TermDev& T = terms[t];
+    const double v0 = c1[I.c1base];
+    const int npairs = np;
+    for (int e = tid; e < T.nq; e += 256) {
+      int rest = e;
+      double s = v0, mag = fabs(v0);
+      bool miss = false;
+      for (int j = 0; j < na; ++j) {
+        const int i = rest % an[j];
+        rest /= an[j];
+        dig[j][tid] = (uint8_t)i;
+        if (af[j] < 0) { miss = true; continue; }
+        const double f = c1[af[j] + i] - v0;
+        s += f;
+        mag += fabs(f);
+      }
+      for (int q = 0; q < npairs; ++q) {
+        if (pf[q] < 0) { miss = true; continue; }
+        const double f = f2[pf[q] + dig[px[q]][tid] + an[px[q]] * dig[py[q]][tid]];
+        s += f;
+        mag += fabs(f);
+      }
+      const double v = V[T.qoff + e];
+      if (miss || !(fabs(v - s) <= TOL_V * (mag + fabs(v)))) *bad = 1;
+    }
+  }
+}
+
+// one-mode matrices at every level: c_a T_a + BtW f_a B
+__global__ __launch_bounds__(256) void k_nm_g1(const NmDev* insts, const int32_t* work, const double* mats,
+                                               const double* c1, double* g1, int kin) {
+  const NmDev& I = insts[work[3 * blockIdx.x]];
+  const int k = work[3 * blockIdx.x + 1], l = work[3 * blockIdx.x + 2];
+  const int n = I.n[k * (I.L + 1) + l], f1 = I.f1off[k * (I.L + 1) + l];
+  const MatDev& md = I.md[k * I.L1 + l];
+  const double* B = mats + md.B;
+  const double* Bt = mats + md.BtW;
+  const double* T = I.T + I.toff[k * (I.L + 1) + l];
+  double* g = g1 + I.g1off[k * (I.L + 1) + l];
+  const double v0 = c1[I.c1base], c = kin ? I.ck[k] : 0.0;
+  for (int e = threadIdx.x; e < n * n; e += 256) {
+    const int i = e / n, j = e % n;
+    double s = 0.0, m = 0.0;
+    if (f1 >= 0 && n > 1)
+      for (int q = 0; q < n; ++q) {
+        const double w = Bt[i * n + q] * B[q * n + j], v = c1[f1 + q];
+        s = fma(w, v - v0, s);
+        m = fma(fabs(w), fabs(v) + fabs(v0), m);
+      }
+    if (!(fabs(s) > TOL_M * m)) s = 0.0;
+    g[e] = fma(c, T[e], s);
+  }
+}
+
+// two-mode matrices E(m) of a pair over the pair indices of level <= m
+__global__ __launch_bounds__(256) void k_nm_e2(const NmDev* insts, const EWork* work, const double* mats,
+                                               const double* c1, const double* f2, double* E) {
+  const EWork w = work[blockIdx.x];
+  const NmDev& I = insts[w.inst];
+  const int p = w.pair, m = w.m, L1 = I.L + 1;
+  const int a = I.pa[p], b = I.pb[p], S = I.s2n[p * L1 + m];
+  const uint16_t* lst = I.s2 + I.s2off[p];
+  const double v0 = c1[I.c1base];
+  for (int e = blockIdx.y * 256 + threadIdx.x; e < S * S; e += gridDim.y * 256) {
+    const int r = lst[e / S], c = lst[e % S];
+    const int ia = r & 255, ib = r >> 8, ja = c & 255, jb = c >> 8;
+    const int la0 = max(I.lam[a * NI + ia], I.lam[a * NI + ja]);
+    const int lb0 = max(I.lam[b * NI + ib], I.lam[b * NI + jb]);
+    double sum = 0.0, mag = 0.0;
+    for (int u = 0; u < 2; ++u) {
+      for (int la = max(la0, 1); la <= m - u - max(lb0, 1); ++la) {
+        const int lb = m - u - la;
+        const int off = I.f2off[(p * L1 + la) * L1 + lb];
+        const int fa = I.f1off[a * L1 + la], fb = I.f1off[b * L1 + lb];
+        if (off < 0 || fa < 0 || fb < 0) continue;   // levels that no row needs
+        const int na = I.n[a * L1 + la], nb = I.n[b * L1 + lb];
+        const MatDev& A = I.md[a * I.L1 + la];
+        const MatDev& Q = I.md[b * I.L1 + lb];
+        double t = 0.0;
+        for (int q = 0; q < nb; ++q) {
+          const double wb = mats[Q.BtW + ib * nb + q] * mats[Q.B + q * nb + jb];
+          double s = 0.0, g = 0.0;
+          for (int o = 0; o < na; ++o) {
+            const double wa = mats[A.BtW + ia * na + o] * mats[A.B + o * na + ja];
+            const double f = f2[off + o + na * q];
+            s = fma(wa, f, s);
+            g = fma(fabs(wa), fabs(f) + fabs(c1[fa + o]) + fabs(c1[fb + q]) + fabs(v0), g);
+          }
+          t = fma(wb, s, t);
+          mag = fma(fabs(wb), g, mag);
+        }
+        sum += u ? -t : t;
+      }
+    }
+    E[w.off + e] = fabs(sum) > TOL_M * mag ? sum : 0.0;
+  }
+}
+
+// What the row kernels read of one grid function.
+struct NmSet {
+  const double* c1;
+  const double* g1;
+  const double* E;
+  const int64_t* eoff;        // [global pair * eld + m]; -1: zero pair
+};
+// nonzero pairs (of V or mu) of every instance, and by mode
+struct NmPairs {
+  const int32_t* nz;          // instance's pairs at nzoff[inst]
+  const int32_t* nzoff;
+  const int32_t* adj;         // pairs holding mode k at adjoff[inst * 33 + k]
+  const int32_t* adjoff;
+  int eld;
+};
+
+// Entries of packed row r: counted (FILL = false) or written.  One thread per
+// row; its mode indices, levels and rank prefixes sit in LDS.
+template <bool FILL, bool MU>
+__global__ __launch_bounds__(RT) void k_nm_rows(const NmDev* insts, const int64_t* row0, int ninst,
+                                                int64_t nrows, NmSet sv, NmSet sm, NmPairs pr, int Dmax,
+                                                int32_t* cnt, const int64_t* ptr, int32_t* col, double* val,
+                                                double* valm) {
+  extern __shared__ char sh[];
+  int32_t* pre = (int32_t*)sh;                     // [k][thread] rank contribution before mode k
+  uint8_t* dg = (uint8_t*)(pre + Dmax * RT);       // mode indices
+  uint8_t* lm = dg + Dmax * RT;                    // their levels
+  uint8_t* bud = lm + Dmax * RT;                   // level budget left before mode k
+  const int tid = threadIdx.x;
+  const int64_t row = (int64_t)blockIdx.x * RT + tid;
+  if (row >= nrows) return;                        // no barriers below
+  const int ii = find_inst(row0, ninst, row);
+  const NmDev& I = insts[ii];
+  const int D = I.D, L = I.L, LB = I.LB, L1 = L + 1;
+  int32_t left = (int32_t)(row - I.row0), done = 0;
+  int b = LB, tot = 0;
+  for (int k = 0; k < D; ++k) {
+    const int32_t* p = I.pre + (k * (LB + 1) + b) * (NI + 1);
+    int i = 0;
+    while (i + 1 < NI && I.lam[k * NI + i + 1] <= b && p[i + 1] <= left) ++i;
+    const int li = I.lam[k * NI + i];
+    pre[k * RT + tid] = done;
+    dg[k * RT + tid] = (uint8_t)i;
+    lm[k * RT + tid] = (uint8_t)li;
+    bud[k * RT + tid] = (uint8_t)b;
+    left -= p[i];
+    done += p[i];
+    b -= li;
+    tot += li;
+  }
+  // rank with the index of mode x replaced by ix (and of mode y > x by iy)
+  auto rank2 = [&](int x, int ix, int y, int iy) {
+    int bb = bud[x * RT + tid];
+    int32_t r = pre[x * RT + tid] + I.pre[(x * (LB + 1) + bb) * (NI + 1) + ix];
+    bb -= I.lam[x * NI + ix];
+    for (int k = x + 1; k < D; ++k) {
+      const int i = (k == y) ? iy : dg[k * RT + tid];
+      r += I.pre[(k * (LB + 1) + bb) * (NI + 1) + i];
+      bb -= I.lam[k * NI + i];
+    }
+    return (int32_t)(r + I.row0);
+  };
+  auto epos = [&](int p, int ia, int ib) {
+    const int bm = I.pb[p];
+    return (int)I.pos[I.posoff[p] + ia * I.n[bm * L1 + L] + ib];
+  };
+  // element of a pair's matrix at its level m, rows (ia, ib) -> (ja, jb)
+  auto eget = [&](const NmSet& s, int p, int m, int ri, int ci) {
+    const int64_t o = s.eoff[(int64_t)(I.pair0 + p) * pr.eld + m];
+    return o < 0 ? 0.0 : s.E[o + (int64_t)ri * I.s2n[p * L1 + m] + ci];
+  };
+  int64_t at = FILL ? ptr[row] : 0;
+  int n = 1;
+  auto put = [&](int32_t c, double v, double vm) {
+    if constexpr (FILL) {
+      col[at] = c;
+      val[at] = v;
+      if constexpr (MU) valm[at] = vm;
+      ++at;
+    }
+    ++n;
+  };
+  const int32_t* nz = pr.nz + pr.nzoff[ii];
+  const int nnz = pr.nzoff[ii + 1] - pr.nzoff[ii];
+  if constexpr (FILL) {   // the diagonal
+    double v = sv.c1[I.c1base], vm = MU ? sm.c1[I.c1base] : 0.0;
+    for (int k = 0; k < D; ++k) {
+      const int i = dg[k * RT + tid], ma = L - (tot - lm[k * RT + tid]);
+      const int o = I.g1off[k * L1 + ma] + i * (I.n[k * L1 + ma] + 1);
+      v += sv.g1[o];
+      if constexpr (MU) vm += sm.g1[o];
+    }
+    for (int z = 0; z < nnz; ++z) {
+      const int p = nz[z], a = I.pa[p], bq = I.pb[p];
+      const int m = L - (tot - lm[a * RT + tid] - lm[bq * RT + tid]);
+      const int e = epos(p, dg[a * RT + tid], dg[bq * RT + tid]);
+      v += eget(sv, p, m, e, e);
+      if constexpr (MU) vm += eget(sm, p, m, e, e);
+    }
+    put((int32_t)row, v, vm);
+    n = 1;
+  }
+  for (int a = 0; a < D; ++a) {   // one index changed
+    const int ia = dg[a * RT + tid], la = lm[a * RT + tid], ma = L - (tot - la);
+    const int na = I.n[a * L1 + ma], room = LB - (tot - la);
+    const double* g = sv.g1 + I.g1off[a * L1 + ma] + ia * na;
+    const double* gm = MU ? sm.g1 + I.g1off[a * L1 + ma] + ia * na : nullptr;
+    const int q0 = pr.adjoff[ii * 33 + a], q1 = pr.adjoff[ii * 33 + a + 1];
+    for (int j = 0; j < na; ++j) {
+      if (j == ia || I.lam[a * NI + j] > room) continue;
+      double v = g[j], vm = MU ? gm[j] : 0.0;
+      for (int q = q0; q < q1; ++q) {
+        const int p = pr.adj[q];
+        const int o = I.pa[p] == a ? I.pb[p] : I.pa[p], io = dg[o * RT + tid];
+        const int m = L - (tot - la - lm[o * RT + tid]);
+        const bool fst = I.pa[p] == a;
+        const int ri = fst ? epos(p, ia, io) : epos(p, io, ia);
+        const int ci = fst ? epos(p, j, io) : epos(p, io, j);
+        v += eget(sv, p, m, ri, ci);
+        if constexpr (MU) vm += eget(sm, p, m, ri, ci);
+      }
+      if (v != 0.0 || vm != 0.0) put(FILL ? rank2(a, j, -1, 0) : 0, v, vm);
+    }
+  }
+  for (int z = 0; z < nnz; ++z) {   // both indices of a pair changed
+    const int p = nz[z], a = I.pa[p], bq = I.pb[p];
+    const int ia = dg[a * RT + tid], ib = dg[bq * RT + tid];
+    const int lab = lm[a * RT + tid] + lm[bq * RT + tid];
+    const int m = L - (tot - lab), room = LB - (tot - lab), S = I.s2n[p * L1 + m];
+    const uint16_t* lst = I.s2 + I.s2off[p];
+    const int ri = epos(p, ia, ib);
+    const int64_t ov = sv.eoff[(int64_t)(I.pair0 + p) * pr.eld + m];
+    const int64_t om = MU ? sm.eoff[(int64_t)(I.pair0 + p) * pr.eld + m] : -1;
+    for (int c = 0; c < S; ++c) {
+      const int ja = lst[c] & 255, jb = lst[c] >> 8;
+      if (ja == ia || jb == ib) continue;
+      if (I.lam[a * NI + ja] + I.lam[bq * NI + jb] > room) continue;
+      const double v = ov < 0 ? 0.0 : sv.E[ov + (int64_t)ri * S + c];
+      const double vm = om < 0 ? 0.0 : sm.E[om + (int64_t)ri * S + c];
+      if (v != 0.0 || vm != 0.0) put(FILL ? rank2(a, ja, bq, jb) : 0, v, vm);
+    }
+  }
+  if constexpr (!FILL) cnt[row] = n;
+}
+
+// row pointers from the row counts: sums of 1024 rows, their scan, the rows
+__global__ __launch_bounds__(256) void k_nm_sum(const int32_t* cnt, int64_t n, int64_t* part) {
+  __shared__ int64_t s[256];
+  int64_t a = 0;
+  for (int k = 0; k < 4; ++k) {
+    const int64_t i = (int64_t)blockIdx.x * 1024 + k * 256 + threadIdx.x;
+    if (i < n) a += cnt[i];
+  }
+  s[threadIdx.x] = a;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+}
+__global__ __launch_bounds__(1024) void k_nm_scan_part(int64_t* part, int np) {
+  __shared__ int64_t s[1024];
+  int64_t carry = 0;
+  for (int b = 0; b < np; b += 1024) {
+    const int i = b + threadIdx.x;
+    const int64_t x = i < np ? part[i] : 0;
+    s[threadIdx.x] = x;
+    __syncthreads();
+    for (int o = 1; o < 1024; o <<= 1) {
+      const int64_t y = (int)threadIdx.x >= o ? s[threadIdx.x - o] : 0;
+      __syncthreads();
+      s[threadIdx.x] += y;
+      __syncthreads();
+    }
+    if (i < np) part[i] = carry + s[threadIdx.x] - x;
+    const int64_t total = s[1023];
+    __syncthreads();
+    carry += total;
+  }
+  if (threadIdx.x == 0) part[np] = carry;
+}
+__global__ __launch_bounds__(1024) void k_nm_ptr(const int32_t* cnt, int64_t n, const int64_t* part,
+                                                 int64_t* ptr) {
+  __shared__ int64_t s[1024];
+  const int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+  const int64_t x = i < n ? cnt[i] : 0;
+  s[threadIdx.x] = x;
+  __syncthreads();
+  for (int o = 1; o < 1024; o <<= 1) {
+    const int64_t y = (int)threadIdx.x >= o ? s[threadIdx.x - o] : 0;
+    __syncthreads();
+    s[threadIdx.x] += y;
+    __syncthreads();
+  }
+  if (i < n) ptr[i] = part[blockIdx.x] + s[threadIdx.x] - x;
+  if (i == n - 1) ptr[n] = part[blockIdx.x] + s[threadIdx.x];
+}
+
+// hpsi(r, v) = sum_e val_e psi(col_e, v): NV * SL lanes per row, NV vectors,
+// the row's entries dealt to SL slices that are added at the end.
+// OUT_COLS: the result goes to the column-major block (nvec <= NV columns),
+// through LDS so that a workgroup writes runs of its 256 / W rows.  IN_COLS:
+// psi is column-major too (a gather of NV values touches NV lines).
+template <int NV, int SL, bool COLS, bool IN_COLS>
+__global__ __launch_bounds__(256) void k_nm_spmm(const int64_t* __restrict__ ptr,
+                                                 const int32_t* __restrict__ col,
+                                                 const double* __restrict__ val,
+                                                 const double* __restrict__ psi,
+                                                 double* __restrict__ hpsi, int64_t rows, int nvec) {
+  constexpr int W = NV * SL, R = 256 / W;
+  __shared__ double tile[COLS ? NV * (R + 1) : 1];
+  const int l = threadIdx.x % W, v = l % NV, s = l / NV;
+  const int64_t r = (int64_t)blockIdx.x * R + threadIdx.x / W;
+  const double* __restrict__ x0 = IN_COLS ? psi + (int64_t)min(v, nvec - 1) * rows : psi + v;
+  constexpr int LD = IN_COLS ? 1 : NV;
+  double a = 0.0;
+  if (r < rows) {
+    const int64_t e1 = ptr[r + 1];
+    int64_t e = ptr[r] + s;
+    double a0 = 0.0, a1 = 0.0;
+    for (; e + 3 * SL < e1; e += 4 * SL) {
+      int32_t c[4];
+      double w[4], x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { c[u] = col[e + u * SL]; w[u] = val[e + u * SL]; }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = x0[(int64_t)c[u] * LD];
+#pragma unroll
+      for (int u = 0; u < 4; u += 2) { a0 = fma(w[u], x[u], a0); a1 = fma(w[u + 1], x[u + 1], a1); }
+    }
+    for (; e < e1; e += SL) a0 = fma(val[e], x0[(int64_t)col[e] * LD], a0);
+    a = a0 + a1;
+#pragma unroll
+    for (int o = NV; o < W; o <<= 1) a += __shfl_xor(a, o, 64);
+    if (!COLS && s == 0) hpsi[r * NV + v] = a;
+  }
+  if constexpr (COLS) {
+    if (s == 0) tile[v * (R + 1) + threadIdx.x / W] = a;
+    __syncthreads();
+    for (int t = threadIdx.x; t < NV * R; t += 256) {
+      const int vv = t / R, rr = t % R;
+      const int64_t ro = (int64_t)blockIdx.x * R + rr;
+      if (vv < nvec && ro < rows) hpsi[(int64_t)vv * rows + ro] = tile[vv * (R + 1) + rr];
+    }
+  }
+}
+// any number of vectors: one thread per (row, vector)
+__global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__ ptr,
+                                                     const int32_t* __restrict__ col,
+                                                     const double* __restrict__ val,
+                                                     const double* __restrict__ psi,
+                                                     double* __restrict__ hpsi, int64_t rows, int nvec) {
+  const int64_t n = rows * nvec;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const int64_t r = i / nvec;
+    const int v = (int)(i - r * nvec);
+    const int64_t e1 = ptr[r + 1];
+    int64_t e = ptr[r];
+    double a0 = 0.0, a1 = 0.0;
+    for (; e + 3 < e1; e += 4) {
+      int32_t c[4];
+      double w[4], x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { c[u] = col[e + u]; w[u] = val[e + u]; }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = psi[(int64_t)c[u] * nvec + v];
+#pragma unroll
+      for (int u = 0; u < 4; u += 2) { a0 = fma(w[u], x[u], a0); a1 = fma(w[u + 1], x[u + 1], a1); }
+    }
+    for (; e < e1; ++e) a0 = fma(val[e], psi[(int64_t)col[e] * nvec + v], a0);
+    hpsi[i] = a0 + a1;
+  }
+}
+
+__global__ void k_nm_zero(int* p, int n) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
+}
+
+// a host byte block whose sections become device pointers after one copy
+struct Blob {
+  std::vector<char> h;
+  template <class T>
+  size_t add(const std::vector<T>& v) {
+    const size_t o = (h.size() + 15) & ~(size_t)15;
+    h.resize(o + sizeof(T) * std::max<size_t>(v.size(), 1));
+    if (!v.empty()) std::memcpy(&h[o], v.data(), sizeof(T) * v.size());
+    return o;
+  }
+};
+
+int upload(const Blob& b, DevBuf& d, hipStream_t st) {
+  int rc;
+  if (d.n < b.h.size() && (rc = d.alloc(b.h.size()))) return rc;
+  NM_TRY(hipMemcpyAsync(d.p, b.h.data(), b.h.size(), hipMemcpyHostToDevice, st));
+  NM_TRY(hipStreamSynchronize(st));   // the host block is pageable and goes away
+  return SG4_OK;
+}
+
+int ensure(DevBuf& d, size_t bytes) { return d.n >= bytes && d.p ? SG4_OK : d.alloc(std::max<size_t>(bytes, 256)); }
+
+}  // namespace
+
+struct NModeTables {
+  bool ok = false;
+  DevBuf blob, insts, work, ck;    // tables; NmDev of every instance; build workspace; c_k
+  DevBuf e_v, e_mu, lists;
+  std::vector<NmDev> dev;          // host copies (device pointers inside)
+  size_t o_term0 = 0, o_row0 = 0, o_cut1 = 0, o_cut2 = 0, o_g1work = 0;
+  int ncut1 = 0, ncut2 = 0, ng1 = 0, npairs = 0, Lmax = 0, Dmax = 0;
+  int64_t nc1 = 0, nf2 = 0, ng1v = 0, nterms = 0;
+  std::vector<int32_t> pair_inst, pair_s2n;   // per global pair: instance; [pair * (Lmax+1) + m]
+};
+
+void nmode_tables_destroy(NModeTables* t) { delete t; }
+
+NModeTables* nmode_tables_create(const NModeIn& in) {
+  auto t = std::make_unique<NModeTables>();
+  const int ni = (int)in.inst.size();
+  t->dev.resize(ni);
+  for (const NModeInst& I : in.inst) {
+    t->Lmax = std::max(t->Lmax, I.L);
+    t->Dmax = std::max(t->Dmax, I.D);
+    t->nterms += I.nterms;
+  }
+  Blob blob;
+  struct Off { size_t n, lam, pre, f1off, f2off, s2n, s2off, s2, posoff, pos, pa, pb, T, toff, g1off; };
+  std::vector<Off> off(ni);
+  std::vector<Cut> cut1, cut2;
+  std::vector<int32_t> g1work;
+  std::vector<int64_t> term0, row0;
+  for (int x = 0; x < ni; ++x) {
+    const NModeInst& I = in.inst[x];
+    NmDev& d = t->dev[x];
+    const int D = I.D, L = I.L, L1 = L + 1, M1 = I.Lmax + 1;
+    d.D = D; d.L = L; d.L1 = M1;
+    d.term0 = I.term0; d.nterms = I.nterms; d.row0 = I.row0; d.nrows = I.nb_ba;
+    auto nn = [&](int k, int l) { return (*in.nq)[I.md0 + (int64_t)k * M1 + l]; };
+    std::vector<int32_t> n(D * L1);
+    for (int k = 0; k < D; ++k)
+      for (int l = 0; l <= L; ++l) {
+        n[k * L1 + l] = nn(k, l);
+        // the middle point is shared by the rules of a mode when they are odd
+        if (n[k * L1 + l] % 2 == 0 || n[k * L1 + l] > NI || (l && n[k * L1 + l] < n[k * L1 + l - 1]) ||
+            n[k * L1] != 1)
+          return t.release();
+      }
+    std::vector<uint8_t> lam(D * NI, 255);
+    for (int k = 0; k < D; ++k)
+      for (int i = 0; i < NI; ++i)
+        for (int l = 0; l <= L; ++l)
+          if (n[k * L1 + l] > i) { lam[k * NI + i] = (uint8_t)l; break; }
+    // basis level from the number of packed rows
+    int LB = -1;
+    std::vector<int64_t> cnt((D + 1) * L1, 0);
+    for (int b = 0; b <= L; ++b) cnt[D * L1 + b] = 1;
+    for (int k = D - 1; k >= 0; --k)
+      for (int b = 0; b <= L; ++b)
+        for (int i = 0; i < NI && lam[k * NI + i] <= b; ++i) cnt[k * L1 + b] += cnt[(k + 1) * L1 + b - lam[k * NI + i]];
+    for (int b = 0; b <= L; ++b)
+      if (cnt[b] == I.nb_ba) LB = b;
+    if (LB < 0 || I.nb_ba > INT32_MAX) return t.release();
+    d.LB = LB;
+    std::vector<int32_t> pre((size_t)D * (LB + 1) * (NI + 1), -1);
+    for (int k = 0; k < D; ++k)
+      for (int b = 0; b <= LB; ++b) {
+        int64_t s = 0;
+        for (int i = 0; i <= NI; ++i) {
+          pre[((size_t)k * (LB + 1) + b) * (NI + 1) + i] = (int32_t)s;
+          if (i == NI || lam[k * NI + i] > b) break;
+          s += cnt[(k + 1) * L1 + b - lam[k * NI + i]];
+        }
+      }
+    // cuts: for every (mode, level) and (pair, levels >= 1) the first term that
+    // has them; the other modes at their middle points
+    const int np = D * (D - 1) / 2;
+    d.npair = np;
+    d.pair0 = t->npairs;
+    std::vector<uint8_t> pa(np), pb(np);
+    for (int a = 0, p = 0; a < D; ++a)
+      for (int b = a + 1; b < D; ++b, ++p) { pa[p] = (uint8_t)a; pb[p] = (uint8_t)b; }
+    std::vector<int32_t> f1off(D * L1, -1), f2off((size_t)np * L1 * L1, -1);
+    d.c1base = t->nc1;
+    t->nc1 += 1;
+    std::vector<int> act;
+    std::vector<int64_t> stride(D);
+    bool centre = false;
+    std::vector<Cut> c2;
+    for (int64_t tt = 0; tt < I.nterms; ++tt) {
+      const int32_t* lev = &(*in.levels)[I.lev0 + tt * D];
+      act.clear();
+      int64_t s = 1, mid = (*in.qoff)[I.term0 + tt];
+      for (int k = 0; k < D; ++k) {
+        const int nk = n[k * L1 + lev[k]];
+        stride[k] = s;
+        mid += s * (nk / 2);
+        s *= nk;
+        if (nk > 1) act.push_back(k);
+      }
+      auto cut = [&](int a, int b) {
+        Cut c{};
+        const int na = n[a * L1 + lev[a]];
+        c.sa = (int32_t)stride[a]; c.na = na; c.sb = 0; c.nb = 1; c.pair = -1;
+        c.off = mid - stride[a] * (na / 2);
+        if (b >= 0) {
+          const int nb = n[b * L1 + lev[b]];
+          c.sb = (int32_t)stride[b]; c.nb = nb;
+          c.off -= stride[b] * (nb / 2);
+        }
+        return c;
+      };
+      if (!centre) {
+        Cut c{};
+        c.off = mid; c.na = 1; c.nb = 1; c.out = d.c1base; c.pair = -1;
+        cut1.push_back(c);
+        centre = true;
+      }
+      for (size_t u = 0; u < act.size(); ++u) {
+        const int a = act[u];
+        if (f1off[a * L1 + lev[a]] < 0) {
+          Cut c = cut(a, -1);
+          c.out = t->nc1;
+          f1off[a * L1 + lev[a]] = (int32_t)c.out;
+          t->nc1 += c.na;
+          cut1.push_back(c);
+        }
+        for (size_t w = u + 1; w < act.size(); ++w) {
+          const int b = act[w], p = a * (2 * D - a - 1) / 2 + (b - a - 1);
+          int32_t& o = f2off[((size_t)p * L1 + lev[a]) * L1 + lev[b]];
+          if (o >= 0) continue;
+          Cut c = cut(a, b);
+          c.out = t->nf2;
+          c.pair = d.pair0 + p;
+          c.v0 = d.c1base;
+          c.fa = lev[a]; c.fb = lev[b];   // resolved below
+          c2.push_back(c);
+          o = (int32_t)t->nf2;
+          t->nf2 += (int64_t)c.na * c.nb;
+        }
+      }
+      if (t->nf2 > INT32_MAX || t->nc1 > INT32_MAX) return t.release();
+    }
+    for (Cut& c : c2) {
+      const int p = c.pair - d.pair0;
+      c.fa = f1off[pa[p] * L1 + (int)c.fa];
+      c.fb = f1off[pb[p] * L1 + (int)c.fb];
+      cut2.push_back(c);
+    }
+    // pair indices by level, and their positions
+    std::vector<int32_t> s2n((size_t)np * L1), s2off(np), posoff(np);
+    std::vector<uint16_t> s2;
+    std::vector<int16_t> pos;
+    std::map<std::vector<int32_t>, std::pair<int32_t, int32_t>> known;   // modes of equal sizes share a list
+    for (int p = 0; p < np; ++p) {
+      const int a = pa[p], b = pb[p], nA = n[a * L1 + L], nB = n[b * L1 + L];
+      std::vector<int32_t> key(n.begin() + a * L1, n.begin() + (a + 1) * L1);
+      key.insert(key.end(), n.begin() + b * L1, n.begin() + (b + 1) * L1);
+      auto f = known.find(key);
+      const bool fresh = f == known.end();
+      if (fresh) f = known.emplace(key, std::make_pair((int32_t)s2.size(), (int32_t)pos.size())).first;
+      s2off[p] = f->second.first;
+      posoff[p] = f->second.second;
+      if (fresh) pos.resize(pos.size() + (size_t)nA * nB, -1);
+      int c = 0;
+      for (int m = 0; m <= L; ++m) {
+        for (int ia = 0; ia < nA; ++ia)
+          for (int ib = 0; ib < nB; ++ib)
+            if (lam[a * NI + ia] + lam[b * NI + ib] == m) {
+              if (fresh) {
+                s2.push_back((uint16_t)(ia | ib << 8));
+                pos[posoff[p] + (size_t)ia * nB + ib] = (int16_t)c;
+              }
+              ++c;
+            }
+        s2n[(size_t)p * L1 + m] = c;
+      }
+      if (c > INT16_MAX) return t.release();
+      t->pair_inst.push_back(x);
+    }
+    std::vector<int32_t> g1off(D * L1), toff(D * L1);
+    std::vector<double> T;
+    for (int k = 0; k < D; ++k) {
+      for (int l = 0; l <= L; ++l) {
+        const int nk = n[k * L1 + l];
+        g1off[k * L1 + l] = (int32_t)t->ng1v;
+        t->ng1v += (int64_t)nk * nk;
+        toff[k * L1 + l] = (int32_t)T.size();
+        const double* src = in.T->data() + (*in.toff)[I.md0 + (int64_t)k * M1 + l];
+        T.insert(T.end(), src, src + (size_t)nk * nk);
+        g1work.insert(g1work.end(), {x, k, l});
+      }
+    }
+    if (t->ng1v > INT32_MAX) return t.release();
+    term0.push_back(I.term0);
+    row0.push_back(I.row0);
+    Off& o = off[x];
+    o.n = blob.add(n); o.lam = blob.add(lam); o.pre = blob.add(pre); o.f1off = blob.add(f1off);
+    o.f2off = blob.add(f2off); o.s2n = blob.add(s2n); o.s2off = blob.add(s2off); o.s2 = blob.add(s2);
+    o.posoff = blob.add(posoff); o.pos = blob.add(pos); o.pa = blob.add(pa); o.pb = blob.add(pb);
+    o.T = blob.add(T); o.toff = blob.add(toff); o.g1off = blob.add(g1off);
+    for (int p = 0; p < np; ++p)
+      for (int m = 0; m <= t->Lmax; ++m) t->pair_s2n.push_back(m <= L ? s2n[(size_t)p * L1 + m] : 0);
+    t->npairs += np;
+  }
+  t->ncut1 = (int)cut1.size();
+  t->ncut2 = (int)cut2.size();
+  t->ng1 = (int)g1work.size() / 3;
+  t->o_term0 = blob.add(term0);
+  t->o_row0 = blob.add(row0);
+  t->o_cut1 = blob.add(cut1);
+  t->o_cut2 = blob.add(cut2);
+  t->o_g1work = blob.add(g1work);
+  if (upload(blob, t->blob, in.stream) != SG4_OK || t->ck.alloc(sizeof(double) * in.ck->size()) != SG4_OK)
+    return nullptr;
+  char* B = t->blob.as<char>();
+  for (int x = 0; x < ni; ++x) {
+    const NModeInst& I = in.inst[x];
+    NmDev& d = t->dev[x];
+    const Off& o = off[x];
+    d.levels = in.d_levels + I.lev0;
+    d.md = in.d_md + I.md0;
+    d.n = (int32_t*)(B + o.n); d.lam = (uint8_t*)(B + o.lam); d.pre = (int32_t*)(B + o.pre);
+    d.f1off = (int32_t*)(B + o.f1off); d.f2off = (int32_t*)(B + o.f2off); d.s2n = (int32_t*)(B + o.s2n);
+    d.s2off = (int32_t*)(B + o.s2off); d.s2 = (uint16_t*)(B + o.s2); d.posoff = (int32_t*)(B + o.posoff);
+    d.pos = (int16_t*)(B + o.pos); d.pa = (uint8_t*)(B + o.pa); d.pb = (uint8_t*)(B + o.pb);
+    d.T = (double*)(B + o.T); d.toff = (int32_t*)(B + o.toff); d.ck = t->ck.as<double>() + I.ck0;
+    d.g1off = (int32_t*)(B + o.g1off);
+  }
+  Blob ib;
+  ib.add(t->dev);
+  if (upload(ib, t->insts, in.stream) != SG4_OK) return nullptr;
+  // the packed rows in lexicographic order?
+  if (ensure(t->work, 256) != SG4_OK) return nullptr;
+  int* bad = t->work.as<int>();
+  hipLaunchKernelGGL(k_nm_zero, dim3(1), dim3(64), 0, in.stream, bad, 1);
+  hipLaunchKernelGGL(k_nm_check_map, dim3((unsigned)std::min<int64_t>(t->nterms, 16384)), dim3(256), 0,
+                     in.stream, t->insts.as<NmDev>(), (const int64_t*)(B + t->o_term0), ni, t->nterms,
+                     in.d_terms, in.d_map, bad);
+  int h = 1;
+  if (hipMemcpyAsync(&h, bad, sizeof(int), hipMemcpyDeviceToHost, in.stream) != hipSuccess ||
+      hipStreamSynchronize(in.stream) != hipSuccess) {
+    set_error("HIP error while checking the packed rows");
+    return nullptr;
+  }
+  t->ok = h == 0;
+  return t.release();
+}
+
+int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double* mu, NModeMat& m) {
+  m.valid = false;
+  if (!t || !t->ok) return SG4_OK;
+  const hipStream_t st = in.stream;
+  const int ni = (int)in.inst.size(), nset = mu ? 2 : 1, eld = t->Lmax + 1;
+  const int64_t rows = in.rows;
+  const int npart = (int)((rows + 1023) / 1024);
+  int rc;
+  // workspace: cuts, functions, one-mode matrices, pair flags of V (and mu), row counts, scan
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t b_c1 = up(8 * t->nc1), b_f2 = up(8 * (t->nf2 + 1)), b_g1 = up(8 * t->ng1v),
+               b_fl = up(4 * ((size_t)t->npairs + 1)), b_set = b_c1 + b_f2 + b_g1 + b_fl,
+               b_cnt = up(4 * rows), b_part = up(8 * ((size_t)npart + 1));
+  if ((rc = ensure(t->work, b_set * nset + b_cnt + b_part))) return SG4_OK;   // no memory: term kernels
+  char* W = t->work.as<char>();
+  char* B = t->blob.as<char>();
+  double *c1[2], *f2[2], *g1[2];
+  int* flag[2];                      // per pair, then the verdict
+  for (int s = 0; s < nset; ++s) {
+    char* w = W + s * b_set;
+    c1[s] = (double*)w; f2[s] = (double*)(w + b_c1); g1[s] = (double*)(w + b_c1 + b_f2);
+    flag[s] = (int*)(w + b_c1 + b_f2 + b_g1);
+  }
+  int32_t* cnt = (int32_t*)(W + b_set * nset);
+  int64_t* part = (int64_t*)(W + b_set * nset + b_cnt);
+  const NmDev* insts = t->insts.as<NmDev>();
+  const int64_t* term0 = (const int64_t*)(B + t->o_term0);
+  const int64_t* row0 = (const int64_t*)(B + t->o_row0);
+  NM_TRY(hipMemcpyAsync(t->ck.p, in.ck->data(), sizeof(double) * in.ck->size(), hipMemcpyHostToDevice, st));
+  std::vector<int> hf[2];
+  for (int s = 0; s < nset; ++s) {
+    const double* G = s ? mu : V;
+    hipLaunchKernelGGL(k_nm_zero, dim3(8), dim3(256), 0, st, flag[s], t->npairs + 1);
+    hipLaunchKernelGGL(k_nm_cut1, dim3(t->ncut1), dim3(64), 0, st, (const Cut*)(B + t->o_cut1), G, c1[s]);
+    if (t->ncut2)
+      hipLaunchKernelGGL(k_nm_cut2, dim3(t->ncut2), dim3(64), 0, st, (const Cut*)(B + t->o_cut2), G, c1[s],
+                         f2[s], flag[s]);
+    hipLaunchKernelGGL(k_nm_verify, dim3((unsigned)std::min<int64_t>(t->nterms, 16384)), dim3(256), 0, st,
+                       insts, term0, ni, t->nterms, in.d_terms, G, c1[s], f2[s], flag[s],
+                       flag[s] + t->npairs);
+    hipLaunchKernelGGL(k_nm_g1, dim3(t->ng1), dim3(256), 0, st, insts, (const int32_t*)(B + t->o_g1work),
+                       in.d_mats, c1[s], g1[s], s == 0);
+    hf[s].resize(t->npairs + 1);
+    NM_TRY(hipMemcpyAsync(hf[s].data(), flag[s], sizeof(int) * hf[s].size(), hipMemcpyDeviceToHost, st));
+  }
+  NM_TRY(hipGetLastError());
+  NM_TRY(hipStreamSynchronize(st));
+  for (int s = 0; s < nset; ++s)
+    if (hf[s][t->npairs]) return SG4_OK;   // not a sum of one- and two-mode functions
+  // two-mode matrices of the nonzero pairs
+  std::vector<EWork> ew[2];
+  std::vector<int64_t> eoff[2];
+  int64_t ne[2] = {0, 0};
+  int Smax = 0;
+  for (int s = 0; s < nset; ++s) {
+    eoff[s].assign((size_t)t->npairs * eld, -1);
+    for (int g = 0; g < t->npairs; ++g) {
+      if (!hf[s][g]) continue;
+      const int x = t->pair_inst[g];
+      for (int l = 0; l <= t->dev[x].L; ++l) {
+        const int S = t->pair_s2n[(size_t)g * eld + l];
+        eoff[s][(size_t)g * eld + l] = ne[s];
+        ew[s].push_back(EWork{x, g - t->dev[x].pair0, l, 0, ne[s]});
+        ne[s] += (int64_t)S * S;
+        Smax = std::max(Smax, S);
+      }
+      if (ne[s] > MAX_E) return SG4_OK;
+    }
+  }
+  std::vector<int32_t> nz, nzoff(1, 0), adj, adjoff((size_t)ni * 33 + 33, 0);
+  for (int x = 0; x < ni; ++x) {
+    const NmDev& d = t->dev[x];
+    std::vector<std::vector<int32_t>> by(d.D);
+    for (int a = 0, p = 0; a < d.D; ++a)
+      for (int b = a + 1; b < d.D; ++b, ++p)
+        if (hf[0][d.pair0 + p] || (mu && hf[1][d.pair0 + p])) {
+          nz.push_back(p);
+          by[a].push_back(p);
+          by[b].push_back(p);
+        }
+    nzoff.push_back((int32_t)nz.size());
+    for (int k = 0; k < d.D; ++k) {
+      adjoff[(size_t)x * 33 + k] = (int32_t)adj.size();
+      adj.insert(adj.end(), by[k].begin(), by[k].end());
+      adjoff[(size_t)x * 33 + k + 1] = (int32_t)adj.size();
+    }
+  }
+  Blob lb;
+  size_t o_ew[2], o_eoff[2];
+  for (int s = 0; s < nset; ++s) { o_ew[s] = lb.add(ew[s]); o_eoff[s] = lb.add(eoff[s]); }
+  const size_t o_nz = lb.add(nz), o_nzoff = lb.add(nzoff), o_adj = lb.add(adj), o_adjoff = lb.add(adjoff);
+  if ((rc = upload(lb, t->lists, st))) return rc == SG4_ERR_OOM ? SG4_OK : rc;
+  if (ensure(t->e_v, 8 * ne[0]) || (mu && ensure(t->e_mu, 8 * ne[1]))) return SG4_OK;
+  char* LB = t->lists.as<char>();
+  DevBuf* eb[2] = {&t->e_v, &t->e_mu};
+  NmSet set[2] = {};
+  for (int s = 0; s < nset; ++s) {
+    set[s] = NmSet{c1[s], g1[s], eb[s]->as<double>(), (const int64_t*)(LB + o_eoff[s])};
+    if (!ew[s].empty())
+      hipLaunchKernelGGL(k_nm_e2, dim3((unsigned)ew[s].size(), (unsigned)std::min(64, (Smax * Smax + 255) / 256)),
+                         dim3(256), 0, st, insts, (const EWork*)(LB + o_ew[s]), in.d_mats, c1[s], f2[s],
+                         eb[s]->as<double>());
+  }
+  const NmPairs pr{(const int32_t*)(LB + o_nz), (const int32_t*)(LB + o_nzoff), (const int32_t*)(LB + o_adj),
+                   (const int32_t*)(LB + o_adjoff), eld};
+  const dim3 rg((unsigned)((rows + RT - 1) / RT));
+  const size_t rl = (size_t)t->Dmax * RT * 7;
+  if (mu)
+    hipLaunchKernelGGL((k_nm_rows<false, true>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+                       t->Dmax, cnt, nullptr, nullptr, nullptr, nullptr);
+  else
+    hipLaunchKernelGGL((k_nm_rows<false, false>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+                       t->Dmax, cnt, nullptr, nullptr, nullptr, nullptr);
+  hipLaunchKernelGGL(k_nm_sum, dim3(npart), dim3(256), 0, st, cnt, rows, part);
+  hipLaunchKernelGGL(k_nm_scan_part, dim3(1), dim3(1024), 0, st, part, npart);
+  int64_t nnz = 0;
+  NM_TRY(hipMemcpyAsync(&nnz, part + npart, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  NM_TRY(hipGetLastError());
+  NM_TRY(hipStreamSynchronize(st));
+  if (nnz > NNZ_SMALL && nnz > NNZ_PER_POINT * (double)in.sum_nq) return SG4_OK;
+  if (ensure(m.ptr, 8 * (rows + 1)) || ensure(m.col, 4 * nnz) || ensure(m.val, 8 * nnz) ||
+      (mu && (ensure(m.val_mu, 8 * nnz) || ensure(m.val_f, 8 * nnz))))
+    return SG4_OK;
+  hipLaunchKernelGGL(k_nm_ptr, dim3(npart), dim3(1024), 0, st, cnt, rows, part, m.ptr.as<int64_t>());
+  if (mu)
+    hipLaunchKernelGGL((k_nm_rows<true, true>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+                       t->Dmax, cnt, m.ptr.as<int64_t>(), m.col.as<int32_t>(), m.val.as<double>(),
+                       m.val_mu.as<double>());
+  else
+    hipLaunchKernelGGL((k_nm_rows<true, false>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+                       t->Dmax, cnt, m.ptr.as<int64_t>(), m.col.as<int32_t>(), m.val.as<double>(), nullptr);
+  NM_TRY(hipGetLastError());
+  m.rows = rows;
+  m.nnz = nnz;
+  m.valid = true;
+  return SG4_OK;
+}
+
+namespace {
+template <bool COLS, bool IN_COLS>
+int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st) {
+  const int64_t* ptr = m.ptr.as<int64_t>();
+  const int32_t* col = m.col.as<int32_t>();
+  const double* val = m.val.as<double>();
+#define SG4_SPMM(NV, SL)                                                                              \
+  hipLaunchKernelGGL((k_nm_spmm<NV, SL, COLS, IN_COLS>), dim3((unsigned)((m.rows * NV * SL + 255) / 256)),     \
+                     dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec)
+  switch (W) {
+    case 1: SG4_SPMM(1, 8); break;
+    case 2: SG4_SPMM(2, 4); break;
+    case 4: SG4_SPMM(4, 4); break;
+    case 8: SG4_SPMM(8, 1); break;
+    case 16: SG4_SPMM(16, 1); break;
+    default: return 1;
+  }
+#undef SG4_SPMM
+  NM_TRY(hipGetLastError());
+  return SG4_OK;
+}
+}  // namespace
+
+int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st) {
+  const int rc = spmm<false, false>(m, nvec, nvec, psi, hpsi, st);
+  if (rc <= 0) return rc;
+  hipLaunchKernelGGL(k_nm_spmm_any, dim3((unsigned)std::min<int64_t>((m.rows * nvec + 255) / 256, (int64_t)1 << 20)),
+                     dim3(256), 0, st, m.ptr.as<int64_t>(), m.col.as<int32_t>(), m.val.as<double>(), psi, hpsi,
+                     m.rows, nvec);
+  NM_TRY(hipGetLastError());
+  return SG4_OK;
+}
+
+bool nmode_cols_direct(const NModeMat& m, int W) {
+  return W <= 16 && (W & (W - 1)) == 0 && m.nnz * W * W <= COLS_DIRECT;
+}
+
+int nmode_apply_cols(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st) {
+  return spmm<true, true>(m, W, nvec, psi, hpsi, st);
+}
+
+int nmode_apply_to_cols(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st) {
+  return spmm<true, false>(m, W, nvec, psi, hpsi, st);
+}
+
+}  // namespace sg4

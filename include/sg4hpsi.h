@@ -379,6 +379,9 @@ int sg4_apply_graph(sg4_plan *p, int32_t nvec, const double *psi, double *hpsi, 
  * sub_module_basis_BtoG_GtoB_SG4.f90:1288-1289); the default here is FP64
  * atomics.  Costs 16 bytes of device memory per result element. */
 #define SG4_OPT_DETERMINISTIC 2
+/* SG4_OPT_SPARSE (default 1): FP64 applies of operators that take the form run
+ * as one sparse matrix (sg4_plan_sparse_info); 0: the term kernels. */
+#define SG4_OPT_SPARSE 3
 int sg4_plan_set_option(sg4_plan *p, int32_t option, int32_t value);
 /* Whether FP64 and FP32 applies of this plan take the split path (split = 1)
  * and the number of stored entries of its kinetic matrix (nonzero whenever
@@ -387,11 +390,27 @@ int sg4_plan_set_option(sg4_plan *p, int32_t option, int32_t value);
  * mode of more than 24 points).  No counterpart in the reference. */
 int sg4_plan_split_info(const sg4_plan *p, int32_t *split, int64_t *kin_nnz);
 
+/* Whether FP64 applies of this plan run as one sparse matrix over the packed
+ * rows (sparse = 1), and its stored entries.  The operator takes that form
+ * when its split algebra holds, its rules have odd sizes, and V is a sum of
+ * one- and two-mode functions to rounding on every grid point (Henon-Heiles,
+ * harmonic, vibronic-coupling and pair force-field models): by the telescoped
+ * Smolyak sums the matrix is the same operator without the sum's
+ * cancellation.  It is built when the operator is set, holds 12 bytes per
+ * entry (32.2 M entries at 10D L=8 Henon-Heiles), and is not used while a
+ * field is set or with SG4_OPT_DETERMINISTIC, SG4_OPT_GROUPING = 0 or
+ * SG4_OPT_SPARSE = 0; other
+ * potentials and precisions keep the term kernels.  No counterpart in the
+ * reference. */
+int sg4_plan_sparse_info(const sg4_plan *p, int32_t *sparse, int64_t *nnz);
+
 /* Statistics of the last apply for roofline reporting: its work items, and
  * the algorithmic flops and HBM bytes of its main H.psi launch (the one that
  * sg4_plan_timing brackets): basis->grid, grid->basis (and, off the split
  * path, kinetic) mode products of the active modes; bytes = potential grid,
- * map, one read of psi and one write of H.psi. */
+ * map, one read of psi and one write of H.psi.  An apply of the sparse matrix
+ * reports the split path's products, which it stands for (2 flops per stored
+ * entry and vector are what it does), and the number of terms as items. */
 int sg4_plan_stats(const sg4_plan *p, int32_t nvec, double *flops, double *bytes,
                    int64_t *items);
 /* Split-precision mode (SG4_PREC_F32X2): flops the matrix cores executed in
