@@ -23,7 +23,9 @@
 // instances of a batch): lambda = a_i target on block i, propagated backwards
 // with U^dagger, and dJ/deps_s = 2 Re <lambda_s | dpsi_s>, dpsi_s being the
 // forward tangent of segment s (dHs/deps = mu/Esc, E0 and Esc fixed), exact
-// for the discrete map.  States at the start of every ckpt_every-th segment
+// for the discrete map.  Where H and mu are one sparse matrix (FP64,
+// sg4_nmode.hip) an order is one launch and a segment only rescales the
+// matrix values.  States at the start of every ckpt_every-th segment
 // are kept; the backward sweep recomputes the others block by block.
 #include <hip/hip_runtime.h>
 
@@ -32,7 +34,7 @@
 #include <string>
 #include <vector>
 
-#include "sg4_internal.h"
+#include "sg4_nmode.h"
 
 namespace sg4 {
 
@@ -275,9 +277,19 @@ struct Prop {
   Buf A4, B4, Y4, E, MW, TACC;   // tangent step
   Buf part;
   std::vector<double> hpart;
+  // H and mu as one sparse matrix where the operator has that form (FP64): an
+  // order is then one launch that forms H w_k and updates the recurrence
+  NModeMat* nm = nullptr;
+  const double* val = nullptr;   // the segment's values
 
   int init(bool tangent) {
     int rc;
+    if (nm) {
+      if ((rc = B.alloc(n)) || (rc = ACC.alloc(n)) || (rc = part.alloc(2 * RED_BLOCKS))) return rc;
+      if (tangent && ((rc = A4.alloc(2 * n)) || (rc = B4.alloc(2 * n)) || (rc = TACC.alloc(n)))) return rc;
+      hpart.resize(2 * RED_BLOCKS);
+      return SG4_OK;
+    }
     if ((rc = A.alloc(n)) || (rc = B.alloc(n)) || (rc = Y.alloc(n)) || (rc = ACC.alloc(n)) ||
         (rc = part.alloc(2 * RED_BLOCKS)))
       return rc;
@@ -285,6 +297,51 @@ struct Prop {
                     (rc = E.alloc(n)) || (rc = MW.alloc(n)) || (rc = TACC.alloc(n))))
       return rc;
     hpart.resize(2 * RED_BLOCKS);
+    return SG4_OK;
+  }
+
+  // A step of the sparse path: the result is in psi afterwards, which trades
+  // places with other (w_0 = psi and w_1 in other alternate as w_{k-1}, w_k; the
+  // last order writes the phased sum over w_{k-1}, which no row gathers).
+  int step_sparse(double*& psi, double*& other, double sgn) {
+    double *wm = other, *wk = psi;
+    const double ph = sgn * p->E0 * p->dt;   // exp(-i E0 dt) forward, its conjugate backward
+    NModeOrder o{};
+    o.val = val; o.acc = ACC.p; o.c0 = p->coef[0]; o.E0 = p->E0; o.sc = 1.0 / p->Esc; o.sgn = sgn;
+    o.pr = std::cos(ph); o.pi = std::sin(ph); o.ns = ns;
+    int rc;
+    for (int k = 1; k < p->ncoef; ++k) {
+      o.wk = wk; o.wm = wm; o.c = p->coef[k];
+      o.first = k == 1; o.last = k + 1 == p->ncoef; o.out = wm;
+      if ((rc = nmode_order(*nm, o, false, st))) return rc;
+      std::swap(wm, wk);
+    }
+    psi = wk;
+    other = wm;
+    return SG4_OK;
+  }
+  int step(Buf& psi, double sgn) {
+    if (nm) return step_sparse(psi.p, B.p, sgn);
+    return step(psi.p, sgn);
+  }
+
+  // (psi, dpsi) <- (U psi, U dpsi + (dU/deps) psi) on the sparse path
+  int tangent_sparse(double* psi, double* dpsi) {
+    const double ph = -p->E0 * p->dt;
+    hipLaunchKernelGGL(k_cb_pack, dim3(blocks_for(n)), dim3(256), 0, st, psi, dpsi, A4.p, rows, ns);
+    CB_TRY(hipGetLastError());
+    double *wm = B4.p, *wk = A4.p;
+    NModeOrder o{};
+    o.val = val; o.acc = ACC.p; o.tacc = TACC.p; o.out = psi; o.tout = dpsi;
+    o.c0 = p->coef[0]; o.E0 = p->E0; o.sc = 1.0 / p->Esc; o.sgn = -1.0;
+    o.pr = std::cos(ph); o.pi = std::sin(ph); o.ns = ns;
+    int rc;
+    for (int k = 1; k < p->ncoef; ++k) {
+      o.wk = wk; o.wm = wm; o.c = p->coef[k];
+      o.first = k == 1; o.last = k + 1 == p->ncoef;
+      if ((rc = nmode_order(*nm, o, true, st))) return rc;
+      std::swap(wm, wk);
+    }
     return SG4_OK;
   }
 
@@ -316,6 +373,7 @@ struct Prop {
 
   // (psi, dpsi) <- (U psi, U dpsi + (dU/deps) psi)
   int step_tangent(double* psi, double* dpsi) {
+    if (nm) return tangent_sparse(psi, dpsi);
     const dim3 g(blocks_for(rows * ns)), b(256);
     const double sc = 1.0 / p->Esc, sgn = -1.0;
     int rc;
@@ -358,7 +416,21 @@ struct Prop {
     return SG4_OK;
   }
 
-  int field(int s) { return sg4_plan_set_field(H, mu, s < 0 ? 0.0 : p->eps[s]); }
+  int field(int s) {
+    if (!nm) return sg4_plan_set_field(H, mu, p->eps[s]);
+    if (!mu) return SG4_OK;
+    val = nm->val_f.as<double>();
+    return nmode_set_field(*nm, p->eps[s], st);
+  }
+
+  // whether the orders run on the sparse matrix (decided once per call)
+  int choose(int ncol, int64_t applies) {
+    int rc;
+    if (p->ncoef < 2 || !nmode_order_width(ncol)) return SG4_OK;
+    if ((rc = plan_field_matrix(H, mu, p->prec, applies, &nm))) return rc;
+    if (nm) val = nm->val.as<double>();
+    return SG4_OK;
+  }
 };
 
 // Restores the field-free potential of H when a propagation leaves on an
@@ -398,7 +470,22 @@ int sg4_cheby_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
   Prop P{};
   P.H = H; P.Mu = nullptr; P.mu = mu; P.ns = ns; P.rows = plan_rows(H);
   P.n = P.rows * 2 * ns; P.st = (hipStream_t)plan_stream(H); P.p = prm;
+  if ((rc = P.choose(2 * ns, (int64_t)prm->nseg * prm->steps_per_seg * (prm->ncoef - 1)))) return rc;
   if ((rc = P.init(false))) return rc;
+  if (P.nm) {
+    double *cur = psi, *other = P.B.p;
+    for (int s = 0; s < prm->nseg; ++s) {
+      if ((rc = P.field(s))) return rc;
+      for (int j = 0; j < prm->steps_per_seg; ++j)
+        if ((rc = P.step_sparse(cur, other, -1.0))) return rc;
+    }
+    if (cur != psi)
+      hipLaunchKernelGGL(k_cb_copy, dim3(blocks_for(P.n)), dim3(256), 0, P.st, cur, psi, P.n);
+    CB_TRY(hipGetLastError());
+    if ((rc = plan_clear_field(H))) return rc;
+    CB_TRY(hipStreamSynchronize(P.st));
+    return SG4_OK;
+  }
   FieldReset reset{H};
   for (int s = 0; s < prm->nseg; ++s) {
     if ((rc = P.field(s))) return rc;
@@ -444,8 +531,14 @@ int sg4_cheby_field_gradient(sg4_plan* H, sg4_plan* Mu, const double* mu, int32_
     sg4_plan* m; void* s;
     ~Restore() { (void)sg4_plan_set_stream(m, s); }
   } restore{Mu, mu_stream};
+  {
+    const int64_t per = (int64_t)prm->nseg * prm->steps_per_seg * (prm->ncoef - 1);
+    bool same = false;
+    if (nmode_order_width(4 * ns) && (rc = plan_is_grid_function(Mu, mu, P.st, &same))) return rc;
+    if (same && (rc = P.choose(2 * ns, 4 * per))) return rc;
+  }
   if ((rc = P.init(true))) return rc;
-  FieldReset reset{H};
+  FieldReset reset{P.nm ? nullptr : H};
   const dim3 b(256);
   // forward, keeping the state at the start of every C-th segment
   std::vector<Buf> ckpt((S + C - 1) / C);
@@ -459,7 +552,7 @@ int sg4_cheby_field_gradient(sg4_plan* H, sg4_plan* Mu, const double* mu, int32_
     }
     if ((rc = P.field(s))) return rc;
     for (int j = 0; j < prm->steps_per_seg; ++j)
-      if ((rc = P.step(cur.p, -1.0))) return rc;
+      if ((rc = P.step(cur, -1.0))) return rc;
   }
   // overlaps and the adjoint seed
   Buf lam, st, dpsi;
@@ -489,7 +582,7 @@ int sg4_cheby_field_gradient(sg4_plan* H, sg4_plan* Mu, const double* mu, int32_
         if (u == s) break;
         if ((rc = P.field(u))) return rc;
         for (int j = 0; j < prm->steps_per_seg; ++j)
-          if ((rc = P.step(st.p, -1.0))) return rc;
+          if ((rc = P.step(st, -1.0))) return rc;
       }
       have = cb;
     }
@@ -502,10 +595,10 @@ int sg4_cheby_field_gradient(sg4_plan* H, sg4_plan* Mu, const double* mu, int32_
     if ((rc = P.cdot(lam.p, dpsi.p, 0, rows, &gr, &gi))) return rc;
     grad[s] = 2.0 * gr;
     for (int j = 0; j < prm->steps_per_seg; ++j)
-      if ((rc = P.step(lam.p, +1.0))) return rc;
+      if ((rc = P.step(lam, +1.0))) return rc;
   }
   reset.H = nullptr;
-  if ((rc = sg4_plan_set_field(H, nullptr, 0.0))) return rc;
+  if ((rc = P.nm ? plan_clear_field(H) : sg4_plan_set_field(H, nullptr, 0.0))) return rc;
   CB_TRY(hipStreamSynchronize(P.st));
   return SG4_OK;
 }
@@ -526,6 +619,9 @@ int sg4_taylor_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
   if ((rc = device_block(H, psi, "psi")) || (mu && (rc = device_block(H, mu, "mu")))) return rc;
   const int64_t rows = plan_rows(H), n = rows * 2 * ns;
   const hipStream_t st = (hipStream_t)plan_stream(H);
+  NModeMat* nm = nullptr;   // H and mu as one sparse matrix (FP64)
+  if ((rc = plan_field_matrix(H, mu, prm->prec, 4 * (int64_t)prm->nseg * prm->steps_per_seg, &nm))) return rc;
+  const double* val = nm ? nm->val.as<double>() : nullptr;
   Buf A, B, Y, part;
   if ((rc = A.alloc(n)) || (rc = B.alloc(n)) || (rc = Y.alloc(n)) ||
       (rc = part.alloc((size_t)NRM_BLOCKS * ns)))
@@ -548,10 +644,14 @@ int sg4_taylor_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
   };
   const dim3 g(blocks_for(rows * ns)), b(256);
   const double ph = -prm->E0 * prm->dt;
-  FieldReset reset{H};
+  FieldReset reset{nm ? nullptr : H};
   int64_t step = 0;
   for (int s = 0; s < prm->nseg; ++s) {
-    if ((rc = sg4_plan_set_field(H, mu, prm->eps[s]))) return rc;
+    if (nm && mu) {
+      val = nm->val_f.as<double>();
+      if ((rc = nmode_set_field(*nm, prm->eps[s], st))) return rc;
+    }
+    if (!nm && (rc = sg4_plan_set_field(H, mu, prm->eps[s]))) return rc;
     for (int j = 0; j < prm->steps_per_seg; ++j, ++step) {
       hipLaunchKernelGGL(k_cb_copy, dim3(blocks_for(n)), b, 0, st, psi, A.p, n);
       double* wk = A.p;
@@ -559,7 +659,8 @@ int sg4_taylor_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
       double m = 0.0;
       int used = 0;
       for (int k = 0; k < prm->npoly; ++k) {
-        if ((rc = sg4_apply_rows(H, 2 * ns, wk, Y.p, prm->prec))) return rc;
+        rc = nm ? nmode_apply(*nm, 2 * ns, wk, Y.p, st, val) : sg4_apply_rows(H, 2 * ns, wk, Y.p, prm->prec);
+        if (rc) return rc;
         hipLaunchKernelGGL(k_tl_order, g, b, 0, st, wk, Y.p, wn, psi, prm->dt / (k + 1), prm->E0, rows, ns);
         if ((rc = max_norm2(wn, &m))) return rc;
         used = k + 1;
@@ -591,7 +692,7 @@ int sg4_taylor_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
     }
   }
   reset.H = nullptr;
-  if ((rc = sg4_plan_set_field(H, nullptr, 0.0))) return rc;
+  if ((rc = nm ? plan_clear_field(H) : sg4_plan_set_field(H, nullptr, 0.0))) return rc;
   CB_TRY(hipStreamSynchronize(st));
   return SG4_OK;
 }

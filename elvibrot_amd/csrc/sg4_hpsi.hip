@@ -79,6 +79,16 @@ __global__ void k_fx_finish(const unsigned long long* __restrict__ fx,
   }
 }
 
+// *flag != 0 when a and b differ somewhere
+__global__ void k_differ(const double* __restrict__ a, const double* __restrict__ b, int64_t n,
+                         unsigned long long* __restrict__ flag) {
+  bool d = false;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    d = d || !(a[i] == b[i]);
+  if (d) *flag = 1ULL;
+}
+
 __global__ void k_to_f32(const double* __restrict__ in, float* __restrict__ out, int64_t n) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
@@ -253,6 +263,11 @@ struct ItemPlan {
                            // (padded Kronecker tiles, six limb products)
 };
 
+// A propagation builds the matrix with the dipole's values once per call
+// (~0.3 ms for small plans, where an apply of the term kernels takes ~25 us):
+// calls of fewer applies keep the term kernels.
+constexpr int64_t NM_MIN_APPLIES = 24;
+
 // Launch configuration of the H.psi kernel; chosen by sg4_plan_autotune.
 struct LaunchCfg {
   int nthreads = 256;          // 256 or 512
@@ -326,10 +341,10 @@ struct sg4_plan {
   std::vector<int64_t> h_toff;
   std::vector<int> inst_L;       // largest |l| of every instance's terms
   double flops_split = 0;        // algorithmic flops per vector of the split path's terms
-  // the field-free H as one sparse matrix (sg4_nmode.hip); field_on: V holds a
-  // field term
+  // H as one sparse matrix (sg4_nmode.hip): the field-free operator and, during
+  // a propagation, the one with the dipole; field_on: V holds a field term
   sg4::NModeTables* nmt = nullptr;
-  sg4::NModeMat nm;
+  sg4::NModeMat nm, nm_field;
   bool field_on = false, nm_off = false;
   bool sparse = true;            // SG4_OPT_SPARSE
   std::set<int> nm_seen;         // block widths applied since the operator was set
@@ -1420,6 +1435,39 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
 using namespace sg4;
 
 namespace sg4 {
+int plan_field_matrix(sg4_plan* P, const double* mu, int prec, int64_t applies, NModeMat** out) {
+  *out = nullptr;
+  if (prec != SG4_PREC_FP64 || !P->nm.valid || !P->sparse || P->nm_off || P->deterministic || !use_split_alg(P) ||
+      applies < NM_MIN_APPLIES)
+    return SG4_OK;
+  if (!mu) { *out = &P->nm; return SG4_OK; }
+  int rc = nmode_build(P->nmt, nmode_in(P), P->d_V0.p ? P->d_V0.as<double>() : P->d_V.as<double>(), mu,
+                       P->nm_field);
+  if (rc) return rc;
+  if (P->nm_field.valid) *out = &P->nm_field;
+  return SG4_OK;
+}
+
+int plan_is_grid_function(const sg4_plan* P, const double* mu, hipStream_t st, bool* same) {
+  *same = false;
+  if (P->type_op != 1 || !P->grouping || !P->split_ok) return SG4_OK;
+  for (double c : P->h_ck)
+    if (c != 0.0) return SG4_OK;
+  DevBuf diff;
+  int rc;
+  if ((rc = diff.alloc(256))) return rc;
+  hipLaunchKernelGGL(k_fx_clear, dim3(1), dim3(64), 0, st, diff.as<unsigned long long>(), (int64_t)1);
+  hipLaunchKernelGGL(k_differ, dim3(grid_blocks(P->sum_nq)), dim3(256), 0, st, P->d_V.as<double>(), mu,
+                     P->sum_nq, diff.as<unsigned long long>());
+  unsigned long long h = 1;
+  HIP_TRY(hipMemcpyAsync(&h, diff.p, sizeof(h), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));
+  *same = h == 0;
+  return SG4_OK;
+}
+
+int plan_clear_field(sg4_plan* P) { return P->field_on ? sg4_plan_set_field(P, nullptr, 0.0) : SG4_OK; }
+
 // The kernels add into their outputs with hardware floating-point atomics
 // compiled with -munsafe-fp-atomics; those are correct on coarse-grained
 // device memory only.  On host (pinned), managed or fine-grained memory the

@@ -57,13 +57,44 @@ void nmode_tables_destroy(NModeTables* t);
 // the matrix small enough to pay.  Synchronises the stream.
 int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double* mu, NModeMat& m);
 
-// hpsi = M psi, nvec vectors in the rows layout
-int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st);
+// hpsi = M psi, nvec vectors in the rows layout (val: other values on M's pattern)
+int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st,
+                const double* val = nullptr);
 // The same to a column-major result, W >= nvec columns at a time: from a
 // column-major block (small blocks, nmode_cols_direct) or from a rows-layout
 // block of W columns.  1: no kernel for this W.
 bool nmode_cols_direct(const NModeMat& m, int W);
 int nmode_apply_cols(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st);
 int nmode_apply_to_cols(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st);
+// val_f = val + eps val_mu
+int nmode_set_field(const NModeMat& m, double eps, hipStream_t st);
+
+// The plan's field-free FP64 operator as such a matrix, with mu's values (mu
+// null: none), for about `applies` applies; *out is null when there is none or
+// it would not pay.  The matrix belongs to the plan and is rebuilt by the next
+// call.
+int plan_field_matrix(sg4_plan* p, const double* mu, int prec, int64_t applies, NModeMat** out);
+// whether the plan is the operator of the grid function mu alone (no kinetic part)
+int plan_is_grid_function(const sg4_plan* p, const double* mu, hipStream_t st, bool* same);
+// takes a field left on the plan back
+int plan_clear_field(sg4_plan* p);
+
+// One Chebyshev order on ns complex states (columns [re | im], 2 ns), or on
+// states and tangents ([re | im | t_re | t_im], 4 ns), in the pass that forms
+// y = H w_k (val: the matrix values of the segment):
+//   z = (y - E0 w_k + [t: mu w_k]) sc,  w_{k+1} = w_{k-1} + 2 r z  (first: r z)
+// with r = sgn i, written over wm; acc = [first: c0 w_0 else acc] + c w_{k+1},
+// of the states in acc, of the tangents in tacc (2 ns columns each).  last:
+// acc times the phase goes to out (and tout) instead.
+struct NModeOrder {
+  const double* val;
+  const double* wk;
+  double* wm;
+  double *acc, *tacc, *out, *tout;
+  double c0, c, E0, sc, sgn, pr, pi;
+  int first, last, ns;
+};
+bool nmode_order_width(int ncol);    // columns the order kernel takes
+int nmode_order(const NModeMat& m, const NModeOrder& a, bool tangent, hipStream_t st);
 
 }  // namespace sg4

@@ -580,6 +580,83 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
   }
 }
 
+// A Chebyshev order (NModeOrder): y and, for tangents, mu w are formed as
+// above (all slices hold the sums after the exchange), the partner column
+// (re <-> im) is NS lanes away.  One launch per order instead of the kinetic
+// rows, the term kernel and the element-wise order (and, with tangents, the
+// dipole operator's two and a copy): 12 uneven instances, 6 steps of 15 orders
+// 35.4 -> 4.9 ms, the adjoint gradient of 3 small ones 8.7 -> 2.1 ms.
+template <int NV, int SL, bool TAN>
+__global__ __launch_bounds__(256) void k_nm_order(const int64_t* __restrict__ ptr,
+                                                  const int32_t* __restrict__ col,
+                                                  const double* __restrict__ mu, NModeOrder a,
+                                                  int64_t rows) {
+  constexpr int W = NV * SL, NS = TAN ? NV / 4 : NV / 2;
+  const int l = threadIdx.x % W, v = l % NV, s = l / NV;
+  const double* __restrict__ val = a.val;
+  const double* __restrict__ x = a.wk;
+  // whole waves stay in the loop: the exchanges need every lane of a row
+  const int64_t r0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) / W;
+  for (int64_t r = r0; r < rows; r += (int64_t)gridDim.x * (256 / W)) {
+    const int64_t e1 = ptr[r + 1];
+    int64_t e = ptr[r] + s;
+    double y0 = 0.0, y1 = 0.0, m0 = 0.0, m1 = 0.0;
+    for (; e + SL < e1; e += 2 * SL) {
+      const double xa = x[(int64_t)col[e] * NV + v], xb = x[(int64_t)col[e + SL] * NV + v];
+      y0 = fma(val[e], xa, y0);
+      y1 = fma(val[e + SL], xb, y1);
+      if constexpr (TAN) {
+        m0 = fma(mu[e], xa, m0);
+        m1 = fma(mu[e + SL], xb, m1);
+      }
+    }
+    if (e < e1) {
+      const double xa = x[(int64_t)col[e] * NV + v];
+      y0 = fma(val[e], xa, y0);
+      if constexpr (TAN) m0 = fma(mu[e], xa, m0);
+    }
+    double y = y0 + y1;
+#pragma unroll
+    for (int o = NV; o < W; o <<= 1) y += __shfl_xor(y, o, 64);
+    const int64_t at = r * NV + v;
+    double z = y - a.E0 * x[at];
+    if constexpr (TAN) {
+      double m = m0 + m1;
+#pragma unroll
+      for (int o = NV; o < W; o <<= 1) m += __shfl_xor(m, o, 64);
+      const double mw = __shfl_xor(m, 2 * NS, 64);
+      if (v >= 2 * NS) z += mw;
+    }
+    z *= a.sc;
+    const double zp = __shfl_xor(z, NS, 64);
+    const double sg = (v & NS) ? a.sgn : -a.sgn;
+    const double wn = a.first ? sg * zp : fma(2.0 * sg, zp, a.wm[at]);
+    double *acc = a.acc, *out = a.out;
+    int64_t ai = at;
+    if constexpr (TAN) {
+      const bool t = v >= 2 * NS;
+      acc = t ? a.tacc : a.acc;
+      out = t ? a.tout : a.out;
+      ai = r * 2 * NS + (t ? v - 2 * NS : v);
+    }
+    const double av = fma(a.c, wn, a.first ? a.c0 * x[at] : acc[ai]);
+    if (a.last) {
+      const double ap = __shfl_xor(av, NS, 64);
+      if (s == 0) out[ai] = (v & NS) ? av * a.pr + ap * a.pi : av * a.pr - ap * a.pi;
+    } else if (s == 0) {
+      a.wm[at] = wn;
+      acc[ai] = av;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_nm_field(const double* __restrict__ val,
+                                                  const double* __restrict__ mu, double eps,
+                                                  double* __restrict__ out, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+    out[i] = fma(eps, mu[i], val[i]);
+}
+
 __global__ void k_nm_zero(int* p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
@@ -993,10 +1070,10 @@ int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double
 
 namespace {
 template <bool COLS, bool IN_COLS>
-int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st) {
+int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st,
+         const double* val) {
   const int64_t* ptr = m.ptr.as<int64_t>();
   const int32_t* col = m.col.as<int32_t>();
-  const double* val = m.val.as<double>();
 #define SG4_SPMM(NV, SL)                                                                              \
   hipLaunchKernelGGL((k_nm_spmm<NV, SL, COLS, IN_COLS>), dim3((unsigned)((m.rows * NV * SL + 255) / 256)),     \
                      dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec)
@@ -1014,12 +1091,12 @@ int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hi
 }
 }  // namespace
 
-int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st) {
-  const int rc = spmm<false, false>(m, nvec, nvec, psi, hpsi, st);
+int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st, const double* val) {
+  if (!val) val = m.val.as<double>();
+  const int rc = spmm<false, false>(m, nvec, nvec, psi, hpsi, st, val);
   if (rc <= 0) return rc;
   hipLaunchKernelGGL(k_nm_spmm_any, dim3((unsigned)std::min<int64_t>((m.rows * nvec + 255) / 256, (int64_t)1 << 20)),
-                     dim3(256), 0, st, m.ptr.as<int64_t>(), m.col.as<int32_t>(), m.val.as<double>(), psi, hpsi,
-                     m.rows, nvec);
+                     dim3(256), 0, st, m.ptr.as<int64_t>(), m.col.as<int32_t>(), val, psi, hpsi, m.rows, nvec);
   NM_TRY(hipGetLastError());
   return SG4_OK;
 }
@@ -1029,11 +1106,45 @@ bool nmode_cols_direct(const NModeMat& m, int W) {
 }
 
 int nmode_apply_cols(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st) {
-  return spmm<true, true>(m, W, nvec, psi, hpsi, st);
+  return spmm<true, true>(m, W, nvec, psi, hpsi, st, m.val.as<double>());
 }
 
 int nmode_apply_to_cols(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st) {
-  return spmm<true, false>(m, W, nvec, psi, hpsi, st);
+  return spmm<true, false>(m, W, nvec, psi, hpsi, st, m.val.as<double>());
+}
+
+bool nmode_order_width(int ncol) { return ncol == 2 || ncol == 4 || ncol == 8 || ncol == 16; }
+
+int nmode_order(const NModeMat& m, const NModeOrder& a, bool tangent, hipStream_t st) {
+  const int64_t* ptr = m.ptr.as<int64_t>();
+  const int32_t* col = m.col.as<int32_t>();
+  const double* mu = m.val_mu.as<double>();
+  auto grid = [&](int w) {
+    return dim3((unsigned)std::min<int64_t>((m.rows * w + 255) / 256, (int64_t)1 << 20));
+  };
+  const int nc = (tangent ? 4 : 2) * a.ns;
+#define SG4_ORDER(NV, SL, TAN) \
+  hipLaunchKernelGGL((k_nm_order<NV, SL, TAN>), grid(NV * SL), dim3(256), 0, st, ptr, col, mu, a, m.rows)
+  if (tangent) {
+    if (nc == 4) SG4_ORDER(4, 4, true);
+    else if (nc == 8) SG4_ORDER(8, 2, true);
+    else SG4_ORDER(16, 1, true);
+  } else {
+    if (nc == 2) SG4_ORDER(2, 8, false);
+    else if (nc == 4) SG4_ORDER(4, 4, false);
+    else if (nc == 8) SG4_ORDER(8, 2, false);
+    else SG4_ORDER(16, 1, false);
+  }
+#undef SG4_ORDER
+  NM_TRY(hipGetLastError());
+  return SG4_OK;
+}
+
+int nmode_set_field(const NModeMat& m, double eps, hipStream_t st) {
+  hipLaunchKernelGGL(k_nm_field, dim3((unsigned)std::min<int64_t>((m.nnz + 255) / 256, 65536)), dim3(256), 0, st,
+                     m.val.as<double>(), m.val_mu.as<double>(), eps, m.val_f.as<double>(), m.nnz);
+  NM_TRY(hipGetLastError());
+  return SG4_OK;
 }
 
 }  // namespace sg4

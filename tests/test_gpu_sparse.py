@@ -146,3 +146,41 @@ def test_field_options_and_graphs_switch_paths(cuda):
     E._capi.check(E.lib().sg4_plan_set_henon_heiles(op._h, 0.2))
     ref = o.hpsi(psi, o.grid_hh(0.2), -0.5 * np.ones(D))
     assert op.sparse_info()[0] and rel(op.apply_host(psi), ref) < TOL
+
+
+@pytest.mark.parametrize("ns", [1, 2, 3, 4])
+@pytest.mark.parametrize("dt,steps", [(0.04, 3), (0.06, 3), (0.1, 4)])
+def test_propagation_on_the_matrix_equals_the_term_kernels(cuda, ns, dt, steps):
+    """Chebyshev steps (odd and even numbers of orders), their field gradient
+    and Taylor steps under a field, on the matrix and by the term kernels, on
+    a batch: the same maps to FP64 rounding over ~100 applies.  Three states
+    have no order kernel and take the term kernels both times."""
+    import torch
+    from elvibrot_amd.propagation import (ChebyshevPropagator, field_gradient_device, propagate_device,
+                                          propagate_taylor_device)
+    op = E.SG4Batch([E.SG4Basis(4, 4), E.SG4Basis(3, 5)], max_nvec=16)
+    assert op.sparse_info()[0]
+    mu = op.grid_dipole()
+    g = torch.Generator(device=cuda).manual_seed(ns)
+    r = lambda: torch.randn(ns, op.nb_ba, device=cuda, dtype=torch.float64, generator=g)
+    psi, target = torch.complex(r(), r()), torch.complex(r(), r())
+    psi, target = (x / torch.linalg.norm(x, dim=1, keepdim=True) for x in (psi, target))
+    eps = [0.05, -0.1, 0.02]
+    blocks = list(zip(op.row0[:-1], op.row0[1:]))
+    prop = ChebyshevPropagator(op, dt, 0.0, 20.0, mu=mu)
+    out = {}
+    for sparse in (True, False):
+        op.set_sparse(sparse)
+        x = propagate_device(prop, psi, eps, steps)
+        J, grad = field_gradient_device(prop, psi, target, eps, steps, checkpoint_every=2, blocks=blocks)
+        t, n = propagate_taylor_device(op, psi, dt, 0.0, 20.0, eps, steps, mu=mu)
+        t0, n0 = propagate_taylor_device(op, psi, dt, 0.0, 20.0, eps, steps)
+        y = torch.empty(op.nb_ba, 2, device=cuda, dtype=torch.float64)
+        op.apply_rows(torch.ones_like(y), y)       # no field is left on the plan
+        out[sparse] = [x, torch.tensor([J]), torch.tensor(grad), t, torch.tensor(n), t0, torch.tensor(n0), y]
+    for a, b in zip(out[True], out[False]):
+        if a.is_floating_point() or a.is_complex():
+            assert (torch.max(torch.abs(a - b)) / torch.max(torch.abs(b))).item() < 1e-11
+        else:
+            assert torch.equal(a, b)
+    print(f"ns={ns} dt={dt}: {prop.nmax} orders", flush=True)
