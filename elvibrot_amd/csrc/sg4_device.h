@@ -509,9 +509,6 @@ struct KGrad {
 // launches.
 __global__ void k_hpsi_t1s_f64(KArgs a, KMats<double> km);
 __global__ void k_hpsi_t1s_f32(KArgs a, KMats<float> km);
-__global__ void k_kin_rows(const int64_t* __restrict__ ptr, const int32_t* __restrict__ col,
-                           const double* __restrict__ val, const double* __restrict__ psi,
-                           double* __restrict__ hpsi, int64_t nrows, int nvec);
 __global__ void k_hpsi_t1_f64(KArgs a, KMats<double> km);
 __global__ void k_hpsi_t1_f32(KArgs a, KMats<float> km);
 __global__ void k_hpsi_t10_f64(KArgs a, KMats10 km);

@@ -50,6 +50,11 @@ struct NModeTables;
 NModeTables* nmode_tables_create(const NModeIn& in);   // null: HIP failure
 void nmode_tables_destroy(NModeTables* t);
 
+// Whether the packed rows are in lexicographic order (the last mode's index
+// fastest), and the kinetic part K alone for such rows.
+bool nmode_rows_ok(const NModeTables* t);
+int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m);
+
 // Builds the matrix of the device grid V and the kinetic part; with mu also
 // the values of the grid function mu as an operator.  m.valid says whether
 // there is one: V (and mu) must be sums of one- and two-mode functions to

@@ -53,7 +53,8 @@ namespace sg4 {
 namespace {
 
 constexpr int NI = SG4_MAX_N;         // 1-D indices per mode
-constexpr int RT = 128;               // rows per workgroup of the row kernels
+constexpr int RL = 4;                // lanes per row and
+constexpr int RT = 256 / RL;          // rows per workgroup of the row kernels
 constexpr double EPS = 2.220446049250313e-16;
 // A grid value may differ from the sum of its parts by the rounding of the
 // parts (each the difference of up to four grid values): 64 eps of the sum of
@@ -235,9 +236,11 @@ __global__ __launch_bounds__(256) void k_nm_verify(const NmDev* insts, const int
   }
 }
 
-// one-mode matrices at every level: c_a T_a + BtW f_a B
+// one-mode matrices at every level: kinetic part c_a T_a, grid part BtW f_a B
+// (KIN | GRID)
+enum { G1_KIN = 1, G1_GRID = 2 };
 __global__ __launch_bounds__(256) void k_nm_g1(const NmDev* insts, const int32_t* work, const double* mats,
-                                               const double* c1, double* g1, int kin) {
+                                               const double* c1, double* g1, int what) {
   const NmDev& I = insts[work[3 * blockIdx.x]];
   const int k = work[3 * blockIdx.x + 1], l = work[3 * blockIdx.x + 2];
   const int n = I.n[k * (I.L + 1) + l], f1 = I.f1off[k * (I.L + 1) + l];
@@ -246,11 +249,11 @@ __global__ __launch_bounds__(256) void k_nm_g1(const NmDev* insts, const int32_t
   const double* Bt = mats + md.BtW;
   const double* T = I.T + I.toff[k * (I.L + 1) + l];
   double* g = g1 + I.g1off[k * (I.L + 1) + l];
-  const double v0 = c1[I.c1base], c = kin ? I.ck[k] : 0.0;
+  const double v0 = c1[I.c1base], c = (what & G1_KIN) ? I.ck[k] : 0.0;
   for (int e = threadIdx.x; e < n * n; e += 256) {
     const int i = e / n, j = e % n;
     double s = 0.0, m = 0.0;
-    if (f1 >= 0 && n > 1)
+    if (f1 >= 0 && n > 1 && (what & G1_GRID))
       for (int q = 0; q < n; ++q) {
         const double w = Bt[i * n + q] * B[q * n + j], v = c1[f1 + q];
         s = fma(w, v - v0, s);
@@ -261,7 +264,8 @@ __global__ __launch_bounds__(256) void k_nm_g1(const NmDev* insts, const int32_t
   }
 }
 
-// two-mode matrices E(m) of a pair over the pair indices of level <= m
+// two-mode matrices E(m) of a pair over the pair indices of level <= m; eight
+// lanes per element share the level pairs (12 instances: 248 us with one)
 __global__ __launch_bounds__(256) void k_nm_e2(const NmDev* insts, const EWork* work, const double* mats,
                                                const double* c1, const double* f2, double* E) {
   const EWork w = work[blockIdx.x];
@@ -270,38 +274,44 @@ __global__ __launch_bounds__(256) void k_nm_e2(const NmDev* insts, const EWork* 
   const int a = I.pa[p], b = I.pb[p], S = I.s2n[p * L1 + m];
   const uint16_t* lst = I.s2 + I.s2off[p];
   const double v0 = c1[I.c1base];
-  for (int e = blockIdx.y * 256 + threadIdx.x; e < S * S; e += gridDim.y * 256) {
+  const int sub = threadIdx.x & 7;
+  for (int e = blockIdx.y * 32 + (threadIdx.x >> 3); e < S * S; e += gridDim.y * 32) {
     const int r = lst[e / S], c = lst[e % S];
     const int ia = r & 255, ib = r >> 8, ja = c & 255, jb = c >> 8;
-    const int la0 = max(I.lam[a * NI + ia], I.lam[a * NI + ja]);
-    const int lb0 = max(I.lam[b * NI + ib], I.lam[b * NI + jb]);
+    const int la0 = max(1, max(I.lam[a * NI + ia], I.lam[a * NI + ja]));
+    const int lb0 = max(1, max(I.lam[b * NI + ib], I.lam[b * NI + jb]));
+    // level pairs l_a + l_b = m (n0 of them), then m - 1 with the minus sign
+    const int n0 = max(0, m - lb0 - la0 + 1), n1 = max(0, n0 - 1);
     double sum = 0.0, mag = 0.0;
-    for (int u = 0; u < 2; ++u) {
-      for (int la = max(la0, 1); la <= m - u - max(lb0, 1); ++la) {
-        const int lb = m - u - la;
-        const int off = I.f2off[(p * L1 + la) * L1 + lb];
-        const int fa = I.f1off[a * L1 + la], fb = I.f1off[b * L1 + lb];
-        if (off < 0 || fa < 0 || fb < 0) continue;   // levels that no row needs
-        const int na = I.n[a * L1 + la], nb = I.n[b * L1 + lb];
-        const MatDev& A = I.md[a * I.L1 + la];
-        const MatDev& Q = I.md[b * I.L1 + lb];
-        double t = 0.0;
-        for (int q = 0; q < nb; ++q) {
-          const double wb = mats[Q.BtW + ib * nb + q] * mats[Q.B + q * nb + jb];
-          double s = 0.0, g = 0.0;
-          for (int o = 0; o < na; ++o) {
-            const double wa = mats[A.BtW + ia * na + o] * mats[A.B + o * na + ja];
-            const double f = f2[off + o + na * q];
-            s = fma(wa, f, s);
-            g = fma(fabs(wa), fabs(f) + fabs(c1[fa + o]) + fabs(c1[fb + q]) + fabs(v0), g);
-          }
-          t = fma(wb, s, t);
-          mag = fma(fabs(wb), g, mag);
+    for (int x = sub; x < n0 + n1; x += 8) {
+      const int u = x >= n0, la = la0 + (u ? x - n0 : x), lb = m - u - la;
+      const int off = I.f2off[(p * L1 + la) * L1 + lb];
+      const int fa = I.f1off[a * L1 + la], fb = I.f1off[b * L1 + lb];
+      if (off < 0 || fa < 0 || fb < 0) continue;   // levels that no row needs
+      const int na = I.n[a * L1 + la], nb = I.n[b * L1 + lb];
+      const MatDev& A = I.md[a * I.L1 + la];
+      const MatDev& Q = I.md[b * I.L1 + lb];
+      double t = 0.0;
+      for (int q = 0; q < nb; ++q) {
+        const double wb = mats[Q.BtW + ib * nb + q] * mats[Q.B + q * nb + jb];
+        double s = 0.0, g = 0.0;
+        for (int o = 0; o < na; ++o) {
+          const double wa = mats[A.BtW + ia * na + o] * mats[A.B + o * na + ja];
+          const double f = f2[off + o + na * q];
+          s = fma(wa, f, s);
+          g = fma(fabs(wa), fabs(f) + fabs(c1[fa + o]) + fabs(c1[fb + q]) + fabs(v0), g);
         }
-        sum += u ? -t : t;
+        t = fma(wb, s, t);
+        mag = fma(fabs(wb), g, mag);
       }
+      sum += u ? -t : t;
     }
-    E[w.off + e] = fabs(sum) > TOL_M * mag ? sum : 0.0;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      sum += __shfl_xor(sum, o, 64);
+      mag += __shfl_xor(mag, o, 64);
+    }
+    if (sub == 0) E[w.off + e] = fabs(sum) > TOL_M * mag ? sum : 0.0;
   }
 }
 
@@ -318,43 +328,85 @@ struct NmPairs {
   const int32_t* nzoff;
   const int32_t* adj;         // pairs holding mode k at adjoff[inst * 33 + k]
   const int32_t* adjoff;
+  // row ri of a pair's matrices at level m: the ecnt[croff + ri] columns at
+  // elist[loff + ri S ..] where both indices change and V or mu is nonzero
+  const int64_t* loff;        // [global pair * eld + m]
+  const int64_t* croff;
+  uint16_t* elist;
+  int32_t* ecnt;
   int eld;
 };
 
-// Entries of packed row r: counted (FILL = false) or written.  One thread per
-// row; its mode indices, levels and rank prefixes sit in LDS.
+// the column lists of NmPairs, one thread per row of a pair's matrix
+__global__ __launch_bounds__(64) void k_nm_elist(const NmDev* __restrict__ insts, const EWork* work, NmSet sv,
+                                                 NmSet sm, NmPairs pr) {
+  const EWork w = work[blockIdx.x];
+  const NmDev& I = insts[w.inst];
+  const int S = I.s2n[w.pair * (I.L + 1) + w.m];
+  const uint16_t* lst = I.s2 + I.s2off[w.pair];
+  const int64_t g = (int64_t)(I.pair0 + w.pair) * pr.eld + w.m;
+  const int64_t ov = sv.eoff[g], om = sm.eoff ? sm.eoff[g] : -1;
+  for (int r = blockIdx.y * 64 + threadIdx.x; r < S; r += gridDim.y * 64) {
+    uint16_t* out = pr.elist + pr.loff[g] + (int64_t)r * S;
+    int n = 0;
+    for (int c = 0; c < S; ++c) {
+      if ((lst[c] & 255) == (lst[r] & 255) || lst[c] >> 8 == lst[r] >> 8) continue;
+      const bool nz = (ov >= 0 && sv.E[ov + (int64_t)r * S + c] != 0.0) ||
+                      (om >= 0 && sm.E[om + (int64_t)r * S + c] != 0.0);
+      if (nz) out[n++] = (uint16_t)c;
+    }
+    pr.ecnt[pr.croff[g] + r] = n;
+  }
+}
+
+// Entries of a packed row: counted (FILL = false) or written.  RL lanes per
+// row take its tasks (one mode changed: D of them; a pair changed: one per
+// nonzero pair) in rounds, a task's entries going after those of the tasks
+// before it; the row's mode indices, levels and rank prefixes sit in LDS.  The
+// chains of dependent table reads bound it; the propagation of 12 instances
+// (which builds once) takes 4.01 / 3.88 / 3.89 / 3.94 / 4.27 ms with 1 / 2 / 4 / 8 /
+// 16 lanes, setting a 6D L=6 operator 1.60 / 1.48 / 1.41 / 1.34 / 1.38 ms.  10D L=8:
+// the two passes take 0.7 and 1.7 ms.  A workgroup's rows belong to one instance (its first workgroup: blk0), whose
+// tables are then addressed by scalars.
 template <bool FILL, bool MU>
-__global__ __launch_bounds__(RT) void k_nm_rows(const NmDev* insts, const int64_t* row0, int ninst,
-                                                int64_t nrows, NmSet sv, NmSet sm, NmPairs pr, int Dmax,
-                                                int32_t* cnt, const int64_t* ptr, int32_t* col, double* val,
-                                                double* valm) {
+__global__ __launch_bounds__(256) void k_nm_rows(const NmDev* __restrict__ insts, const int64_t* __restrict__ blk0,
+                                                 int ninst, NmSet sv, NmSet sm, NmPairs pr, int Dmax,
+                                                 int32_t* cnt, const int64_t* ptr, int32_t* col, double* val,
+                                                 double* valm) {
   extern __shared__ char sh[];
-  int32_t* pre = (int32_t*)sh;                     // [k][thread] rank contribution before mode k
+  int32_t* pre = (int32_t*)sh;                     // [k][row] rank contribution before mode k
   uint8_t* dg = (uint8_t*)(pre + Dmax * RT);       // mode indices
   uint8_t* lm = dg + Dmax * RT;                    // their levels
   uint8_t* bud = lm + Dmax * RT;                   // level budget left before mode k
-  const int tid = threadIdx.x;
-  const int64_t row = (int64_t)blockIdx.x * RT + tid;
-  if (row >= nrows) return;                        // no barriers below
-  const int ii = find_inst(row0, ninst, row);
+  __shared__ int tots[RT];
+  const int sub = threadIdx.x % RL, tid = threadIdx.x / RL;
+  const int ii = __builtin_amdgcn_readfirstlane(find_inst(blk0, ninst, blockIdx.x));
   const NmDev& I = insts[ii];
+  const int64_t lrow = ((int64_t)blockIdx.x - blk0[ii]) * RT + tid, row = I.row0 + lrow;
+  const bool on = lrow < I.nrows;
   const int D = I.D, L = I.L, LB = I.LB, L1 = L + 1;
-  int32_t left = (int32_t)(row - I.row0), done = 0;
-  int b = LB, tot = 0;
-  for (int k = 0; k < D; ++k) {
-    const int32_t* p = I.pre + (k * (LB + 1) + b) * (NI + 1);
-    int i = 0;
-    while (i + 1 < NI && I.lam[k * NI + i + 1] <= b && p[i + 1] <= left) ++i;
-    const int li = I.lam[k * NI + i];
-    pre[k * RT + tid] = done;
-    dg[k * RT + tid] = (uint8_t)i;
-    lm[k * RT + tid] = (uint8_t)li;
-    bud[k * RT + tid] = (uint8_t)b;
-    left -= p[i];
-    done += p[i];
-    b -= li;
-    tot += li;
+  if (on && sub == 0) {
+    int32_t left = (int32_t)lrow, done = 0;
+    int b = LB, tot = 0;
+    for (int k = 0; k < D; ++k) {
+      const int32_t* p = I.pre + (k * (LB + 1) + b) * (NI + 1);
+      int i = 0;
+      while (i + 1 < NI && I.lam[k * NI + i + 1] <= b && p[i + 1] <= left) ++i;
+      const int li = I.lam[k * NI + i];
+      pre[k * RT + tid] = done;
+      dg[k * RT + tid] = (uint8_t)i;
+      lm[k * RT + tid] = (uint8_t)li;
+      bud[k * RT + tid] = (uint8_t)b;
+      left -= p[i];
+      done += p[i];
+      b -= li;
+      tot += li;
+    }
+    tots[tid] = tot;
   }
+  __syncthreads();
+  if (!on) return;                                 // no barriers below; whole rows leave
+  const int tot = tots[tid];
   // rank with the index of mode x replaced by ix (and of mode y > x by iy)
   auto rank2 = [&](int x, int ix, int y, int iy) {
     int bb = bud[x * RT + tid];
@@ -368,86 +420,113 @@ __global__ __launch_bounds__(RT) void k_nm_rows(const NmDev* insts, const int64_
     return (int32_t)(r + I.row0);
   };
   auto epos = [&](int p, int ia, int ib) {
-    const int bm = I.pb[p];
-    return (int)I.pos[I.posoff[p] + ia * I.n[bm * L1 + L] + ib];
+    return (int)I.pos[I.posoff[p] + ia * I.n[I.pb[p] * L1 + L] + ib];
   };
   // element of a pair's matrix at its level m, rows (ia, ib) -> (ja, jb)
   auto eget = [&](const NmSet& s, int p, int m, int ri, int ci) {
     const int64_t o = s.eoff[(int64_t)(I.pair0 + p) * pr.eld + m];
     return o < 0 ? 0.0 : s.E[o + (int64_t)ri * I.s2n[p * L1 + m] + ci];
   };
-  int64_t at = FILL ? ptr[row] : 0;
-  int n = 1;
-  auto put = [&](int32_t c, double v, double vm) {
-    if constexpr (FILL) {
-      col[at] = c;
-      val[at] = v;
-      if constexpr (MU) valm[at] = vm;
-      ++at;
-    }
-    ++n;
-  };
   const int32_t* nz = pr.nz + pr.nzoff[ii];
-  const int nnz = pr.nzoff[ii + 1] - pr.nzoff[ii];
-  if constexpr (FILL) {   // the diagonal
-    double v = sv.c1[I.c1base], vm = MU ? sm.c1[I.c1base] : 0.0;
-    for (int k = 0; k < D; ++k) {
-      const int i = dg[k * RT + tid], ma = L - (tot - lm[k * RT + tid]);
-      const int o = I.g1off[k * L1 + ma] + i * (I.n[k * L1 + ma] + 1);
-      v += sv.g1[o];
-      if constexpr (MU) vm += sm.g1[o];
-    }
-    for (int z = 0; z < nnz; ++z) {
-      const int p = nz[z], a = I.pa[p], bq = I.pb[p];
-      const int m = L - (tot - lm[a * RT + tid] - lm[bq * RT + tid]);
-      const int e = epos(p, dg[a * RT + tid], dg[bq * RT + tid]);
-      v += eget(sv, p, m, e, e);
-      if constexpr (MU) vm += eget(sm, p, m, e, e);
-    }
-    put((int32_t)row, v, vm);
-    n = 1;
-  }
-  for (int a = 0; a < D; ++a) {   // one index changed
-    const int ia = dg[a * RT + tid], la = lm[a * RT + tid], ma = L - (tot - la);
-    const int na = I.n[a * L1 + ma], room = LB - (tot - la);
-    const double* g = sv.g1 + I.g1off[a * L1 + ma] + ia * na;
-    const double* gm = MU ? sm.g1 + I.g1off[a * L1 + ma] + ia * na : nullptr;
-    const int q0 = pr.adjoff[ii * 33 + a], q1 = pr.adjoff[ii * 33 + a + 1];
-    for (int j = 0; j < na; ++j) {
-      if (j == ia || I.lam[a * NI + j] > room) continue;
-      double v = g[j], vm = MU ? gm[j] : 0.0;
-      for (int q = q0; q < q1; ++q) {
-        const int p = pr.adj[q];
-        const int o = I.pa[p] == a ? I.pb[p] : I.pa[p], io = dg[o * RT + tid];
-        const int m = L - (tot - la - lm[o * RT + tid]);
-        const bool fst = I.pa[p] == a;
-        const int ri = fst ? epos(p, ia, io) : epos(p, io, ia);
-        const int ci = fst ? epos(p, j, io) : epos(p, io, j);
-        v += eget(sv, p, m, ri, ci);
-        if constexpr (MU) vm += eget(sm, p, m, ri, ci);
+  const int ntask = D + pr.nzoff[ii + 1] - pr.nzoff[ii];
+  // the entries of a task: put(x, ix, y, iy, v, vm) for each
+  auto each = [&](int task, auto&& put) {
+    if (task < D) {
+      const int a = task, ia = dg[a * RT + tid], la = lm[a * RT + tid], ma = L - (tot - la);
+      const int na = I.n[a * L1 + ma], room = LB - (tot - la);
+      const double* g = sv.g1 + I.g1off[a * L1 + ma] + ia * na;
+      const double* gm = MU ? sm.g1 + I.g1off[a * L1 + ma] + ia * na : nullptr;
+      const int q0 = pr.adjoff[ii * 33 + a], q1 = pr.adjoff[ii * 33 + a + 1];
+      for (int j = 0; j < na; ++j) {
+        if (j == ia || I.lam[a * NI + j] > room) continue;
+        double v = g[j], vm = MU ? gm[j] : 0.0;
+        for (int q = q0; q < q1; ++q) {
+          const int p = pr.adj[q];
+          const bool fst = I.pa[p] == a;
+          const int o = fst ? I.pb[p] : I.pa[p], io = dg[o * RT + tid];
+          const int m = L - (tot - la - lm[o * RT + tid]);
+          const int ri = fst ? epos(p, ia, io) : epos(p, io, ia);
+          const int ci = fst ? epos(p, j, io) : epos(p, io, j);
+          v += eget(sv, p, m, ri, ci);
+          if constexpr (MU) vm += eget(sm, p, m, ri, ci);
+        }
+        if (v != 0.0 || vm != 0.0) put(a, j, -1, 0, v, vm);
       }
-      if (v != 0.0 || vm != 0.0) put(FILL ? rank2(a, j, -1, 0) : 0, v, vm);
+    } else {
+      const int p = nz[task - D], a = I.pa[p], bq = I.pb[p];
+      const int ia = dg[a * RT + tid], ib = dg[bq * RT + tid];
+      const int lab = lm[a * RT + tid] + lm[bq * RT + tid];
+      const int m = L - (tot - lab), room = LB - (tot - lab), S = I.s2n[p * L1 + m];
+      const uint16_t* lst = I.s2 + I.s2off[p];
+      const int ri = epos(p, ia, ib);
+      const int64_t ov = sv.eoff[(int64_t)(I.pair0 + p) * pr.eld + m];
+      const int64_t om = MU ? sm.eoff[(int64_t)(I.pair0 + p) * pr.eld + m] : -1;
+      const int64_t g = (int64_t)(I.pair0 + p) * pr.eld + m;
+      const uint16_t* el = pr.elist + pr.loff[g] + (int64_t)ri * S;
+      const int ne = pr.ecnt[pr.croff[g] + ri];
+      for (int x = 0; x < ne; ++x) {
+        const int c = el[x], ja = lst[c] & 255, jb = lst[c] >> 8;
+        if (room < m && I.lam[a * NI + ja] + I.lam[bq * NI + jb] > room) continue;   // LB < L
+        const double v = ov < 0 ? 0.0 : sv.E[ov + (int64_t)ri * S + c];
+        const double vm = om < 0 ? 0.0 : sm.E[om + (int64_t)ri * S + c];
+        put(a, ja, bq, jb, v, vm);
+      }
+    }
+  };
+  if constexpr (!FILL) {
+    int n = 0;
+    for (int task = sub; task < ntask; task += RL)
+      each(task, [&](int, int, int, int, double, double) { ++n; });
+    for (int o = 1; o < RL; o <<= 1) n += __shfl_xor(n, o, 64);
+    if (sub == 0) cnt[row] = n + 1;
+  } else {
+    int64_t at = ptr[row];
+    double dv = 0.0, dm = 0.0;                     // the diagonal, first in its row
+    for (int task = sub; task < ntask; task += RL) {
+      if (task < D) {
+        const int i = dg[task * RT + tid], ma = L - (tot - lm[task * RT + tid]);
+        const int o = I.g1off[task * L1 + ma] + i * (I.n[task * L1 + ma] + 1);
+        dv += sv.g1[o];
+        if constexpr (MU) dm += sm.g1[o];
+      } else {
+        const int p = nz[task - D], a = I.pa[p], bq = I.pb[p];
+        const int m = L - (tot - lm[a * RT + tid] - lm[bq * RT + tid]);
+        const int e = epos(p, dg[a * RT + tid], dg[bq * RT + tid]);
+        dv += eget(sv, p, m, e, e);
+        if constexpr (MU) dm += eget(sm, p, m, e, e);
+      }
+    }
+    for (int o = 1; o < RL; o <<= 1) {
+      dv += __shfl_xor(dv, o, 64);
+      if constexpr (MU) dm += __shfl_xor(dm, o, 64);
+    }
+    if (sub == 0) {
+      col[at] = (int32_t)row;
+      val[at] = dv + sv.c1[I.c1base];
+      if constexpr (MU) valm[at] = dm + sm.c1[I.c1base];
+    }
+    ++at;
+    for (int base = 0; base < ntask; base += RL) {   // the same number of rounds in every lane of a row
+      const int task = base + sub;
+      int n = 0;
+      if (task < ntask) each(task, [&](int, int, int, int, double, double) { ++n; });
+      int before = 0, all = n;
+      for (int o = 1; o < RL; o <<= 1) {
+        const int y = __shfl_up(all, o, RL);
+        if (sub >= o) all += y;
+      }
+      before = all - n;
+      int64_t w = at + before;
+      if (n)
+        each(task, [&](int x, int ix, int y, int iy, double v, double vm) {
+          col[w] = rank2(x, ix, y, iy);
+          val[w] = v;
+          if constexpr (MU) valm[w] = vm;
+          ++w;
+        });
+      at += __shfl(all, RL - 1, RL);
     }
   }
-  for (int z = 0; z < nnz; ++z) {   // both indices of a pair changed
-    const int p = nz[z], a = I.pa[p], bq = I.pb[p];
-    const int ia = dg[a * RT + tid], ib = dg[bq * RT + tid];
-    const int lab = lm[a * RT + tid] + lm[bq * RT + tid];
-    const int m = L - (tot - lab), room = LB - (tot - lab), S = I.s2n[p * L1 + m];
-    const uint16_t* lst = I.s2 + I.s2off[p];
-    const int ri = epos(p, ia, ib);
-    const int64_t ov = sv.eoff[(int64_t)(I.pair0 + p) * pr.eld + m];
-    const int64_t om = MU ? sm.eoff[(int64_t)(I.pair0 + p) * pr.eld + m] : -1;
-    for (int c = 0; c < S; ++c) {
-      const int ja = lst[c] & 255, jb = lst[c] >> 8;
-      if (ja == ia || jb == ib) continue;
-      if (I.lam[a * NI + ja] + I.lam[bq * NI + jb] > room) continue;
-      const double v = ov < 0 ? 0.0 : sv.E[ov + (int64_t)ri * S + c];
-      const double vm = om < 0 ? 0.0 : sm.E[om + (int64_t)ri * S + c];
-      if (v != 0.0 || vm != 0.0) put(FILL ? rank2(a, ja, bq, jb) : 0, v, vm);
-    }
-  }
-  if constexpr (!FILL) cnt[row] = n;
 }
 
 // row pointers from the row counts: sums of 1024 rows, their scan, the rows
@@ -585,7 +664,8 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
 // (re <-> im) is NS lanes away.  One launch per order instead of the kinetic
 // rows, the term kernel and the element-wise order (and, with tangents, the
 // dipole operator's two and a copy): 12 uneven instances, 6 steps of 15 orders
-// 35.4 -> 4.9 ms, the adjoint gradient of 3 small ones 8.7 -> 2.1 ms.
+// 35.4 -> 3.9 ms (30 us an order), the adjoint gradient of 3 small ones 8.6 ->
+// 1.9 ms (4.5 us an order: launch latency).
 template <int NV, int SL, bool TAN>
 __global__ __launch_bounds__(256) void k_nm_order(const int64_t* __restrict__ ptr,
                                                   const int32_t* __restrict__ col,
@@ -686,13 +766,16 @@ int ensure(DevBuf& d, size_t bytes) { return d.n >= bytes && d.p ? SG4_OK : d.al
 }  // namespace
 
 struct NModeTables {
-  bool ok = false;
+  bool rows_ok = false;            // the packed rows are in lexicographic order
+  bool cuts = true, ok = false;    // V can be cut through middle points; both
   DevBuf blob, insts, work, ck;    // tables; NmDev of every instance; build workspace; c_k
-  DevBuf e_v, e_mu, lists;
+  DevBuf e_v, e_mu, elist, lists;
   std::vector<NmDev> dev;          // host copies (device pointers inside)
-  size_t o_term0 = 0, o_row0 = 0, o_cut1 = 0, o_cut2 = 0, o_g1work = 0;
+  size_t o_term0 = 0, o_blk0 = 0, o_cut1 = 0, o_cut2 = 0, o_g1work = 0, o_none = 0;
   int ncut1 = 0, ncut2 = 0, ng1 = 0, npairs = 0, Lmax = 0, Dmax = 0;
-  int64_t nc1 = 0, nf2 = 0, ng1v = 0, nterms = 0;
+  int64_t nc1 = 0, nf2 = 0, ng1v = 0, nterms = 0, nblk = 0;
+  bool v_ready = false;            // V's part of work, e_v and v_flags hold the plan's operator
+  std::vector<int> v_flags;
   std::vector<int32_t> pair_inst, pair_s2n;   // per global pair: instance; [pair * (Lmax+1) + m]
 };
 
@@ -712,7 +795,7 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
   std::vector<Off> off(ni);
   std::vector<Cut> cut1, cut2;
   std::vector<int32_t> g1work;
-  std::vector<int64_t> term0, row0;
+  std::vector<int64_t> term0, blk0;
   for (int x = 0; x < ni; ++x) {
     const NModeInst& I = in.inst[x];
     NmDev& d = t->dev[x];
@@ -724,10 +807,9 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
     for (int k = 0; k < D; ++k)
       for (int l = 0; l <= L; ++l) {
         n[k * L1 + l] = nn(k, l);
+        if (n[k * L1 + l] > NI || (l && n[k * L1 + l] < n[k * L1 + l - 1])) return t.release();
         // the middle point is shared by the rules of a mode when they are odd
-        if (n[k * L1 + l] % 2 == 0 || n[k * L1 + l] > NI || (l && n[k * L1 + l] < n[k * L1 + l - 1]) ||
-            n[k * L1] != 1)
-          return t.release();
+        if (n[k * L1 + l] % 2 == 0 || n[k * L1] != 1) t->cuts = false;
       }
     std::vector<uint8_t> lam(D * NI, 255);
     for (int k = 0; k < D; ++k)
@@ -757,11 +839,11 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
       }
     // cuts: for every (mode, level) and (pair, levels >= 1) the first term that
     // has them; the other modes at their middle points
-    const int np = D * (D - 1) / 2;
+    const int np = t->cuts ? D * (D - 1) / 2 : 0;
     d.npair = np;
     d.pair0 = t->npairs;
     std::vector<uint8_t> pa(np), pb(np);
-    for (int a = 0, p = 0; a < D; ++a)
+    for (int a = 0, p = 0; a < D && np; ++a)
       for (int b = a + 1; b < D; ++b, ++p) { pa[p] = (uint8_t)a; pb[p] = (uint8_t)b; }
     std::vector<int32_t> f1off(D * L1, -1), f2off((size_t)np * L1 * L1, -1);
     d.c1base = t->nc1;
@@ -770,7 +852,7 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
     std::vector<int64_t> stride(D);
     bool centre = false;
     std::vector<Cut> c2;
-    for (int64_t tt = 0; tt < I.nterms; ++tt) {
+    for (int64_t tt = 0; tt < I.nterms && t->cuts; ++tt) {
       const int32_t* lev = &(*in.levels)[I.lev0 + tt * D];
       act.clear();
       int64_t s = 1, mid = (*in.qoff)[I.term0 + tt];
@@ -876,7 +958,8 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
     }
     if (t->ng1v > INT32_MAX) return t.release();
     term0.push_back(I.term0);
-    row0.push_back(I.row0);
+    blk0.push_back(t->nblk);
+    t->nblk += (I.nb_ba + RT - 1) / RT;
     Off& o = off[x];
     o.n = blob.add(n); o.lam = blob.add(lam); o.pre = blob.add(pre); o.f1off = blob.add(f1off);
     o.f2off = blob.add(f2off); o.s2n = blob.add(s2n); o.s2off = blob.add(s2off); o.s2 = blob.add(s2);
@@ -890,10 +973,11 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
   t->ncut2 = (int)cut2.size();
   t->ng1 = (int)g1work.size() / 3;
   t->o_term0 = blob.add(term0);
-  t->o_row0 = blob.add(row0);
+  t->o_blk0 = blob.add(blk0);
   t->o_cut1 = blob.add(cut1);
   t->o_cut2 = blob.add(cut2);
   t->o_g1work = blob.add(g1work);
+  t->o_none = blob.add(std::vector<int32_t>((size_t)ni * 33 + 33, 0));   // no pairs
   if (upload(blob, t->blob, in.stream) != SG4_OK || t->ck.alloc(sizeof(double) * in.ck->size()) != SG4_OK)
     return nullptr;
   char* B = t->blob.as<char>();
@@ -926,41 +1010,117 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
     set_error("HIP error while checking the packed rows");
     return nullptr;
   }
-  t->ok = h == 0;
+  t->rows_ok = h == 0;
+  t->ok = t->rows_ok && t->cuts;
   return t.release();
+}
+
+namespace {
+size_t up(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Build workspace: for V and for mu the cuts, two-mode functions, one-mode
+// matrices and pair flags (then the verdict); the row counts and their scan.
+struct Work {
+  double *c1[2], *f2[2], *g1[2];
+  int* flag[2];
+  int32_t* cnt;
+  int64_t* part;
+  int npart;
+  int layout(NModeTables* t, int64_t rows) {
+    npart = (int)((rows + 1023) / 1024);
+    const size_t b_c1 = up(8 * t->nc1), b_f2 = up(8 * (t->nf2 + 1)), b_g1 = up(8 * t->ng1v),
+                 b_fl = up(4 * ((size_t)t->npairs + 1)), b_set = b_c1 + b_f2 + b_g1 + b_fl,
+                 b_cnt = up(4 * rows), b_part = up(8 * ((size_t)npart + 1));
+    if (int rc = ensure(t->work, 2 * b_set + b_cnt + b_part)) return rc;
+    char* W = t->work.as<char>();
+    for (int s = 0; s < 2; ++s) {
+      char* w = W + s * b_set;
+      c1[s] = (double*)w;
+      f2[s] = (double*)(w + b_c1);
+      g1[s] = (double*)(w + b_c1 + b_f2);
+      flag[s] = (int*)(w + b_c1 + b_f2 + b_g1);
+    }
+    cnt = (int32_t*)(W + 2 * b_set);
+    part = (int64_t*)(W + 2 * b_set + b_cnt);
+    return SG4_OK;
+  }
+};
+
+// the row counts' sum (synchronises) and the row pointers
+int scan_rows(const Work& w, int64_t rows, hipStream_t st, int64_t* nnz) {
+  hipLaunchKernelGGL(k_nm_sum, dim3(w.npart), dim3(256), 0, st, w.cnt, rows, w.part);
+  hipLaunchKernelGGL(k_nm_scan_part, dim3(1), dim3(1024), 0, st, w.part, w.npart);
+  NM_TRY(hipMemcpyAsync(nnz, w.part + w.npart, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  NM_TRY(hipGetLastError());
+  NM_TRY(hipStreamSynchronize(st));
+  return SG4_OK;
+}
+}  // namespace
+
+bool nmode_rows_ok(const NModeTables* t) { return t && t->rows_ok; }
+
+int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m) {
+  m.valid = false;
+  const hipStream_t st = in.stream;
+  const int64_t rows = in.rows;
+  Work w;
+  int rc;
+  if ((rc = w.layout(t, rows))) return rc;
+  char* B = t->blob.as<char>();
+  const NmDev* insts = t->insts.as<NmDev>();
+  t->v_ready = false;
+  NM_TRY(hipMemcpyAsync(t->ck.p, in.ck->data(), sizeof(double) * in.ck->size(), hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_nm_zero, dim3(8), dim3(256), 0, st, (int*)w.c1[1], (int)(2 * t->nc1));   // V0 = 0
+  hipLaunchKernelGGL(k_nm_g1, dim3(t->ng1), dim3(256), 0, st, insts, (const int32_t*)(B + t->o_g1work),
+                     in.d_mats, w.c1[1], w.g1[1], G1_KIN);
+  const NmSet set{w.c1[1], w.g1[1], nullptr, nullptr};
+  const int32_t* none = (const int32_t*)(B + t->o_none);
+  const NmPairs pr{none, none, none, none, nullptr, nullptr, nullptr, nullptr, 0};
+  const dim3 rg((unsigned)t->nblk);
+  const size_t rl = (size_t)t->Dmax * RT * 7;
+  const int64_t* blk0 = (const int64_t*)(B + t->o_blk0);
+  const int ni = (int)in.inst.size();
+  hipLaunchKernelGGL((k_nm_rows<false, false>), rg, dim3(256), rl, st, insts, blk0, ni, set, set, pr, t->Dmax,
+                     w.cnt, nullptr, nullptr, nullptr, nullptr);
+  int64_t nnz = 0;
+  if ((rc = scan_rows(w, rows, st, &nnz))) return rc;
+  if ((rc = ensure(m.ptr, 8 * (rows + 1))) || (rc = ensure(m.col, 4 * nnz)) || (rc = ensure(m.val, 8 * nnz)))
+    return rc;
+  hipLaunchKernelGGL(k_nm_ptr, dim3(w.npart), dim3(1024), 0, st, w.cnt, rows, w.part, m.ptr.as<int64_t>());
+  hipLaunchKernelGGL((k_nm_rows<true, false>), rg, dim3(256), rl, st, insts, blk0, ni, set, set, pr, t->Dmax,
+                     w.cnt, m.ptr.as<int64_t>(), m.col.as<int32_t>(), m.val.as<double>(), nullptr);
+  NM_TRY(hipGetLastError());
+  m.rows = rows;
+  m.nnz = nnz;
+  m.valid = true;
+  return SG4_OK;
 }
 
 int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double* mu, NModeMat& m) {
   m.valid = false;
   if (!t || !t->ok) return SG4_OK;
+  const bool have_v = mu && t->v_ready;   // V's functions and matrices, made when the operator was set
+  if (!have_v) t->v_ready = false;
   const hipStream_t st = in.stream;
   const int ni = (int)in.inst.size(), nset = mu ? 2 : 1, eld = t->Lmax + 1;
   const int64_t rows = in.rows;
-  const int npart = (int)((rows + 1023) / 1024);
   int rc;
-  // workspace: cuts, functions, one-mode matrices, pair flags of V (and mu), row counts, scan
-  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t b_c1 = up(8 * t->nc1), b_f2 = up(8 * (t->nf2 + 1)), b_g1 = up(8 * t->ng1v),
-               b_fl = up(4 * ((size_t)t->npairs + 1)), b_set = b_c1 + b_f2 + b_g1 + b_fl,
-               b_cnt = up(4 * rows), b_part = up(8 * ((size_t)npart + 1));
-  if ((rc = ensure(t->work, b_set * nset + b_cnt + b_part))) return SG4_OK;   // no memory: term kernels
-  char* W = t->work.as<char>();
+  Work w;
+  if (w.layout(t, rows)) return SG4_OK;   // no memory: term kernels
   char* B = t->blob.as<char>();
-  double *c1[2], *f2[2], *g1[2];
-  int* flag[2];                      // per pair, then the verdict
-  for (int s = 0; s < nset; ++s) {
-    char* w = W + s * b_set;
-    c1[s] = (double*)w; f2[s] = (double*)(w + b_c1); g1[s] = (double*)(w + b_c1 + b_f2);
-    flag[s] = (int*)(w + b_c1 + b_f2 + b_g1);
-  }
-  int32_t* cnt = (int32_t*)(W + b_set * nset);
-  int64_t* part = (int64_t*)(W + b_set * nset + b_cnt);
+  auto& c1 = w.c1;
+  auto& f2 = w.f2;
+  auto& g1 = w.g1;
+  auto& flag = w.flag;
+  int32_t* cnt = w.cnt;
+  int64_t* part = w.part;
   const NmDev* insts = t->insts.as<NmDev>();
   const int64_t* term0 = (const int64_t*)(B + t->o_term0);
-  const int64_t* row0 = (const int64_t*)(B + t->o_row0);
-  NM_TRY(hipMemcpyAsync(t->ck.p, in.ck->data(), sizeof(double) * in.ck->size(), hipMemcpyHostToDevice, st));
+  const int64_t* blk0 = (const int64_t*)(B + t->o_blk0);
+  if (!have_v)
+    NM_TRY(hipMemcpyAsync(t->ck.p, in.ck->data(), sizeof(double) * in.ck->size(), hipMemcpyHostToDevice, st));
   std::vector<int> hf[2];
-  for (int s = 0; s < nset; ++s) {
+  for (int s = have_v ? 1 : 0; s < nset; ++s) {
     const double* G = s ? mu : V;
     hipLaunchKernelGGL(k_nm_zero, dim3(8), dim3(256), 0, st, flag[s], t->npairs + 1);
     hipLaunchKernelGGL(k_nm_cut1, dim3(t->ncut1), dim3(64), 0, st, (const Cut*)(B + t->o_cut1), G, c1[s]);
@@ -971,10 +1131,11 @@ int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double
                        insts, term0, ni, t->nterms, in.d_terms, G, c1[s], f2[s], flag[s],
                        flag[s] + t->npairs);
     hipLaunchKernelGGL(k_nm_g1, dim3(t->ng1), dim3(256), 0, st, insts, (const int32_t*)(B + t->o_g1work),
-                       in.d_mats, c1[s], g1[s], s == 0);
+                       in.d_mats, c1[s], g1[s], s ? G1_GRID : G1_GRID | G1_KIN);
     hf[s].resize(t->npairs + 1);
     NM_TRY(hipMemcpyAsync(hf[s].data(), flag[s], sizeof(int) * hf[s].size(), hipMemcpyDeviceToHost, st));
   }
+  if (have_v) hf[0] = t->v_flags;
   NM_TRY(hipGetLastError());
   NM_TRY(hipStreamSynchronize(st));
   for (int s = 0; s < nset; ++s)
@@ -1017,54 +1178,76 @@ int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double
       adjoff[(size_t)x * 33 + k + 1] = (int32_t)adj.size();
     }
   }
+  // column lists of the pairs that are nonzero in V or mu
+  std::vector<EWork> uw;
+  std::vector<int64_t> loff((size_t)t->npairs * eld, 0), croff((size_t)t->npairs * eld, 0);
+  int64_t nl = 0, nr = 0;
+  for (int g = 0; g < t->npairs; ++g) {
+    if (!hf[0][g] && !(mu && hf[1][g])) continue;
+    const int x = t->pair_inst[g];
+    for (int l = 0; l <= t->dev[x].L; ++l) {
+      const int S = t->pair_s2n[(size_t)g * eld + l];
+      loff[(size_t)g * eld + l] = nl;
+      croff[(size_t)g * eld + l] = nr;
+      uw.push_back(EWork{x, g - t->dev[x].pair0, l, 0, 0});
+      nl += (int64_t)S * S;
+      nr += S;
+    }
+  }
   Blob lb;
   size_t o_ew[2], o_eoff[2];
   for (int s = 0; s < nset; ++s) { o_ew[s] = lb.add(ew[s]); o_eoff[s] = lb.add(eoff[s]); }
-  const size_t o_nz = lb.add(nz), o_nzoff = lb.add(nzoff), o_adj = lb.add(adj), o_adjoff = lb.add(adjoff);
+  const size_t o_nz = lb.add(nz), o_nzoff = lb.add(nzoff), o_adj = lb.add(adj), o_adjoff = lb.add(adjoff),
+               o_uw = lb.add(uw), o_loff = lb.add(loff), o_croff = lb.add(croff);
   if ((rc = upload(lb, t->lists, st))) return rc == SG4_ERR_OOM ? SG4_OK : rc;
-  if (ensure(t->e_v, 8 * ne[0]) || (mu && ensure(t->e_mu, 8 * ne[1]))) return SG4_OK;
+  if (ensure(t->e_v, 8 * ne[0]) || (mu && ensure(t->e_mu, 8 * ne[1])) ||
+      ensure(t->elist, up(2 * nl) + 4 * nr))
+    return SG4_OK;
   char* LB = t->lists.as<char>();
   DevBuf* eb[2] = {&t->e_v, &t->e_mu};
   NmSet set[2] = {};
   for (int s = 0; s < nset; ++s) {
     set[s] = NmSet{c1[s], g1[s], eb[s]->as<double>(), (const int64_t*)(LB + o_eoff[s])};
-    if (!ew[s].empty())
-      hipLaunchKernelGGL(k_nm_e2, dim3((unsigned)ew[s].size(), (unsigned)std::min(64, (Smax * Smax + 255) / 256)),
+    if (!ew[s].empty() && (s || !have_v))
+      hipLaunchKernelGGL(k_nm_e2, dim3((unsigned)ew[s].size(), (unsigned)std::min(256, (Smax * Smax + 31) / 32)),
                          dim3(256), 0, st, insts, (const EWork*)(LB + o_ew[s]), in.d_mats, c1[s], f2[s],
                          eb[s]->as<double>());
   }
   const NmPairs pr{(const int32_t*)(LB + o_nz), (const int32_t*)(LB + o_nzoff), (const int32_t*)(LB + o_adj),
-                   (const int32_t*)(LB + o_adjoff), eld};
-  const dim3 rg((unsigned)((rows + RT - 1) / RT));
+                   (const int32_t*)(LB + o_adjoff), (const int64_t*)(LB + o_loff),
+                   (const int64_t*)(LB + o_croff), t->elist.as<uint16_t>(),
+                   (int32_t*)(t->elist.as<char>() + up(2 * nl)), eld};
+  if (!uw.empty())
+    hipLaunchKernelGGL(k_nm_elist, dim3((unsigned)uw.size(), (unsigned)((Smax + 63) / 64)), dim3(64), 0, st, insts,
+                       (const EWork*)(LB + o_uw), set[0], set[1], pr);
+  const dim3 rg((unsigned)t->nblk);
   const size_t rl = (size_t)t->Dmax * RT * 7;
   if (mu)
-    hipLaunchKernelGGL((k_nm_rows<false, true>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+    hipLaunchKernelGGL((k_nm_rows<false, true>), rg, dim3(256), rl, st, insts, blk0, ni, set[0], set[1], pr,
                        t->Dmax, cnt, nullptr, nullptr, nullptr, nullptr);
   else
-    hipLaunchKernelGGL((k_nm_rows<false, false>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+    hipLaunchKernelGGL((k_nm_rows<false, false>), rg, dim3(256), rl, st, insts, blk0, ni, set[0], set[1], pr,
                        t->Dmax, cnt, nullptr, nullptr, nullptr, nullptr);
-  hipLaunchKernelGGL(k_nm_sum, dim3(npart), dim3(256), 0, st, cnt, rows, part);
-  hipLaunchKernelGGL(k_nm_scan_part, dim3(1), dim3(1024), 0, st, part, npart);
   int64_t nnz = 0;
-  NM_TRY(hipMemcpyAsync(&nnz, part + npart, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  NM_TRY(hipGetLastError());
-  NM_TRY(hipStreamSynchronize(st));
+  if ((rc = scan_rows(w, rows, st, &nnz))) return rc;
   if (nnz > NNZ_SMALL && nnz > NNZ_PER_POINT * (double)in.sum_nq) return SG4_OK;
   if (ensure(m.ptr, 8 * (rows + 1)) || ensure(m.col, 4 * nnz) || ensure(m.val, 8 * nnz) ||
       (mu && (ensure(m.val_mu, 8 * nnz) || ensure(m.val_f, 8 * nnz))))
     return SG4_OK;
-  hipLaunchKernelGGL(k_nm_ptr, dim3(npart), dim3(1024), 0, st, cnt, rows, part, m.ptr.as<int64_t>());
+  hipLaunchKernelGGL(k_nm_ptr, dim3(w.npart), dim3(1024), 0, st, cnt, rows, part, m.ptr.as<int64_t>());
   if (mu)
-    hipLaunchKernelGGL((k_nm_rows<true, true>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+    hipLaunchKernelGGL((k_nm_rows<true, true>), rg, dim3(256), rl, st, insts, blk0, ni, set[0], set[1], pr,
                        t->Dmax, cnt, m.ptr.as<int64_t>(), m.col.as<int32_t>(), m.val.as<double>(),
                        m.val_mu.as<double>());
   else
-    hipLaunchKernelGGL((k_nm_rows<true, false>), rg, dim3(RT), rl, st, insts, row0, ni, rows, set[0], set[1], pr,
+    hipLaunchKernelGGL((k_nm_rows<true, false>), rg, dim3(256), rl, st, insts, blk0, ni, set[0], set[1], pr,
                        t->Dmax, cnt, m.ptr.as<int64_t>(), m.col.as<int32_t>(), m.val.as<double>(), nullptr);
   NM_TRY(hipGetLastError());
   m.rows = rows;
   m.nnz = nnz;
   m.valid = true;
+  t->v_ready = true;
+  t->v_flags = hf[0];
   return SG4_OK;
 }
 
@@ -1130,7 +1313,7 @@ int nmode_order(const NModeMat& m, const NModeOrder& a, bool tangent, hipStream_
     else if (nc == 8) SG4_ORDER(8, 2, true);
     else SG4_ORDER(16, 1, true);
   } else {
-    if (nc == 2) SG4_ORDER(2, 8, false);
+    if (nc == 2) SG4_ORDER(2, 4, false);
     else if (nc == 4) SG4_ORDER(4, 4, false);
     else if (nc == 8) SG4_ORDER(8, 2, false);
     else SG4_ORDER(16, 1, false);

@@ -12,7 +12,7 @@ namespace sg4 {
 // c_k T_k(l_k) with T_k(l) = BtW D2 B (nb x nb), the identity in the other
 // modes.  Summed over the Smolyak terms with the combination weights, the
 // kinetic part of H becomes one sparse matrix K between packed rows that
-// differ in one mode index (built on the host, applied by k_kin_rows), and a
+// differ in one mode index (sg4_nmode.hip), and a
 // term only needs  W_t P_t^T B^T W V_t B P_t :  basis->grid products, the
 // potential, grid->basis products.  The grid->basis groups run in reverse
 // order so that the last basis->grid group, the potential and the first
