@@ -513,6 +513,7 @@ __global__ void k_hpsi_t1_f64(KArgs a, KMats<double> km);
 __global__ void k_hpsi_t1_f32(KArgs a, KMats<float> km);
 __global__ void k_hpsi_t10_f64(KArgs a, KMats10 km);
 __global__ void k_grad_v(KArgs a, KGrad kg);
+__global__ void k_grad_groups(KArgs a, KGrad kg);
 __global__ void k_hpsi_t1g_f64(KArgs a, KMats1G km);
 
 }  // namespace sg4
