@@ -479,6 +479,21 @@ __device__ __forceinline__ void term_t1_grouped(const KArgs& a, const KMats<T>& 
 
 constexpr int NT32 = 768;
 
+// Type-10 and general type-1 kernels: workgroup (x, y) does term order[x] for
+// vectors y 2^lg .. of the nvec; psi and hpsi element (row, vector) at
+// row rs + vector vs.
+struct PArgs {
+  const int32_t* order;
+  const TermDev* terms;
+  const MatDev* md;
+  const int32_t* map;
+  const double* psi;
+  double* hpsi;
+  int64_t rs, vs;
+  int nvec, lg;
+  int stage;   // the matrices of a term in LDS
+};
+
 struct KMats10 {
   const double* mats;
   const double* V;
@@ -511,9 +526,9 @@ __global__ void k_hpsi_t1s_f64(KArgs a, KMats<double> km);
 __global__ void k_hpsi_t1s_f32(KArgs a, KMats<float> km);
 __global__ void k_hpsi_t1_f64(KArgs a, KMats<double> km);
 __global__ void k_hpsi_t1_f32(KArgs a, KMats<float> km);
-__global__ void k_hpsi_t10_f64(KArgs a, KMats10 km);
+__global__ void k_hpsi_t10_f64(PArgs a, KMats10 km);
 __global__ void k_grad_v(KArgs a, KGrad kg);
 __global__ void k_grad_groups(KArgs a, KGrad kg);
-__global__ void k_hpsi_t1g_f64(KArgs a, KMats1G km);
+__global__ void k_hpsi_t1g_f64(PArgs a, KMats1G km);
 
 }  // namespace sg4

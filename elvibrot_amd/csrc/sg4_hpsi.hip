@@ -19,7 +19,7 @@
 //   per-mode grid path (k_hpsi_t1_*, term_t1): one pass per mode, any sizes.
 //   sparse path (sg4_nmode.hip): FP64, potentials that are sums of one- and
 //     two-mode functions: all of H as one sparse matrix over the packed rows.
-// Type 10 (d1 G d1): k_hpsi_t10_f64.  Eigenvalue gradients: k_grad_v.
+// Type 10 (d1 G d1) and general type 1: sg4_k_points.hip.  Eigenvalue gradients: k_grad_v.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -339,6 +339,11 @@ struct sg4_plan {
   std::vector<double> h_T;       // T_k(m) per (mode, level), rounding entries zeroed
   std::vector<int64_t> h_toff;
   std::vector<int> inst_L;       // largest |l| of every instance's terms
+  // type 10 and general type 1: the terms by decreasing work, the largest
+  // term, the padded block widths applied since the operator was set
+  sg4::DevBuf d_order;
+  int64_t pt_nmax = 0, pt_mats = 0;   // points, matrix entries
+  std::set<int> pt_seen;
   double flops_split = 0;        // algorithmic flops per vector of the split path's terms
   // H as one sparse matrix (sg4_nmode.hip): the field-free operator and, during
   // a propagation, the one with the dipole; field_on: V holds a field term
@@ -400,6 +405,7 @@ static void invalidate(sg4_plan* P) {
   P->mfma_valid = false;
   P->nm.valid = false;
   P->nm_seen.clear();
+  P->pt_seen.clear();
 }
 
 // Greedy grouping of consecutive active modes into the shapes of
@@ -667,6 +673,33 @@ static int build_nmode(sg4_plan* P) {
   return nmode_build(P->nmt, in, P->d_V0.p ? P->d_V0.as<double>() : P->d_V.as<double>(), nullptr, P->nm);
 }
 
+// Term order of the type-10 and general type-1 kernels.
+static int build_points(sg4_plan* P) {
+  P->split_ok = P->split_fp = false;
+  std::vector<int32_t> ord(P->nterms);
+  std::vector<double> cost(P->nterms);
+  P->pt_nmax = P->pt_mats = 0;
+  for (int64_t t = 0; t < P->nterms; ++t) {
+    const TermDev& T = P->h_terms[t];
+    double w = 0;
+    int64_t mats = 0;
+    for (int q = 0; q < T.nact; ++q) {
+      const MatDev& m = P->h_md[T.mat[q]];
+      w += m.nq;
+      mats += 2 * m.nq * m.nb + (P->type_op == 10 ? 1 : 2) * m.nq * m.nq;
+    }
+    ord[t] = (int32_t)t;
+    cost[t] = w * std::max(T.nq, T.nb);
+    P->pt_nmax = std::max<int64_t>(P->pt_nmax, std::max(T.nq, T.nb));
+    P->pt_mats = std::max(P->pt_mats, mats);
+  }
+  std::stable_sort(ord.begin(), ord.end(), [&](int32_t x, int32_t y) { return cost[x] > cost[y]; });
+  int rc = P->d_order.alloc(sizeof(int32_t) * ord.size());
+  if (rc) return rc;
+  HIP_TRY(hipMemcpy(P->d_order.p, ord.data(), sizeof(int32_t) * ord.size(), hipMemcpyHostToDevice));
+  return SG4_OK;
+}
+
 static int build_terms(sg4_plan* P) {
   P->mfma_valid = false;
   P->flops_split = 0.0;
@@ -716,6 +749,7 @@ static int build_terms(sg4_plan* P) {
   if (rc) return rc;
   HIP_TRY(hipMemcpy(P->d_terms.p, P->h_terms.data(), sizeof(TermDev) * P->h_terms.size(),
                     hipMemcpyHostToDevice));
+  if (P->type_op != 1) return build_points(P);
   if ((rc = build_kinetic(P))) return rc;
   return build_nmode(P);
 }
@@ -855,10 +889,10 @@ static int get_items(sg4_plan* P, int nvec, int esize, ItemPlan** out, int nbuf_
   for (int64_t t = 0; t < (split ? 0 : P->nterms); ++t) {
     const TermDev& T = P->h_terms[t];
     const int64_t nmax = std::max(T.nq, T.nb);
-    const int nbuf = nbuf_force ? nbuf_force : ((P->type_op == 10) ? P->D + 3 : 2);
+    const int nbuf = nbuf_force ? nbuf_force : 2;
     const int64_t per = nbuf * nmax * esize;  // bytes per vector (work buffers)
     const bool big = per > budget;
-    if (big && (P->type_op == 10 || nbuf_force)) {
+    if (big && nbuf_force) {
       set_error("term too large for the LDS work buffers of this kernel");
       return SG4_ERR_UNSUPPORTED;
     }
@@ -899,8 +933,7 @@ static int get_items(sg4_plan* P, int nvec, int esize, ItemPlan** out, int nbuf_
   ip->lds = lds;
   ip->nitems2 = (int64_t)h2.size();
   ip->lds2 = lds2;
-  ip->flops_main = split ? flops_main
-                         : (P->type_op == 10 ? 4.0 : 3.0) * P->flops_per_vec * nvec;
+  ip->flops_main = split ? flops_main : 3.0 * P->flops_per_vec * nvec;
   int rc = ip->items.alloc(sizeof(Item) * h.size());
   if (rc) return rc;
   HIP_TRY(hipMemcpy(ip->items.p, h.data(), sizeof(Item) * h.size(), hipMemcpyHostToDevice));
@@ -913,6 +946,13 @@ static int get_items(sg4_plan* P, int nvec, int esize, ItemPlan** out, int nbuf_
   P->items[key] = std::move(ip);
   return SG4_OK;
 }
+
+// Launch of the type-10 and general type-1 kernels (apply_points): the vectors
+// of a term are cut into 2^lg as long as POINT_ITEMS workgroups remain and the
+// buffers stay within POINT_LDS; matrices of at most POINT_MATS entries a term
+// are staged in LDS.
+constexpr int64_t POINT_ITEMS = 1024, POINT_LDS = 32 * 1024, POINT_MATS = 2048;
+constexpr int POINT_LDS_MAX = LDS_MAX - 4096;   // beside the kernels' static LDS
 
 static int grid_blocks(int64_t n) {
   int64_t b = (n + 255) / 256;
@@ -1289,16 +1329,15 @@ static int prepare(sg4_plan* P, int nvec, int prec, const LaunchCfg& cfg, ItemPl
       if ((rc = P->d_fx.alloc(need))) return rc;
     }
   }
+  *ip = nullptr;
+  if (P->type_op != 1) return SG4_OK;
   const int esize = (prec == SG4_PREC_FP64) ? 8 : 4;
   if (esize == 4 && (rc = ensure_f32(P))) return rc;
   if (prec == SG4_PREC_F32X2) {
     if ((rc = build_mfma(P))) return rc;
     return get_items_mfma(P, nvec, cfg.lds_budget, cfg.xcd, ip);
   }
-  if (P->type_op == 11) return get_items(P, nvec, esize, ip, 4, LDS_MAX, 0, false);
-  const bool t10 = P->type_op == 10;
-  return get_items(P, nvec, esize, ip, 0, t10 ? LDS_SMALL : cfg.lds_budget, t10 ? 0 : cfg.xcd,
-                   use_split(P));
+  return get_items(P, nvec, esize, ip, 0, cfg.lds_budget, cfg.xcd, use_split(P));
 }
 
 // Width of the rows-layout staging block of a column-major apply of nvec
@@ -1363,10 +1402,55 @@ static int apply_nmode(sg4_plan* P, int nvec, int W, const double* psi, double* 
   return SG4_OK;
 }
 
+// Apply of a type-10 or general type-1 operator to nvec vectors, element
+// (row, vector) at row rs + vector vs; W: the padded width the block counts as.
+static int apply_points(sg4_plan* P, int nvec, int W, const double* psi, double* hpsi, int64_t rs, int64_t vs) {
+  if (P->deterministic) {
+    set_error("deterministic accumulation is available on the split type-1 path only");
+    return SG4_ERR_UNSUPPORTED;
+  }
+  // accepted term sizes: D + 3 (type 10) buffers of a term within 64 KiB, four within the LDS
+  const bool t10 = P->type_op == 10;
+  if ((t10 ? P->D + 3 : 4) * 8 * P->pt_nmax > (t10 ? LDS_SMALL : LDS_MAX)) {
+    set_error("term too large for the LDS work buffers of this kernel");
+    return SG4_ERR_UNSUPPORTED;
+  }
+  if (P->no_alloc && !P->pt_seen.count(W)) return not_prepared();
+  if (!P->no_alloc) P->pt_seen.insert(W);
+  const int64_t per = 8 * (t10 ? P->D + 3 : 3) * P->pt_nmax;
+  int lg = 0;
+  while ((2 << lg) <= nvec && per * (2 << lg) <= POINT_LDS && P->nterms * ((nvec - 1) / (2 << lg) + 1) >= POINT_ITEMS) ++lg;
+  const int64_t n = P->nb_ba * nvec;
+  hipLaunchKernelGGL(k_fill, dim3(grid_blocks(n)), dim3(256), 0, P->stream, hpsi, n, 0.0);
+  PArgs a{P->d_order.as<int32_t>(), P->d_terms.as<TermDev>(), P->d_md.as<MatDev>(), P->d_map.as<int32_t>(),
+          psi, hpsi, rs, vs, nvec, lg, P->pt_mats <= POINT_MATS};
+  const size_t lds = (size_t)(per << lg) + (a.stage ? 8 * P->pt_mats : 0);
+  const dim3 grid((unsigned)P->nterms, (unsigned)((nvec + (1 << lg) - 1) >> lg));
+  P->last_items = (int64_t)grid.x * grid.y;
+  P->last_flops = (t10 ? 4.0 : 3.0) * P->flops_per_vec * W;
+  int rc;
+  if (P->timing) {
+    if ((rc = next_events(P))) return rc;
+    HIP_TRY(hipEventRecord(P->ev0, P->stream));
+  }
+  if (t10) {
+    KMats10 km{P->d_mats.as<double>(), P->d_V.as<double>(), P->d_G.as<double>(), P->d_Jac.as<double>(),
+               P->d_sqRJ.as<double>()};
+    hipLaunchKernelGGL(k_hpsi_t10_f64, grid, dim3(t10 ? 384 : 256), lds, P->stream, a, km);
+  } else {
+    KMats1G km{P->d_mats.as<double>(), P->d_F.as<double>(), P->d_der.as<int32_t>(), P->nder, P->sum_nq};
+    hipLaunchKernelGGL(k_hpsi_t1g_f64, grid, dim3(t10 ? 384 : 256), lds, P->stream, a, km);
+  }
+  if (P->timing) HIP_TRY(hipEventRecord(P->ev1, P->stream));
+  HIP_TRY(hipGetLastError());
+  return SG4_OK;
+}
+
 static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, int prec,
                       const LaunchCfg* cfgp = nullptr) {
   int rc;
   if ((rc = check_apply(P, nvec, prec))) return rc;
+  if (P->type_op != 1) return apply_points(P, nvec, nvec, psi, hpsi, nvec, 1);
   if (use_nmode(P, prec)) return apply_nmode(P, nvec, nvec, psi, hpsi, nullptr, nullptr);
   const LaunchCfg cfg = cfgp ? *cfgp : cfg_for(P, nvec, prec);
   ItemPlan* ip = nullptr;
@@ -1404,7 +1488,7 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
     if (!split) HIP_TRY(hipEventRecord(P->ev0, P->stream));
   }
   const unsigned grid = (unsigned)((cfg.grid > 0 && cfg.grid < ip->nitems) ? cfg.grid : ip->nitems);
-  const dim3 blk(P->type_op == 10 ? 256 : (split ? cfg.nthreads : std::min(cfg.nthreads, NT)));
+  const dim3 blk(split ? cfg.nthreads : std::min(cfg.nthreads, NT));
   if (prec == SG4_PREC_F32X2) {
     // kinetic rows in FP64 (initialise hpsi), then the terms on the matrix cores
     if ((rc = nmode_apply(P->kin, nvec, psi, hpsi, P->stream))) return rc;
@@ -1466,14 +1550,6 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
     if (fx)
       hipLaunchKernelGGL(k_fx_finish, dim3(grid_blocks(n)), dim3(256), 0, P->stream, fx, fxflag,
                          hpsi, n);
-  } else if (P->type_op == 11) {
-    KMats1G km{P->d_mats.as<double>(), P->d_F.as<double>(), P->d_der.as<int32_t>(), P->nder,
-               P->sum_nq};
-    hipLaunchKernelGGL(k_hpsi_t1g_f64, dim3(grid), dim3(256), ip->lds, P->stream, a, km);
-  } else if (P->type_op == 10) {
-    KMats10 km{P->d_mats.as<double>(), P->d_V.as<double>(), P->d_G.as<double>(),
-               P->d_Jac.as<double>(), P->d_sqRJ.as<double>()};
-    hipLaunchKernelGGL(k_hpsi_t10_f64, dim3((unsigned)ip->nitems), blk, ip->lds, P->stream, a, km);
   } else if (esize == 8) {
     KMats<double> km{P->d_mats.as<double>(), P->d_V.as<double>(), P->d_ck.as<double>()};
     hipLaunchKernelGGL(k_hpsi_t1_f64, dim3(grid), blk, ip->lds, P->stream, a, km);
@@ -1683,7 +1759,7 @@ int sg4_plan_create_batch(int32_t ninst, const sg4_tables* tabs, int32_t max_nve
     (void)hipFuncSetAttribute((const void*)k_hpsi_t1s_f32,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     (void)hipFuncSetAttribute((const void*)k_hpsi_t10_f64,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
+                              hipFuncAttributeMaxDynamicSharedMemorySize, POINT_LDS_MAX);
     (void)hipFuncSetAttribute((const void*)k_grad_v,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     (void)hipFuncSetAttribute((const void*)k_grad_groups,
@@ -1691,7 +1767,7 @@ int sg4_plan_create_batch(int32_t ninst, const sg4_tables* tabs, int32_t max_nve
     (void)hipFuncSetAttribute((const void*)k_hpsi_mfma,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     (void)hipFuncSetAttribute((const void*)k_hpsi_t1g_f64,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
+                              hipFuncAttributeMaxDynamicSharedMemorySize, POINT_LDS_MAX);
   });
   std::unique_ptr<sg4_plan> P(new sg4_plan);
   HIP_TRY(hipGetDevice(&P->device));
@@ -2010,6 +2086,7 @@ int sg4_apply(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi, int32_
     return apply_rows(p, 1, psi, hpsi, prec);
   }
   const int W = pad_width(p, nvec);
+  if (p->type_op > 1 && prec == SG4_PREC_FP64) return apply_points(p, nvec, W, psi, hpsi, 1, p->nb_ba);
   if (p->type_op && use_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
   hipLaunchKernelGGL(k_cols_to_rows, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, psi, ri, p->nb_ba, nvec, W);
   int rc = apply_rows(p, W, ri, ro, prec);
@@ -2074,6 +2151,7 @@ int sg4_apply_noalloc(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi
   if (nvec == 1) return apply_rows(p, 1, psi, hpsi, prec);
   double* ri = base;
   double* ro = base + n;
+  if (p->type_op > 1 && prec == SG4_PREC_FP64) return apply_points(p, nvec, W, psi, hpsi, 1, p->nb_ba);
   if (use_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
   hipLaunchKernelGGL(k_cols_to_rows, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, psi, ri, p->nb_ba, nvec, W);
   if ((rc = apply_rows(p, W, ri, ro, prec))) return rc;
