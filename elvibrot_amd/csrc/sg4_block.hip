@@ -3,25 +3,24 @@
 // product is a pass over HBM with a tiny output.
 //
 //   gram:    C (m x q) = A B^T, A: m rows, B: q rows (stride lda, ldb), the
-//            inner dimension n long.  Each workgroup takes 32-column tiles in
-//            a grid-stride loop, stages the rows of a tile in LDS (sized for
-//            this m and q, so that small grams keep several workgroups per
-//            CU and their tile loads in flight) and keeps 4 x 4 register
-//            blocks of C: with fewer blocks than threads the tile's columns
-//            are dealt to slices of threads, summed in LDS at the end; the
-//            workgroup partials go to a work array and a second kernel adds
-//            them, one wave per output, in a fixed order (deterministic, no
-//            atomics).
-//   combine: Y (k x n) = beta Y + U X, U (k x d) small, X: d rows; one
-//            column per thread, coalesced across the wave, U entries from
-//            scalar loads (wave-uniform addresses) as FMA operands.
-// Measured at 10D L=8 (n = 1.26 M): gram 8 x 8 0.065 ms, 16 x 20 0.16 ms,
-// 20 x 20 0.19 ms, 4 x 84 0.32 ms (HBM floor 0.02, 0.05, 0.05, 0.11 ms; with
-// LDS for 124 rows at two workgroups per CU and no column slices: 0.22, 0.28 ms
-// for 8 x 8 and 20 x 20); combine 8 x 8 0.031 ms, 16 x 48 0.16 ms, 20 x 84
-// 0.34 ms, 36 x 84 0.69 ms (U broadcast from LDS instead: 0.05, 0.20, 0.48,
-// 0.83 ms).  The Davidson driver uses them for the small grams and the
-// rotations to at most 20 rows, and the library GEMM for the others.
+//            inner dimension n long, on the FP64 matrix cores: a wave keeps up
+//            to 4 x 2 tiles of 16 x 16 and takes 16 columns at a time straight
+//            from memory into operand registers (no LDS, no barrier in the
+//            loop); the workgroups' partials go to a work array and a second
+//            kernel adds them, one wave per output, in a fixed order
+//            (deterministic, no atomics).
+//   combine: Y (k x n) = beta Y + U X, U (k x d) small, X: d rows: 32 columns
+//            per wave and step, X straight into operand registers, U in LDS in
+//            operand order (up to 64 KiB; larger U by scalar loads, one column
+//            per thread).
+// Bound by HBM for the Davidson's shapes.  At 10D L=8 (n = 1.26 M), us, before
+// (LDS tiles and 4 x 4 register blocks; one column per thread with U from
+// scalar loads) -> now, and the floor at the copy rate of 4.9 TB/s: gram 8 x 8
+// 65 -> 34 (33), 20 x 20 191 -> 86 (82), 60 x 16 305 -> 165 (156), 100 x 16 465 ->
+// 283 (238), 84 x 84 1825 -> 1111 (library split-K product 300-600); combine 8 x 8
+// 29 -> 28, 16 x 48 158 -> 149 (131), 20 x 60 244 -> 193 (164), 36 x 84 703 -> 352
+// (246), 64 x 64 1035 -> 367 (262).  1024 or 2048 gram workgroups: 187, 209 for
+// 60 x 16 (more partials).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,109 +31,91 @@
 namespace sg4 {
 namespace {
 
-constexpr int GT = 32;         // columns per gram tile
-constexpr int GMAX = 124;      // rows of A or B (LDS: 32 x (4 ceil(rows/4) + 1) doubles each)
-constexpr int GBLK = 512;      // 4 x 4 output blocks per workgroup (two per thread)
-constexpr int GNB = 2048;      // workgroups of the gram's first kernel (at most)
+constexpr int GMAX = 124;      // rows of A or B
+constexpr int GBLK = 512;      // 4 x 4 output blocks at most
+constexpr int GNB = 2048;      // partials per output that the work array is sized for
+constexpr int GWGS = 512;      // workgroups of a gram (per group of tiles)
+constexpr int64_t CWG = 2048;  // workgroups of a combine
 constexpr int CMAXU = 8192;    // entries of U (k d) at most
-constexpr int CK = 16;         // outputs of the combine per pass over X (k <= 16)
+constexpr int CK = 16;         // outputs of the scalar combine per pass over X (k <= 16)
 constexpr int CKW = 48;        // the same for wider k (k > 48: several passes)
 
-// column slices of the gram's workgroup for nblk 4 x 4 output blocks
-__host__ __device__ constexpr int gram_slices(int nblk) {
-  return nblk >= 256 ? 1 : (256 / nblk < GT ? 256 / nblk : GT);
-}
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+struct __attribute__((packed, aligned(8))) D4 { double v[4]; };   // 32 bytes at 8-byte alignment
 
+// Partial sums of C = A B^T over the columns of this workgroup: TA x TB tiles
+// of 16 x 16 on v_mfma_f64_16x16x4.  A wave takes 16 columns at a time; lane l
+// holds columns 4 (l/16) .. +3 of row l%16 of every tile (a row's 16 columns
+// are one 128-byte line), and product s of the four uses column 4 (l/16) + s
+// of both operands, so nothing goes through LDS.  blockIdx.y: group of tiles;
+// swap: A and B are exchanged (the wider one in the TA tiles).
+template <int TA, int TB>
 __global__ __launch_bounds__(256) void k_gram_part(int m, int q, int64_t n, const double* __restrict__ A,
                                                    int64_t lda, const double* __restrict__ B, int64_t ldb,
-                                                   double* __restrict__ part) {
-  // As[c pa + i]: column c of the tile, row i (rows padded to a multiple of 4
-  // with zeros; pitch pa = 4 m4 + 1), Bs likewise with pitch pb = 4 q4 + 1
-  extern __shared__ double gl[];
-  const int m4 = (m + 3) >> 2, q4 = (q + 3) >> 2, nblk = m4 * q4;
-  const int pa = 4 * m4 + 1, pb = 4 * q4 + 1;
-  double* As = gl;
-  double* Bs = gl + GT * pa;
-  const int tid = threadIdx.x;
-  // with fewer than 256 output blocks the columns of a tile are dealt to ns
-  // slices of threads (block tid % nblk, slice tid / nblk: columns slice,
-  // slice + ns, ...), whose sums are added in LDS at the end in slice order;
-  // otherwise a thread keeps output blocks tid and tid + 256 over all columns
-  const int ns = gram_slices(nblk);
-  const int b0 = ns > 1 ? tid % nblk : tid, b1 = tid + 256;
-  const int sl = ns > 1 ? tid / nblk : 0;
-  const bool on0 = ns > 1 ? tid < ns * nblk : b0 < nblk;
-  double acc0[16], acc1[16];
+                                                   int swap, double* __restrict__ part) {
+  __shared__ double red[4][256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, kq = lane >> 4;
+  const int gb = (q + 16 * TB - 1) / (16 * TB);
+  const int i0 = (blockIdx.y / gb) * 16 * TA, j0 = (blockIdx.y % gb) * 16 * TB;
+  const double* pa[TA];
+  const double* pb[TB];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) { acc0[e] = 0.0; acc1[e] = 0.0; }
-  const int64_t ntile = (n + GT - 1) / GT;
-  for (int64_t t = blockIdx.x; t < ntile; t += gridDim.x) {
-    const int64_t c0 = t * GT;
-    __syncthreads();                            // previous tile consumed
-    for (int e = tid; e < GT * 4 * m4; e += 256) {
-      const int i = e / GT, c = e % GT;         // consecutive threads: consecutive columns
-      As[c * pa + i] = (i < m && c0 + c < n) ? A[(int64_t)i * lda + c0 + c] : 0.0;
-    }
-    for (int e = tid; e < GT * 4 * q4; e += 256) {
-      const int i = e / GT, c = e % GT;
-      Bs[c * pb + i] = (i < q && c0 + c < n) ? B[(int64_t)i * ldb + c0 + c] : 0.0;
-    }
-    __syncthreads();
-    if (on0) {
-      const int bi = (b0 / q4) * 4, bj = (b0 % q4) * 4;
-      for (int c = sl; c < GT; c += ns) {
-        double a[4], b[4];
+  for (int t = 0; t < TA; ++t) pa[t] = A + (int64_t)min(i0 + 16 * t + r, m - 1) * lda + 4 * kq;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) { a[u] = As[c * pa + bi + u]; b[u] = Bs[c * pb + bj + u]; }
+  for (int t = 0; t < TB; ++t) pb[t] = B + (int64_t)min(j0 + 16 * t + r, q - 1) * ldb + 4 * kq;
+  f64x4 acc[TA][TB];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+  for (int x = 0; x < TA; ++x)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) acc0[4 * u + v] = fma(a[u], b[v], acc0[4 * u + v]);
-      }
-    }
-    if (ns == 1 && b1 < nblk) {
-      const int bi = (b1 / q4) * 4, bj = (b1 % q4) * 4;
-      for (int c = 0; c < GT; ++c) {
-        double a[4], b[4];
+    for (int y = 0; y < TB; ++y) acc[x][y] = f64x4{0.0, 0.0, 0.0, 0.0};
+  auto products = [&](const D4 (&a)[TA], const D4 (&b)[TB]) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) { a[u] = As[c * pa + bi + u]; b[u] = Bs[c * pb + bj + u]; }
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+      for (int x = 0; x < TA; ++x)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) acc1[4 * u + v] = fma(a[u], b[v], acc1[4 * u + v]);
-      }
-    }
+        for (int y = 0; y < TB; ++y)
+          acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x].v[s], b[y].v[s], acc[x][y], 0, 0, 0);
+  };
+  const int64_t full = n / 16, step = (int64_t)gridDim.x * 4;
+  int64_t t = (int64_t)blockIdx.x * 4 + wave;
+  for (; t < full; t += step) {
+    D4 a[TA], b[TB];
+#pragma unroll
+    for (int x = 0; x < TA; ++x) a[x] = *(const D4*)(pa[x] + 16 * t);
+#pragma unroll
+    for (int y = 0; y < TB; ++y) b[y] = *(const D4*)(pb[y] + 16 * t);
+    products(a, b);
   }
-  // partial of output e = i q + j at part[e * nb + workgroup]
+  if (t == full && 16 * full < n) {   // the columns beyond the last whole block, the others zero
+    D4 a[TA], b[TB];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const bool in = 16 * full + 4 * kq + s < n;
+#pragma unroll
+      for (int x = 0; x < TA; ++x) a[x].v[s] = in ? pa[x][16 * full + s] : 0.0;
+#pragma unroll
+      for (int y = 0; y < TB; ++y) b[y].v[s] = in ? pb[y][16 * full + s] : 0.0;
+    }
+    products(a, b);
+  }
+  // the four waves' sums in wave order; output (i, j) of a tile: value i / 4 of
+  // lane 16 (i % 4) + j
   const int64_t nb = gridDim.x;
-  if (ns > 1) {
-    __syncthreads();                            // the last tile consumed: LDS reused
-    double* red = gl;                           // [slice][block][16]
-    if (on0)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) red[(sl * nblk + b0) * 16 + e] = acc0[e];
-    __syncthreads();
-    for (int o = tid; o < nblk * 16; o += 256) {
-      const int b = o >> 4, e = o & 15;
-      double sum = 0.0;
-      for (int k = 0; k < ns; ++k) sum += red[(k * nblk + b) * 16 + e];
-      const int i = (b / q4) * 4 + (e >> 2), j = (b % q4) * 4 + (e & 3);
-      if (i < m && j < q) part[((int64_t)i * q + j) * nb + blockIdx.x] = sum;
+  for (int x = 0; x < TA; ++x)
+#pragma unroll
+    for (int y = 0; y < TB; ++y) {
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 4; ++u) red[wave][(4 * u + kq) * 16 + r] = acc[x][y][u];
+      __syncthreads();
+      const int i = i0 + 16 * x + threadIdx.x / 16, j = j0 + 16 * y + threadIdx.x % 16;
+      if (i < m && j < q) {
+        const double s = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+        part[(swap ? (int64_t)j * m + i : (int64_t)i * q + j) * nb + blockIdx.x] = s;
+      }
     }
-    return;
-  }
-  if (b0 < nblk) {
-    const int bi = (b0 / q4) * 4, bj = (b0 % q4) * 4;
-    for (int u = 0; u < 4; ++u)
-      for (int v = 0; v < 4; ++v)
-        if (bi + u < m && bj + v < q) part[((int64_t)(bi + u) * q + bj + v) * nb + blockIdx.x] = acc0[4 * u + v];
-  }
-  if (b1 < nblk) {
-    const int bi = (b1 / q4) * 4, bj = (b1 % q4) * 4;
-    for (int u = 0; u < 4; ++u)
-      for (int v = 0; v < 4; ++v)
-        if (bi + u < m && bj + v < q) part[((int64_t)(bi + u) * q + bj + v) * nb + blockIdx.x] = acc1[4 * u + v];
-  }
 }
 
 // C[e] = sum over the nb workgroup partials of output e: one wave per output,
@@ -149,6 +130,77 @@ __global__ __launch_bounds__(256) void k_gram_sum(int mq, int nb, const double* 
   for (int b = lane; b < nb; b += 64) s += part[(int64_t)e * nb + b];
   for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
   if (lane == 0) C[e] = s;
+}
+
+// Y (16 RT rows from i0) = beta Y + U X for 32 columns per wave and step, on
+// v_mfma_f64_16x16x4: lane l holds columns 2 (l%16), +1 of row 4 s + l/16 of X
+// (256 bytes of a row per wave and load) for two column tiles, U sits in LDS in
+// operand order, zero beyond k and d.
+template <int RT>
+__global__ __launch_bounds__(256) void k_combine_mfma(int k, int d, int64_t n, const double* __restrict__ U,
+                                                      const double* __restrict__ X, int64_t ldx, double beta,
+                                                      double* __restrict__ Y, int64_t ldy) {
+  extern __shared__ double ul[];   // [(s RT + rt) 64 + lane]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, kq = lane >> 4;
+  const int ks = (d + 3) >> 2, i0 = blockIdx.y * 16 * RT;
+  for (int e = threadIdx.x; e < ks * RT * 64; e += 256) {
+    const int l = e & 63, st = e >> 6, rt = st % RT, s = st / RT;
+    const int i = i0 + 16 * rt + (l & 15), j = 4 * s + (l >> 4);
+    ul[e] = (i < k && j < d) ? U[(int64_t)i * d + j] : 0.0;
+  }
+  __syncthreads();
+  const int64_t nblk = (n + 31) / 32;
+  for (int64_t t = (int64_t)blockIdx.x * 4 + wave; t < nblk; t += (int64_t)gridDim.x * 4) {
+    const int64_t c = 32 * t + 2 * r;
+    const bool in0 = c < n, in1 = c + 1 < n;
+    f64x4 acc[RT][2];
+#pragma unroll
+    for (int x = 0; x < RT; ++x) acc[x][0] = acc[x][1] = f64x4{0.0, 0.0, 0.0, 0.0};
+    auto product = [&](int s, double x0, double x1) {
+#pragma unroll
+      for (int x = 0; x < RT; ++x) {
+        const double u = ul[(s * RT + x) * 64 + lane];
+        acc[x][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u, x0, acc[x][0], 0, 0, 0);
+        acc[x][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u, x1, acc[x][1], 0, 0, 0);
+      }
+    };
+    if (32 * t + 32 <= n) {   // uniform over the wave: a matrix instruction takes all lanes
+      const double* p = X + (int64_t)kq * ldx + c;
+      int s = 0;
+      for (; 4 * s + 16 <= d; s += 4) {     // four steps' loads in flight
+        double a[4], b[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const double* w = p + (int64_t)4 * (s + u) * ldx;
+          a[u] = w[0];
+          b[u] = w[1];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) product(s + u, a[u], b[u]);
+      }
+      for (; s < ks; ++s) {
+        const bool row = 4 * s + kq < d;
+        const double* w = p + (int64_t)4 * s * ldx;
+        product(s, row ? w[0] : 0.0, row ? w[1] : 0.0);
+      }
+    } else {                                // the last columns
+      for (int s = 0; s < ks; ++s) {
+        const bool row = 4 * s + kq < d;
+        const double* w = X + (int64_t)(4 * s + kq) * ldx + c;
+        product(s, row && in0 ? w[0] : 0.0, row && in1 ? w[1] : 0.0);
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < RT; ++x)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + 16 * x + 4 * u + kq;
+        if (i >= k) continue;
+        double* y = Y + (int64_t)i * ldy + c;
+        if (in0) y[0] = beta == 0.0 ? acc[x][0][u] : fma(beta, y[0], acc[x][0][u]);
+        if (in1) y[1] = beta == 0.0 ? acc[x][1][u] : fma(beta, y[1], acc[x][1][u]);
+      }
+  }
 }
 
 // Y rows i0..i0+CK-1 for the columns of this thread; U entries are read
@@ -230,14 +282,22 @@ int sg4_block_gram(sg4_plan* p, int32_t m, int32_t q, int64_t n, const double* A
       (rc = device_block(p, C, "C")) || (rc = device_block(p, work, "work")))
     return rc;
   const hipStream_t st = (hipStream_t)plan_stream(p);
-  const int64_t ntile = (n + GT - 1) / GT;
-  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)GNB, ntile, nwork / ((int64_t)m * q)}));
-  // LDS: the tile's rows, or the slice sums at the end if larger (<= 32 KiB)
-  const int m4 = (m + 3) / 4, q4 = (q + 3) / 4, ns = gram_slices(m4 * q4);
-  const size_t tile = sizeof(double) * GT * ((size_t)(4 * m4 + 1) + (4 * q4 + 1));
-  const size_t red = ns > 1 ? sizeof(double) * 16 * (size_t)ns * m4 * q4 : 0;
-  const size_t lds = std::max(tile, red);
-  hipLaunchKernelGGL(k_gram_part, dim3(nb), dim3(256), lds, st, m, q, n, A, lda, B, ldb, work);
+  const int64_t nwave = (n + 63) / 64;
+  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)GWGS, (nwave + 3) / 4, nwork / ((int64_t)m * q)}));
+  const bool swap = q > m;                     // the wider block in the row tiles
+  const int M = swap ? q : m, Q = swap ? m : q;
+  const double *a = swap ? B : A, *b = swap ? A : B;
+  const int64_t la = swap ? ldb : lda, lb = swap ? lda : ldb;
+  const int ta = M <= 16 ? 1 : M <= 32 ? 2 : 4, tb = Q <= 16 ? 1 : 2;
+  const dim3 grid((unsigned)nb, (unsigned)(((M + 16 * ta - 1) / (16 * ta)) * ((Q + 16 * tb - 1) / (16 * tb))));
+#define SG4_GRAM(TA, TB) \
+  hipLaunchKernelGGL((k_gram_part<TA, TB>), grid, dim3(256), 0, st, M, Q, n, a, la, b, lb, swap, work)
+  if (tb == 1) {
+    if (ta == 1) SG4_GRAM(1, 1); else if (ta == 2) SG4_GRAM(2, 1); else SG4_GRAM(4, 1);
+  } else {
+    if (ta == 2) SG4_GRAM(2, 2); else SG4_GRAM(4, 2);
+  }
+#undef SG4_GRAM
   BK_TRY(hipGetLastError());
   const int mq = m * q;
   hipLaunchKernelGGL(k_gram_sum, dim3((mq + 3) / 4), dim3(256), 0, st, mq, nb, work, C);
@@ -260,6 +320,16 @@ int sg4_block_combine(sg4_plan* p, int32_t k, int32_t d, int64_t n, const double
   const int64_t xe = 8 * ((int64_t)(d - 1) * ldx + n), ye = 8 * ((int64_t)(k - 1) * ldy + n);
   if (xb < yb + ye && yb < xb + xe) { set_error("sg4_block_combine: X and Y overlap"); return SG4_ERR_ARG; }
   const hipStream_t st = (hipStream_t)plan_stream(p);
+  const int rt = k <= 16 ? 1 : k <= 32 ? 2 : 4;
+  const size_t lds = sizeof(double) * 64 * rt * (size_t)((d + 3) / 4);
+  if (lds <= 64 * 1024) {
+    const dim3 grid((unsigned)std::min<int64_t>((n + 127) / 128, CWG), (unsigned)((k + 16 * rt - 1) / (16 * rt)));
+    if (rt == 1) hipLaunchKernelGGL(k_combine_mfma<1>, grid, dim3(256), lds, st, k, d, n, U, X, ldx, beta, Y, ldy);
+    else if (rt == 2) hipLaunchKernelGGL(k_combine_mfma<2>, grid, dim3(256), lds, st, k, d, n, U, X, ldx, beta, Y, ldy);
+    else hipLaunchKernelGGL(k_combine_mfma<4>, grid, dim3(256), lds, st, k, d, n, U, X, ldx, beta, Y, ldy);
+    BK_TRY(hipGetLastError());
+    return SG4_OK;
+  }
   const unsigned nb = (unsigned)std::min<int64_t>((n + 255) / 256, 65535);
   if (k <= CK)
     hipLaunchKernelGGL(k_combine<CK>, dim3(nb), dim3(256), 0, st, k, d, n, U, X, ldx, beta, Y, ldy);

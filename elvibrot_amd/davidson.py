@@ -75,14 +75,13 @@ def _gram(A, B, chunks=256):
 
 class _Dense:
     """Products over packed vectors (rows of length nb_ba) on the device.
-    Grams with at most 400 outputs or at most 16 columns (up to 124 rows)
-    and rotations to at most 20 rows go through the library's block kernels
-    (sg4_block_gram, sg4_block_combine, on the operator's plan and stream);
-    the others through the split-K batched product and the library GEMM,
-    which are faster there (10D L=8: gram 20 x 20 0.19 against 0.32 ms,
-    100 x 16 0.47 against 0.57 ms, 16 x 100 0.56 against 0.31 ms, 36 x 36
-    0.37 against 0.30 ms; rotation 20 x 84 0.34 against 0.59 ms, 36 x 84
-    0.69 against 0.64 ms).
+    Grams with at most 400 outputs or at most 16 rows or columns (up to 124)
+    and rotations go through the library's block kernels (sg4_block_gram,
+    sg4_block_combine, on the operator's plan and stream); wider grams through
+    the split-K batched product, which is faster there (10D L=8, us, kernel
+    against library: gram 20 x 20 86 / 320, 100 x 16 283 / 570, 16 x 100 285 /
+    310, 36 x 36 297 / 300, 84 x 84 1110 / 300-600; rotation 20 x 84 245 / 590,
+    36 x 84 352 / 640).
     CPU tensors (host tests of the driver with a dense matrix) use plain
     torch products."""
 
@@ -101,7 +100,7 @@ class _Dense:
         m, n = A.shape
         q = B.shape[0]
         need = C.c_int64()
-        if (m * q > 400 and q > 16) or lib().sg4_block_gram_work(m, q, C.byref(need)) != 0:
+        if (m * q > 400 and min(m, q) > 16) or lib().sg4_block_gram_work(m, q, C.byref(need)) != 0:
             return _gram(A, B)
         if self.work is None or self.work.numel() < need.value:
             self.work = torch.empty(need.value, device=A.device, dtype=torch.float64)
@@ -116,7 +115,7 @@ class _Dense:
         """beta Y + U @ X (into Y when given; U: k x d, X: d rows)"""
         U = torch.as_tensor(U, dtype=torch.float64, device=X.device)
         k, d = U.shape
-        if X.device.type != "cuda" or self.h is None or k > 20 or k * d > 8192:
+        if X.device.type != "cuda" or self.h is None or k * d > 8192:
             R = U @ X
             if Y is None:
                 return R
