@@ -43,12 +43,23 @@ struct Item {
   int16_t v0;
   int8_t lgnv;
   int8_t big;     // second buffer in global scratch (slot) instead of LDS
-  int32_t slot;
+  int32_t slot;   // split path: index of the term's records
   int32_t pad;
 };
 
+// Split path: a term's header (boff, qoff, wgt as two words each, N, groups) and
+// then one record per group (shape, points P, point stride A, offsets of up to
+// three B and three BtW matrices), read through the scalar cache.  Chasing
+// TermDev -> MatDev with vector loads instead cost a chain of dependent waits
+// before every pass and 56 VGPRs: 10D L=5 x1 78 -> 43 us, 8D L=6 x1 79 -> 54,
+// 9D L=7 x1 308 -> 207 (results to a block, 256 threads).
+struct SRec { int32_t w[8]; };
+enum { SR_BOFF = 0, SR_QOFF = 2, SR_WGT = 4, SR_N = 6, SR_G = 7 };       // header
+enum { SR_SHAPE = 0, SR_A = 1, SR_B = 2, SR_BTW = 5 };                   // group (shape | P << 8)
+
 struct KArgs {
   const Item* items;
+  const SRec* recs = nullptr;
   const TermDev* terms;
   const MatDev* md;
   const int32_t* map;
@@ -62,6 +73,8 @@ struct KArgs {
   // per result element (two words) and an overflow counter; nullptr: FP64 atomics
   unsigned long long* fx = nullptr;
   unsigned long long* fxflag = nullptr;
+  // the terms' results by place in the map (sg4_rowsum.h), instead of atomics
+  void* out = nullptr;
 };
 
 // Deterministic scatter-add: c * 2^64 as a 128-bit two's complement integer
@@ -108,6 +121,21 @@ enum { OUT_STORE = 0, OUT_ADD = 1, OUT_VSTORE = 2, OUT_SCATTER = 3 };
 
 template <class T>
 using cptr = const __attribute__((address_space(4))) T*;   // scalar (constant) loads
+
+// A work item through the scalar cache.  Vector loads of the item and of its
+// term's record wait for the stores and atomics of the item before (one
+// in-order counter); scalar loads do not.
+__device__ __forceinline__ Item load_item(const Item* items, int w) {
+  cptr<int32_t> p = (cptr<int32_t>)(items + w);
+  Item it;
+  it.term = p[0];
+  const int x = p[1];
+  it.v0 = (int16_t)(x & 0xffff);
+  it.lgnv = (int8_t)((x >> 16) & 0xff);
+  it.big = (int8_t)(x >> 24);
+  it.slot = p[2];
+  return it;
+}
 
 // the value is the same in every lane (it derives from the work item);
 // readfirstlane states that so the pointer can live in scalar registers
@@ -524,6 +552,8 @@ struct KGrad {
 // launches.
 __global__ void k_hpsi_t1s_f64(KArgs a, KMats<double> km);
 __global__ void k_hpsi_t1s_f32(KArgs a, KMats<float> km);
+__global__ void k_hpsi_t1s_out_f64(KArgs a, KMats<double> km);   // results to a.out
+__global__ void k_hpsi_t1s_out_f32(KArgs a, KMats<float> km);
 __global__ void k_hpsi_t1_f64(KArgs a, KMats<double> km);
 __global__ void k_hpsi_t1_f32(KArgs a, KMats<float> km);
 __global__ void k_hpsi_t10_f64(PArgs a, KMats10 km);

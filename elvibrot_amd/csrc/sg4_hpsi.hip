@@ -37,6 +37,7 @@
 
 #include "sg4_mfma.h"
 #include "sg4_nmode.h"
+#include "sg4_rowsum.h"
 
 namespace sg4 {
 
@@ -268,9 +269,14 @@ struct ItemPlan {
 // calls of fewer applies keep the term kernels.
 constexpr int64_t NM_MIN_APPLIES = 24;
 
+constexpr int64_t XCD_BLOCK = 16 << 20;   // bytes of a block of vectors (default_cfg)
+constexpr int64_t ROWSUM_MIN = 1 << 16;   // places of the map (use_rowsum)
+constexpr int ROWSUM_AFTER = 8;           // applies of the term kernels before it
+constexpr int LARGE_THREADS = 512;        // threads for the terms beyond the LDS budget
+
 // Launch configuration of the H.psi kernel; chosen by sg4_plan_autotune.
 struct LaunchCfg {
-  int nthreads = 256;          // 256 or 512
+  int nthreads = 256;          // 256 or 512 (default_cfg: from 64)
   int lds_budget = LDS_SMALL;  // bytes of work buffers per workgroup
   int grid = 0;                // 0: one workgroup per item, else persistent grid
   int xcd = 0;                 // 1: keep the items of a term on one XCD; k >= 2: keep a
@@ -307,9 +313,13 @@ struct sg4_plan {
   bool have_qw = false;
   bool f32_valid = false;
   int64_t nmats = 0;
+  sg4::DevBuf d_recs;                    // split path: records of the terms (ensure_recs)
+  std::vector<int32_t> h_rec0;           // first record of each term
+  bool recs_valid = false;
   sg4::DevBuf d_rows_in, d_rows_out, d_cols_in, d_cols_out;
   std::map<int64_t, std::unique_ptr<sg4::ItemPlan>> items;  // per (nvec, size, budget, order)
   std::map<int, sg4::LaunchCfg> tuned;                       // per (nvec, precision)
+  std::map<int, sg4::LaunchCfg> defaults;                    // likewise, of default_cfg
   hipStream_t own_stream = nullptr;                          // for graph capture on the null stream
   struct GraphEntry { int nvec, prec; const double* psi; double* hpsi; hipGraphExec_t exec; };
   std::vector<GraphEntry> graphs;
@@ -324,6 +334,8 @@ struct sg4_plan {
   // overflow counter at the end
   bool deterministic = false;
   sg4::DevBuf d_fx;
+  int term_applies = 0;      // applies of the term kernels, up to ROWSUM_AFTER
+  sg4::RowSum rowsum;        // sums over the terms without atomics (use_rowsum)
   // general type-1 operator (type_op 11): derivative terms and their grids
   int nder = 0;
   sg4::DevBuf d_der, d_F;
@@ -702,6 +714,8 @@ static int build_points(sg4_plan* P) {
 
 static int build_terms(sg4_plan* P) {
   P->mfma_valid = false;
+  P->recs_valid = false;
+  P->defaults.clear();
   P->flops_split = 0.0;
   P->h_terms.resize(P->nterms);
   std::vector<double> ck = P->h_ck;
@@ -827,6 +841,49 @@ static std::vector<Item> order_items(const sg4_plan* P, const std::vector<HItem>
   return h;
 }
 
+// The records the split kernels read of a term (see SRec).
+static int ensure_recs(sg4_plan* P) {
+  if (P->recs_valid) return SG4_OK;
+  if (P->no_alloc) return not_prepared();
+  std::vector<SRec> rec;
+  rec.reserve(P->nterms * 4);
+  P->h_rec0.resize(P->nterms);
+  auto words = [](SRec& r, int i, const void* v) { std::memcpy(&r.w[i], v, 8); };
+  for (int64_t t = 0; t < P->nterms; ++t) {
+    const TermDev& T = P->h_terms[t];
+    P->h_rec0[t] = (int32_t)rec.size();
+    SRec h{};
+    words(h, SR_BOFF, &T.boff);
+    words(h, SR_QOFF, &T.qoff);
+    words(h, SR_WGT, &T.wgt);
+    h.w[SR_N] = T.nq;
+    const int G = T.nact ? T.ngrp : 0;
+    h.w[SR_G] = G;
+    rec.push_back(h);
+    int A = 1;
+    for (int g = 0; g < G; ++g) {
+      const int p0 = T.gfirst[g], p1 = g + 1 < G ? T.gfirst[g + 1] : T.nact;
+      SRec r{};
+      int np = 1;
+      for (int q = 0; q < 3; ++q) {
+        const MatDev& m = P->h_md[T.mat[p0 + q < p1 ? p0 + q : p0]];
+        if (p0 + q < p1) np *= m.nq;
+        r.w[SR_B + q] = (int32_t)m.B;
+        r.w[SR_BTW + q] = (int32_t)m.BtW;
+      }
+      r.w[SR_SHAPE] = T.gshape[g] | np << 8;
+      r.w[SR_A] = A;
+      rec.push_back(r);
+      A *= np;
+    }
+  }
+  int rc = P->d_recs.alloc(sizeof(SRec) * rec.size());
+  if (rc) return rc;
+  HIP_TRY(hipMemcpy(P->d_recs.p, rec.data(), sizeof(SRec) * rec.size(), hipMemcpyHostToDevice));
+  P->recs_valid = true;
+  return SG4_OK;
+}
+
 // Work items for a block of nvec vectors: for every term the vectors are cut
 // into power-of-two chunks so that the work buffers fit the LDS budget; a
 // term too large for that even with one vector keeps its second buffer in a
@@ -848,6 +905,8 @@ static int get_items(sg4_plan* P, int nvec, int esize, ItemPlan** out, int nbuf_
   auto itp = P->items.find(key);
   if (itp != P->items.end()) { *out = itp->second.get(); return SG4_OK; }
   if (P->no_alloc) return not_prepared();
+  if (split)
+    if (int rc = ensure_recs(P)) return rc;
   std::vector<HItem> all;
   double flops_main = 0;
   all.reserve(P->nterms * 2);
@@ -872,6 +931,7 @@ static int get_items(sg4_plan* P, int nvec, int esize, ItemPlan** out, int nbuf_
         h.it.term = (int32_t)t;
         h.it.v0 = (int16_t)v0;
         h.it.lgnv = (int8_t)g;
+        h.it.slot = P->h_rec0[t];
         h.cost = work * (1 << g);
         h.large = large;
         if (!large) {   // basis->grid + grid->basis products and the potential
@@ -1295,12 +1355,50 @@ static bool use_nmode(const sg4_plan* P, int prec) {
          use_split_alg(P);
 }
 
+// Launch of the term kernels when nothing is tuned or set and the results go
+// to a block (use_rowsum).  The kernels wait for latencies, so the LDS budget
+// is what lets their registers fill the CU: FP64 three workgroups of 256 (9D
+// L=7 x8 337 us; 64 KiB 406, 40 KiB 397), FP32 five (265; 64 KiB 323, 40 KiB
+// 287), split precision four (240; 64 KiB 260, 32 KiB 242), there less where
+// the largest item would be more than 2.5 times a fair share of the whole among
+// 1024 workgroups (6D L=6 x16: 39 -> 27 us; FP64 and FP32 gain nothing sure).  A workgroup is about as wide as its largest item has slabs of 27
+// points: 10D L=5 x1 26.4 / 31.6 / 43 us with 64 / 128 / 256 threads, 8D L=6
+// x2 42.1 / 42.4 / 57, 9D L=7 x8 412 / 345 / 327.  Blocks beyond the L2s keep a class of terms on one
+// XCD (10D L=8 x16 6.1 -> 4.7 ms, 10D L=7 x8 656 -> 629 us, 8D L=6 x32 in
+// FP32 94 -> 99).  With atomics the smaller budgets only add contention (10D
+// L=8 x16 9.1 -> 11.4 ms).
+static LaunchCfg default_cfg(sg4_plan* P, int nvec, int prec) {
+  const int key = nvec * 16 + prec;
+  auto it = P->defaults.find(key);
+  if (it != P->defaults.end()) return it->second;
+  LaunchCfg c;
+  const int64_t esize = prec == SG4_PREC_FP64 ? 8 : 4;
+  c.lds_budget = (prec == SG4_PREC_FP64 ? 53 : prec == SG4_PREC_F32 ? 32 : 40) * 1024;
+  if (prec == SG4_PREC_F32X2) {
+    const int64_t fair = 5 * (P->sum_nb * nvec / 1024) / 2 * esize;
+    c.lds_budget = (int)std::min<int64_t>(c.lds_budget, std::max<int64_t>(fair, 16 * 1024));
+  }
+  if (P->D >= 6 && P->nb_ba * nvec * 8 > XCD_BLOCK) c.xcd = 3;
+  if (prec != SG4_PREC_F32X2) {
+    int64_t e = 0;
+    for (const TermDev& T : P->h_terms) {
+      int g = 0;
+      while ((2 << g) <= nvec && ((2 << g) + 1) * T.nq * esize + 4 * T.nq <= c.lds_budget) ++g;
+      e = std::max(e, (int64_t)T.nq << g);
+    }
+    c.nthreads = e <= 64 * 27 ? 64 : e <= (esize == 8 ? 4900 : 3456) ? 128 : 256;
+  }
+  P->defaults[key] = c;
+  return c;
+}
+
 // Launch configuration for (nvec, prec): the one tuned or set for it, else
 // the one set for the nearest block width of the same precision (the
 // narrowest wider one first): the best launch shape depends on the term set
 // far more than on the block width, so a block of 8 vectors in a Davidson
-// iteration runs with the launch tuned for 16.  Defaults when none is set.
-static LaunchCfg cfg_for(const sg4_plan* P, int nvec, int prec) {
+// iteration runs with the launch tuned for 16.  When none is set: default_cfg
+// if the terms' results are summed row by row, else LaunchCfg's values.
+static LaunchCfg cfg_for(sg4_plan* P, int nvec, int prec, bool rowsum) {
   auto it = P->tuned.find(nvec * 16 + prec);
   if (it != P->tuned.end()) return it->second;
   const LaunchCfg* best = nullptr;
@@ -1311,7 +1409,35 @@ static LaunchCfg cfg_for(const sg4_plan* P, int nvec, int prec) {
     const bool better = !best || (w > nvec && (bw < nvec || w < bw)) || (w < nvec && bw < nvec && w > bw);
     if (better) { best = &kv.second; bw = w; }
   }
-  return best ? *best : LaunchCfg{};
+  return best ? *best : rowsum ? default_cfg(P, nvec, prec) : LaunchCfg{};
+}
+
+// The block for the terms' results when they are summed row by row, or null:
+// the kernels then add into H.psi with atomics, ~187 G/s on the whole chip
+// whatever their addresses.  Storing and summing moves a result twice instead
+// of once but streams: split precision 8D L=6 x2 62 -> 33 us, x16 131 -> 80,
+// 9D L=7 x8 355 -> 281, 10D L=8 x16 (256 threads) 7.7 -> 3.9 ms; FP64 8D L=6 x1
+// 71 -> 54, 9D L=6 x16 198 -> 148.  Small term sets would only pay for the
+// launch: 6D L=5 (26 k places) x1 / x4 15.6 -> 15.7 / 14.3 -> 16.8 us, 6D L=6
+// (94 k) 27.1 -> 19.2 / 26.4 -> 21.1.
+// The inverted map costs as much as the sums save in some ten applies (9D L=7
+// 2.7 ms against 0.13 per apply of 5 vectors), so a plan builds it at the apply
+// after ROWSUM_AFTER, or for a graph (now).
+// The block belongs to the plan's stream: an apply that the caller captures
+// keeps the atomics, since its graph may run beside the plan's other work.
+static void* use_rowsum(sg4_plan* P, int nvec, int prec, bool now = false) {
+  if (P->deterministic || !use_split_for(P, prec) || P->sum_nb < ROWSUM_MIN) return nullptr;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const bool busy = hipStreamIsCapturing(P->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+  if (busy) (void)hipGetLastError();
+  if (busy && (!P->own_stream || P->stream != P->own_stream)) return nullptr;
+  const bool alloc = !P->no_alloc && !busy;
+  if (alloc && !P->rowsum.tried && !now && P->term_applies++ < ROWSUM_AFTER) return nullptr;
+  if (alloc && rowsum_build(P->rowsum, P->d_map.as<int32_t>(), P->sum_nb, P->nb_ba, P->d_terms.as<TermDev>(),
+                            P->h_terms, P->stream))
+    return nullptr;
+  if (!P->rowsum.ok) return nullptr;
+  return rowsum_block(P->rowsum, P->stream, (size_t)P->sum_nb * nvec * (prec == SG4_PREC_FP64 ? 8 : 4), alloc);
 }
 
 // Everything an apply needs that may allocate or copy (FP32 copies, item
@@ -1338,6 +1464,14 @@ static int prepare(sg4_plan* P, int nvec, int prec, const LaunchCfg& cfg, ItemPl
     return get_items_mfma(P, nvec, cfg.lds_budget, cfg.xcd, ip);
   }
   return get_items(P, nvec, esize, ip, 0, cfg.lds_budget, cfg.xcd, use_split(P));
+}
+
+// The same, and the lists of an apply with atomics beside those of one without
+// (a captured apply finds them prepared).
+static int prepare_all(sg4_plan* P, int nvec, int prec, const LaunchCfg& cfg, bool one, ItemPlan** ip) {
+  int rc;
+  if (!one && !P->no_alloc && (rc = prepare(P, nvec, prec, cfg_for(P, nvec, prec, false), ip))) return rc;
+  return prepare(P, nvec, prec, cfg, ip);
 }
 
 // Width of the rows-layout staging block of a column-major apply of nvec
@@ -1452,9 +1586,10 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
   if ((rc = check_apply(P, nvec, prec))) return rc;
   if (P->type_op != 1) return apply_points(P, nvec, nvec, psi, hpsi, nvec, 1);
   if (use_nmode(P, prec)) return apply_nmode(P, nvec, nvec, psi, hpsi, nullptr, nullptr);
-  const LaunchCfg cfg = cfgp ? *cfgp : cfg_for(P, nvec, prec);
+  void* out = use_rowsum(P, nvec, prec);
+  const LaunchCfg cfg = cfgp ? *cfgp : cfg_for(P, nvec, prec, out != nullptr);
   ItemPlan* ip = nullptr;
-  if ((rc = prepare(P, nvec, prec, cfg, &ip))) return rc;
+  if ((rc = prepare_all(P, nvec, prec, cfg, cfgp || !out, &ip))) return rc;
   const int esize = (prec == SG4_PREC_FP64) ? 8 : 4;
   const int64_t n = P->nb_ba * nvec;
   const bool split = use_split_for(P, prec);
@@ -1502,16 +1637,18 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
     m.fx = fx;
     m.fxflag = fxflag;
     m.nvec = nvec;
-    for (int list = 0; list < 2; ++list) {
+    m.out = (float*)out;
+    for (int list = 1; list >= 0; --list) {
       const int64_t ni = list ? ip->nitems2 : ip->nitems;
       if (P->timing && list == 0) HIP_TRY(hipEventRecord(P->ev0, P->stream));
       if (ni > 0) {
         m.nitems = (int)ni;
         m.items = list ? ip->items2.as<Item>() : ip->items.as<Item>();
         const unsigned gr = (unsigned)((cfg.grid > 0 && cfg.grid < ni) ? cfg.grid : ni);
-        hipLaunchKernelGGL(k_hpsi_mfma, dim3(gr), dim3(std::min(cfg.nthreads, NT_MFMA)),
+        hipLaunchKernelGGL(out ? k_hpsi_mfma_out : k_hpsi_mfma, dim3(gr), dim3(list ? std::max(cfg.nthreads, LARGE_THREADS) : cfg.nthreads),
                            list ? ip->lds2 : ip->lds, P->stream, m);
       }
+      if (out && list == 0 && (rc = rowsum_add(P->rowsum, m.out, nvec, hpsi, P->stream))) return rc;
       if (P->timing && list == 0) HIP_TRY(hipEventRecord(P->ev1, P->stream));
     }
     if (fx)
@@ -1523,27 +1660,28 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
   if (split) {
     // kinetic rows (initialise hpsi), then the potential part of the terms
     if ((rc = nmode_apply(P->kin, nvec, psi, hpsi, P->stream))) return rc;
-    for (int list = 0; list < 2; ++list) {
+    a.out = out;
+    a.recs = P->d_recs.as<SRec>();
+    for (int list = 1; list >= 0; --list) {
       const int64_t ni = list ? ip->nitems2 : ip->nitems;
-      if (ni == 0) {
-        if (P->timing && list == 0) {
-          HIP_TRY(hipEventRecord(P->ev0, P->stream));
-          HIP_TRY(hipEventRecord(P->ev1, P->stream));
-        }
-        continue;
-      }
+      if (P->timing && list == 0) HIP_TRY(hipEventRecord(P->ev0, P->stream));
       KArgs b = a;
       b.nitems = (int)ni;
       b.items = list ? ip->items2.as<Item>() : ip->items.as<Item>();
       const unsigned gr = (unsigned)((cfg.grid > 0 && cfg.grid < ni) ? cfg.grid : ni);
       const int lds = list ? ip->lds2 : ip->lds;
-      if (P->timing && list == 0) HIP_TRY(hipEventRecord(P->ev0, P->stream));
-      if (esize == 8) {
+      if (ni == 0) {
+      } else if (esize == 8) {
         KMats<double> km{P->d_mats.as<double>(), P->d_V.as<double>(), P->d_ck.as<double>()};
-        hipLaunchKernelGGL(k_hpsi_t1s_f64, dim3(gr), blk, lds, P->stream, b, km);
+        hipLaunchKernelGGL(out ? k_hpsi_t1s_out_f64 : k_hpsi_t1s_f64, dim3(gr), list ? dim3(std::max(cfg.nthreads, LARGE_THREADS)) : blk, lds, P->stream, b, km);
       } else {
         KMats<float> km{P->d_mats32.as<float>(), P->d_V32.as<float>(), P->d_ck32.as<float>()};
-        hipLaunchKernelGGL(k_hpsi_t1s_f32, dim3(gr), blk, lds, P->stream, b, km);
+        hipLaunchKernelGGL(out ? k_hpsi_t1s_out_f32 : k_hpsi_t1s_f32, dim3(gr), list ? dim3(std::max(cfg.nthreads, LARGE_THREADS)) : blk, lds, P->stream, b, km);
+      }
+      if (out && list == 0) {
+        rc = esize == 8 ? rowsum_add(P->rowsum, (const double*)out, nvec, hpsi, P->stream)
+                        : rowsum_add(P->rowsum, (const float*)out, nvec, hpsi, P->stream);
+        if (rc) return rc;
       }
       if (P->timing && list == 0) HIP_TRY(hipEventRecord(P->ev1, P->stream));
     }
@@ -1757,6 +1895,12 @@ int sg4_plan_create_batch(int32_t ninst, const sg4_tables* tabs, int32_t max_nve
     (void)hipFuncSetAttribute((const void*)k_hpsi_t1s_f64,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     (void)hipFuncSetAttribute((const void*)k_hpsi_t1s_f32,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
+    (void)hipFuncSetAttribute((const void*)k_hpsi_t1s_out_f64,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
+    (void)hipFuncSetAttribute((const void*)k_hpsi_t1s_out_f32,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
+    (void)hipFuncSetAttribute((const void*)k_hpsi_mfma_out,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     (void)hipFuncSetAttribute((const void*)k_hpsi_t10_f64,
                               hipFuncAttributeMaxDynamicSharedMemorySize, POINT_LDS_MAX);
@@ -2344,8 +2488,9 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
 
 int sg4_plan_config(const sg4_plan* p, int32_t nvec, int32_t prec, int32_t* cfg4) {
   if (!p || !cfg4) { set_error("null argument"); return SG4_ERR_ARG; }
-  const LaunchCfg c = cfg_for(p, nvec, prec);
-  cfg4[0] = c.nthreads; cfg4[1] = c.lds_budget; cfg4[2] = c.grid; cfg4[3] = c.xcd;
+  sg4_plan* q = const_cast<sg4_plan*>(p);   // default_cfg keeps what it derives
+  const LaunchCfg c = cfg_for(q, nvec, prec, !p->deterministic && use_split_for(p, prec));
+  cfg4[0] = std::max(c.nthreads, 256); cfg4[1] = c.lds_budget; cfg4[2] = c.grid; cfg4[3] = c.xcd;
   return SG4_OK;
 }
 
@@ -2380,9 +2525,14 @@ int sg4_apply_graph(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi, 
     if (e.nvec == nvec && e.prec == prec && e.psi == psi && e.hpsi == hpsi) g = &e;
   if (!g) {
     ItemPlan* ip = nullptr;
-    if ((rc = prepare(p, nvec, prec, cfg_for(p, nvec, prec), &ip))) return rc;
     HIP_TRY(hipStreamSynchronize(user));
     const bool timing = p->timing;
+    p->stream = p->own_stream;
+    const bool sums = p->type_op == 1 && !use_nmode(p, prec) && use_rowsum(p, nvec, prec, true);
+    rc = prepare(p, nvec, prec, cfg_for(p, nvec, prec, sums), &ip);
+    p->stream = user;
+    if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(p->own_stream));
     p->timing = false;
     p->stream = p->own_stream;
     hipGraph_t graph;

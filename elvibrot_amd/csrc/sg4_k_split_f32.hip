@@ -4,6 +4,7 @@
 
 namespace sg4 {
 
-__global__ __launch_bounds__(NT32) void k_hpsi_t1s_f32(KArgs a, KMats<float> km) { split_items(a, km); }
+__global__ __launch_bounds__(NT32) void k_hpsi_t1s_f32(KArgs a, KMats<float> km) { split_items<float, false>(a, km); }
+__global__ __launch_bounds__(NT32) void k_hpsi_t1s_out_f32(KArgs a, KMats<float> km) { split_items<float, true>(a, km); }
 
 }  // namespace sg4

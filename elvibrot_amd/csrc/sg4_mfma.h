@@ -63,6 +63,7 @@ struct MArgs {
   double* hpsi;           // rows layout H.psi (holds the kinetic part; terms are added)
   unsigned long long* fx;       // deterministic accumulator (or nullptr), see fx_add
   unsigned long long* fxflag;
+  float* out;                   // the terms' results by place in the map (sg4_rowsum.h)
   int nvec;
   int nitems;
 };
@@ -159,7 +160,7 @@ __device__ __forceinline__ int slot_k(int j, int s) {
 }
 
 enum { MIN_LDS = 0, MIN_GATHER = 1 };
-enum { MOUT_LDS = 0, MOUT_SCATTER = 1 };
+enum { MOUT_LDS = 0, MOUT_SCATTER = 1, MOUT_PLACE = 2 };
 
 // LDS row stride (floats) of an item with nv vectors: nv + 4 from 16 vectors
 // on (20, 36, 68), so that the four lane groups of a B-operand read (rows 4A
@@ -174,6 +175,7 @@ struct MCtx {
   const uint16_t* matB;     // fused pass: grid->basis matrix
   const double* psi;
   double* hpsi;
+  float* out;               // MOUT_PLACE: the term's results by place, from vector v0 on
   unsigned long long* fx;
   unsigned long long* fxflag;
   uint32_t dummy;           // byte address of a per-lane scratch word (masked-out rows)
@@ -268,6 +270,10 @@ __device__ __forceinline__ void mpass(const MCtx& c) {
         const uint32_t ad = kval[s] ? base + kofb[s] : c.dummy;
         *(__attribute__((address_space(3))) float*)(uintptr_t)ad = y[s >> 2][s & 3];
       }
+    } else if constexpr (OUT == MOUT_PLACE) {
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+        if (cv && kval[s]) c.out[(int64_t)(pb + koff[s]) * c.nvec + v] = y[s >> 2][s & 3];
     } else {
       const uint32_t rowb = (uint32_t)c.nvec * 8u, vb = (uint32_t)(c.v0 + v) * 8u;
 #pragma unroll
@@ -290,8 +296,9 @@ __device__ __forceinline__ void mpass_k(const MCtx& c) {
 }
 
 // The potential part of one term for one chunk of vectors.
+template <int OUT>
 __device__ __forceinline__ void term_mfma(const MArgs& a, const Item& it, float* lds) {
-  const TermM* T = &a.terms[it.term];
+  cptr<TermM> T = (cptr<TermM>)(a.terms + it.term);
   const int lg = it.lgnv, nv = 1 << lg;
   const int32_t* map = a.map + T->boff;
   const float* V = a.V + T->qoff;
@@ -302,7 +309,12 @@ __device__ __forceinline__ void term_mfma(const MArgs& a, const Item& it, float*
     if (m >= 0)
       for (int v = threadIdx.x; v < nv; v += blockDim.x) {
         const int64_t r = (int64_t)m * a.nvec + it.v0 + v;
-        const double val = w * (double)(V[0] * (float)a.psi[r]);
+        const float x = V[0] * (float)a.psi[r];
+        if constexpr (OUT == MOUT_PLACE) {
+          a.out[T->boff * a.nvec + it.v0 + v] = x;
+          continue;
+        }
+        const double val = w * (double)x;
         if (a.fx) fx_add(a.fx + 2 * r, a.fxflag, val);
         else atomicAdd(&a.hpsi[r], val);
       }
@@ -326,6 +338,7 @@ __device__ __forceinline__ void term_mfma(const MArgs& a, const Item& it, float*
   c.dummy = (uint32_t)(uintptr_t)(dummy + (threadIdx.x & 63));
   c.psi = a.psi;
   c.hpsi = a.hpsi;
+  c.out = OUT == MOUT_PLACE ? a.out + T->boff * a.nvec + it.v0 : nullptr;
   c.fx = a.fx;
   c.fxflag = a.fxflag;
   c.nvec = a.nvec;
@@ -348,27 +361,29 @@ __device__ __forceinline__ void term_mfma(const MArgs& a, const Item& it, float*
     __syncthreads();
   }
   set(G - 1, T->mB[G - 1], T->mB[G - 1] + 1);
-  if (G == 1) mpass_k<MIN_GATHER, MOUT_SCATTER, true>(c);
+  if (G == 1) mpass_k<MIN_GATHER, OUT, true>(c);
   else mpass_k<MIN_LDS, MOUT_LDS, true>(c);
   for (int g = G - 2; g >= 0; --g) {
     __syncthreads();
     set(g, T->mB[g] + 1, T->mB[g] + 1);
-    if (g == 0) mpass_k<MIN_LDS, MOUT_SCATTER, false>(c);
+    if (g == 0) mpass_k<MIN_LDS, OUT, false>(c);
     else mpass_k<MIN_LDS, MOUT_LDS, false>(c);
   }
 }
 
+template <int OUT>
 __device__ __forceinline__ void mfma_items(const MArgs& a) {
   extern __shared__ double lds_d[];
   float* lds = (float*)lds_d;
   for (int w = blockIdx.x; w < a.nitems; w += gridDim.x) {
     if (w != (int)blockIdx.x) __syncthreads();   // LDS reuse between items
-    const Item it = a.items[w];
+    const Item it = load_item(a.items, w);
     if (it.term < 0) continue;
-    term_mfma(a, it, lds);
+    term_mfma<OUT>(a, it, lds);
   }
 }
 
 __global__ void k_hpsi_mfma(MArgs a);
+__global__ void k_hpsi_mfma_out(MArgs a);   // results to a.out
 
 }  // namespace sg4

@@ -30,6 +30,7 @@ struct SCtx {
   const int32_t* Ms;     // the term's map, staged in LDS
   const double* psi;     // gather: slabs read from the packed block (group 0 only)
   double* hpsi;          // scatter: slabs added into the packed result (group 0 only)
+  T* out;                // or stored by place in the map
   double w;
   int nvec, v0;
   int gather, scatter;
@@ -39,10 +40,15 @@ struct SCtx {
   int lgnv;
 };
 
+// A result of the output block: FP64 with the term's weight, FP32 without (the
+// row sums multiply it in FP64).
+__device__ __forceinline__ double out_value(double w, double x) { return w * x; }
+__device__ __forceinline__ float out_value(double, float x) { return x; }
+
 // A pass over group 0 (A = 1, AV = nv) may read its slabs straight from the
 // packed block (gather) and add them straight into the result (scatter):
 // element J of slab (b, av) is grid point P b + J, vector av.
-template <class T, int N0, int N1, int N2, bool FUSED>
+template <class T, bool OUT, int N0, int N1, int N2, bool FUSED>
 __device__ __forceinline__ void split_pass(const SCtx<T>& c) {
   constexpr int P = N0 * N1 * N2;
   for (int f = threadIdx.x; f < c.nfib; f += blockDim.x) {
@@ -83,6 +89,10 @@ __device__ __forceinline__ void split_pass(const SCtx<T>& c) {
     if (c.scatter) {
 #pragma unroll
       for (int J = 0; J < P; ++J) {
+        if constexpr (OUT) {
+          c.out[(int64_t)(P * b + J) * c.nvec + av] = out_value(c.w, x[J]);
+          continue;
+        }
         const int m = c.Ms[P * b + J];
         if (m >= 0) atomicAdd(&c.hpsi[(int64_t)m * c.nvec + c.v0 + av], c.w * (double)x[J]);
       }
@@ -93,10 +103,10 @@ __device__ __forceinline__ void split_pass(const SCtx<T>& c) {
   }
 }
 
-template <class T, bool FUSED>
+template <class T, bool OUT, bool FUSED>
 __device__ __forceinline__ void dispatch_split(const SCtx<T>& c, int shape) {
   switch (shape) {
-#define SG4_SCASE(id, a, b, d) case id: split_pass<T, a, b, d, FUSED>(c); return;
+#define SG4_SCASE(id, a, b, d) case id: split_pass<T, OUT, a, b, d, FUSED>(c); return;
     SG4_SHAPES(SG4_SCASE)
 #undef SG4_SCASE
     default: return;
@@ -108,26 +118,34 @@ __device__ __forceinline__ void dispatch_split(const SCtx<T>& c, int shape) {
 // gathering from the packed block) -> fused group G-1 -> grid->basis groups
 // G-2..0 (group 0 scatter-adding into the result).  A term with one group
 // does all of it in one register pass.
-template <class T>
+template <class T, bool OUT>
 __device__ __forceinline__ void term_t1_split(const KArgs& a, const KMats<T>& km, const Item& it,
                                               T* lds) {
-  const TermDev* Td = &a.terms[it.term];
+  cptr<SRec> R = (cptr<SRec>)(a.recs + it.slot);
   const int lg = it.lgnv, nv = 1 << lg;
-  const int32_t* map = a.map + Td->boff;
-  const T* V = km.V + Td->qoff;
-  const double w = Td->wgt;
-  if (Td->nact == 0) {  // the one-point term
+  auto word2 = [&](int i) { return (int64_t)((uint64_t)(uint32_t)R->w[i] | ((uint64_t)(uint32_t)R->w[i + 1] << 32)); };
+  const int64_t boff = word2(SR_BOFF);
+  const int32_t* map = a.map + boff;
+  const T* V = km.V + word2(SR_QOFF);
+  const double w = __longlong_as_double(word2(SR_WGT));
+  const int G = R->w[SR_G];
+  if (G == 0) {  // the one-point term
     const int m = map[0];
     if (m >= 0)
       for (int v = threadIdx.x; v < nv; v += blockDim.x) {
         const int64_t r = (int64_t)m * a.nvec + it.v0 + v;
-        const double val = w * (double)(V[0] * (T)a.psi[r]);
+        const T x = V[0] * (T)a.psi[r];
+        if constexpr (OUT) {
+          ((T*)a.out)[boff * a.nvec + it.v0 + v] = out_value(w, x);
+          continue;
+        }
+        const double val = w * (double)x;
         if (a.fx) fx_add(a.fx + 2 * r, a.fxflag, val);
         else atomicAdd(&a.hpsi[r], val);
       }
     return;
   }
-  const int N = Td->nq;
+  const int N = R->w[SR_N];
   const int NE = N * nv;
   const int nt = blockDim.x;
   T* X = lds;
@@ -152,68 +170,51 @@ __device__ __forceinline__ void term_t1_split(const KArgs& a, const KMats<T>& km
     }
   }
   __syncthreads();
-  const int G = Td->ngrp;
   SCtx<T> c;
   c.X = X;
   c.Vs = Vs;
   c.Ms = Ms;
   c.psi = a.psi;
   c.hpsi = a.hpsi;
+  c.out = OUT ? (T*)a.out + boff * a.nvec + it.v0 : nullptr;
   c.w = w;
   c.nvec = a.nvec;
   c.v0 = it.v0;
   c.lgnv = lg;
-  int Ag[MAXACT];
-  {
-    int A = 1;
-    for (int g = 0; g < G; ++g) {
-      Ag[g] = A;
-      const int p1 = (g + 1 < G) ? Td->gfirst[g + 1] : Td->nact;
-      for (int pm = Td->gfirst[g]; pm < p1; ++pm) A *= a.md[Td->mat[pm]].nq;
-    }
-  }
-  auto setup = [&](int g, bool fused, bool btw) {
-    const int p0 = Td->gfirst[g];
-    const int p1 = (g + 1 < G) ? Td->gfirst[g + 1] : Td->nact;
-    int P = 1;
+  auto setup = [&](int g, bool btw) {
+    cptr<SRec> r = R + 1 + g;
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
-      const int pm = p0 + q;
-      if (pm < p1) {
-        const MatDev* md = &a.md[Td->mat[pm]];
-        P *= md->nq;
-        c.M[q] = km.mats + (btw ? md->BtW : md->B);
-        c.Mt[q] = km.mats + md->BtW;
-      } else {
-        c.M[q] = c.M[0];
-        c.Mt[q] = c.Mt[0];
-      }
+      c.M[q] = km.mats + r->w[(btw ? SR_BTW : SR_B) + q];
+      c.Mt[q] = km.mats + r->w[SR_BTW + q];
     }
-    (void)fused;
-    c.AV = Ag[g] * nv;
+    const int P = r->w[SR_SHAPE] >> 8;
+    c.AV = r->w[SR_A] * nv;
     c.invAV = 1.0f / (float)c.AV;
     c.nfib = NE / P;
+    return r->w[SR_SHAPE] & 255;
   };
   // group 0 gathers; the last grid->basis pass (group 0) scatter-adds (FP64
   // atomics), or, with the deterministic accumulator, leaves its output in X
   // for one fixed-point pass below (kept out of the unrolled shape passes)
   const int scat = (a.fx == nullptr);
   for (int g = 0; g + 1 < G; ++g) {
-    setup(g, false, false);
+    const int shape = setup(g, false);
     c.gather = (g == 0);
     c.scatter = 0;
-    dispatch_split<T, false>(c, Td->gshape[g]);
+    dispatch_split<T, OUT, false>(c, shape);
     __syncthreads();
   }
-  setup(G - 1, true, false);
+  const int shape = setup(G - 1, false);
   c.gather = (G == 1);
   c.scatter = (G == 1) && scat;
-  dispatch_split<T, true>(c, Td->gshape[G - 1]);
+  dispatch_split<T, OUT, true>(c, shape);
   for (int g = G - 2; g >= 0; --g) {
     __syncthreads();
-    setup(g, false, true);
+    const int shape = setup(g, true);
     c.gather = 0;
     c.scatter = (g == 0) && scat;
-    dispatch_split<T, false>(c, Td->gshape[g]);
+    dispatch_split<T, OUT, false>(c, shape);
   }
   if (!scat) {
     // group 0's layout: X[av + nv p] is grid point p, vector av
@@ -226,15 +227,15 @@ __device__ __forceinline__ void term_t1_split(const KArgs& a, const KMats<T>& km
   }
 }
 
-template <class T>
+template <class T, bool OUT>
 __device__ __forceinline__ void split_items(const KArgs& a, const KMats<T>& km) {
   extern __shared__ double lds_d[];
   T* lds = (T*)lds_d;
   for (int w = blockIdx.x; w < a.nitems; w += gridDim.x) {
     if (w != (int)blockIdx.x) __syncthreads();   // LDS reuse between items
-    const Item it = a.items[w];
+    const Item it = load_item(a.items, w);
     if (it.term < 0) continue;
-    term_t1_split<T>(a, km, it, lds);
+    term_t1_split<T, OUT>(a, km, it, lds);
   }
 }
 
