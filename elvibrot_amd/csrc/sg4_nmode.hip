@@ -659,73 +659,106 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
   }
 }
 
-// A Chebyshev order (NModeOrder): y and, for tangents, mu w are formed as
-// above (all slices hold the sums after the exchange), the partner column
-// (re <-> im) is NS lanes away.  One launch per order instead of the kinetic
-// rows, the term kernel and the element-wise order (and, with tangents, the
-// dipole operator's two and a copy): 12 uneven instances, 6 steps of 15 orders
-// 35.4 -> 3.9 ms (30 us an order), the adjoint gradient of 3 small ones 8.6 ->
-// 1.9 ms (4.5 us an order: launch latency).
-template <int NV, int SL, bool TAN>
+struct alignas(8) Two { double x, y; };
+
+// Rows that leave the chip idle with four slices: eight shorten the chain (3
+// small instances 4.0 -> 3.4 us an order, tangents 5.2 -> 4.1; 12 uneven ones,
+// 130 k rows, 19.7 -> 22.3).
+constexpr int64_t ORDER_FEW = 32768;
+
+// A Chebyshev order (NModeOrder).  A lane holds two neighbouring columns (one
+// 16-byte load per entry), NC * SL lanes a row; the row's entries are dealt to
+// SL slices, OU of them in flight per lane, and all slices hold the sums after
+// the exchange.  The partner column (re <-> im) is the lane's other one for one
+// state, NS / 2 lanes away else; mu w comes from NS lanes away.  One launch per
+// order instead of the kinetic rows, the term kernel and the element-wise order
+// (and, with tangents, the dipole operator's two and a copy).  Bound by the
+// latency of the chain row -> column -> vector for small instances and by the
+// gathers for large ones: 12 uneven instances, 6 steps of 15 orders, 35.4 -> 2.9
+// ms, 20 us an order (one column per lane, two entries in flight: 3.9 and 30; SL
+// 2 / 8 / 16: 3.3 / 3.1 / 3.4 ms; 2 or 6 entries: 3.1, 2.9), the adjoint gradient
+// of 3 small ones 8.6 -> 1.8.
+template <int NC, int SL, bool TAN>
 __global__ __launch_bounds__(256) void k_nm_order(const int64_t* __restrict__ ptr,
                                                   const int32_t* __restrict__ col,
                                                   const double* __restrict__ mu, NModeOrder a,
                                                   int64_t rows) {
-  constexpr int W = NV * SL, NS = TAN ? NV / 4 : NV / 2;
-  const int l = threadIdx.x % W, v = l % NV, s = l / NV;
+  constexpr int W = NC * SL, NS = TAN ? NC / 2 : NC, OU = 4;
+  const int l = threadIdx.x % W, j = l % NC, s = l / NC;
   const double* __restrict__ val = a.val;
-  const double* __restrict__ x = a.wk;
+  const Two* __restrict__ x = (const Two*)a.wk;
   // whole waves stay in the loop: the exchanges need every lane of a row
   const int64_t r0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) / W;
   for (int64_t r = r0; r < rows; r += (int64_t)gridDim.x * (256 / W)) {
-    const int64_t e1 = ptr[r + 1];
-    int64_t e = ptr[r] + s;
-    double y0 = 0.0, y1 = 0.0, m0 = 0.0, m1 = 0.0;
-    for (; e + SL < e1; e += 2 * SL) {
-      const double xa = x[(int64_t)col[e] * NV + v], xb = x[(int64_t)col[e + SL] * NV + v];
-      y0 = fma(val[e], xa, y0);
-      y1 = fma(val[e + SL], xb, y1);
-      if constexpr (TAN) {
-        m0 = fma(mu[e], xa, m0);
-        m1 = fma(mu[e + SL], xb, m1);
+    const int64_t e0 = ptr[r], e1 = ptr[r + 1], at = r * NC + j;
+    const bool tan = TAN && j >= NS;
+    const int64_t ai = TAN ? r * NS + (tan ? j - NS : j) : at;
+    Two* acc = (Two*)(tan ? a.tacc : a.acc);
+    Two* out = (Two*)(tan ? a.tout : a.out);
+    const Two xr = x[at];
+    Two wm{0.0, 0.0}, ac{a.c0 * xr.x, a.c0 * xr.y};
+    if (!a.first) {
+      wm = ((const Two*)a.wm)[at];
+      ac = acc[ai];
+    }
+    Two y{0.0, 0.0}, m{0.0, 0.0};
+    for (int64_t e = e0 + s; e < e1; e += OU * SL) {
+      Two xv[OU];
+      double w[OU], u[OU];
+#pragma unroll
+      for (int k = 0; k < OU; ++k) {
+        const int64_t i = min(e + k * SL, e1 - 1);
+        xv[k] = x[(int64_t)col[i] * NC + j];
+        w[k] = val[i];
+        if constexpr (TAN) u[k] = mu[i];
+      }
+#pragma unroll
+      for (int k = 0; k < OU; ++k) {
+        if (e + k * SL >= e1) continue;
+        y.x = fma(w[k], xv[k].x, y.x);
+        y.y = fma(w[k], xv[k].y, y.y);
+        if constexpr (TAN) {
+          m.x = fma(u[k], xv[k].x, m.x);
+          m.y = fma(u[k], xv[k].y, m.y);
+        }
       }
     }
-    if (e < e1) {
-      const double xa = x[(int64_t)col[e] * NV + v];
-      y0 = fma(val[e], xa, y0);
-      if constexpr (TAN) m0 = fma(mu[e], xa, m0);
-    }
-    double y = y0 + y1;
 #pragma unroll
-    for (int o = NV; o < W; o <<= 1) y += __shfl_xor(y, o, 64);
-    const int64_t at = r * NV + v;
-    double z = y - a.E0 * x[at];
-    if constexpr (TAN) {
-      double m = m0 + m1;
-#pragma unroll
-      for (int o = NV; o < W; o <<= 1) m += __shfl_xor(m, o, 64);
-      const double mw = __shfl_xor(m, 2 * NS, 64);
-      if (v >= 2 * NS) z += mw;
+    for (int o = NC; o < W; o <<= 1) {
+      y.x += __shfl_xor(y.x, o, 64);
+      y.y += __shfl_xor(y.y, o, 64);
+      if constexpr (TAN) {
+        m.x += __shfl_xor(m.x, o, 64);
+        m.y += __shfl_xor(m.y, o, 64);
+      }
     }
-    z *= a.sc;
-    const double zp = __shfl_xor(z, NS, 64);
-    const double sg = (v & NS) ? a.sgn : -a.sgn;
-    const double wn = a.first ? sg * zp : fma(2.0 * sg, zp, a.wm[at]);
-    double *acc = a.acc, *out = a.out;
-    int64_t ai = at;
+    Two z{y.x - a.E0 * xr.x, y.y - a.E0 * xr.y};
     if constexpr (TAN) {
-      const bool t = v >= 2 * NS;
-      acc = t ? a.tacc : a.acc;
-      out = t ? a.tout : a.out;
-      ai = r * 2 * NS + (t ? v - 2 * NS : v);
+      const double mx = __shfl_xor(m.x, NS, 64), my = __shfl_xor(m.y, NS, 64);
+      if (tan) {
+        z.x += mx;
+        z.y += my;
+      }
     }
-    const double av = fma(a.c, wn, a.first ? a.c0 * x[at] : acc[ai]);
+    z.x *= a.sc;
+    z.y *= a.sc;
+    // the partner's z and the sign of the imaginary unit on this column
+    const bool im = NS > 1 && (j & (NS / 2));
+    const double sx = im ? a.sgn : -a.sgn, sy = NS == 1 ? a.sgn : sx;
+    Two zp{z.y, z.x};
+    if constexpr (NS > 1) zp = Two{__shfl_xor(z.x, NS / 2, 64), __shfl_xor(z.y, NS / 2, 64)};
+    Two wn{sx * zp.x, sy * zp.y};
+    if (!a.first) wn = Two{fma(2.0 * sx, zp.x, wm.x), fma(2.0 * sy, zp.y, wm.y)};
+    ac.x = fma(a.c, wn.x, ac.x);
+    ac.y = fma(a.c, wn.y, ac.y);
     if (a.last) {
-      const double ap = __shfl_xor(av, NS, 64);
-      if (s == 0) out[ai] = (v & NS) ? av * a.pr + ap * a.pi : av * a.pr - ap * a.pi;
+      Two ap{ac.y, ac.x};
+      if constexpr (NS > 1) ap = Two{__shfl_xor(ac.x, NS / 2, 64), __shfl_xor(ac.y, NS / 2, 64)};
+      const double px = im ? a.pi : -a.pi, py = NS == 1 ? a.pi : px;
+      if (s == 0) out[ai] = Two{ac.x * a.pr + ap.x * px, ac.y * a.pr + ap.y * py};
     } else if (s == 0) {
-      a.wm[at] = wn;
-      acc[ai] = av;
+      ((Two*)a.wm)[at] = wn;
+      acc[ai] = ac;
     }
   }
 }
@@ -1306,17 +1339,21 @@ int nmode_order(const NModeMat& m, const NModeOrder& a, bool tangent, hipStream_
     return dim3((unsigned)std::min<int64_t>((m.rows * w + 255) / 256, (int64_t)1 << 20));
   };
   const int nc = (tangent ? 4 : 2) * a.ns;
-#define SG4_ORDER(NV, SL, TAN) \
-  hipLaunchKernelGGL((k_nm_order<NV, SL, TAN>), grid(NV * SL), dim3(256), 0, st, ptr, col, mu, a, m.rows)
+  const bool few = m.rows <= ORDER_FEW;
+#define SG4_ORDER(NC, SL, TAN) \
+  hipLaunchKernelGGL((k_nm_order<NC, SL, TAN>), grid(NC * SL), dim3(256), 0, st, ptr, col, mu, a, m.rows)
   if (tangent) {
-    if (nc == 4) SG4_ORDER(4, 4, true);
-    else if (nc == 8) SG4_ORDER(8, 2, true);
-    else SG4_ORDER(16, 1, true);
+    if (nc == 4 && few) SG4_ORDER(2, 8, true);
+    else if (nc == 4) SG4_ORDER(2, 4, true);
+    else if (nc == 8) SG4_ORDER(4, 4, true);
+    else SG4_ORDER(8, 2, true);
   } else {
-    if (nc == 2) SG4_ORDER(2, 4, false);
-    else if (nc == 4) SG4_ORDER(4, 4, false);
-    else if (nc == 8) SG4_ORDER(8, 2, false);
-    else SG4_ORDER(16, 1, false);
+    if (nc == 2 && few) SG4_ORDER(1, 8, false);
+    else if (nc == 2) SG4_ORDER(1, 4, false);
+    else if (nc == 4 && few) SG4_ORDER(2, 8, false);
+    else if (nc == 4) SG4_ORDER(2, 4, false);
+    else if (nc == 8) SG4_ORDER(4, 4, false);
+    else SG4_ORDER(8, 2, false);
   }
 #undef SG4_ORDER
   NM_TRY(hipGetLastError());
