@@ -66,12 +66,12 @@ constexpr double TOL_V = 64 * EPS, TOL_M = 16 * EPS;
 // ~9.5 ps in the FP64 term kernel.
 constexpr double NNZ_PER_POINT = 4.0;
 constexpr int64_t NNZ_SMALL = 1 << 18;        // always taken: the apply is one short launch
-// A column-major block is read in place while nnz W^2 <= 2^26 (W columns, a
+// A column-major block is read in place while nnz W^2 <= 2^24 (W columns, a
 // gather touches W lines instead of one), else staged in the rows layout (one
-// more launch).  In place / staged, us: 6D L=6 x16 9.4 / 11.3, 8D L=6 x8
-// 17.8 / 17.8, x16 36.6 / 30.4, 10D L=6 x4 46.9 / 47.8, x8 60.5 / 48.0, 12D L=6
-// x2 50.5 / 52.8, x4 127 / 114.
-constexpr int64_t COLS_DIRECT = (int64_t)1 << 26;
+// more launch).  In place / staged, us: 6D L=6 (160 k entries) x8 6.8 / 7.5, x16
+// 9.3 / 9.4, 8D L=6 (760 k) x4 11.5 / 10.8, x8 17.5 / 15.1, 9D L=7 (5.0 M) x2
+// 31.0 / 28.3.
+constexpr int64_t COLS_DIRECT = (int64_t)1 << 24;
 constexpr int64_t MAX_E = (int64_t)1 << 27;   // entries of the two-mode tables
 
 // Device view of an instance.
@@ -583,6 +583,8 @@ __global__ __launch_bounds__(1024) void k_nm_ptr(const int32_t* cnt, int64_t n, 
   if (i == n - 1) ptr[n] = part[blockIdx.x] + s[threadIdx.x];
 }
 
+struct alignas(8) Two { double x, y; };
+
 // hpsi(r, v) = sum_e val_e psi(col_e, v): NV * SL lanes per row, NV vectors,
 // the row's entries dealt to SL slices that are added at the end.
 // OUT_COLS: the result goes to the column-major block (nvec <= NV columns),
@@ -631,6 +633,88 @@ __global__ __launch_bounds__(256) void k_nm_spmm(const int64_t* __restrict__ ptr
     }
   }
 }
+// The same from a rows-layout block: a lane holds PV pairs of columns (16-byte
+// loads), NC lanes a row and slice, SL slices, SU entries in flight per lane.
+// WIDE: blocks of NV columns of a wider block (blockIdx.y; multiples of 8: 9D
+// L=7 x32 162 -> 112 us; three blocks of 4 at x12 85 -> 127, not taken).  Bound by the rate
+// at which lines are requested: few lanes per line, many entries of a row per
+// wave.  10D L=8 (32 M entries) x16 440 us, x8 286, x4 207, x2 155; with one
+// column per lane 750, 446, 306, 197; one pair 497, 338, 225, 155; two pairs and
+// 1 / 2 / 8 slices at x16 624 / 474 / 437, four pairs 452-528.
+template <int NC, int PV, int SL, int SU, bool COLS, bool WIDE>
+__global__ __launch_bounds__(256) void k_nm_spmm_pairs(const int64_t* __restrict__ ptr,
+                                                       const int32_t* __restrict__ col,
+                                                       const double* __restrict__ val,
+                                                       const double* __restrict__ psi,
+                                                       double* __restrict__ hpsi, int64_t rows, int nvec) {
+  constexpr int W = NC * SL, R = 256 / W, NV = 2 * NC * PV;
+  __shared__ double tile[COLS ? NV * (R + 1) : 1];
+  const int l = threadIdx.x % W, j = l % NC, s = l / NC, rr = threadIdx.x / W;
+  const int64_t r = (int64_t)blockIdx.x * R + rr;
+  const int64_t ld = WIDE ? nvec / 2 : NC * PV;           // pairs per row
+  const int64_t j0 = j + (WIDE ? (int64_t)blockIdx.y * (NC * PV) : 0);
+  const Two* __restrict__ x = (const Two*)psi + j0;
+  Two y[PV];
+#pragma unroll
+  for (int p = 0; p < PV; ++p) y[p] = Two{0.0, 0.0};
+  if (r < rows) {
+    const int64_t e1 = ptr[r + 1];
+    int64_t e = ptr[r] + s;
+    for (; e + (SU - 1) * SL < e1; e += SU * SL) {
+      int32_t c[SU];
+      double w[SU];
+      Two xv[SU][PV];
+#pragma unroll
+      for (int u = 0; u < SU; ++u) { c[u] = col[e + u * SL]; w[u] = val[e + u * SL]; }
+#pragma unroll
+      for (int u = 0; u < SU; ++u)
+#pragma unroll
+        for (int p = 0; p < PV; ++p) xv[u][p] = x[c[u] * ld + p * NC];
+#pragma unroll
+      for (int u = 0; u < SU; ++u)
+#pragma unroll
+        for (int p = 0; p < PV; ++p) {
+          y[p].x = fma(w[u], xv[u][p].x, y[p].x);
+          y[p].y = fma(w[u], xv[u][p].y, y[p].y);
+        }
+    }
+    for (; e < e1; e += SL) {
+      const double w = val[e];
+      const int64_t c = col[e] * ld;
+#pragma unroll
+      for (int p = 0; p < PV; ++p) {
+        const Two xv = x[c + p * NC];
+        y[p].x = fma(w, xv.x, y[p].x);
+        y[p].y = fma(w, xv.y, y[p].y);
+      }
+    }
+  }
+#pragma unroll
+  for (int o = NC; o < W; o <<= 1)
+#pragma unroll
+    for (int p = 0; p < PV; ++p) {
+      y[p].x += __shfl_xor(y[p].x, o, 64);
+      y[p].y += __shfl_xor(y[p].y, o, 64);
+    }
+  if constexpr (!COLS) {
+    if (r < rows && s == 0)
+#pragma unroll
+      for (int p = 0; p < PV; ++p) ((Two*)hpsi)[r * ld + j0 + p * NC] = y[p];
+  } else {
+    if (s == 0)
+#pragma unroll
+      for (int p = 0; p < PV; ++p) {
+        tile[2 * (p * NC + j) * (R + 1) + rr] = y[p].x;
+        tile[(2 * (p * NC + j) + 1) * (R + 1) + rr] = y[p].y;
+      }
+    __syncthreads();
+    for (int t = threadIdx.x; t < NV * R; t += 256) {
+      const int vv = t / R, ro = t % R;
+      const int64_t row = (int64_t)blockIdx.x * R + ro;
+      if (vv < nvec && row < rows) hpsi[(int64_t)vv * rows + row] = tile[vv * (R + 1) + ro];
+    }
+  }
+}
 // any number of vectors: one thread per (row, vector)
 __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__ ptr,
                                                      const int32_t* __restrict__ col,
@@ -658,8 +742,6 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
     hpsi[i] = a0 + a1;
   }
 }
-
-struct alignas(8) Two { double x, y; };
 
 // Rows that leave the chip idle with four slices: eight shorten the chain (3
 // small instances 4.0 -> 3.4 us an order, tangents 5.2 -> 4.1; 12 uneven ones,
@@ -1293,14 +1375,34 @@ int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hi
 #define SG4_SPMM(NV, SL)                                                                              \
   hipLaunchKernelGGL((k_nm_spmm<NV, SL, COLS, IN_COLS>), dim3((unsigned)((m.rows * NV * SL + 255) / 256)),     \
                      dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec)
-  switch (W) {
-    case 1: SG4_SPMM(1, 8); break;
-    case 2: SG4_SPMM(2, 4); break;
-    case 4: SG4_SPMM(4, 4); break;
-    case 8: SG4_SPMM(8, 1); break;
-    case 16: SG4_SPMM(16, 1); break;
-    default: return 1;
+#define SG4_PAIRS(NC, PV, SL, SU, WIDE)                                                                \
+  hipLaunchKernelGGL((k_nm_spmm_pairs<NC, PV, SL, SU, COLS, WIDE>),                                    \
+                     dim3((unsigned)((m.rows * NC * SL + 255) / 256), WIDE ? W / (2 * NC * PV) : 1),   \
+                     dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec)
+  if constexpr (IN_COLS) {
+    switch (W) {
+      case 1: SG4_SPMM(1, 8); break;
+      case 2: SG4_SPMM(2, 4); break;
+      case 4: SG4_SPMM(4, 4); break;
+      case 8: SG4_SPMM(8, 1); break;
+      case 16: SG4_SPMM(16, 1); break;
+      default: return 1;
+    }
+  } else {
+    switch (W) {
+      case 1: SG4_SPMM(1, 8); break;
+      case 2: SG4_PAIRS(1, 1, 8, 2, false); break;
+      case 4: SG4_PAIRS(1, 2, 8, 2, false); break;
+      case 8: SG4_PAIRS(2, 2, 8, 2, false); break;
+      case 16: SG4_PAIRS(4, 2, 4, 2, false); break;
+      default:
+        if constexpr (COLS) return 1;
+        else if (W % 16 == 0) SG4_PAIRS(4, 2, 4, 2, true);
+        else if (W % 8 == 0) SG4_PAIRS(2, 2, 8, 2, true);
+        else return 1;
+    }
   }
+#undef SG4_PAIRS
 #undef SG4_SPMM
   NM_TRY(hipGetLastError());
   return SG4_OK;
