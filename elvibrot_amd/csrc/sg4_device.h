@@ -75,6 +75,7 @@ struct KArgs {
   unsigned long long* fxflag = nullptr;
   // the terms' results by place in the map (sg4_rowsum.h), instead of atomics
   void* out = nullptr;
+  const float* psi32 = nullptr;   // FP32 kernel with out: psi in FP32
 };
 
 // Deterministic scatter-add: c * 2^64 as a 128-bit two's complement integer

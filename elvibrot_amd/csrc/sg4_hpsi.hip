@@ -1412,6 +1412,11 @@ static LaunchCfg cfg_for(sg4_plan* P, int nvec, int prec, bool rowsum) {
   return best ? *best : rowsum ? default_cfg(P, nvec, prec) : LaunchCfg{};
 }
 
+// Bytes of the terms' results; the FP32 mode's copy of psi follows them.
+static size_t rowsum_bytes(const sg4_plan* P, int nvec, int esize) {
+  return ((size_t)P->sum_nb * nvec * esize + 255) & ~(size_t)255;
+}
+
 // The block for the terms' results when they are summed row by row, or null:
 // the kernels then add into H.psi with atomics, ~187 G/s on the whole chip
 // whatever their addresses.  Storing and summing moves a result twice instead
@@ -1437,7 +1442,9 @@ static void* use_rowsum(sg4_plan* P, int nvec, int prec, bool now = false) {
                             P->h_terms, P->stream))
     return nullptr;
   if (!P->rowsum.ok) return nullptr;
-  return rowsum_block(P->rowsum, P->stream, (size_t)P->sum_nb * nvec * (prec == SG4_PREC_FP64 ? 8 : 4), alloc);
+  const size_t bytes = rowsum_bytes(P, nvec, prec == SG4_PREC_FP64 ? 8 : 4) +
+                       (prec == SG4_PREC_F32 ? sizeof(float) * P->nb_ba * nvec : 0);
+  return rowsum_block(P->rowsum, P->stream, bytes, alloc);
 }
 
 // Everything an apply needs that may allocate or copy (FP32 copies, item
@@ -1659,7 +1666,9 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
   }
   if (split) {
     // kinetic rows (initialise hpsi), then the potential part of the terms
-    if ((rc = nmode_apply(P->kin, nvec, psi, hpsi, P->stream))) return rc;
+    float* psi32 = out && esize == 4 ? (float*)((char*)out + rowsum_bytes(P, nvec, esize)) : nullptr;
+    if ((rc = nmode_apply(P->kin, nvec, psi, hpsi, P->stream, nullptr, psi32))) return rc;
+    a.psi32 = psi32;
     a.out = out;
     a.recs = P->d_recs.as<SRec>();
     for (int list = 1; list >= 0; --list) {

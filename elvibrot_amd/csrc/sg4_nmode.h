@@ -62,9 +62,10 @@ int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m);
 // the matrix small enough to pay.  Synchronises the stream.
 int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double* mu, NModeMat& m);
 
-// hpsi = M psi, nvec vectors in the rows layout (val: other values on M's pattern)
+// hpsi = M psi, nvec vectors in the rows layout (val: other values on M's pattern;
+// psi32: psi in FP32, written beside it)
 int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st,
-                const double* val = nullptr);
+                const double* val = nullptr, float* psi32 = nullptr);
 // The same to a column-major result, W >= nvec columns at a time: from a
 // column-major block (small blocks, nmode_cols_direct) or from a rows-layout
 // block of W columns.  1: no kernel for this W.

@@ -595,7 +595,8 @@ __global__ __launch_bounds__(256) void k_nm_spmm(const int64_t* __restrict__ ptr
                                                  const int32_t* __restrict__ col,
                                                  const double* __restrict__ val,
                                                  const double* __restrict__ psi,
-                                                 double* __restrict__ hpsi, int64_t rows, int nvec) {
+                                                 double* __restrict__ hpsi, int64_t rows, int nvec,
+                                                 float* __restrict__ psi32) {
   constexpr int W = NV * SL, R = 256 / W;
   __shared__ double tile[COLS ? NV * (R + 1) : 1];
   const int l = threadIdx.x % W, v = l % NV, s = l / NV;
@@ -621,7 +622,10 @@ __global__ __launch_bounds__(256) void k_nm_spmm(const int64_t* __restrict__ ptr
     a = a0 + a1;
 #pragma unroll
     for (int o = NV; o < W; o <<= 1) a += __shfl_xor(a, o, 64);
-    if (!COLS && s == 0) hpsi[r * NV + v] = a;
+    if (!COLS && s == 0) {
+      hpsi[r * NV + v] = a;
+      if (psi32) psi32[r * NV + v] = (float)psi[r * NV + v];
+    }
   }
   if constexpr (COLS) {
     if (s == 0) tile[v * (R + 1) + threadIdx.x / W] = a;
@@ -646,7 +650,8 @@ __global__ __launch_bounds__(256) void k_nm_spmm_pairs(const int64_t* __restrict
                                                        const int32_t* __restrict__ col,
                                                        const double* __restrict__ val,
                                                        const double* __restrict__ psi,
-                                                       double* __restrict__ hpsi, int64_t rows, int nvec) {
+                                                       double* __restrict__ hpsi, int64_t rows, int nvec,
+                                                       float* __restrict__ psi32) {
   constexpr int W = NC * SL, R = 256 / W, NV = 2 * NC * PV;
   __shared__ double tile[COLS ? NV * (R + 1) : 1];
   const int l = threadIdx.x % W, j = l % NC, s = l / NC, rr = threadIdx.x / W;
@@ -699,7 +704,14 @@ __global__ __launch_bounds__(256) void k_nm_spmm_pairs(const int64_t* __restrict
   if constexpr (!COLS) {
     if (r < rows && s == 0)
 #pragma unroll
-      for (int p = 0; p < PV; ++p) ((Two*)hpsi)[r * ld + j0 + p * NC] = y[p];
+      for (int p = 0; p < PV; ++p) {
+        const int64_t at = r * ld + j0 + p * NC;
+        ((Two*)hpsi)[at] = y[p];
+        if (psi32) {
+          const Two v = ((const Two*)psi)[at];
+          *(float2*)(psi32 + 2 * at) = make_float2((float)v.x, (float)v.y);
+        }
+      }
   } else {
     if (s == 0)
 #pragma unroll
@@ -720,7 +732,8 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
                                                      const int32_t* __restrict__ col,
                                                      const double* __restrict__ val,
                                                      const double* __restrict__ psi,
-                                                     double* __restrict__ hpsi, int64_t rows, int nvec) {
+                                                     double* __restrict__ hpsi, int64_t rows, int nvec,
+                                                     float* __restrict__ psi32) {
   const int64_t n = rows * nvec;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const int64_t r = i / nvec;
@@ -740,6 +753,7 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
     }
     for (; e < e1; ++e) a0 = fma(val[e], psi[(int64_t)col[e] * nvec + v], a0);
     hpsi[i] = a0 + a1;
+    if (psi32) psi32[i] = (float)psi[i];
   }
 }
 
@@ -1369,16 +1383,16 @@ int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double
 namespace {
 template <bool COLS, bool IN_COLS>
 int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st,
-         const double* val) {
+         const double* val, float* psi32 = nullptr) {
   const int64_t* ptr = m.ptr.as<int64_t>();
   const int32_t* col = m.col.as<int32_t>();
 #define SG4_SPMM(NV, SL)                                                                              \
   hipLaunchKernelGGL((k_nm_spmm<NV, SL, COLS, IN_COLS>), dim3((unsigned)((m.rows * NV * SL + 255) / 256)),     \
-                     dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec)
+                     dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec, psi32)
 #define SG4_PAIRS(NC, PV, SL, SU, WIDE)                                                                \
   hipLaunchKernelGGL((k_nm_spmm_pairs<NC, PV, SL, SU, COLS, WIDE>),                                    \
                      dim3((unsigned)((m.rows * NC * SL + 255) / 256), WIDE ? W / (2 * NC * PV) : 1),   \
-                     dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec)
+                     dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec, psi32)
   if constexpr (IN_COLS) {
     switch (W) {
       case 1: SG4_SPMM(1, 8); break;
@@ -1409,12 +1423,13 @@ int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hi
 }
 }  // namespace
 
-int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st, const double* val) {
+int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st, const double* val,
+                float* psi32) {
   if (!val) val = m.val.as<double>();
-  const int rc = spmm<false, false>(m, nvec, nvec, psi, hpsi, st, val);
+  const int rc = spmm<false, false>(m, nvec, nvec, psi, hpsi, st, val, psi32);
   if (rc <= 0) return rc;
   hipLaunchKernelGGL(k_nm_spmm_any, dim3((unsigned)std::min<int64_t>((m.rows * nvec + 255) / 256, (int64_t)1 << 20)),
-                     dim3(256), 0, st, m.ptr.as<int64_t>(), m.col.as<int32_t>(), val, psi, hpsi, m.rows, nvec);
+                     dim3(256), 0, st, m.ptr.as<int64_t>(), m.col.as<int32_t>(), val, psi, hpsi, m.rows, nvec, psi32);
   NM_TRY(hipGetLastError());
   return SG4_OK;
 }

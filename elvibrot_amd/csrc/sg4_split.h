@@ -29,6 +29,7 @@ struct SCtx {
   const T* Vs;
   const int32_t* Ms;     // the term's map, staged in LDS
   const double* psi;     // gather: slabs read from the packed block (group 0 only)
+  const float* psi32;    // FP32 with OUT: from its FP32 copy
   double* hpsi;          // scatter: slabs added into the packed result (group 0 only)
   T* out;                // or stored by place in the map
   double w;
@@ -45,6 +46,11 @@ struct SCtx {
 __device__ __forceinline__ double out_value(double w, double x) { return w * x; }
 __device__ __forceinline__ float out_value(double, float x) { return x; }
 
+// The FP32 kernel that stores its results gathers from an FP32 copy of psi (a
+// by-product of the kinetic rows, the same rounding): 27 loads of 8 bytes a slab
+// held twice the registers and lines (8D L=6 x24 107 -> 91 us, 9D L=7 x8 262 ->
+// 225; split precision gains 0-2 % and reads psi).
+//
 // A pass over group 0 (A = 1, AV = nv) may read its slabs straight from the
 // packed block (gather) and add them straight into the result (scatter):
 // element J of slab (b, av) is grid point P b + J, vector av.
@@ -60,7 +66,9 @@ __device__ __forceinline__ void split_pass(const SCtx<T>& c) {
 #pragma unroll
       for (int J = 0; J < P; ++J) {
         const int m = c.Ms[P * b + J];
-        x[J] = (m >= 0) ? (T)c.psi[(int64_t)m * c.nvec + c.v0 + av] : (T)0;
+        const int64_t r = (int64_t)m * c.nvec + c.v0 + av;
+        if constexpr (OUT && sizeof(T) == 4) x[J] = (m >= 0) ? c.psi32[r] : 0.0f;
+        else x[J] = (m >= 0) ? (T)c.psi[r] : (T)0;
       }
     } else {
 #pragma unroll
@@ -175,6 +183,7 @@ __device__ __forceinline__ void term_t1_split(const KArgs& a, const KMats<T>& km
   c.Vs = Vs;
   c.Ms = Ms;
   c.psi = a.psi;
+  c.psi32 = a.psi32;
   c.hpsi = a.hpsi;
   c.out = OUT ? (T*)a.out + boff * a.nvec + it.v0 : nullptr;
   c.w = w;
