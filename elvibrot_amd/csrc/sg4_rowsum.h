@@ -19,6 +19,7 @@ struct RowSum {
   int64_t nseg = 0;
   int shift = 0, nw = 0;
   DevBuf pos;      // uint32, rows after rows: place | (index of its term's weight << shift)
+  DevBuf wi;       // uint8 weight indices where they do not fit beside the place (shift = 32)
   DevBuf wtab;     // the distinct term weights
   DevBuf seg;      // int32: nseg + 1 starts in pos, then nseg rows
   // the terms' results of one apply, one block per stream; a block stays until

@@ -20,7 +20,7 @@ constexpr int RS_SEG = 64;                       // places per segment (one per 
 constexpr int RS_LOADS = 8;                      // places in flight per lane
 constexpr int RS_LANES = 4;                      // log2 of the lanes per segment, at least
 constexpr int RS_BATCH = 8;                      // fill launches
-constexpr size_t RS_MAX_BYTES = size_t(8) << 30; // results held per plan
+constexpr size_t RS_MAX_BYTES = size_t(16) << 30; // results held per plan
 constexpr size_t RS_MAX_BLOCKS = 8;
 constexpr int RS_WEIGHTS = 256;                 // distinct term weights
 constexpr uint32_t RS_MULTI = 0x80000000u;
@@ -83,34 +83,40 @@ __global__ __launch_bounds__(256) void k_rs_first(const int32_t* map, const int3
 
 // places of the terms [t0, t1); the launches go up the terms
 __global__ __launch_bounds__(256) void k_rs_fill(const int32_t* map, const TermDev* terms, const uint8_t* tw,
-                                                 int64_t t0, int64_t t1, int shift, int32_t* cursor, uint32_t* pos) {
+                                                 int64_t t0, int64_t t1, int shift, int32_t* cursor, uint32_t* pos,
+                                                 uint8_t* wi) {
   for (int64_t t = t0 + blockIdx.x; t < t1; t += gridDim.x) {
     const int64_t b = terms[t].boff;
     const int n = terms[t].nb;
-    const uint32_t w = (uint32_t)((uint64_t)tw[t] << shift);
+    const uint32_t w = wi ? 0u : (uint32_t)((uint64_t)tw[t] << shift);
     for (int p = threadIdx.x; p < n; p += 256) {
       const int m = map[b + p];
-      if (m >= 0) pos[atomicAdd(&cursor[m], 1)] = (uint32_t)(b + p) | w;
+      if (m < 0) continue;
+      const int e = atomicAdd(&cursor[m], 1);
+      pos[e] = (uint32_t)(b + p) | w;
+      if (wi) wi[e] = tw[t];
     }
   }
 }
 
 // one wave per segment: its places in increasing order
-__global__ __launch_bounds__(256) void k_rs_sort(uint32_t* pos, const int32_t* seg, int64_t nseg, uint32_t mask) {
+__global__ __launch_bounds__(256) void k_rs_sort(uint32_t* pos, uint8_t* wi, const int32_t* seg, int64_t nseg,
+                                                 uint32_t mask) {
   const int64_t s = (blockIdx.x * 256LL + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   if (s >= nseg) return;                // whole waves
   const int e = seg[s] + lane;
   const bool on = e < seg[s + 1];
   const uint32_t full = on ? pos[e] : 0u;
-  uint32_t key = on ? (full & mask) : 0xffffffffu, val = full;
+  uint32_t key = on ? (full & mask) : 0xffffffffu, val = full, w = on && wi ? wi[e] : 0u;
   for (int k = 2; k <= 64; k <<= 1)
     for (int j = k >> 1; j > 0; j >>= 1) {
-      const uint32_t ok = __shfl_xor(key, j), ov = __shfl_xor(val, j);
+      const uint32_t ok = __shfl_xor(key, j), ov = __shfl_xor(val, j), ow = __shfl_xor(w, j);
       const bool low = ((lane & j) == 0) == ((lane & k) == 0);
-      if (low ? ok < key : ok > key) { key = ok; val = ov; }
+      if (low ? ok < key : ok > key) { key = ok; val = ov; w = ow; }
     }
   if (on) pos[e] = val;
+  if (on && wi) wi[e] = (uint8_t)w;
 }
 
 template <class T, int V> struct alignas(sizeof(T) * V) Pack { T x[V]; };
@@ -119,7 +125,8 @@ template <class T, int V> struct alignas(sizeof(T) * V) Pack { T x[V]; };
 // to 2^ls slices, RS_LOADS places in flight per lane.  A row of one segment is
 // added without an atomic.
 template <class T, int V>
-__global__ __launch_bounds__(256) void k_rs_add(const uint32_t* __restrict__ pos, const double* __restrict__ wtab,
+__global__ __launch_bounds__(256) void k_rs_add(const uint32_t* __restrict__ pos, const uint8_t* __restrict__ wi,
+                                                const double* __restrict__ wtab,
                                                 int nw, int shift, const int32_t* __restrict__ seg, int64_t nseg,
                                                 const T* __restrict__ out, int nvec, int lg, int ls,
                                                 double* hpsi) {
@@ -151,7 +158,7 @@ __global__ __launch_bounds__(256) void k_rs_add(const uint32_t* __restrict__ pos
     for (int k = 0; k < RS_LOADS; ++k) {
       if (e + (k << ls) >= e1) continue;
       double w = 1.0;
-      if constexpr (sizeof(T) == 4) w = wt[(uint64_t)p[k] >> shift];
+      if constexpr (sizeof(T) == 4) w = wt[wi ? wi[e + (k << ls)] : (uint64_t)p[k] >> shift];
 #pragma unroll
       for (int j = 0; j < V; ++j) {
         if constexpr (sizeof(T) == 4) acc[j] += w * (double)x[k].x[j];
@@ -178,7 +185,7 @@ int add(const RowSum& s, const T* out, int nvec, double* hpsi, hipStream_t st) {
   const int ls = RS_LANES > lg ? RS_LANES - lg : 0;
   const int64_t nb = ((s.nseg << (lg + ls)) + 255) / 256;
   hipLaunchKernelGGL((k_rs_add<T, V>), dim3((unsigned)nb, (unsigned)((nvec + (V << lg) - 1) / (V << lg))), dim3(256),
-                     0, st, s.pos.as<uint32_t>(), s.wtab.as<double>(), s.nw, s.shift, s.seg.as<int32_t>(), s.nseg,
+                     0, st, s.pos.as<uint32_t>(), s.wi.as<uint8_t>(), s.wtab.as<double>(), s.nw, s.shift, s.seg.as<int32_t>(), s.nseg,
                      out, nvec, lg, ls, hpsi);
   RS_TRY(hipGetLastError());
   return SG4_OK;
@@ -202,7 +209,8 @@ int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, 
   }
   int shift = 0;
   while (sum_nb >> shift) ++shift;
-  if (((uint64_t)(tab.size() - 1) << shift) >> 32) return SG4_OK;
+  const bool apart = ((uint64_t)(tab.size() - 1) << shift) >> 32;
+  if (apart) shift = 32;
   const int64_t nt = (int64_t)terms.size();
   DevBuf cnt, first, dtw, num, order;
   if (cnt.alloc(4 * (size_t)rows) || first.alloc(4 * (size_t)rows) || order.alloc(4 * (size_t)rows) ||
@@ -246,17 +254,17 @@ int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, 
     at += n;
   }
   sg[nseg] = at;
-  if (s.pos.alloc(4 * (size_t)at) || s.seg.alloc(4 * sg.size())) return SG4_OK;
+  if (s.pos.alloc(4 * (size_t)at) || (apart && s.wi.alloc((size_t)at)) || s.seg.alloc(4 * sg.size())) return SG4_OK;
   RS_TRY(hipMemcpyAsync(cnt.p, c.data(), 4 * (size_t)rows, hipMemcpyHostToDevice, st));
   RS_TRY(hipMemcpyAsync(s.seg.p, sg.data(), 4 * sg.size(), hipMemcpyHostToDevice, st));
   for (int i = 0; i < RS_BATCH; ++i) {
     const int64_t t0 = nt * i / RS_BATCH, t1 = nt * (i + 1) / RS_BATCH;
     if (t1 > t0)
       hipLaunchKernelGGL(k_rs_fill, dim3((unsigned)std::min<int64_t>(t1 - t0, 8192)), blk, 0, st, d_map, d_terms,
-                         dtw.as<uint8_t>(), t0, t1, shift, cnt.as<int32_t>(), s.pos.as<uint32_t>());
+                         dtw.as<uint8_t>(), t0, t1, shift, cnt.as<int32_t>(), s.pos.as<uint32_t>(), s.wi.as<uint8_t>());
   }
   hipLaunchKernelGGL(k_rs_sort, dim3((unsigned)((nseg + 3) / 4)), blk, 0, st, s.pos.as<uint32_t>(),
-                     s.seg.as<int32_t>(), nseg, (uint32_t)((1ull << shift) - 1));
+                     s.wi.as<uint8_t>(), s.seg.as<int32_t>(), nseg, (uint32_t)((1ull << shift) - 1));
   RS_TRY(hipGetLastError());
   RS_TRY(hipStreamSynchronize(st));
   s.nseg = nseg;

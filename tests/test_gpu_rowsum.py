@@ -95,3 +95,18 @@ def test_block_of_a_batch_graphs_and_streams(prec):
     E._capi.check(E.lib().sg4_apply_noalloc(op._h, 4, C.c_void_p(xc.data_ptr()), C.c_void_p(rc.data_ptr()), prec))
     torch.cuda.synchronize()
     assert float((rc.t() - z).abs().max()) <= lim
+
+
+@pytest.mark.parametrize("prec", [E.PREC_F32, E.PREC_F32X2])
+def test_weight_indices_apart_from_the_places(prec):
+    """A batch whose places and distinct term weights do not fit 32 bits
+    together: the weight indices are kept beside the places."""
+    bs = [E.SG4Basis(D, L) for D, L in [(12, 8), (11, 4), (10, 4), (9, 4), (8, 4), (7, 4), (6, 4), (5, 5), (4, 6)]]
+    weights = {float(w) for b in bs for w in b.weights()}
+    assert (len(weights) - 1).bit_length() + sum(b.sum_nb for b in bs).bit_length() > 32
+    op = E.SG4Batch(bs, max_nvec=2)
+    op.set_sparse(False)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(op.nb_ba, 2, device="cuda", dtype=torch.float64, generator=g)
+    y, z = pair(op, x, prec)
+    assert float((y - z).abs().max()) <= tol(max(b.nterms for b in bs), z)
