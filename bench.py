@@ -50,13 +50,14 @@ UNIT = {"fp64": "FP64 VALU (= FP64 MFMA peak)", "f32": "FP32 VALU",
 # threads, LDS budget, persistent grid, item order (3: classes of terms with
 # equal levels in modes 3..D-1 on one XCD; 2: modes 2..D-1)
 PINNED = {(10, 8, 16): {"fp64": (512, 163840, 2048, 3), "f32": (768, 163840, 2048, 2),
-                        "f32x2": (1024, 163840, 512, 2)}}
+                        "f32x2": (512, 81920, 0, 3)}}
 # the propagation workload's 2-column applies (64-instance batch below):
 # sg4_plan_autotune's best launches, timed over whole applies on MI355X
-PINNED_PROP = {"f32x2": (256, 32768, 2048, 3), "fp64": (256, 65536, 0, 3)}
+PINNED_PROP = {"f32x2": (256, 40960, 0, 3), "fp64": (256, 54272, 0, 3)}
 PREC = {"fp64": 0, "f32": 1, "f32x2": 2}
 DTYPE = {"fp64": "f64", "f32": "f32", "f32x2": "bf16x3-split/f32-acc"}
-KERNEL = {"fp64": "k_hpsi_t1s_f64", "f32": "k_hpsi_t1s_f32", "f32x2": "k_hpsi_mfma"}
+# the kernels of the main launch: the terms, then the sums of their rows
+KERNEL = {"fp64": "k_hpsi_t1s_out_f64", "f32": "k_hpsi_t1s_out_f32", "f32x2": "k_hpsi_mfma_out"}
 
 
 def cpu_model():
@@ -309,7 +310,7 @@ def main():
         dts, kavgs = timed(PREC["fp64"], args.steps, args.warmup)
         moved = 12.0 * nnz + 16.0 * b.nb_ba * nvec
         sparse = {"H·psi/s": nvec * args.steps / dts, "ms_per_step": dts / args.steps * 1e3,
-                  "kernel": "k_nm_spmm", "kernel_ms": kavgs * 1e3, "entries": nnz,
+                  "kernel": "k_nm_spmm_pairs", "kernel_ms": kavgs * 1e3, "entries": nnz,
                   "bytes": moved, "GBps": moved / kavgs / 1e9, "peak_GBps": PEAK_HBM_GBPS}
     op.set_sparse(False)
     # the apply replayed from one captured HIP graph, in the rows layout the
@@ -355,9 +356,9 @@ def main():
                      "intensity_flop_per_byte": st["flops"] / st["bytes"],
                      "ridge_flop_per_byte": PEAK["f32x2"] * 1e12 / (PEAK_HBM_GBPS * 1e9),
                      "limit": "latency of the LDS passes (one dependency chain per tile, a "
-                              "barrier per pass, 4 waves per SIMD); the scatter's memory-side "
-                              "FP64 atomics add ~20 %",
-                     "atomic_adds_per_launch": b.sum_nb * nvec,   # every map entry (LB = L)
+                              "barrier per pass, 4 waves per SIMD); the row sums, bound by "
+                              "the rate of their line fetches, add ~20 %",
+                     "results_per_launch": b.sum_nb * nvec,   # every map entry (LB = L)
                      "traffic_GBps": (traffic / kavg / 1e9) if traffic else None,
                      "algorithmic_TFLOPs": achieved,
                      "algorithmic_frac_of_bf16_peak": achieved / PEAK["f32x2"]})

@@ -271,7 +271,7 @@ constexpr int64_t NM_MIN_APPLIES = 24;
 
 constexpr int64_t XCD_BLOCK = 16 << 20;   // bytes of a block of vectors (default_cfg)
 constexpr int64_t ROWSUM_MIN = 1 << 16;   // places of the map (use_rowsum)
-constexpr int ROWSUM_AFTER = 8;           // applies of the term kernels before it
+constexpr int ROWSUM_AFTER = 4;           // applies of the term kernels before it
 constexpr int LARGE_THREADS = 512;        // threads for the terms beyond the LDS budget
 
 // Launch configuration of the H.psi kernel; chosen by sg4_plan_autotune.
@@ -2450,7 +2450,7 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
   const int threads3[] = {256, 512, NT32};
   std::vector<int> threads(threads3, threads3 + ((use_split(p) && prec == SG4_PREC_F32) ? 3 : 2));
   if (prec == SG4_PREC_F32X2) threads.push_back(NT_MFMA);
-  const int budgets[] = {32 * 1024, 48 * 1024, 64 * 1024, 80 * 1024, 112 * 1024, 160 * 1024};
+  const int budgets[] = {32 * 1024, 40 * 1024, 53 * 1024, 64 * 1024, 80 * 1024, 112 * 1024, 160 * 1024};
   const int grids[] = {0, 4, 8};   // 0: one per item; k: k workgroups per CU, persistent
   for (int nt : threads)
     for (int bu : budgets)
