@@ -10,10 +10,11 @@
 // three modes whose slabs a thread holds in registers while it multiplies
 // them by the small 1-D matrices (entries wave-uniform, read through the
 // scalar cache).  Four type-1 paths:
-//   split path (k_nm_spmm + k_hpsi_t1s_*): the kinetic part as one sparse
+//   split path (kinetic rows + k_hpsi_t1s_*): the kinetic part as one sparse
 //     matrix over the packed rows, the terms keep only basis->grid, the
-//     potential and grid->basis, with the gather and the weighted scatter-add
-//     folded into the first and last passes;
+//     potential and grid->basis, with the gather folded into the first pass and
+//     the last one storing its results for the row sums (sg4_rowsum.hip) or
+//     adding them with atomics;
 //   grouped grid path (k_hpsi_t1_*, term_t1_grouped): the reference's
 //     structure with the kinetic derivatives on the grid;
 //   per-mode grid path (k_hpsi_t1_*, term_t1): one pass per mode, any sizes.
@@ -1577,10 +1578,10 @@ static int apply_points(sg4_plan* P, int nvec, int W, const double* psi, double*
   if (t10) {
     KMats10 km{P->d_mats.as<double>(), P->d_V.as<double>(), P->d_G.as<double>(), P->d_Jac.as<double>(),
                P->d_sqRJ.as<double>()};
-    hipLaunchKernelGGL(k_hpsi_t10_f64, grid, dim3(t10 ? 384 : 256), lds, P->stream, a, km);
+    hipLaunchKernelGGL(k_hpsi_t10_f64, grid, dim3(384), lds, P->stream, a, km);
   } else {
     KMats1G km{P->d_mats.as<double>(), P->d_F.as<double>(), P->d_der.as<int32_t>(), P->nder, P->sum_nq};
-    hipLaunchKernelGGL(k_hpsi_t1g_f64, grid, dim3(t10 ? 384 : 256), lds, P->stream, a, km);
+    hipLaunchKernelGGL(k_hpsi_t1g_f64, grid, dim3(256), lds, P->stream, a, km);
   }
   if (P->timing) HIP_TRY(hipEventRecord(P->ev1, P->stream));
   HIP_TRY(hipGetLastError());

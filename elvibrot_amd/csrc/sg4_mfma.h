@@ -30,7 +30,8 @@
 // then the last group fused in registers (basis->grid, times V, grid->basis:
 // the C tile is the next B operand), then grid->basis groups G-2..0.  Group 0
 // gathers its B operands from the packed block through the term's map and
-// the last pass adds W_t times its output into H.psi with FP64 atomics (the
+// the last pass stores its output by place in the map (the row sums multiply
+// W_t in FP64) or adds W_t times it into H.psi with FP64 atomics (the
 // partial sums of the Smolyak combination are up to ~1e3 times larger than
 // the result, so the sum over terms is accumulated in FP64).
 #pragma once

@@ -19,7 +19,8 @@ namespace sg4 {
 // grid->basis group are one register pass.
 // LDS: X (N nv values of the item), Vs (the N potential values), Ms (the N
 // map entries, so that the psi gathers and the scatter-adds only wait for
-// LDS, not for a global map load).
+// LDS, not for a global map load).  OUT: the results are stored by place in the
+// map for the row sums instead of added.
 // ---------------------------------------------------------------------------
 template <class T>
 struct SCtx {

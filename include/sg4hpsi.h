@@ -127,8 +127,11 @@ int sg4_setup_destroy(sg4_setup *s);
 
 /* ---- device plan ----------------------------------------------------------
  * Owns device copies of the tables, the 1-D matrices and the grids, plus
- * pre-sized work buffers for blocks of up to max_nvec vectors: no device
- * allocation happens inside sg4_apply.                                       */
+ * pre-sized work buffers for blocks of up to max_nvec vectors.  An apply
+ * allocates its work items at the first call for a block width and, where the
+ * terms' results are summed row by row, the inverted map (a plan's fifth apply)
+ * and a results block per stream and wider block (at most 16 GiB; without it,
+ * and in applies that the caller captures, the sums are FP64 atomics).        */
 int sg4_plan_create(const sg4_tables *tables, int32_t max_nvec, sg4_plan **out);
 /* A batch of ninst independent SG4 operators (different D, L, grids) in one
  * plan: the operator is block-diagonal over the concatenated packed rows
@@ -342,7 +345,8 @@ int sg4_plan_autotune(sg4_plan *p, int32_t nvec, int32_t prec, float *best_ms);
 /* the launch parameters in use for (nvec, prec): threads, LDS budget, grid, xcd.
  * A block width with no parameters of its own (tuned or set) uses those of the
  * nearest configured width of the same precision (the narrowest wider one
- * first), else the defaults. */
+ * first), else the defaults (which follow the sizes; fewer than 256 threads
+ * are reported as 256). */
 int sg4_plan_config(const sg4_plan *p, int32_t nvec, int32_t prec, int32_t *cfg4);
 /* set the launch parameters for (nvec, prec) (e.g. a configuration saved from
  * an earlier autotune): threads 256 or 512 (768 for the FP32 mode on the split
