@@ -1595,9 +1595,15 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
   if (P->type_op != 1) return apply_points(P, nvec, nvec, psi, hpsi, nvec, 1);
   if (use_nmode(P, prec)) return apply_nmode(P, nvec, nvec, psi, hpsi, nullptr, nullptr);
   void* out = use_rowsum(P, nvec, prec);
-  const LaunchCfg cfg = cfgp ? *cfgp : cfg_for(P, nvec, prec, out != nullptr);
+  LaunchCfg cfg = cfgp ? *cfgp : cfg_for(P, nvec, prec, out != nullptr);
   ItemPlan* ip = nullptr;
-  if ((rc = prepare_all(P, nvec, prec, cfg, cfgp || !out, &ip))) return rc;
+  rc = prepare_all(P, nvec, prec, cfg, cfgp || !out, &ip);
+  if (rc && out && P->no_alloc && !cfgp) {   // this width was only applied with atomics so far
+    out = nullptr;
+    cfg = cfg_for(P, nvec, prec, false);
+    rc = prepare(P, nvec, prec, cfg, &ip);
+  }
+  if (rc) return rc;
   const int esize = (prec == SG4_PREC_FP64) ? 8 : 4;
   const int64_t n = P->nb_ba * nvec;
   const bool split = use_split_for(P, prec);
@@ -2439,6 +2445,7 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
   const bool timing = p->timing;
   p->timing = false;
   p->nm_off = true;    // tune the term kernels also where FP64 takes the sparse path
+  (void)use_rowsum(p, nvec, prec, true);   // every launch is timed on the path that later applies take
   LaunchCfg best;
   float bms = 1e30f;
   int cus = 256;
@@ -2539,7 +2546,7 @@ int sg4_apply_graph(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi, 
     const bool timing = p->timing;
     p->stream = p->own_stream;
     const bool sums = p->type_op == 1 && !use_nmode(p, prec) && use_rowsum(p, nvec, prec, true);
-    rc = prepare(p, nvec, prec, cfg_for(p, nvec, prec, sums), &ip);
+    rc = prepare_all(p, nvec, prec, cfg_for(p, nvec, prec, sums), !sums, &ip);
     p->stream = user;
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(p->own_stream));

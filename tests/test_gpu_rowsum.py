@@ -110,3 +110,30 @@ def test_weight_indices_apart_from_the_places(prec):
     x = torch.randn(op.nb_ba, 2, device="cuda", dtype=torch.float64, generator=g)
     y, z = pair(op, x, prec)
     assert float((y - z).abs().max()) <= tol(max(b.nterms for b in bs), z)
+
+
+def test_first_call_a_graph_and_noalloc_of_an_early_width():
+    """A plan's first call may be its graph entry, and the allocation-free entry
+    takes a width that was applied before the row sums were there."""
+    b = E.SG4Basis(6, 6)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    x = torch.randn(b.nb_ba, 8, device="cuda", dtype=torch.float64, generator=g)
+    for prec in (E.PREC_FP64, E.PREC_F32, E.PREC_F32X2):
+        first = E.SG4Operator(b, max_nvec=16)
+        first.set_sparse(False)
+        r = torch.full_like(x, float("nan"))
+        for _ in range(3):
+            first.apply_graph(x, r, prec)
+        op = E.SG4Operator(b, max_nvec=16)
+        op.set_sparse(False)
+        xc = x.t().contiguous()
+        rc = torch.empty_like(xc)
+        op.apply(xc, rc, prec)                       # eight vectors: with atomics
+        wide = torch.randn(b.nb_ba, 16, device="cuda", dtype=torch.float64, generator=g)
+        y, z = pair(op, wide, prec)
+        rc.fill_(float("nan"))
+        torch.cuda.synchronize()
+        E._capi.check(E.lib().sg4_apply_noalloc(op._h, 8, C.c_void_p(xc.data_ptr()), C.c_void_p(rc.data_ptr()), prec))
+        y, z = pair(op, x, prec)
+        assert float((r - z).abs().max()) <= tol(b.nterms, z), prec
+        assert float((rc.t() - z).abs().max()) <= tol(b.nterms, z), prec
