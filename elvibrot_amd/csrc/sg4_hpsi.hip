@@ -1445,7 +1445,8 @@ static void* use_rowsum(sg4_plan* P, int nvec, int prec, bool now = false) {
   if (!P->rowsum.ok) return nullptr;
   const size_t bytes = rowsum_bytes(P, nvec, prec == SG4_PREC_FP64 ? 8 : 4) +
                        (prec == SG4_PREC_F32 ? sizeof(float) * P->nb_ba * nvec : 0);
-  return rowsum_block(P->rowsum, P->stream, bytes, alloc);
+  // graphs of the plan's own stream hold their blocks
+  return rowsum_block(P->rowsum, P->stream, bytes, alloc, P->stream && P->stream == P->own_stream);
 }
 
 // Everything an apply needs that may allocate or copy (FP32 copies, item

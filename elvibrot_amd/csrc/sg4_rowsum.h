@@ -22,8 +22,8 @@ struct RowSum {
   DevBuf wi;       // uint8 weight indices where they do not fit beside the place (shift = 32)
   DevBuf wtab;     // the distinct term weights
   DevBuf seg;      // int32: nseg + 1 starts in pos, then nseg rows
-  // the terms' results of one apply, one block per stream; a block stays until
-  // the plan's operator changes (a larger one is added beside it)
+  // the terms' results of one apply: a block per stream, replaced by a larger one
+  // when a wider apply needs it, unless graphs hold it (keep)
   struct Out { hipStream_t stream; DevBuf buf; };
   std::vector<std::unique_ptr<Out>> out;
 };
@@ -32,8 +32,9 @@ struct RowSum {
 // fit the index types or the device memory
 int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, const TermDev* d_terms,
                  const std::vector<TermDev>& terms, hipStream_t st);
-// the stream's block of at least `bytes`, or null (none within the limits; alloc = false: none held)
-void* rowsum_block(RowSum& s, hipStream_t st, size_t bytes, bool alloc);
+// the stream's block of at least `bytes`, or null (none within the limits; alloc = false: none held);
+// keep: the stream's smaller blocks stay
+void* rowsum_block(RowSum& s, hipStream_t st, size_t bytes, bool alloc, bool keep);
 // hpsi(r, v) += the row's places of out (float: times the term weights)
 int rowsum_add(const RowSum& s, const double* out, int nvec, double* hpsi, hipStream_t st);
 int rowsum_add(const RowSum& s, const float* out, int nvec, double* hpsi, hipStream_t st);

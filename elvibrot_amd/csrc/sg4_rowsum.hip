@@ -274,13 +274,16 @@ int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, 
   return SG4_OK;
 }
 
-void* rowsum_block(RowSum& s, hipStream_t st, size_t bytes, bool alloc) {
-  size_t held = 0;
-  for (const auto& o : s.out) {
+void* rowsum_block(RowSum& s, hipStream_t st, size_t bytes, bool alloc, bool keep) {
+  for (const auto& o : s.out)
     if (o->stream == st && o->buf.n >= bytes) return o->buf.p;
-    held += o->buf.n;
-  }
-  if (!alloc || s.out.size() >= RS_MAX_BLOCKS || held + bytes > RS_MAX_BYTES) return nullptr;
+  if (!alloc || bytes > RS_MAX_BYTES) return nullptr;
+  if (!keep)   // freeing waits for the applies that still use it
+    s.out.erase(std::remove_if(s.out.begin(), s.out.end(), [&](const auto& o) { return o->stream == st; }),
+                s.out.end());
+  size_t held = 0;
+  for (const auto& o : s.out) held += o->buf.n;
+  if (s.out.size() >= RS_MAX_BLOCKS || held + bytes > RS_MAX_BYTES) return nullptr;
   auto o = std::make_unique<RowSum::Out>();
   o->stream = st;
   if (o->buf.alloc(bytes)) return nullptr;
