@@ -765,8 +765,11 @@ static int build_terms(sg4_plan* P) {
   HIP_TRY(hipMemcpy(P->d_terms.p, P->h_terms.data(), sizeof(TermDev) * P->h_terms.size(),
                     hipMemcpyHostToDevice));
   if (P->type_op != 1) return build_points(P);
-  if ((rc = build_kinetic(P))) return rc;
-  return build_nmode(P);
+  if ((rc = build_kinetic(P)) || (rc = build_nmode(P))) return rc;
+  // the matrices are filled by kernels on the plan's stream; the next apply may
+  // run on another one (sg4_plan_set_stream)
+  HIP_TRY(hipStreamSynchronize(P->stream));
+  return SG4_OK;
 }
 
 struct HItem { Item it; double cost; bool large; };

@@ -51,7 +51,8 @@ NModeTables* nmode_tables_create(const NModeIn& in);   // null: HIP failure
 void nmode_tables_destroy(NModeTables* t);
 
 // Whether the packed rows are in lexicographic order (the last mode's index
-// fastest), and the kinetic part K alone for such rows.
+// fastest), and the kinetic part K alone for such rows.  Both builders return
+// with the last kernels enqueued on in.stream.
 bool nmode_rows_ok(const NModeTables* t);
 int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m);
 
@@ -59,7 +60,7 @@ int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m);
 // the values of the grid function mu as an operator.  m.valid says whether
 // there is one: V (and mu) must be sums of one- and two-mode functions to
 // rounding on every grid point, the packed rows in lexicographic order, and
-// the matrix small enough to pay.  Synchronises the stream.
+// the matrix small enough to pay.
 int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double* mu, NModeMat& m);
 
 // hpsi = M psi, nvec vectors in the rows layout (val: other values on M's pattern;
