@@ -364,7 +364,7 @@ struct sg4_plan {
   sg4::NModeMat nm, nm_field;
   bool field_on = false, nm_off = false;
   bool sparse = true;            // SG4_OPT_SPARSE
-  std::set<int> nm_seen;         // block widths applied since the operator was set
+  std::set<int> nm_seen;         // block widths that the sparse path prepared (apply_nmode)
   // split-precision MFMA path (SG4_PREC_F32X2): terms cut into mode groups,
   // group matrices in A-operand lane order
   bool mfma_valid = false;
@@ -1522,8 +1522,13 @@ static int next_events(sg4_plan* P) {
 // column-major blocks of nvec vectors (W columns, or null: rows layout).
 static int apply_nmode(sg4_plan* P, int nvec, int W, const double* psi, double* hpsi, double* ri, double* ro) {
   int rc;
-  if (P->no_alloc && !P->nm_seen.count(W)) return not_prepared();
-  if (!P->no_alloc) P->nm_seen.insert(W);
+  // the term kernels' lists too: a field or an option may send the next apply,
+  // also one that may not allocate, to them
+  ItemPlan* ip = nullptr;
+  if (P->no_alloc || P->nm_seen.insert(W).second) {
+    rc = prepare(P, W, SG4_PREC_FP64, cfg_for(P, W, SG4_PREC_FP64, false), &ip);
+    if (rc && P->no_alloc) return rc;
+  }
   P->last_items = P->nterms;
   P->last_flops = P->flops_split * W;
   const bool direct = ri && nmode_cols_direct(P->nm, W);
@@ -2502,6 +2507,7 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
   p->timing = timing;
   if (rc) return rc;
   drop_graphs(p);
+  p->nm_seen.clear();
   p->tuned[nvec * 16 + prec] = best;
   if (best_ms) *best_ms = bms;
   return SG4_OK;
@@ -2529,6 +2535,7 @@ int sg4_plan_set_config(sg4_plan* p, int32_t nvec, int32_t prec, const int32_t* 
   LaunchCfg c;
   c.nthreads = cfg4[0]; c.lds_budget = cfg4[1]; c.grid = cfg4[2]; c.xcd = cfg4[3];
   drop_graphs(p);
+  p->nm_seen.clear();
   p->tuned[nvec * 16 + prec] = c;
   return SG4_OK;
 }
