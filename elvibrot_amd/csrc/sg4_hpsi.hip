@@ -1359,6 +1359,23 @@ static bool use_nmode(const sg4_plan* P, int prec) {
          use_split_alg(P);
 }
 
+// Whether the plan's stream is being captured, and by the caller (the plan
+// captures its own stream for sg4_apply_graph).
+static bool captured(const sg4_plan* P) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(P->stream, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+static bool caller_captures(const sg4_plan* P) {
+  return !(P->own_stream && P->stream == P->own_stream) && captured(P);
+}
+
+// use_nmode for one apply.  A caller's graph outlives the call: a field set
+// later changes V in place, which the term kernels read at every replay and the
+// matrix does not hold.
+static bool take_nmode(const sg4_plan* P, int prec) { return use_nmode(P, prec) && !caller_captures(P); }
+
 // Launch of the term kernels when nothing is tuned or set and the results go
 // to a block (use_rowsum).  The kernels wait for latencies, so the LDS budget
 // is what lets their registers fill the CU: FP64 three workgroups of 256 (9D
@@ -1436,11 +1453,8 @@ static size_t rowsum_bytes(const sg4_plan* P, int nvec, int esize) {
 // keeps the atomics, since its graph may run beside the plan's other work.
 static void* use_rowsum(sg4_plan* P, int nvec, int prec, bool now = false) {
   if (P->deterministic || !use_split_for(P, prec) || P->sum_nb < ROWSUM_MIN) return nullptr;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const bool busy = hipStreamIsCapturing(P->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
-  if (busy) (void)hipGetLastError();
-  if (busy && (!P->own_stream || P->stream != P->own_stream)) return nullptr;
-  const bool alloc = !P->no_alloc && !busy;
+  if (caller_captures(P)) return nullptr;
+  const bool alloc = !P->no_alloc && !captured(P);
   if (alloc && !P->rowsum.tried && !now && P->term_applies++ < ROWSUM_AFTER) return nullptr;
   if (alloc && rowsum_build(P->rowsum, P->d_map.as<int32_t>(), P->sum_nb, P->nb_ba, P->d_terms.as<TermDev>(),
                             P->h_terms, P->stream))
@@ -1602,7 +1616,7 @@ static int apply_rows(sg4_plan* P, int nvec, const double* psi, double* hpsi, in
   int rc;
   if ((rc = check_apply(P, nvec, prec))) return rc;
   if (P->type_op != 1) return apply_points(P, nvec, nvec, psi, hpsi, nvec, 1);
-  if (use_nmode(P, prec)) return apply_nmode(P, nvec, nvec, psi, hpsi, nullptr, nullptr);
+  if (take_nmode(P, prec)) return apply_nmode(P, nvec, nvec, psi, hpsi, nullptr, nullptr);
   void* out = use_rowsum(P, nvec, prec);
   LaunchCfg cfg = cfgp ? *cfgp : cfg_for(P, nvec, prec, out != nullptr);
   ItemPlan* ip = nullptr;
@@ -2256,7 +2270,7 @@ int sg4_apply(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi, int32_
   }
   const int W = pad_width(p, nvec);
   if (p->type_op > 1 && prec == SG4_PREC_FP64) return apply_points(p, nvec, W, psi, hpsi, 1, p->nb_ba);
-  if (p->type_op && use_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
+  if (p->type_op && take_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
   hipLaunchKernelGGL(k_cols_to_rows, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, psi, ri, p->nb_ba, nvec, W);
   int rc = apply_rows(p, W, ri, ro, prec);
   if (rc) return rc;
@@ -2321,7 +2335,7 @@ int sg4_apply_noalloc(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi
   double* ri = base;
   double* ro = base + n;
   if (p->type_op > 1 && prec == SG4_PREC_FP64) return apply_points(p, nvec, W, psi, hpsi, 1, p->nb_ba);
-  if (use_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
+  if (take_nmode(p, prec)) return apply_nmode(p, nvec, W, psi, hpsi, ri, ro);
   hipLaunchKernelGGL(k_cols_to_rows, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, psi, ri, p->nb_ba, nvec, W);
   if ((rc = apply_rows(p, W, ri, ro, prec))) return rc;
   hipLaunchKernelGGL(k_rows_to_cols, tile_grid(p->nb_ba, W), dim3(256), 0, p->stream, ro, hpsi, p->nb_ba, nvec, W);
