@@ -434,7 +434,9 @@ struct Prop {
 };
 
 // Restores the field-free potential of H when a propagation leaves on an
-// error path (the normal end restores it itself and clears H).
+// error path (the normal end restores it itself and clears H).  On the matrix
+// the propagation sets no field; one left on the plan before is taken back at
+// its start.
 struct FieldReset {
   sg4_plan* H;
   ~FieldReset() { if (H) (void)sg4_plan_set_field(H, nullptr, 0.0); }
@@ -473,6 +475,7 @@ int sg4_cheby_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
   if ((rc = P.choose(2 * ns, (int64_t)prm->nseg * prm->steps_per_seg * (prm->ncoef - 1)))) return rc;
   if ((rc = P.init(false))) return rc;
   if (P.nm) {
+    if ((rc = plan_clear_field(H))) return rc;
     double *cur = psi, *other = P.B.p;
     for (int s = 0; s < prm->nseg; ++s) {
       if ((rc = P.field(s))) return rc;
@@ -482,7 +485,6 @@ int sg4_cheby_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
     if (cur != psi)
       hipLaunchKernelGGL(k_cb_copy, dim3(blocks_for(P.n)), dim3(256), 0, P.st, cur, psi, P.n);
     CB_TRY(hipGetLastError());
-    if ((rc = plan_clear_field(H))) return rc;
     CB_TRY(hipStreamSynchronize(P.st));
     return SG4_OK;
   }
@@ -538,6 +540,7 @@ int sg4_cheby_field_gradient(sg4_plan* H, sg4_plan* Mu, const double* mu, int32_
     if (same && (rc = P.choose(2 * ns, 4 * per))) return rc;
   }
   if ((rc = P.init(true))) return rc;
+  if (P.nm && (rc = plan_clear_field(H))) return rc;
   FieldReset reset{P.nm ? nullptr : H};
   const dim3 b(256);
   // forward, keeping the state at the start of every C-th segment
@@ -598,7 +601,7 @@ int sg4_cheby_field_gradient(sg4_plan* H, sg4_plan* Mu, const double* mu, int32_
       if ((rc = P.step(lam, +1.0))) return rc;
   }
   reset.H = nullptr;
-  if ((rc = P.nm ? plan_clear_field(H) : sg4_plan_set_field(H, nullptr, 0.0))) return rc;
+  if (!P.nm && (rc = sg4_plan_set_field(H, nullptr, 0.0))) return rc;
   CB_TRY(hipStreamSynchronize(P.st));
   return SG4_OK;
 }
@@ -644,6 +647,7 @@ int sg4_taylor_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
   };
   const dim3 g(blocks_for(rows * ns)), b(256);
   const double ph = -prm->E0 * prm->dt;
+  if (nm && (rc = plan_clear_field(H))) return rc;
   FieldReset reset{nm ? nullptr : H};
   int64_t step = 0;
   for (int s = 0; s < prm->nseg; ++s) {
@@ -692,7 +696,7 @@ int sg4_taylor_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
     }
   }
   reset.H = nullptr;
-  if ((rc = nm ? plan_clear_field(H) : sg4_plan_set_field(H, nullptr, 0.0))) return rc;
+  if (!nm && (rc = sg4_plan_set_field(H, nullptr, 0.0))) return rc;
   CB_TRY(hipStreamSynchronize(st));
   return SG4_OK;
 }
