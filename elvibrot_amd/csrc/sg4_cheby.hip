@@ -536,7 +536,7 @@ int sg4_cheby_field_gradient(sg4_plan* H, sg4_plan* Mu, const double* mu, int32_
   {
     const int64_t per = (int64_t)prm->nseg * prm->steps_per_seg * (prm->ncoef - 1);
     bool same = false;
-    if (nmode_order_width(4 * ns) && (rc = plan_is_grid_function(Mu, mu, P.st, &same))) return rc;
+    if (nmode_order_width(4 * ns) && (rc = plan_is_grid_function(Mu, H, mu, P.st, &same))) return rc;
     if (same && (rc = P.choose(2 * ns, 4 * per))) return rc;
   }
   if ((rc = P.init(true))) return rc;

@@ -1757,9 +1757,20 @@ int plan_field_matrix(sg4_plan* P, const double* mu, int prec, int64_t applies, 
   return SG4_OK;
 }
 
-int plan_is_grid_function(const sg4_plan* P, const double* mu, hipStream_t st, bool* same) {
+// Two plans over the same terms, grids, 1-D matrices and packed rows.
+static bool same_tables(const sg4_plan* A, const sg4_plan* B) {
+  if (A->inst.size() != B->inst.size() || A->sum_nq != B->sum_nq) return false;
+  for (size_t i = 0; i < A->inst.size(); ++i) {
+    const sg4_plan::Inst &a = A->inst[i], &b = B->inst[i];
+    if (a.D != b.D || a.Lmax != b.Lmax || a.nterms != b.nterms || a.nb_ba != b.nb_ba) return false;
+  }
+  return A->h_levels == B->h_levels && A->h_weights == B->h_weights && A->h_nq == B->h_nq && A->h_nb == B->h_nb &&
+         A->h_mats == B->h_mats && A->h_map == B->h_map;
+}
+
+int plan_is_grid_function(const sg4_plan* P, const sg4_plan* H, const double* mu, hipStream_t st, bool* same) {
   *same = false;
-  if (P->type_op != 1 || !P->grouping || !P->split_ok) return SG4_OK;
+  if (P->type_op != 1 || !use_split_alg(P) || !P->sparse || P->deterministic || !same_tables(P, H)) return SG4_OK;
   for (double c : P->h_ck)
     if (c != 0.0) return SG4_OK;
   DevBuf diff;

@@ -81,8 +81,10 @@ int nmode_set_field(const NModeMat& m, double eps, hipStream_t st);
 // it would not pay.  The matrix belongs to the plan and is rebuilt by the next
 // call.
 int plan_field_matrix(sg4_plan* p, const double* mu, int prec, int64_t applies, NModeMat** out);
-// whether the plan is the operator of the grid function mu alone (no kinetic part)
-int plan_is_grid_function(const sg4_plan* p, const double* mu, hipStream_t st, bool* same);
+// whether the plan is the operator of the grid function mu alone (no kinetic
+// part), over H's terms and grids (mu has a value per grid point of H) and free
+// to run as a matrix
+int plan_is_grid_function(const sg4_plan* p, const sg4_plan* H, const double* mu, hipStream_t st, bool* same);
 // takes a field left on the plan back
 int plan_clear_field(sg4_plan* p);
 
