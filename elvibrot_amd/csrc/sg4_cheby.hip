@@ -300,6 +300,12 @@ struct Prop {
     return SG4_OK;
   }
 
+  int order(const NModeOrder& o, bool tangent) {
+    int rc;
+    if ((rc = plan_product_begin(H, (tangent ? 4 : 2) * ns)) || (rc = nmode_order(*nm, o, tangent, st))) return rc;
+    return plan_product_end(H);
+  }
+
   // A step of the sparse path: the result is in psi afterwards, which trades
   // places with other (w_0 = psi and w_1 in other alternate as w_{k-1}, w_k; the
   // last order writes the phased sum over w_{k-1}, which no row gathers).
@@ -313,7 +319,7 @@ struct Prop {
     for (int k = 1; k < p->ncoef; ++k) {
       o.wk = wk; o.wm = wm; o.c = p->coef[k];
       o.first = k == 1; o.last = k + 1 == p->ncoef; o.out = wm;
-      if ((rc = nmode_order(*nm, o, false, st))) return rc;
+      if ((rc = order(o, false))) return rc;
       std::swap(wm, wk);
     }
     psi = wk;
@@ -339,7 +345,7 @@ struct Prop {
     for (int k = 1; k < p->ncoef; ++k) {
       o.wk = wk; o.wm = wm; o.c = p->coef[k];
       o.first = k == 1; o.last = k + 1 == p->ncoef;
-      if ((rc = nmode_order(*nm, o, true, st))) return rc;
+      if ((rc = order(o, true))) return rc;
       std::swap(wm, wk);
     }
     return SG4_OK;
@@ -663,8 +669,13 @@ int sg4_taylor_propagate(sg4_plan* H, const double* mu, int32_t ns, double* psi,
       double m = 0.0;
       int used = 0;
       for (int k = 0; k < prm->npoly; ++k) {
-        rc = nm ? nmode_apply(*nm, 2 * ns, wk, Y.p, st, val) : sg4_apply_rows(H, 2 * ns, wk, Y.p, prm->prec);
-        if (rc) return rc;
+        if (nm) {
+          if ((rc = plan_product_begin(H, 2 * ns)) || (rc = nmode_apply(*nm, 2 * ns, wk, Y.p, st, val)) ||
+              (rc = plan_product_end(H)))
+            return rc;
+        } else if ((rc = sg4_apply_rows(H, 2 * ns, wk, Y.p, prm->prec))) {
+          return rc;
+        }
         hipLaunchKernelGGL(k_tl_order, g, b, 0, st, wk, Y.p, wn, psi, prm->dt / (k + 1), prm->E0, rows, ns);
         if ((rc = max_norm2(wn, &m))) return rc;
         used = k + 1;

@@ -1532,6 +1532,19 @@ static int next_events(sg4_plan* P) {
   return SG4_OK;
 }
 
+int plan_product_begin(sg4_plan* P, int nvec) {
+  P->last_items = P->nterms;
+  P->last_flops = P->flops_split * nvec;
+  if (!P->timing) return SG4_OK;
+  if (int rc = next_events(P)) return rc;
+  HIP_TRY(hipEventRecord(P->ev0, P->stream));
+  return SG4_OK;
+}
+int plan_product_end(sg4_plan* P) {
+  if (P->timing) HIP_TRY(hipEventRecord(P->ev1, P->stream));
+  return SG4_OK;
+}
+
 // FP64 apply of the sparse path.  ri: a rows-layout staging block for
 // column-major blocks of nvec vectors (W columns, or null: rows layout).
 static int apply_nmode(sg4_plan* P, int nvec, int W, const double* psi, double* hpsi, double* ri, double* ro) {
@@ -1543,15 +1556,10 @@ static int apply_nmode(sg4_plan* P, int nvec, int W, const double* psi, double* 
     rc = prepare(P, W, SG4_PREC_FP64, cfg_for(P, W, SG4_PREC_FP64, false), &ip);
     if (rc && P->no_alloc) return rc;
   }
-  P->last_items = P->nterms;
-  P->last_flops = P->flops_split * W;
   const bool direct = ri && nmode_cols_direct(P->nm, W);
   if (ri && !direct)
     hipLaunchKernelGGL(k_cols_to_rows, tile_grid(P->nb_ba, W), dim3(256), 0, P->stream, psi, ri, P->nb_ba, nvec, W);
-  if (P->timing) {
-    if ((rc = next_events(P))) return rc;
-    HIP_TRY(hipEventRecord(P->ev0, P->stream));
-  }
+  if ((rc = plan_product_begin(P, W))) return rc;
   bool back = false;
   if (!ri) rc = nmode_apply(P->nm, nvec, psi, hpsi, P->stream);
   else if (direct) rc = nmode_apply_cols(P->nm, W, nvec, psi, hpsi, P->stream);
@@ -1559,8 +1567,7 @@ static int apply_nmode(sg4_plan* P, int nvec, int W, const double* psi, double* 
     rc = nmode_apply(P->nm, W, ri, ro, P->stream);
     back = true;
   }
-  if (rc) return rc;
-  if (P->timing) HIP_TRY(hipEventRecord(P->ev1, P->stream));
+  if (rc || (rc = plan_product_end(P))) return rc;
   if (back)
     hipLaunchKernelGGL(k_rows_to_cols, tile_grid(P->nb_ba, W), dim3(256), 0, P->stream, ro, hpsi, P->nb_ba, nvec, W);
   HIP_TRY(hipGetLastError());

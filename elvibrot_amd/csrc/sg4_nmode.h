@@ -85,6 +85,10 @@ int plan_field_matrix(sg4_plan* p, const double* mu, int prec, int64_t applies, 
 // part), over H's terms and grids (mu has a value per grid point of H) and free
 // to run as a matrix
 int plan_is_grid_function(const sg4_plan* p, const sg4_plan* H, const double* mu, hipStream_t st, bool* same);
+// around a product with such a matrix, what an apply of the plan records: the
+// statistics and, with timing on, the events
+int plan_product_begin(sg4_plan* p, int nvec);
+int plan_product_end(sg4_plan* p);
 // takes a field left on the plan back
 int plan_clear_field(sg4_plan* p);
 
