@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdio>
 #include <cstdlib>
 #include <cmath>
@@ -34,6 +35,7 @@
 #include <set>
 #include <stdexcept>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "sg4_mfma.h"
@@ -272,7 +274,6 @@ constexpr int64_t NM_MIN_APPLIES = 24;
 
 constexpr int64_t XCD_BLOCK = 16 << 20;   // bytes of a block of vectors (default_cfg)
 constexpr int64_t ROWSUM_MIN = 1 << 16;   // places of the map (use_rowsum)
-constexpr int ROWSUM_AFTER = 4;           // applies of the term kernels before it
 constexpr int LARGE_THREADS = 512;        // threads for the terms beyond the LDS budget
 
 // Launch configuration of the H.psi kernel; chosen by sg4_plan_autotune.
@@ -335,7 +336,7 @@ struct sg4_plan {
   // overflow counter at the end
   bool deterministic = false;
   sg4::DevBuf d_fx;
-  int term_applies = 0;      // applies of the term kernels, up to ROWSUM_AFTER
+  double rowsum_gain = 0;    // us that the row sums would have saved so far (rowsum_pays)
   sg4::RowSum rowsum;        // sums over the terms without atomics (use_rowsum)
   // general type-1 operator (type_op 11): derivative terms and their grids
   int nder = 0;
@@ -774,6 +775,17 @@ static int build_terms(sg4_plan* P) {
 
 struct HItem { Item it; double cost; bool large; };
 
+// Instance and levels (6 bits each) of a class of terms.
+typedef std::array<uint64_t, 1 + (SG4_MAX_D + 9) / 10> ClassKey;
+static_assert(SG4_MAX_L < 64, "levels take 6 bits");
+struct ClassHash {
+  size_t operator()(const ClassKey& k) const {
+    uint64_t h = 0;
+    for (uint64_t w : k) h = (h ^ w) * 0x9e3779b97f4a7c15ull, h ^= h >> 29;
+    return (size_t)h;
+  }
+};
+
 // Item order of a launch: by decreasing cost, or (xcd >= 1) dealt to the
 // eight XCDs (workgroups go round-robin to the XCDs) so that the items of a
 // term (xcd = 1) or of a class of terms with equal levels in modes
@@ -792,24 +804,23 @@ static std::vector<Item> order_items(const sg4_plan* P, const std::vector<HItem>
     // terms with equal levels in modes xcd..D-1 share the rows that agree in
     // those modes: put such a class on one XCD, its items next to each other
     // (classes by decreasing largest item, items by decreasing cost)
-    std::map<std::vector<int32_t>, int> cls_of;
+    std::unordered_map<ClassKey, int, ClassHash> cls_of;
+    std::vector<int> term_cls(P->nterms, -1);
     std::vector<std::vector<const HItem*>> cls;
     for (auto& x : all) {
       if (x.large != large) continue;
-      int64_t t = x.it.term;
-      size_t ii = 0;
-      while (ii + 1 < P->inst.size() && t >= P->inst[ii + 1].term0) ++ii;
-      const sg4_plan::Inst& I = P->inst[ii];
-      std::vector<int32_t> key(1, (int32_t)ii);
-      for (int k = xcd; k < I.D; ++k) key.push_back(P->h_levels[I.lev0 + (t - I.term0) * I.D + k]);
-      auto f = cls_of.find(key);
-      int c;
-      if (f == cls_of.end()) {
-        c = (int)cls.size();
-        cls_of[key] = c;
-        cls.emplace_back();
-      } else {
-        c = f->second;
+      const int64_t t = x.it.term;
+      int& c = term_cls[t];
+      if (c < 0) {
+        size_t ii = 0;
+        while (ii + 1 < P->inst.size() && t >= P->inst[ii + 1].term0) ++ii;
+        const sg4_plan::Inst& I = P->inst[ii];
+        ClassKey key{{ii}};
+        for (int k = xcd; k < I.D; ++k)
+          key[1 + (k - xcd) / 10] |= (uint64_t)P->h_levels[I.lev0 + (t - I.term0) * I.D + k] << 6 * ((k - xcd) % 10);
+        const auto f = cls_of.emplace(key, (int)cls.size());
+        if (f.second) cls.emplace_back();
+        c = f.first->second;
       }
       cls[c].push_back(&x);
     }
@@ -1438,6 +1449,19 @@ static size_t rowsum_bytes(const sg4_plan* P, int nvec, int esize) {
   return ((size_t)P->sum_nb * nvec * esize + 255) & ~(size_t)255;
 }
 
+// Whether the applies so far would have saved what inverting the map (and the
+// lists of another launch) costs, this one included: a plan of few applies then
+// never pays for it, and a longer one at most twice.  us, one apply with atomics
+// / with sums, and the apply that changes over: 6D L=6 (94 k places) x1 41 / 32,
+// 600; 8D L=6 (439 k) x1 72 / 50, 540, FP32 x24 203 / 102, 920; 9D L=7 (3.7 M) x1
+// 310 / 208, 2100, x5 438 / 355, 2400, x16 704 / 521, 2700; 10D L=8 (31 M) split x1
+// 2059 / 834, 8800, FP64 x16 9178 / 4716, 15500.  The estimates below are low on
+// the savings where they are far apart (10D).
+static bool rowsum_pays(sg4_plan* P, int nvec) {
+  P->rowsum_gain += 8.0 + 1e-6 * (20.0 + 1.5 * nvec) * (double)P->sum_nb;
+  return P->rowsum_gain > 800.0 + 3.5e-4 * (double)P->sum_nb;
+}
+
 // The block for the terms' results when they are summed row by row, or null:
 // the kernels then add into H.psi with atomics, ~187 G/s on the whole chip
 // whatever their addresses.  Storing and summing moves a result twice instead
@@ -1446,16 +1470,16 @@ static size_t rowsum_bytes(const sg4_plan* P, int nvec, int esize) {
 // 71 -> 54, 9D L=6 x16 198 -> 148.  Small term sets would only pay for the
 // launch: 6D L=5 (26 k places) x1 / x4 15.6 -> 15.7 / 14.3 -> 16.8 us, 6D L=6
 // (94 k) 27.1 -> 19.2 / 26.4 -> 21.1.
-// The inverted map costs as much as the sums save in some ten applies (9D L=7
-// 2.7 ms against 0.13 per apply of 5 vectors), so a plan builds it at the apply
-// after ROWSUM_AFTER, or for a graph (now).
+// The inverted map costs as much as the sums save in some ten to eighty applies,
+// so a plan builds it once they would have saved that much (rowsum_pays), or for
+// a graph or the autotuner (now).
 // The block belongs to the plan's stream: an apply that the caller captures
 // keeps the atomics, since its graph may run beside the plan's other work.
 static void* use_rowsum(sg4_plan* P, int nvec, int prec, bool now = false) {
   if (P->deterministic || !use_split_for(P, prec) || P->sum_nb < ROWSUM_MIN) return nullptr;
   if (caller_captures(P)) return nullptr;
   const bool alloc = !P->no_alloc && !captured(P);
-  if (alloc && !P->rowsum.tried && !now && P->term_applies++ < ROWSUM_AFTER) return nullptr;
+  if (alloc && !P->rowsum.tried && !now && !rowsum_pays(P, nvec)) return nullptr;
   if (alloc && rowsum_build(P->rowsum, P->d_map.as<int32_t>(), P->sum_nb, P->nb_ba, P->d_terms.as<TermDev>(),
                             P->h_terms, P->stream))
     return nullptr;

@@ -7,6 +7,11 @@
 // places in the same order, so rows are numbered by first appearance in the
 // map and their places sorted: split precision 8D L=6 x2 56 us (rows in packed
 // order, places as the atomics of the fill left them), 39 (places sorted), 34.
+//
+// The map is inverted on the device, one number (the totals) read back: 9D L=7
+// 1.1 ms of kernels, 10D L=8 6.7 (counts and fill 4.7: atomics on the rows that
+// most terms hold; sort 1.1).  With the rows' order and segments made on the host
+// the whole took 1.9 and 16 ms.
 #include "sg4_rowsum.h"
 
 #include <algorithm>
@@ -20,6 +25,7 @@ constexpr int RS_SEG = 64;                       // places per segment (one per 
 constexpr int RS_LOADS = 8;                      // places in flight per lane
 constexpr int RS_LANES = 4;                      // log2 of the lanes per segment, at least
 constexpr int RS_BATCH = 8;                      // fill launches
+constexpr int SCAN = 1024;                       // items per workgroup of a scan
 constexpr size_t RS_MAX_BYTES = size_t(16) << 30; // results held per plan
 constexpr size_t RS_MAX_BLOCKS = 8;
 constexpr int RS_WEIGHTS = 256;                 // distinct term weights
@@ -34,10 +40,11 @@ constexpr uint32_t RS_MULTI = 0x80000000u;
     }                                                 \
   } while (0)
 
-__global__ __launch_bounds__(256) void k_rs_init(int32_t* cnt, int32_t* first, int64_t n) {
+__global__ __launch_bounds__(256) void k_rs_init(int32_t* cnt, int32_t* first, int32_t* order, int64_t n) {
   for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) {
     cnt[i] = 0;
     first[i] = INT32_MAX;
+    order[i] = -1;
   }
 }
 
@@ -79,6 +86,75 @@ __global__ __launch_bounds__(256) void k_rs_first(const int32_t* map, const int3
     }
     if (!FILL && threadIdx.x == 0) num[t] = done;
   }
+}
+
+// What a scan adds up: the rows that first appear in term i, or (order) the
+// places of the row that is i-th in the order and, in the upper half, its segments.
+__device__ __forceinline__ uint64_t scan_item(const int32_t* num, const int32_t* order, int64_t i) {
+  if (!order) return (uint32_t)num[i];
+  const int r = order[i];
+  if (r < 0) return 0;                // rows that no term holds
+  const uint32_t n = (uint32_t)num[r];
+  return (uint64_t)((n + RS_SEG - 1) / RS_SEG) << 32 | n;
+}
+
+// inclusive scan over the workgroup (SCAN threads); s: SCAN values of LDS
+__device__ __forceinline__ uint64_t scan_block(uint64_t x, uint64_t* s) {
+  s[threadIdx.x] = x;
+  __syncthreads();
+  for (int o = 1; o < SCAN; o <<= 1) {
+    const uint64_t y = (int)threadIdx.x >= o ? s[threadIdx.x - o] : 0;
+    __syncthreads();
+    s[threadIdx.x] += y;
+    __syncthreads();
+  }
+  return s[threadIdx.x];
+}
+
+// sums of SCAN items each, then their exclusive scan with the total behind it
+__global__ __launch_bounds__(SCAN) void k_rs_sums(const int32_t* num, const int32_t* order, int64_t n, uint64_t* part) {
+  __shared__ uint64_t s[SCAN];
+  const int64_t i = (int64_t)blockIdx.x * SCAN + threadIdx.x;
+  const uint64_t x = scan_block(i < n ? scan_item(num, order, i) : 0, s);
+  if (threadIdx.x == SCAN - 1) part[blockIdx.x] = x;
+}
+__global__ __launch_bounds__(SCAN) void k_rs_scan(uint64_t* part, int np) {
+  __shared__ uint64_t s[SCAN];
+  uint64_t carry = 0;
+  for (int b = 0; b < np; b += SCAN) {
+    const int i = b + threadIdx.x;
+    const uint64_t x = i < np ? part[i] : 0, y = scan_block(x, s);
+    if (i < np) part[i] = carry + y - x;
+    carry += s[SCAN - 1];
+    __syncthreads();                  // s is written again
+  }
+  if (threadIdx.x == 0) part[np] = carry;
+}
+
+// the terms' first rows in the order (from num, in place)
+__global__ __launch_bounds__(SCAN) void k_rs_base(int32_t* num, int64_t n, const uint64_t* part) {
+  __shared__ uint64_t s[SCAN];
+  const int64_t i = (int64_t)blockIdx.x * SCAN + threadIdx.x;
+  const uint64_t x = i < n ? scan_item(num, nullptr, i) : 0, y = part[blockIdx.x] + scan_block(x, s) - x;
+  if (i < n) num[i] = (int32_t)y;
+}
+
+// the segments of the rows in the order, and (in place of the counts) where a
+// row's places start; nseg, places: the totals that seg was sized for
+__global__ __launch_bounds__(SCAN) void k_rs_segs(int32_t* cnt, const int32_t* order, int64_t n, const uint64_t* part,
+                                                  int32_t* seg, int64_t nseg, int32_t places) {
+  __shared__ uint64_t s[SCAN];
+  const int64_t i = (int64_t)blockIdx.x * SCAN + threadIdx.x;
+  const uint64_t x = i < n ? scan_item(cnt, order, i) : 0, y = part[blockIdx.x] + scan_block(x, s) - x;
+  if (i == 0) seg[nseg] = places;
+  if (x == 0) return;
+  const int r = order[i], at = (int)(uint32_t)y, num = (int)(uint32_t)x;
+  int64_t k = (int64_t)(y >> 32);
+  for (int o = 0; o < num; o += RS_SEG, ++k) {
+    seg[k] = at + o;
+    seg[nseg + 1 + k] = (int32_t)((uint32_t)r | (num > RS_SEG ? RS_MULTI : 0u));
+  }
+  cnt[r] = at;
 }
 
 // places of the terms [t0, t1); the launches go up the terms
@@ -212,56 +288,46 @@ int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, 
   const bool apart = ((uint64_t)(tab.size() - 1) << shift) >> 32;
   if (apart) shift = 32;
   const int64_t nt = (int64_t)terms.size();
-  DevBuf cnt, first, dtw, num, order;
-  if (cnt.alloc(4 * (size_t)rows) || first.alloc(4 * (size_t)rows) || order.alloc(4 * (size_t)rows) ||
-      dtw.alloc(nt) || num.alloc(4 * nt) || s.wtab.alloc(8 * tab.size()))
-    return SG4_OK;
-  const dim3 blk(256), tg((unsigned)std::min<int64_t>(nt, 8192));
-  RS_TRY(hipMemcpyAsync(dtw.p, tw.data(), nt, hipMemcpyHostToDevice, st));
+  const int ntp = (int)((nt + SCAN - 1) / SCAN), nrp = (int)((rows + SCAN - 1) / SCAN);
+  // one workspace: partial sums, then counts, first places and order of the
+  // rows, the terms' first rows, the terms' weight indices
+  const size_t b_part = 8 * ((size_t)std::max(ntp, nrp) + 1), b_rows = 4 * (size_t)rows;
+  DevBuf ws;
+  if (ws.alloc(b_part + 3 * b_rows + 4 * (size_t)nt + (size_t)nt) || s.wtab.alloc(8 * tab.size())) return SG4_OK;
+  uint64_t* part = ws.as<uint64_t>();
+  int32_t *cnt = (int32_t*)(ws.as<char>() + b_part), *first = cnt + rows, *order = first + rows, *num = order + rows;
+  uint8_t* dtw = (uint8_t*)(num + nt);
+  const dim3 blk(256), sblk(SCAN), tg((unsigned)std::min<int64_t>(nt, 8192));
+  RS_TRY(hipMemcpyAsync(dtw, tw.data(), nt, hipMemcpyHostToDevice, st));
   RS_TRY(hipMemcpyAsync(s.wtab.p, tab.data(), 8 * tab.size(), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_rs_init, dim3(512), blk, 0, st, cnt.as<int32_t>(), first.as<int32_t>(), rows);
-  hipLaunchKernelGGL(k_rs_count, dim3(2048), blk, 0, st, d_map, sum_nb, cnt.as<int32_t>(), first.as<int32_t>());
-  hipLaunchKernelGGL(k_rs_first<false>, tg, blk, 0, st, d_map, first.as<int32_t>(), d_terms, nt, num.as<int32_t>(),
-                     (const int32_t*)nullptr, (int32_t*)nullptr);
-  std::vector<int32_t> c(rows), base(nt), ord(rows);
-  RS_TRY(hipMemcpyAsync(base.data(), num.p, 4 * nt, hipMemcpyDeviceToHost, st));
+  hipLaunchKernelGGL(k_rs_init, dim3(512), blk, 0, st, cnt, first, order, rows);
+  hipLaunchKernelGGL(k_rs_count, dim3(2048), blk, 0, st, d_map, sum_nb, cnt, first);
+  hipLaunchKernelGGL(k_rs_first<false>, tg, blk, 0, st, d_map, first, d_terms, nt, num, (const int32_t*)nullptr,
+                     (int32_t*)nullptr);
+  hipLaunchKernelGGL(k_rs_sums, dim3(ntp), sblk, 0, st, num, (const int32_t*)nullptr, nt, part);
+  hipLaunchKernelGGL(k_rs_scan, dim3(1), sblk, 0, st, part, ntp);
+  hipLaunchKernelGGL(k_rs_base, dim3(ntp), sblk, 0, st, num, nt, part);
+  hipLaunchKernelGGL(k_rs_first<true>, tg, blk, 0, st, d_map, first, d_terms, nt, (int32_t*)nullptr, num, order);
+  hipLaunchKernelGGL(k_rs_sums, dim3(nrp), sblk, 0, st, cnt, order, rows, part);
+  hipLaunchKernelGGL(k_rs_scan, dim3(1), sblk, 0, st, part, nrp);
+  RS_TRY(hipGetLastError());
+  uint64_t total = 0;
+  RS_TRY(hipMemcpyAsync(&total, part + nrp, sizeof(total), hipMemcpyDeviceToHost, st));
   RS_TRY(hipStreamSynchronize(st));
-  int32_t nord = 0;
-  for (int64_t t = 0; t < nt; ++t) {
-    const int32_t n = base[t];
-    base[t] = nord;
-    nord += n;
-  }
-  RS_TRY(hipMemcpyAsync(num.p, base.data(), 4 * nt, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_rs_first<true>, tg, blk, 0, st, d_map, first.as<int32_t>(), d_terms, nt, (int32_t*)nullptr,
-                     num.as<int32_t>(), order.as<int32_t>());
-  RS_TRY(hipMemcpyAsync(ord.data(), order.p, 4 * (size_t)nord, hipMemcpyDeviceToHost, st));
-  RS_TRY(hipMemcpyAsync(c.data(), cnt.p, 4 * (size_t)rows, hipMemcpyDeviceToHost, st));
-  RS_TRY(hipStreamSynchronize(st));
-  int64_t nseg = 0;
-  for (int32_t i = 0; i < nord; ++i) nseg += (c[ord[i]] + RS_SEG - 1) / RS_SEG;
+  const int64_t nseg = (int64_t)(total >> 32), places = (int64_t)(uint32_t)total;
   if (nseg == 0) return SG4_OK;
-  std::vector<int32_t> sg(2 * nseg + 1);
-  int32_t at = 0;
-  int64_t k = 0;
-  for (int32_t i = 0; i < nord; ++i) {
-    const int32_t r = ord[i], n = c[r];
-    c[r] = at;
-    for (int32_t o = 0; o < n; o += RS_SEG, ++k) {
-      sg[k] = at + o;
-      sg[nseg + 1 + k] = (int32_t)((uint32_t)r | (n > RS_SEG ? RS_MULTI : 0u));
-    }
-    at += n;
+  if (s.pos.alloc(4 * (size_t)places) || (apart && s.wi.alloc((size_t)places)) ||
+      s.seg.alloc(4 * (2 * (size_t)nseg + 1))) {
+    (void)s.pos.alloc(0);
+    (void)s.wi.alloc(0);
+    return SG4_OK;
   }
-  sg[nseg] = at;
-  if (s.pos.alloc(4 * (size_t)at) || (apart && s.wi.alloc((size_t)at)) || s.seg.alloc(4 * sg.size())) return SG4_OK;
-  RS_TRY(hipMemcpyAsync(cnt.p, c.data(), 4 * (size_t)rows, hipMemcpyHostToDevice, st));
-  RS_TRY(hipMemcpyAsync(s.seg.p, sg.data(), 4 * sg.size(), hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_rs_segs, dim3(nrp), sblk, 0, st, cnt, order, rows, part, s.seg.as<int32_t>(), nseg, (int32_t)places);
   for (int i = 0; i < RS_BATCH; ++i) {
     const int64_t t0 = nt * i / RS_BATCH, t1 = nt * (i + 1) / RS_BATCH;
     if (t1 > t0)
       hipLaunchKernelGGL(k_rs_fill, dim3((unsigned)std::min<int64_t>(t1 - t0, 8192)), blk, 0, st, d_map, d_terms,
-                         dtw.as<uint8_t>(), t0, t1, shift, cnt.as<int32_t>(), s.pos.as<uint32_t>(), s.wi.as<uint8_t>());
+                         dtw, t0, t1, shift, cnt, s.pos.as<uint32_t>(), s.wi.as<uint8_t>());
   }
   hipLaunchKernelGGL(k_rs_sort, dim3((unsigned)((nseg + 3) / 4)), blk, 0, st, s.pos.as<uint32_t>(),
                      s.wi.as<uint8_t>(), s.seg.as<int32_t>(), nseg, (uint32_t)((1ull << shift) - 1));
