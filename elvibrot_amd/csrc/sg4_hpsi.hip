@@ -403,12 +403,14 @@ static int not_prepared() {
 // lists, the term and matrix tables, the kinetic matrix, the FP32 copies) and
 // the launch configuration of their capture: every call that reallocates
 // those buffers or changes the configuration destroys them, and the next
-// sg4_apply_graph captures again.
+// sg4_apply_graph captures again.  The block of results that they share goes
+// with them.
 static void drop_graphs(sg4_plan* P) {
-  if (P->graphs.empty()) return;
-  if (P->own_stream) (void)hipStreamSynchronize(P->own_stream);
+  if (!P->own_stream) return;
+  if (!P->graphs.empty()) (void)hipStreamSynchronize(P->own_stream);
   for (auto& g : P->graphs) (void)hipGraphExecDestroy(g.exec);
   P->graphs.clear();
+  rowsum_drop(P->rowsum, P->own_stream);
 }
 
 // The operator or the term set changed: everything derived from them.
@@ -420,6 +422,7 @@ static void invalidate(sg4_plan* P) {
   P->nm.valid = false;
   P->nm_seen.clear();
   P->pt_seen.clear();
+  P->rowsum.failed = SIZE_MAX;
 }
 
 // Greedy grouping of consecutive active modes into the shapes of
@@ -1486,8 +1489,12 @@ static void* use_rowsum(sg4_plan* P, int nvec, int prec, bool now = false) {
   if (!P->rowsum.ok) return nullptr;
   const size_t bytes = rowsum_bytes(P, nvec, prec == SG4_PREC_FP64 ? 8 : 4) +
                        (prec == SG4_PREC_F32 ? sizeof(float) * P->nb_ba * nvec : 0);
-  // graphs of the plan's own stream hold their blocks
-  return rowsum_block(P->rowsum, P->stream, bytes, alloc, P->stream && P->stream == P->own_stream);
+  if (void* o = rowsum_held(P->rowsum, P->stream, bytes)) return o;
+  if (!alloc || !rowsum_fits(P->rowsum, P->stream, bytes)) return nullptr;
+  // the plan's graphs share the block of its own stream: the narrower ones are
+  // captured again with the larger one
+  if (P->own_stream && P->stream == P->own_stream) drop_graphs(P);
+  return rowsum_alloc(P->rowsum, P->stream, bytes);
 }
 
 // Everything an apply needs that may allocate or copy (FP32 copies, item
@@ -2561,6 +2568,7 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   p->timing = timing;
+  if (use_nmode(p, prec)) rowsum_drop(p->rowsum, p->stream);   // later applies leave it unused
   if (rc) return rc;
   drop_graphs(p);
   p->nm_seen.clear();

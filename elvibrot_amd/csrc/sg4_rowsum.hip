@@ -340,21 +340,37 @@ int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, 
   return SG4_OK;
 }
 
-void* rowsum_block(RowSum& s, hipStream_t st, size_t bytes, bool alloc, bool keep) {
+void* rowsum_held(const RowSum& s, hipStream_t st, size_t bytes) {
   for (const auto& o : s.out)
     if (o->stream == st && o->buf.n >= bytes) return o->buf.p;
-  if (!alloc || bytes > RS_MAX_BYTES) return nullptr;
-  if (!keep)   // freeing waits for the applies that still use it
-    s.out.erase(std::remove_if(s.out.begin(), s.out.end(), [&](const auto& o) { return o->stream == st; }),
-                s.out.end());
-  size_t held = 0;
-  for (const auto& o : s.out) held += o->buf.n;
-  if (s.out.size() >= RS_MAX_BLOCKS || held + bytes > RS_MAX_BYTES) return nullptr;
-  auto o = std::make_unique<RowSum::Out>();
-  o->stream = st;
-  if (o->buf.alloc(bytes)) return nullptr;
-  s.out.push_back(std::move(o));
-  return s.out.back()->buf.p;
+  return nullptr;
+}
+
+bool rowsum_fits(const RowSum& s, hipStream_t st, size_t bytes) {
+  size_t held = 0, blocks = 0;
+  for (const auto& o : s.out)
+    if (o->stream != st) { held += o->buf.n; ++blocks; }
+  return bytes < s.failed && blocks < RS_MAX_BLOCKS && held + bytes <= RS_MAX_BYTES;
+}
+
+void* rowsum_alloc(RowSum& s, hipStream_t st, size_t bytes) {
+  RowSum::Out* o = nullptr;
+  for (const auto& x : s.out)
+    if (x->stream == st) o = x.get();
+  const size_t had = o ? o->buf.n : 0;
+  if (!o) {
+    s.out.push_back(std::make_unique<RowSum::Out>());
+    o = s.out.back().get();
+    o->stream = st;
+  }
+  if (o->buf.alloc(bytes) == SG4_OK) return o->buf.p;   // freeing waits for the applies that still use it
+  s.failed = bytes;
+  if (!had || o->buf.alloc(had)) rowsum_drop(s, st);
+  return nullptr;
+}
+
+void rowsum_drop(RowSum& s, hipStream_t st) {
+  s.out.erase(std::remove_if(s.out.begin(), s.out.end(), [&](const auto& o) { return o->stream == st; }), s.out.end());
 }
 
 int rowsum_add(const RowSum& s, const double* out, int nvec, double* hpsi, hipStream_t st) {
