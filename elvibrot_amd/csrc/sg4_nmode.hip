@@ -585,6 +585,15 @@ __global__ __launch_bounds__(1024) void k_nm_ptr(const int32_t* cnt, int64_t n, 
 
 struct alignas(8) Two { double x, y; };
 
+// Workgroups of the products in x and z: a launch takes fewer than 2^32 threads
+// in a direction, which 16 lanes a row reach at 2^28 rows.
+constexpr int64_t MAX_BLOCKS_X = (int64_t)1 << 23;
+__device__ __forceinline__ int64_t block_xz() { return blockIdx.x + (int64_t)gridDim.x * blockIdx.z; }
+dim3 grid_xz(int64_t blocks, int y) {
+  const int64_t z = (blocks + MAX_BLOCKS_X - 1) / MAX_BLOCKS_X;
+  return dim3((unsigned)((blocks + z - 1) / z), (unsigned)y, (unsigned)z);
+}
+
 // hpsi(r, v) = sum_e val_e psi(col_e, v): NV * SL lanes per row, NV vectors,
 // the row's entries dealt to SL slices that are added at the end.
 // OUT_COLS: the result goes to the column-major block (nvec <= NV columns),
@@ -600,7 +609,7 @@ __global__ __launch_bounds__(256) void k_nm_spmm(const int64_t* __restrict__ ptr
   constexpr int W = NV * SL, R = 256 / W;
   __shared__ double tile[COLS ? NV * (R + 1) : 1];
   const int l = threadIdx.x % W, v = l % NV, s = l / NV;
-  const int64_t r = (int64_t)blockIdx.x * R + threadIdx.x / W;
+  const int64_t r = block_xz() * R + threadIdx.x / W;
   const double* __restrict__ x0 = IN_COLS ? psi + (int64_t)min(v, nvec - 1) * rows : psi + v;
   constexpr int LD = IN_COLS ? 1 : NV;
   double a = 0.0;
@@ -632,7 +641,7 @@ __global__ __launch_bounds__(256) void k_nm_spmm(const int64_t* __restrict__ ptr
     __syncthreads();
     for (int t = threadIdx.x; t < NV * R; t += 256) {
       const int vv = t / R, rr = t % R;
-      const int64_t ro = (int64_t)blockIdx.x * R + rr;
+      const int64_t ro = block_xz() * R + rr;
       if (vv < nvec && ro < rows) hpsi[(int64_t)vv * rows + ro] = tile[vv * (R + 1) + rr];
     }
   }
@@ -655,7 +664,7 @@ __global__ __launch_bounds__(256) void k_nm_spmm_pairs(const int64_t* __restrict
   constexpr int W = NC * SL, R = 256 / W, NV = 2 * NC * PV;
   __shared__ double tile[COLS ? NV * (R + 1) : 1];
   const int l = threadIdx.x % W, j = l % NC, s = l / NC, rr = threadIdx.x / W;
-  const int64_t r = (int64_t)blockIdx.x * R + rr;
+  const int64_t r = block_xz() * R + rr;
   const int64_t ld = WIDE ? nvec / 2 : NC * PV;           // pairs per row
   const int64_t j0 = j + (WIDE ? (int64_t)blockIdx.y * (NC * PV) : 0);
   const Two* __restrict__ x = (const Two*)psi + j0;
@@ -722,7 +731,7 @@ __global__ __launch_bounds__(256) void k_nm_spmm_pairs(const int64_t* __restrict
     __syncthreads();
     for (int t = threadIdx.x; t < NV * R; t += 256) {
       const int vv = t / R, ro = t % R;
-      const int64_t row = (int64_t)blockIdx.x * R + ro;
+      const int64_t row = block_xz() * R + ro;
       if (vv < nvec && row < rows) hpsi[(int64_t)vv * rows + row] = tile[vv * (R + 1) + ro];
     }
   }
@@ -1387,11 +1396,11 @@ int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hi
   const int64_t* ptr = m.ptr.as<int64_t>();
   const int32_t* col = m.col.as<int32_t>();
 #define SG4_SPMM(NV, SL)                                                                              \
-  hipLaunchKernelGGL((k_nm_spmm<NV, SL, COLS, IN_COLS>), dim3((unsigned)((m.rows * NV * SL + 255) / 256)),     \
+  hipLaunchKernelGGL((k_nm_spmm<NV, SL, COLS, IN_COLS>), grid_xz((m.rows * NV * SL + 255) / 256, 1),           \
                      dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec, psi32)
 #define SG4_PAIRS(NC, PV, SL, SU, WIDE)                                                                \
   hipLaunchKernelGGL((k_nm_spmm_pairs<NC, PV, SL, SU, COLS, WIDE>),                                    \
-                     dim3((unsigned)((m.rows * NC * SL + 255) / 256), WIDE ? W / (2 * NC * PV) : 1),   \
+                     grid_xz((m.rows * NC * SL + 255) / 256, WIDE ? W / (2 * NC * PV) : 1),            \
                      dim3(256), 0, st, ptr, col, val, psi, hpsi, m.rows, nvec, psi32)
   if constexpr (IN_COLS) {
     switch (W) {

@@ -3,8 +3,10 @@
 // do not run, and every call that matters is kept in a log.  Loaded with global
 // visibility before the library, its symbols take the place of the runtime's.
 // Fresh memory is filled with one 32-bit word (hh_fill), so that a test chooses
-// what the kernels that did not run have left behind.
+// what the kernels that did not run have left behind (allocations beyond 1 GiB
+// are zeros and take no memory until they are written).
 #include <hip/hip_runtime_api.h>
+#include <sys/mman.h>
 
 #include <cstdlib>
 #include <cstring>
@@ -20,6 +22,8 @@ long g_allow = -1;          // allocations that succeed before one fails; -1: al
 size_t g_limit = 0;         // bytes of device memory; 0: unlimited
 size_t g_held = 0;
 int g_handles = 0;
+hipError_t g_last = hipSuccess;
+constexpr size_t BIG = size_t(1) << 30;
 struct Cfg { dim3 g, b; size_t lds; hipStream_t st; } g_cfg;
 
 void note(const std::string& s) { g_log += s + "\n"; }
@@ -50,6 +54,9 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t st) {
   note("launch " + g_names[f] + " " + num(g.x) + " " + num(g.y) + " " + num(g.z) + " " + num(b.x) + " " + at(st));
+  // the runtime's limit: fewer than 2^32 threads in every direction
+  if ((size_t)g.x * b.x >> 32 || (size_t)g.y * b.y >> 32 || g.y > 65535 || g.z > 65535)
+    return g_last = hipErrorInvalidConfiguration;
   return hipSuccess;
 }
 hipError_t hipMalloc(void** p, size_t n) {
@@ -58,8 +65,12 @@ hipError_t hipMalloc(void** p, size_t n) {
     note("nomem " + num(n));
     return hipErrorOutOfMemory;
   }
-  *p = std::malloc(n + 256);
-  for (size_t i = 0; i < n / 4; ++i) ((int*)*p)[i] = g_fill;
+  if (n > BIG) {
+    *p = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  } else {
+    *p = std::malloc(n + 256);
+    for (size_t i = 0; i < n / 4; ++i) ((int*)*p)[i] = g_fill;
+  }
   g_mem[*p] = n;
   g_held += n;
   note("malloc " + num(n) + " " + at(*p));
@@ -70,8 +81,9 @@ hipError_t hipFree(void* p) {
   if (i == g_mem.end()) return hipErrorInvalidValue;
   note("free " + num(i->second) + " " + at(p));
   g_held -= i->second;
+  if (i->second > BIG) munmap(p, i->second);
+  else std::free(p);
   g_mem.erase(i);
-  std::free(p);
   return hipSuccess;
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { note("memcpy " + num(n)); std::memcpy(d, s, n); return hipSuccess; }
@@ -107,7 +119,11 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1.0f; 
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600*, int) { return hipErrorUnknown; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { static void* s = std::malloc(size_t(256) << 20); *p = s; return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
