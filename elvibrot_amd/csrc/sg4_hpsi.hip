@@ -321,7 +321,7 @@ struct sg4_plan {
   sg4::DevBuf d_rows_in, d_rows_out, d_cols_in, d_cols_out;
   std::map<int64_t, std::unique_ptr<sg4::ItemPlan>> items;  // per (nvec, size, budget, order)
   std::map<int, sg4::LaunchCfg> tuned;                       // per (nvec, precision)
-  std::map<int, sg4::LaunchCfg> defaults;                    // likewise, of default_cfg
+  mutable std::map<int, sg4::LaunchCfg> defaults;            // likewise, of default_cfg
   hipStream_t own_stream = nullptr;                          // for graph capture on the null stream
   struct GraphEntry { int nvec, prec; const double* psi; double* hpsi; hipGraphExec_t exec; };
   std::vector<GraphEntry> graphs;
@@ -1402,7 +1402,7 @@ static bool take_nmode(const sg4_plan* P, int prec) { return use_nmode(P, prec) 
 // XCD (10D L=8 x16 6.1 -> 4.7 ms, 10D L=7 x8 656 -> 629 us, 8D L=6 x32 in
 // FP32 94 -> 99).  With atomics the smaller budgets only add contention (10D
 // L=8 x16 9.1 -> 11.4 ms).
-static LaunchCfg default_cfg(sg4_plan* P, int nvec, int prec) {
+static LaunchCfg default_cfg(const sg4_plan* P, int nvec, int prec) {
   const int key = nvec * 16 + prec;
   auto it = P->defaults.find(key);
   if (it != P->defaults.end()) return it->second;
@@ -1433,7 +1433,7 @@ static LaunchCfg default_cfg(sg4_plan* P, int nvec, int prec) {
 // far more than on the block width, so a block of 8 vectors in a Davidson
 // iteration runs with the launch tuned for 16.  When none is set: default_cfg
 // if the terms' results are summed row by row, else LaunchCfg's values.
-static LaunchCfg cfg_for(sg4_plan* P, int nvec, int prec, bool rowsum) {
+static LaunchCfg cfg_for(const sg4_plan* P, int nvec, int prec, bool rowsum) {
   auto it = P->tuned.find(nvec * 16 + prec);
   if (it != P->tuned.end()) return it->second;
   const LaunchCfg* best = nullptr;
@@ -1450,6 +1450,13 @@ static LaunchCfg cfg_for(sg4_plan* P, int nvec, int prec, bool rowsum) {
 // Bytes of the terms' results; the FP32 mode's copy of psi follows them.
 static size_t rowsum_bytes(const sg4_plan* P, int nvec, int esize) {
   return ((size_t)P->sum_nb * nvec * esize + 255) & ~(size_t)255;
+}
+static size_t rowsum_block_bytes(const sg4_plan* P, int nvec, int prec) {
+  return rowsum_bytes(P, nvec, prec == SG4_PREC_FP64 ? 8 : 4) +
+         (prec == SG4_PREC_F32 ? sizeof(float) * P->nb_ba * nvec : 0);
+}
+static bool rowsum_able(const sg4_plan* P, int prec) {
+  return !P->deterministic && use_split_for(P, prec) && P->sum_nb >= ROWSUM_MIN;
 }
 
 // Whether the applies so far would have saved what inverting the map (and the
@@ -1479,16 +1486,14 @@ static bool rowsum_pays(sg4_plan* P, int nvec) {
 // The block belongs to the plan's stream: an apply that the caller captures
 // keeps the atomics, since its graph may run beside the plan's other work.
 static void* use_rowsum(sg4_plan* P, int nvec, int prec, bool now = false) {
-  if (P->deterministic || !use_split_for(P, prec) || P->sum_nb < ROWSUM_MIN) return nullptr;
-  if (caller_captures(P)) return nullptr;
+  if (!rowsum_able(P, prec) || caller_captures(P)) return nullptr;
   const bool alloc = !P->no_alloc && !captured(P);
   if (alloc && !P->rowsum.tried && !now && !rowsum_pays(P, nvec)) return nullptr;
   if (alloc && rowsum_build(P->rowsum, P->d_map.as<int32_t>(), P->sum_nb, P->nb_ba, P->d_terms.as<TermDev>(),
                             P->h_terms, P->stream))
     return nullptr;
   if (!P->rowsum.ok) return nullptr;
-  const size_t bytes = rowsum_bytes(P, nvec, prec == SG4_PREC_FP64 ? 8 : 4) +
-                       (prec == SG4_PREC_F32 ? sizeof(float) * P->nb_ba * nvec : 0);
+  const size_t bytes = rowsum_block_bytes(P, nvec, prec);
   if (void* o = rowsum_held(P->rowsum, P->stream, bytes)) return o;
   if (!alloc || !rowsum_fits(P->rowsum, P->stream, bytes)) return nullptr;
   // the plan's graphs share the block of its own stream: the narrower ones are
@@ -2579,8 +2584,10 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
 
 int sg4_plan_config(const sg4_plan* p, int32_t nvec, int32_t prec, int32_t* cfg4) {
   if (!p || !cfg4) { set_error("null argument"); return SG4_ERR_ARG; }
-  sg4_plan* q = const_cast<sg4_plan*>(p);   // default_cfg keeps what it derives
-  const LaunchCfg c = cfg_for(q, nvec, prec, !p->deterministic && use_split_for(p, prec));
+  const size_t bytes = rowsum_block_bytes(p, nvec, prec);
+  const bool sums = rowsum_able(p, prec) && p->rowsum.ok &&
+                    (rowsum_held(p->rowsum, p->stream, bytes) || rowsum_fits(p->rowsum, p->stream, bytes));
+  const LaunchCfg c = cfg_for(p, nvec, prec, sums);
   cfg4[0] = std::max(c.nthreads, 256); cfg4[1] = c.lds_budget; cfg4[2] = c.grid; cfg4[3] = c.xcd;
   return SG4_OK;
 }

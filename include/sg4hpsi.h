@@ -346,8 +346,9 @@ int sg4_plan_autotune(sg4_plan *p, int32_t nvec, int32_t prec, float *best_ms);
 /* the launch parameters in use for (nvec, prec): threads, LDS budget, grid, xcd.
  * A block width with no parameters of its own (tuned or set) uses those of the
  * nearest configured width of the same precision (the narrowest wider one
- * first), else the defaults (which follow the sizes; fewer than 256 threads
- * are reported as 256). */
+ * first), else the defaults: 256 threads and 64 KiB while the terms add with
+ * atomics, and a launch that follows the sizes (fewer than 256 threads are
+ * reported as 256) once their results are summed row by row. */
 int sg4_plan_config(const sg4_plan *p, int32_t nvec, int32_t prec, int32_t *cfg4);
 /* set the launch parameters for (nvec, prec) (e.g. a configuration saved from
  * an earlier autotune): threads 256 or 512 (768 for the FP32 mode on the split
