@@ -579,10 +579,14 @@ static int build_kinetic(sg4_plan* P) {
   const NModeIn in = nmode_in(P);
   if (!P->nmt && !(P->nmt = nmode_tables_create(in))) return SG4_ERR_HIP;
   if (nmode_rows_ok(P->nmt)) {
-    if ((rc = nmode_build_kinetic(P->nmt, in, P->kin))) return rc;
-    P->split_ok = true;
-    P->split_fp = fp;
-    return SG4_OK;
+    rc = nmode_build_kinetic(P->nmt, in, P->kin);
+    if (rc && rc != SG4_ERR_OOM) return rc;
+    if (rc == SG4_OK) {
+      P->split_ok = true;
+      P->split_fp = fp;
+      return SG4_OK;
+    }
+    // no memory for its workspace: the host's sweeps need the matrix alone
   }
   // two sweeps over (row, mode) pairs: count, then fill
   const int64_t nrows = P->nb_ba;

@@ -47,7 +47,7 @@ struct NModeIn {
 
 // Index tables of a plan (they depend on its tables only, not on V).
 struct NModeTables;
-NModeTables* nmode_tables_create(const NModeIn& in);   // null: HIP failure
+NModeTables* nmode_tables_create(const NModeIn& in);   // null: HIP failure; without rows_ok where memory is short
 void nmode_tables_destroy(NModeTables* t);
 
 // Whether the packed rows are in lexicographic order (the last mode's index

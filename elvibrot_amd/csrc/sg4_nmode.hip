@@ -921,6 +921,8 @@ void nmode_tables_destroy(NModeTables* t) { delete t; }
 
 NModeTables* nmode_tables_create(const NModeIn& in) {
   auto t = std::make_unique<NModeTables>();
+  // a plan without them: no sparse matrices, K from the host
+  auto no_memory = [] { return new NModeTables; };
   const int ni = (int)in.inst.size();
   t->dev.resize(ni);
   for (const NModeInst& I : in.inst) {
@@ -1116,8 +1118,9 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
   t->o_cut2 = blob.add(cut2);
   t->o_g1work = blob.add(g1work);
   t->o_none = blob.add(std::vector<int32_t>((size_t)ni * 33 + 33, 0));   // no pairs
-  if (upload(blob, t->blob, in.stream) != SG4_OK || t->ck.alloc(sizeof(double) * in.ck->size()) != SG4_OK)
-    return nullptr;
+  int rc = upload(blob, t->blob, in.stream);
+  if (!rc) rc = t->ck.alloc(sizeof(double) * in.ck->size());
+  if (rc) return rc == SG4_ERR_OOM ? no_memory() : nullptr;
   char* B = t->blob.as<char>();
   for (int x = 0; x < ni; ++x) {
     const NModeInst& I = in.inst[x];
@@ -1134,9 +1137,10 @@ NModeTables* nmode_tables_create(const NModeIn& in) {
   }
   Blob ib;
   ib.add(t->dev);
-  if (upload(ib, t->insts, in.stream) != SG4_OK) return nullptr;
+  rc = upload(ib, t->insts, in.stream);
+  if (!rc) rc = ensure(t->work, 256);
+  if (rc) return rc == SG4_ERR_OOM ? no_memory() : nullptr;
   // the packed rows in lexicographic order?
-  if (ensure(t->work, 256) != SG4_OK) return nullptr;
   int* bad = t->work.as<int>();
   hipLaunchKernelGGL(k_nm_zero, dim3(1), dim3(64), 0, in.stream, bad, 1);
   hipLaunchKernelGGL(k_nm_check_map, dim3((unsigned)std::min<int64_t>(t->nterms, 16384)), dim3(256), 0,
