@@ -2523,7 +2523,17 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
-  const bool timing = p->timing;
+  struct Restore {     // on every way out
+    sg4_plan* p;
+    bool timing;
+    hipEvent_t e0, e1;
+    ~Restore() {
+      p->nm_off = false;
+      p->timing = timing;
+      (void)hipEventDestroy(e0);
+      (void)hipEventDestroy(e1);
+    }
+  } restore{p, p->timing, e0, e1};
   p->timing = false;
   p->nm_off = true;    // tune the term kernels also where FP64 takes the sparse path
   (void)use_rowsum(p, nvec, prec, true);   // every launch is timed on the path that later applies take
@@ -2574,9 +2584,6 @@ int sg4_plan_autotune(sg4_plan* p, int32_t nvec, int32_t prec, float* best_ms) {
     HIP_TRY(hipEventElapsedTime(&bms, e0, e1));
     bms /= 3;
   }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  p->timing = timing;
   if (use_nmode(p, prec)) rowsum_drop(p->rowsum, p->stream);   // later applies leave it unused
   if (rc) return rc;
   drop_graphs(p);
