@@ -29,6 +29,9 @@ constexpr int SCAN = 1024;                       // items per workgroup of a sca
 constexpr size_t RS_MAX_BYTES = size_t(16) << 30; // results held per plan
 constexpr size_t RS_MAX_BLOCKS = 8;
 constexpr int RS_WEIGHTS = 256;                 // distinct term weights
+// A segment's indices run up to RS_LOADS times its lanes beyond its end, in 32
+// bits; a launch with a lane per place of every segment takes 2^32 threads.
+constexpr int64_t RS_PLACES = INT32_MAX - 4096, RS_SEGMENTS = (int64_t(1) << 32) / RS_SEG - 4;
 constexpr uint32_t RS_MULTI = 0x80000000u;
 
 #define RS_TRY(x)                                     \
@@ -273,7 +276,7 @@ int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, 
                  const std::vector<TermDev>& terms, hipStream_t st) {
   if (s.tried) return SG4_OK;
   s.tried = true;
-  if (sum_nb >= INT32_MAX || rows >= INT32_MAX) return SG4_OK;
+  if (sum_nb >= RS_PLACES || rows >= INT32_MAX) return SG4_OK;
   std::map<double, int> ids;
   std::vector<double> tab;
   std::vector<uint8_t> tw(terms.size());
@@ -315,7 +318,7 @@ int rowsum_build(RowSum& s, const int32_t* d_map, int64_t sum_nb, int64_t rows, 
   RS_TRY(hipMemcpyAsync(&total, part + nrp, sizeof(total), hipMemcpyDeviceToHost, st));
   RS_TRY(hipStreamSynchronize(st));
   const int64_t nseg = (int64_t)(total >> 32), places = (int64_t)(uint32_t)total;
-  if (nseg == 0) return SG4_OK;
+  if (nseg == 0 || nseg >= RS_SEGMENTS) return SG4_OK;
   if (s.pos.alloc(4 * (size_t)places) || (apart && s.wi.alloc((size_t)places)) ||
       s.seg.alloc(4 * (2 * (size_t)nseg + 1))) {
     (void)s.pos.alloc(0);
