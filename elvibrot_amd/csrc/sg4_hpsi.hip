@@ -360,10 +360,12 @@ struct sg4_plan {
   std::set<int> pt_seen;
   double flops_split = 0;        // algorithmic flops per vector of the split path's terms
   // H as one sparse matrix (sg4_nmode.hip): the field-free operator and, during
-  // a propagation, the one with the dipole; field_on: V holds a field term
+  // a propagation, the one with the dipole; field_on: V holds a field term;
+  // field_graph: a graph of the caller sets fields, so V may hold one at any time
   sg4::NModeTables* nmt = nullptr;
   sg4::NModeMat nm, nm_field;
-  bool field_on = false, nm_off = false;
+  bool field_on = false, field_graph = false, nm_off = false;
+  bool graphs_stale = false;     // a field changed the path: the next sg4_apply_graph drops the graphs
   bool sparse = true;            // SG4_OPT_SPARSE
   std::set<int> nm_seen;         // block widths that the sparse path prepared (apply_nmode)
   // split-precision MFMA path (SG4_PREC_F32X2): terms cut into mode groups,
@@ -406,6 +408,7 @@ static int not_prepared() {
 // sg4_apply_graph captures again.  The block of results that they share goes
 // with them.
 static void drop_graphs(sg4_plan* P) {
+  P->graphs_stale = false;
   if (!P->own_stream) return;
   if (!P->graphs.empty()) (void)hipStreamSynchronize(P->own_stream);
   for (auto& g : P->graphs) (void)hipGraphExecDestroy(g.exec);
@@ -1373,8 +1376,8 @@ static bool use_split_for(const sg4_plan* P, int prec) {
 
 // FP64 applies of a field-free operator that is a sparse matrix.
 static bool use_nmode(const sg4_plan* P, int prec) {
-  return prec == SG4_PREC_FP64 && P->nm.valid && P->sparse && !P->field_on && !P->nm_off && !P->deterministic &&
-         use_split_alg(P);
+  return prec == SG4_PREC_FP64 && P->nm.valid && P->sparse && !P->field_on && !P->field_graph && !P->nm_off &&
+         !P->deterministic && use_split_alg(P);
 }
 
 // Whether the plan's stream is being captured, and by the caller (the plan
@@ -1833,7 +1836,9 @@ int plan_is_grid_function(const sg4_plan* P, const sg4_plan* H, const double* mu
   return SG4_OK;
 }
 
-int plan_clear_field(sg4_plan* P) { return P->field_on ? sg4_plan_set_field(P, nullptr, 0.0) : SG4_OK; }
+int plan_clear_field(sg4_plan* P) {
+  return P->field_on || P->field_graph ? sg4_plan_set_field(P, nullptr, 0.0) : SG4_OK;
+}
 
 // The kernels add into their outputs with hardware floating-point atomics
 // compiled with -munsafe-fp-atomics; those are correct on coarse-grained
@@ -2193,7 +2198,7 @@ int sg4_plan_set_operator(sg4_plan* p, const sg4_operator* op) {
   p->type_op = op->type_op;
   HIP_TRY(hipMemcpy(p->d_V.p, op->V, sizeof(double) * p->sum_nq, hipMemcpyHostToDevice));
   (void)p->d_V0.alloc(0);
-  p->field_on = false;
+  p->field_on = p->field_graph = false;
   return build_terms(p);
 }
 
@@ -2216,7 +2221,7 @@ int sg4_plan_set_operator_type1(sg4_plan* p, int32_t nder, const int32_t* der, c
   p->type_op = 11;
   p->h_ck.assign(p->nck, 0.0);
   (void)p->d_V0.alloc(0);
-  p->field_on = false;
+  p->field_on = p->field_graph = false;
   return build_terms(p);
 }
 
@@ -2239,7 +2244,7 @@ int sg4_plan_set_henon_heiles(sg4_plan* p, double lambda) {
   HIP_TRY(hipGetLastError());
   p->type_op = 1;
   (void)p->d_V0.alloc(0);
-  p->field_on = false;
+  p->field_on = p->field_graph = false;
   p->h_ck.assign(p->nck, -0.5);
   int rc;
   if ((rc = p->d_ck.alloc(sizeof(double) * p->nck))) return rc;
@@ -2301,7 +2306,7 @@ int sg4_plan_set_jacobi_triatomic(sg4_plan* p, const double* prm) {
   HIP_TRY(hipGetLastError());
   p->type_op = 10;
   (void)p->d_V0.alloc(0);
-  p->field_on = false;
+  p->field_on = p->field_graph = false;
   p->h_ck.assign(p->nck, 0.0);
   rc = build_terms(p);
   if (rc) return rc;
@@ -2469,9 +2474,13 @@ int sg4_plan_set_field(sg4_plan* p, const double* mu, double eps) {
                      p->d_V0.as<double>(), mu, eps, p->d_V.as<double>(), p->sum_nq);
   HIP_TRY(hipGetLastError());
   p->f32_valid = false;
-  // FP64 graphs of the sparse path do not read V: a field changes the path
-  if (p->field_on != (mu != nullptr) && p->nm.valid) drop_graphs(p);
+  // FP64 graphs of the sparse path do not read V: a field changes the path.  They
+  // are dropped later, since this call may be part of a capture; then V changes
+  // at every replay, whatever the last call here said.
+  const bool graph = p->field_graph || caller_captures(p);
+  if ((p->field_on != (mu != nullptr) || p->field_graph != graph) && p->nm.valid) p->graphs_stale = true;
   p->field_on = mu != nullptr;
+  p->field_graph = graph;
   return SG4_OK;
 }
 
@@ -2628,6 +2637,7 @@ int sg4_apply_graph(sg4_plan* p, int32_t nvec, const double* psi, double* hpsi, 
   if ((rc = device_blocks(p, psi, hpsi))) return rc;
   if ((rc = check_apply(p, nvec, prec))) return rc;
   if (blocks_overlap(p, nvec, psi, hpsi)) return SG4_ERR_ARG;
+  if (p->graphs_stale) drop_graphs(p);
   hipStream_t user = p->stream;
   if (!p->own_stream) HIP_TRY(hipStreamCreateWithFlags(&p->own_stream, hipStreamNonBlocking));
   sg4_plan::GraphEntry* g = nullptr;

@@ -405,7 +405,8 @@ int sg4_plan_split_info(const sg4_plan *p, int32_t *split, int64_t *kin_nnz);
  * cancellation.  It is built when the operator is set, holds 12 bytes per
  * entry (32.2 M entries at 10D L=8 Henon-Heiles), and is not used while a
  * field is set, in applies that the caller captures into a graph (their replays
- * follow a field set later), or with SG4_OPT_DETERMINISTIC, SG4_OPT_GROUPING = 0 or
+ * follow a field set later), once the caller has captured sg4_plan_set_field
+ * (until the next operator), or with SG4_OPT_DETERMINISTIC, SG4_OPT_GROUPING = 0 or
  * SG4_OPT_SPARSE = 0; other
  * potentials and precisions keep the term kernels.  No counterpart in the
  * reference. */
