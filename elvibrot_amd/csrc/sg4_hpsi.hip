@@ -683,6 +683,8 @@ static int build_kinetic(sg4_plan* P) {
   HIP_TRY(hipMemcpy(P->kin.val.p, val.data(), sizeof(double) * val.size(), hipMemcpyHostToDevice));
   P->kin.rows = nrows;
   P->kin.nnz = (int64_t)col.size();
+  P->kin.longest = 0;
+  for (int64_t r = 0; r < nrows; ++r) P->kin.longest = std::max(P->kin.longest, ptr[r + 1] - ptr[r]);
   P->kin.valid = true;
   P->split_ok = true;
   P->split_fp = fp;
@@ -1389,7 +1391,7 @@ static bool captured(const sg4_plan* P) {
   return true;
 }
 static bool caller_captures(const sg4_plan* P) {
-  return !(P->own_stream && P->stream == P->own_stream) && captured(P);
+  return P->stream && P->stream != P->own_stream && captured(P);
 }
 
 // use_nmode for one apply.  A caller's graph outlives the call: a field set

@@ -16,7 +16,7 @@ namespace sg4 {
 // The buffers are kept and reused when the matrix is built again.
 struct NModeMat {
   bool valid = false;
-  int64_t rows = 0, nnz = 0;
+  int64_t rows = 0, nnz = 0, longest = 0;   // longest: entries of the longest row
   DevBuf ptr, col, val;   // int64 row pointers, int32 columns, FP64 values
   DevBuf val_mu, val_f;   // field matrices: values of mu; val + eps val_mu of the segment
 };

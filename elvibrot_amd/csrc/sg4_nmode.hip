@@ -529,28 +529,40 @@ __global__ __launch_bounds__(256) void k_nm_rows(const NmDev* __restrict__ insts
   }
 }
 
-// row pointers from the row counts: sums of 1024 rows, their scan, the rows
-__global__ __launch_bounds__(256) void k_nm_sum(const int32_t* cnt, int64_t n, int64_t* part) {
+// row pointers from the row counts: sums (and the longest row) of 1024 rows,
+// their scan with the total and the longest row of all behind it, the rows
+__global__ __launch_bounds__(256) void k_nm_sum(const int32_t* cnt, int64_t n, int64_t* part, int32_t* most) {
   __shared__ int64_t s[256];
+  __shared__ int m[256];
   int64_t a = 0;
+  int b = 0;
   for (int k = 0; k < 4; ++k) {
     const int64_t i = (int64_t)blockIdx.x * 1024 + k * 256 + threadIdx.x;
-    if (i < n) a += cnt[i];
+    if (i < n) { a += cnt[i]; b = max(b, cnt[i]); }
   }
   s[threadIdx.x] = a;
+  m[threadIdx.x] = b;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+    if ((int)threadIdx.x < o) {
+      s[threadIdx.x] += s[threadIdx.x + o];
+      m[threadIdx.x] = max(m[threadIdx.x], m[threadIdx.x + o]);
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+  if (threadIdx.x == 0) { part[blockIdx.x] = s[0]; most[blockIdx.x] = m[0]; }
 }
-__global__ __launch_bounds__(1024) void k_nm_scan_part(int64_t* part, int np) {
+__global__ __launch_bounds__(1024) void k_nm_scan_part(int64_t* part, const int32_t* most, int np) {
   __shared__ int64_t s[1024];
+  __shared__ int longest;
+  if (threadIdx.x == 0) longest = 0;
+  __syncthreads();
   int64_t carry = 0;
+  int len = 0;
   for (int b = 0; b < np; b += 1024) {
     const int i = b + threadIdx.x;
     const int64_t x = i < np ? part[i] : 0;
+    if (i < np) len = max(len, most[i]);
     s[threadIdx.x] = x;
     __syncthreads();
     for (int o = 1; o < 1024; o <<= 1) {
@@ -564,7 +576,9 @@ __global__ __launch_bounds__(1024) void k_nm_scan_part(int64_t* part, int np) {
     __syncthreads();
     carry += total;
   }
-  if (threadIdx.x == 0) part[np] = carry;
+  atomicMax(&longest, len);
+  __syncthreads();
+  if (threadIdx.x == 0) { part[np] = carry; part[np + 1] = longest; }
 }
 __global__ __launch_bounds__(1024) void k_nm_ptr(const int32_t* cnt, int64_t n, const int64_t* part,
                                                  int64_t* ptr) {
@@ -736,7 +750,8 @@ __global__ __launch_bounds__(256) void k_nm_spmm_pairs(const int64_t* __restrict
     }
   }
 }
-// any number of vectors: one thread per (row, vector)
+// any number of vectors: SL threads per (row, vector)
+template <int SL>
 __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__ ptr,
                                                      const int32_t* __restrict__ col,
                                                      const double* __restrict__ val,
@@ -744,24 +759,30 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
                                                      double* __restrict__ hpsi, int64_t rows, int nvec,
                                                      float* __restrict__ psi32) {
   const int64_t n = rows * nvec;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+  const int s = threadIdx.x % SL;
+  // whole groups of SL lanes stay in the loop
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) / SL; i < n; i += (int64_t)gridDim.x * (256 / SL)) {
     const int64_t r = i / nvec;
     const int v = (int)(i - r * nvec);
     const int64_t e1 = ptr[r + 1];
-    int64_t e = ptr[r];
+    int64_t e = ptr[r] + s;
     double a0 = 0.0, a1 = 0.0;
-    for (; e + 3 < e1; e += 4) {
+    for (; e + 3 * SL < e1; e += 4 * SL) {
       int32_t c[4];
       double w[4], x[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) { c[u] = col[e + u]; w[u] = val[e + u]; }
+      for (int u = 0; u < 4; ++u) { c[u] = col[e + u * SL]; w[u] = val[e + u * SL]; }
 #pragma unroll
       for (int u = 0; u < 4; ++u) x[u] = psi[(int64_t)c[u] * nvec + v];
 #pragma unroll
       for (int u = 0; u < 4; u += 2) { a0 = fma(w[u], x[u], a0); a1 = fma(w[u + 1], x[u + 1], a1); }
     }
-    for (; e < e1; ++e) a0 = fma(val[e], psi[(int64_t)col[e] * nvec + v], a0);
-    hpsi[i] = a0 + a1;
+    for (; e < e1; e += SL) a0 = fma(val[e], psi[(int64_t)col[e] * nvec + v], a0);
+    a0 += a1;
+#pragma unroll
+    for (int o = 1; o < SL; o <<= 1) a0 += __shfl_xor(a0, o, 64);
+    if (s != 0) continue;
+    hpsi[i] = a0;
     if (psi32) psi32[i] = (float)psi[i];
   }
 }
@@ -770,6 +791,14 @@ __global__ __launch_bounds__(256) void k_nm_spmm_any(const int64_t* __restrict__
 // small instances 4.0 -> 3.4 us an order, tangents 5.2 -> 4.1; 12 uneven ones,
 // 130 k rows, 19.7 -> 22.3).
 constexpr int64_t ORDER_FEW = 32768;
+
+// Few rows of which one is long: its chain decides, and a wave takes a row (16 to
+// 64 slices).  Many modes all coupled in pairs, us, before -> so (the term kernels
+// in brackets): 32D L=2 (row of 2113 entries) x8 58 -> 13 (28), x16 61 -> 17 (29),
+// 16D L=3 (1537) x8 47 -> 13 (34), 12D L=3 (865) x16 29 -> 13 (24); an order of one
+// state 40 -> 5 (24) at 32D.  Rows up to 250 entries (6D L=4, 5D L=5) are faster in
+// place: x8 16-18 (23).
+constexpr int64_t LONG_ROW = 256;
 
 // A Chebyshev order (NModeOrder).  A lane holds two neighbouring columns (one
 // 16-byte load per entry), NC * SL lanes a row; the row's entries are dealt to
@@ -1165,15 +1194,15 @@ size_t up(size_t b) { return (b + 255) & ~(size_t)255; }
 struct Work {
   double *c1[2], *f2[2], *g1[2];
   int* flag[2];
-  int32_t* cnt;
+  int32_t *cnt, *most;
   int64_t* part;
   int npart;
   int layout(NModeTables* t, int64_t rows) {
     npart = (int)((rows + 1023) / 1024);
     const size_t b_c1 = up(8 * t->nc1), b_f2 = up(8 * (t->nf2 + 1)), b_g1 = up(8 * t->ng1v),
                  b_fl = up(4 * ((size_t)t->npairs + 1)), b_set = b_c1 + b_f2 + b_g1 + b_fl,
-                 b_cnt = up(4 * rows), b_part = up(8 * ((size_t)npart + 1));
-    if (int rc = ensure(t->work, 2 * b_set + b_cnt + b_part)) return rc;
+                 b_cnt = up(4 * rows), b_part = up(8 * ((size_t)npart + 2));
+    if (int rc = ensure(t->work, 2 * b_set + b_cnt + b_part + 4 * (size_t)npart)) return rc;
     char* W = t->work.as<char>();
     for (int s = 0; s < 2; ++s) {
       char* w = W + s * b_set;
@@ -1184,17 +1213,21 @@ struct Work {
     }
     cnt = (int32_t*)(W + 2 * b_set);
     part = (int64_t*)(W + 2 * b_set + b_cnt);
+    most = (int32_t*)(W + 2 * b_set + b_cnt + b_part);
     return SG4_OK;
   }
 };
 
-// the row counts' sum (synchronises) and the row pointers
-int scan_rows(const Work& w, int64_t rows, hipStream_t st, int64_t* nnz) {
-  hipLaunchKernelGGL(k_nm_sum, dim3(w.npart), dim3(256), 0, st, w.cnt, rows, w.part);
-  hipLaunchKernelGGL(k_nm_scan_part, dim3(1), dim3(1024), 0, st, w.part, w.npart);
-  NM_TRY(hipMemcpyAsync(nnz, w.part + w.npart, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+// the row counts' sum and the longest row (synchronises)
+int scan_rows(const Work& w, int64_t rows, hipStream_t st, int64_t* nnz, int64_t* longest) {
+  hipLaunchKernelGGL(k_nm_sum, dim3(w.npart), dim3(256), 0, st, w.cnt, rows, w.part, w.most);
+  hipLaunchKernelGGL(k_nm_scan_part, dim3(1), dim3(1024), 0, st, w.part, w.most, w.npart);
+  int64_t h[2] = {0, 0};
+  NM_TRY(hipMemcpyAsync(h, w.part + w.npart, sizeof(h), hipMemcpyDeviceToHost, st));
   NM_TRY(hipGetLastError());
   NM_TRY(hipStreamSynchronize(st));
+  *nnz = h[0];
+  *longest = h[1];
   return SG4_OK;
 }
 }  // namespace
@@ -1224,8 +1257,8 @@ int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m) {
   const int ni = (int)in.inst.size();
   hipLaunchKernelGGL((k_nm_rows<false, false>), rg, dim3(256), rl, st, insts, blk0, ni, set, set, pr, t->Dmax,
                      w.cnt, nullptr, nullptr, nullptr, nullptr);
-  int64_t nnz = 0;
-  if ((rc = scan_rows(w, rows, st, &nnz))) return rc;
+  int64_t nnz = 0, longest = 0;
+  if ((rc = scan_rows(w, rows, st, &nnz, &longest))) return rc;
   if ((rc = ensure(m.ptr, 8 * (rows + 1))) || (rc = ensure(m.col, 4 * nnz)) || (rc = ensure(m.val, 8 * nnz)))
     return rc;
   hipLaunchKernelGGL(k_nm_ptr, dim3(w.npart), dim3(1024), 0, st, w.cnt, rows, w.part, m.ptr.as<int64_t>());
@@ -1234,6 +1267,7 @@ int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m) {
   NM_TRY(hipGetLastError());
   m.rows = rows;
   m.nnz = nnz;
+  m.longest = longest;
   m.valid = true;
   return SG4_OK;
 }
@@ -1370,8 +1404,8 @@ int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double
   else
     hipLaunchKernelGGL((k_nm_rows<false, false>), rg, dim3(256), rl, st, insts, blk0, ni, set[0], set[1], pr,
                        t->Dmax, cnt, nullptr, nullptr, nullptr, nullptr);
-  int64_t nnz = 0;
-  if ((rc = scan_rows(w, rows, st, &nnz))) return rc;
+  int64_t nnz = 0, longest = 0;
+  if ((rc = scan_rows(w, rows, st, &nnz, &longest))) return rc;
   if (nnz > NNZ_SMALL && nnz > NNZ_PER_POINT * (double)in.sum_nq) return SG4_OK;
   if (ensure(m.ptr, 8 * (rows + 1)) || ensure(m.col, 4 * nnz) || ensure(m.val, 8 * nnz) ||
       (mu && (ensure(m.val_mu, 8 * nnz) || ensure(m.val_f, 8 * nnz))))
@@ -1387,6 +1421,7 @@ int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double
   NM_TRY(hipGetLastError());
   m.rows = rows;
   m.nnz = nnz;
+  m.longest = longest;
   m.valid = true;
   t->v_ready = true;
   t->v_flags = hf[0];
@@ -1394,6 +1429,8 @@ int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double
 }
 
 namespace {
+bool long_rows(const NModeMat& m) { return m.longest > LONG_ROW && m.rows <= ORDER_FEW; }
+
 template <bool COLS, bool IN_COLS>
 int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st,
          const double* val, float* psi32 = nullptr) {
@@ -1416,15 +1453,24 @@ int spmm(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hi
       default: return 1;
     }
   } else {
+    const bool lg = long_rows(m);
     switch (W) {
       case 1: SG4_SPMM(1, 8); break;
       case 2: SG4_PAIRS(1, 1, 8, 2, false); break;
       case 4: SG4_PAIRS(1, 2, 8, 2, false); break;
-      case 8: SG4_PAIRS(2, 2, 8, 2, false); break;
-      case 16: SG4_PAIRS(4, 2, 4, 2, false); break;
+      case 8:
+        if (lg) SG4_PAIRS(2, 2, 32, 2, false);
+        else SG4_PAIRS(2, 2, 8, 2, false);
+        break;
+      case 16:
+        if (lg) SG4_PAIRS(4, 2, 16, 2, false);
+        else SG4_PAIRS(4, 2, 4, 2, false);
+        break;
       default:
         if constexpr (COLS) return 1;
+        else if (W % 16 == 0 && lg) SG4_PAIRS(4, 2, 16, 2, true);
         else if (W % 16 == 0) SG4_PAIRS(4, 2, 4, 2, true);
+        else if (W % 8 == 0 && lg) SG4_PAIRS(2, 2, 32, 2, true);
         else if (W % 8 == 0) SG4_PAIRS(2, 2, 8, 2, true);
         else return 1;
     }
@@ -1441,14 +1487,16 @@ int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hi
   if (!val) val = m.val.as<double>();
   const int rc = spmm<false, false>(m, nvec, nvec, psi, hpsi, st, val, psi32);
   if (rc <= 0) return rc;
-  hipLaunchKernelGGL(k_nm_spmm_any, dim3((unsigned)std::min<int64_t>((m.rows * nvec + 255) / 256, (int64_t)1 << 20)),
-                     dim3(256), 0, st, m.ptr.as<int64_t>(), m.col.as<int32_t>(), val, psi, hpsi, m.rows, nvec, psi32);
+  const int sl = long_rows(m) ? 16 : 1;
+  hipLaunchKernelGGL(sl == 1 ? k_nm_spmm_any<1> : k_nm_spmm_any<16>,
+                     dim3((unsigned)std::min<int64_t>((m.rows * nvec * sl + 255) / 256, (int64_t)1 << 20)), dim3(256), 0,
+                     st, m.ptr.as<int64_t>(), m.col.as<int32_t>(), val, psi, hpsi, m.rows, nvec, psi32);
   NM_TRY(hipGetLastError());
   return SG4_OK;
 }
 
 bool nmode_cols_direct(const NModeMat& m, int W) {
-  return W <= 16 && (W & (W - 1)) == 0 && m.nnz * W * W <= COLS_DIRECT;
+  return W <= 16 && (W & (W - 1)) == 0 && m.nnz * W * W <= COLS_DIRECT && (W < 8 || !long_rows(m));
 }
 
 int nmode_apply_cols(const NModeMat& m, int W, int nvec, const double* psi, double* hpsi, hipStream_t st) {
@@ -1472,7 +1520,18 @@ int nmode_order(const NModeMat& m, const NModeOrder& a, bool tangent, hipStream_
   const bool few = m.rows <= ORDER_FEW;
 #define SG4_ORDER(NC, SL, TAN) \
   hipLaunchKernelGGL((k_nm_order<NC, SL, TAN>), grid(NC * SL), dim3(256), 0, st, ptr, col, mu, a, m.rows)
-  if (tangent) {
+  if (long_rows(m)) {   // a wave per row
+    if (tangent) {
+      if (nc == 4) SG4_ORDER(2, 32, true);
+      else if (nc == 8) SG4_ORDER(4, 16, true);
+      else SG4_ORDER(8, 8, true);
+    } else {
+      if (nc == 2) SG4_ORDER(1, 64, false);
+      else if (nc == 4) SG4_ORDER(2, 32, false);
+      else if (nc == 8) SG4_ORDER(4, 16, false);
+      else SG4_ORDER(8, 8, false);
+    }
+  } else if (tangent) {
     if (nc == 4 && few) SG4_ORDER(2, 8, true);
     else if (nc == 4) SG4_ORDER(2, 4, true);
     else if (nc == 8) SG4_ORDER(4, 4, true);
