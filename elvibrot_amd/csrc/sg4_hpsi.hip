@@ -267,10 +267,11 @@ struct ItemPlan {
                            // (padded Kronecker tiles, six limb products)
 };
 
-// A propagation builds the matrix with the dipole's values once per call
-// (~0.3 ms for small plans, where an apply of the term kernels takes ~25 us):
-// calls of fewer applies keep the term kernels.
-constexpr int64_t NM_MIN_APPLIES = 24;
+// A propagation builds the matrix with the dipole's values once per call; a call
+// whose applies save less than that keeps the term kernels.  An order of one state,
+// term kernels -> matrix, us: 6D L=3 15.6 -> 3.1, 32D L=2 23.9 -> 5, 6D L=6 33 -> 3.7,
+// 8D L=6 (0.44 M points) 80 -> 6.3, 9D L=7 (3.7 M) 351 -> 22, 10D L=8 (31 M) 2108 -> 166.
+constexpr double NM_SAVED = 10.0, NM_SAVED_POINT = 6e-5;
 
 constexpr int64_t XCD_BLOCK = 16 << 20;   // bytes of a block of vectors (default_cfg)
 constexpr int64_t ROWSUM_MIN = 1 << 16;   // places of the map (use_rowsum)
@@ -1798,10 +1799,10 @@ using namespace sg4;
 namespace sg4 {
 int plan_field_matrix(sg4_plan* P, const double* mu, int prec, int64_t applies, NModeMat** out) {
   *out = nullptr;
-  if (prec != SG4_PREC_FP64 || !P->nm.valid || !P->sparse || P->nm_off || P->deterministic || !use_split_alg(P) ||
-      applies < NM_MIN_APPLIES)
+  if (prec != SG4_PREC_FP64 || !P->nm.valid || !P->sparse || P->nm_off || P->deterministic || !use_split_alg(P))
     return SG4_OK;
   if (!mu) { *out = &P->nm; return SG4_OK; }
+  if ((double)applies * (NM_SAVED + NM_SAVED_POINT * (double)P->sum_nq) < nmode_field_cost(P->nmt, P->nm)) return SG4_OK;
   int rc = nmode_build(P->nmt, nmode_in(P), P->d_V0.p ? P->d_V0.as<double>() : P->d_V.as<double>(), mu,
                        P->nm_field);
   if (rc) return rc;

@@ -63,6 +63,9 @@ int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m);
 // the matrix small enough to pay.
 int nmode_build(NModeTables* t, const NModeIn& in, const double* V, const double* mu, NModeMat& m);
 
+// us that building the plan's matrix m again with a grid function's values takes
+double nmode_field_cost(const NModeTables* t, const NModeMat& m);
+
 // hpsi = M psi, nvec vectors in the rows layout (val: other values on M's pattern;
 // psi32: psi in FP32, written beside it)
 int nmode_apply(const NModeMat& m, int nvec, const double* psi, double* hpsi, hipStream_t st,

@@ -1232,6 +1232,15 @@ int scan_rows(const Work& w, int64_t rows, hipStream_t st, int64_t* nnz, int64_t
 }
 }  // namespace
 
+// Host lists, cuts and the check of every pair, and a row's tasks, one per pair:
+// beyond the launches and copies of any build (150 us) 32D L=2 (496 pairs) takes
+// 3290 us, 21D 1500, 12D L=3 (66) 570; then the entries: 10D L=8 (32 M) 4100.
+double nmode_field_cost(const NModeTables* t, const NModeMat& m) {
+  int pairs = 0;
+  for (int g = 0; g < t->npairs && g < (int)t->v_flags.size(); ++g) pairs += t->v_flags[g] != 0;
+  return 150.0 + 6.5 * pairs + 1.3e-4 * (double)m.nnz;
+}
+
 bool nmode_rows_ok(const NModeTables* t) { return t && t->rows_ok; }
 
 int nmode_build_kinetic(NModeTables* t, const NModeIn& in, NModeMat& m) {
