@@ -11,15 +11,15 @@
 //            (deterministic, no atomics).
 //   combine: Y (k x n) = beta Y + U X, U (k x d) small, X: d rows: 32 columns
 //            per wave and step, X straight into operand registers, U in LDS in
-//            operand order (up to 64 KiB; larger U by scalar loads, one column
-//            per thread).
+//            operand order; one column per thread with U by scalar loads where U
+//            exceeds 64 KiB and where the matrix cores have little to do.
 // Bound by HBM for the Davidson's shapes.  At 10D L=8 (n = 1.26 M), us, before
 // (LDS tiles and 4 x 4 register blocks; one column per thread with U from
 // scalar loads) -> now, and the floor at the copy rate of 4.9 TB/s: gram 8 x 8
 // 65 -> 34 (33), 20 x 20 191 -> 86 (82), 60 x 16 305 -> 165 (156), 100 x 16 465 ->
-// 283 (238), 84 x 84 1825 -> 1111 (library split-K product 300-600); combine 8 x 8
-// 29 -> 28, 16 x 48 158 -> 149 (131), 20 x 60 244 -> 193 (164), 36 x 84 703 -> 352
-// (246), 64 x 64 1035 -> 367 (262).  1024 or 2048 gram workgroups: 187, 209 for
+// 283 (238), 84 x 84 1825 -> 1111 (library split-K product 300-600); combine 16 x 48
+// 158 -> 149 (131), 20 x 60 244 -> 193 (164), 36 x 84 703 -> 352 (246), 64 x 64 1035
+// -> 367 (262).  1024 or 2048 gram workgroups: 187, 209 for
 // 60 x 16 (more partials).
 #include <hip/hip_runtime.h>
 
@@ -35,7 +35,17 @@ constexpr int GMAX = 124;      // rows of A or B
 constexpr int GBLK = 512;      // 4 x 4 output blocks at most
 constexpr int GNB = 2048;      // partials per output that the work array is sized for
 constexpr int GWGS = 512;      // workgroups of a gram (per group of tiles)
-constexpr int64_t CWG = 2048;  // workgroups of a combine
+// Workgroups of a combine: with U of more than 16 rows 2048 that stay and load it
+// once (n = 1.26 M, 36 x 84 352 us, one per tile 468), with fewer rows one per tile
+// of columns (8 x 8 of the same, beta = 1, 47 -> 42, 16 x 16 120 -> 111).
+constexpr int64_t CWG = 2048, CWG16 = 65535;
+// A combine with one thread per column where the matrix cores have little to do:
+// few rows of X, which the writes of whole Y rows bound (n = 1.26 M, us, matrix
+// cores / threads: 16 x 4 beta 1 64 / 58, 32 x 8 146 / 106, 36 x 8 159 / 120), and
+// few rows of Y beyond the caches (1 x 60 115 / 107, 4 x 124 253 / 233; 4 x 60 of
+// 400 k 35 / 39) or one or two of them (1 x 124 of 100 k 26 / 22).
+constexpr int64_t THREADS_N = 1 << 19, THREADS_X = 48000000;
+constexpr int THREADS_D = 8, THREADS_K = 4, THREADS_K2 = 2, THREADS_D2 = 48;
 constexpr int CMAXU = 8192;    // entries of U (k d) at most
 constexpr int CK = 16;         // outputs of the scalar combine per pass over X (k <= 16)
 constexpr int CKW = 48;        // the same for wider k (k > 48: several passes)
@@ -90,12 +100,20 @@ __global__ __launch_bounds__(256) void k_gram_part(int m, int q, int64_t n, cons
   if (t == full && 16 * full < n) {   // the columns beyond the last whole block, the others zero
     D4 a[TA], b[TB];
 #pragma unroll
+    for (int s = 0; s < 4; ++s) {       // without a branch, so that the loads go out together
+      const int64_t o = min(16 * full + s, n - 1 - 4 * kq);
+#pragma unroll
+      for (int x = 0; x < TA; ++x) a[x].v[s] = pa[x][o];
+#pragma unroll
+      for (int y = 0; y < TB; ++y) b[y].v[s] = pb[y][o];
+    }
+#pragma unroll
     for (int s = 0; s < 4; ++s) {
       const bool in = 16 * full + 4 * kq + s < n;
 #pragma unroll
-      for (int x = 0; x < TA; ++x) a[x].v[s] = in ? pa[x][16 * full + s] : 0.0;
+      for (int x = 0; x < TA; ++x) a[x].v[s] = in ? a[x].v[s] : 0.0;
 #pragma unroll
-      for (int y = 0; y < TB; ++y) b[y].v[s] = in ? pb[y][16 * full + s] : 0.0;
+      for (int y = 0; y < TB; ++y) b[y].v[s] = in ? b[y].v[s] : 0.0;
     }
     products(a, b);
   }
@@ -322,8 +340,10 @@ int sg4_block_combine(sg4_plan* p, int32_t k, int32_t d, int64_t n, const double
   const hipStream_t st = (hipStream_t)plan_stream(p);
   const int rt = k <= 16 ? 1 : k <= 32 ? 2 : 4;
   const size_t lds = sizeof(double) * 64 * rt * (size_t)((d + 3) / 4);
-  if (lds <= 64 * 1024) {
-    const dim3 grid((unsigned)std::min<int64_t>((n + 127) / 128, CWG), (unsigned)((k + 16 * rt - 1) / (16 * rt)));
+  const bool threads = (d <= THREADS_D && n >= THREADS_N) || (k <= THREADS_K && d * n > THREADS_X) ||
+                       (k <= THREADS_K2 && d >= THREADS_D2);
+  if (lds <= 64 * 1024 && !threads) {
+    const dim3 grid((unsigned)std::min<int64_t>((n + 127) / 128, rt == 1 ? CWG16 : CWG), (unsigned)((k + 16 * rt - 1) / (16 * rt)));
     if (rt == 1) hipLaunchKernelGGL(k_combine_mfma<1>, grid, dim3(256), lds, st, k, d, n, U, X, ldx, beta, Y, ldy);
     else if (rt == 2) hipLaunchKernelGGL(k_combine_mfma<2>, grid, dim3(256), lds, st, k, d, n, U, X, ldx, beta, Y, ldy);
     else hipLaunchKernelGGL(k_combine_mfma<4>, grid, dim3(256), lds, st, k, d, n, U, X, ldx, beta, Y, ldy);
