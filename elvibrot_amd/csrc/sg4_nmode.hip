@@ -600,12 +600,14 @@ __global__ __launch_bounds__(1024) void k_nm_ptr(const int32_t* cnt, int64_t n, 
 struct alignas(8) Two { double x, y; };
 
 // Workgroups of the products in x and z: a launch takes fewer than 2^32 threads
-// in a direction, which 16 lanes a row reach at 2^28 rows.
+// in a direction, which 16 lanes a row reach at 2^28 rows.  The stride is a
+// constant: a product of few rows would wait for the grid's size (6D L=3 x1
+// 4.65 -> 4.8 us).
 constexpr int64_t MAX_BLOCKS_X = (int64_t)1 << 23;
-__device__ __forceinline__ int64_t block_xz() { return blockIdx.x + (int64_t)gridDim.x * blockIdx.z; }
+__device__ __forceinline__ int64_t block_xz() { return blockIdx.x + MAX_BLOCKS_X * blockIdx.z; }
 dim3 grid_xz(int64_t blocks, int y) {
-  const int64_t z = (blocks + MAX_BLOCKS_X - 1) / MAX_BLOCKS_X;
-  return dim3((unsigned)((blocks + z - 1) / z), (unsigned)y, (unsigned)z);
+  return dim3((unsigned)std::min(blocks, MAX_BLOCKS_X), (unsigned)y,
+              (unsigned)((blocks + MAX_BLOCKS_X - 1) / MAX_BLOCKS_X));
 }
 
 // hpsi(r, v) = sum_e val_e psi(col_e, v): NV * SL lanes per row, NV vectors,
