@@ -1475,10 +1475,12 @@ static bool rowsum_able(const sg4_plan* P, int prec) {
 // / with sums, and the apply that changes over: 6D L=6 (94 k places) x1 41 / 32,
 // 600; 8D L=6 (439 k) x1 72 / 50, 540, FP32 x24 203 / 102, 920; 9D L=7 (3.7 M) x1
 // 310 / 208, 2100, x5 438 / 355, 2400, x16 704 / 521, 2700; 10D L=8 (31 M) split x1
-// 2059 / 834, 8800, FP64 x16 9178 / 4716, 15500.  The estimates below are low on
-// the savings where they are far apart (10D).
+// 2059 / 834, 8800, x16 6796 / 3757, 14500, FP64 x16 9178 / 4716, 15500.  A place
+// saves 20 ps and 1.5 for each vector, more where the block of vectors outgrows the
+// caches.
 static bool rowsum_pays(sg4_plan* P, int nvec) {
-  P->rowsum_gain += 8.0 + 1e-6 * (20.0 + 1.5 * nvec) * (double)P->sum_nb;
+  const double beyond = 1.0 + 8.0 * (double)P->nb_ba * nvec / 96e6;
+  P->rowsum_gain += 8.0 + 1e-6 * (20.0 + 1.5 * nvec) * beyond * (double)P->sum_nb;
   return P->rowsum_gain > 800.0 + 3.5e-4 * (double)P->sum_nb;
 }
 
@@ -1490,7 +1492,7 @@ static bool rowsum_pays(sg4_plan* P, int nvec) {
 // 71 -> 54, 9D L=6 x16 198 -> 148.  Small term sets would only pay for the
 // launch: 6D L=5 (26 k places) x1 / x4 15.6 -> 15.7 / 14.3 -> 16.8 us, 6D L=6
 // (94 k) 27.1 -> 19.2 / 26.4 -> 21.1.
-// The inverted map costs as much as the sums save in some ten to eighty applies,
+// The inverted map costs as much as the sums save in some three to eighty applies,
 // so a plan builds it once they would have saved that much (rowsum_pays), or for
 // a graph or the autotuner (now).
 // The block belongs to the plan's stream: an apply that the caller captures

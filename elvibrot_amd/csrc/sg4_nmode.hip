@@ -22,14 +22,13 @@
 // (parity, band structure of polynomials) and are not stored.
 //
 // What bounds it: the gathers of psi rows, one 128-byte line per stored entry
-// and 16 vectors, from beyond L2.  10D L=8 Henon-Heiles (32.2 M entries, 0.39
-// GB): 0.75 ms at 16 vectors (4.1 GB of gathers, 5.5 TB/s), 0.14 ms at one
-// (matrix 2.8 TB/s); the term kernels and the kinetic rows take 5.1 and 1.2 ms.
-// sg4_apply of 16 column-major vectors: 0.85 ms against 5.2.  One group of W
-// lanes per row (W vectors, the entries loaded once per group) in row order;
-// measured slower at 16 / 1 vectors: 8 loads in flight 0.77 / 0.16 ms, a
-// contiguous chunk of rows per XCD 0.80 / 0.15, non-temporal matrix loads 0.94 /
-// 0.18, two slices of entries per row (16 vectors) 0.87.
+// and 16 vectors.  10D L=8 Henon-Heiles (32.2 M entries, 0.39 GB): 0.44 ms at 16
+// vectors (2.64 GB read, 0.19 written: 5.8 TB/s with the result to columns), 0.14
+// ms at one (matrix 2.8 TB/s); the term kernels and the kinetic rows take 4.7 and
+// 0.8 ms.  sg4_apply of 16 column-major vectors: 0.54 ms against 4.8.  Rows in
+// order; measured slower at 16 / 1 vectors with the kernel of one column per lane
+// (0.75 / 0.14 ms): 8 loads in flight 0.77 / 0.16 ms, a contiguous chunk of rows
+// per XCD 0.80 / 0.15, non-temporal matrix loads 0.94 / 0.18.
 #include "sg4_nmode.h"
 
 #include <algorithm>
@@ -62,8 +61,10 @@ constexpr double EPS = 2.220446049250313e-16;
 // quadrature terms is rounding.
 constexpr double TOL_V = 64 * EPS, TOL_M = 16 * EPS;
 // Stored entries per grid point up to which the matrix is taken: an entry
-// costs ~1.5 ps per vector at 10D L=8 (gather of one psi value), a grid point
-// ~9.5 ps in the FP64 term kernel.
+// cost ~1.5 ps per vector at 10D L=8 (gather of one psi value) with one column per
+// lane, ~0.85 with pairs of columns, a grid point 9.2 to 9.5 ps in the FP64 term
+// kernel: matrices of four to some eight entries per point would still pay, which
+// the memory and the building of the larger ones speak against.
 constexpr double NNZ_PER_POINT = 4.0;
 constexpr int64_t NNZ_SMALL = 1 << 18;        // always taken: the apply is one short launch
 // A column-major block is read in place while nnz W^2 <= 2^24 (W columns, a

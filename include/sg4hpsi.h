@@ -130,7 +130,7 @@ int sg4_setup_destroy(sg4_setup *s);
  * pre-sized work buffers for blocks of up to max_nvec vectors.  An apply
  * allocates its work items at the first call for a block width and, where the
  * terms' results are summed row by row, the inverted map (once the applies so
- * far would have saved its cost, some 10 to 80 of them)
+ * far would have saved its cost, some 3 to 80 of them)
  * and a results block per stream and wider block (at most 16 GiB; without it,
  * and in applies that the caller captures, the sums are FP64 atomics).        */
 int sg4_plan_create(const sg4_tables *tables, int32_t max_nvec, sg4_plan **out);
